@@ -20,64 +20,15 @@
 // that prefix, so no host synchronisation is needed and empty groups cost nothing.  Workgroup ids
 // are remapped so that each XCD (ids congruent mod 8) walks a contiguous run of tiles that share
 // weight panels in its own L2.
-#include <atomic>
 #include <type_traits>
-#include <vector>
 
-#include "mx_common.h"
+#include "mx_gemm_common.h"
+#include "mx_gemm_ksplit.h"
+#include "mx_launch.h"
 
 namespace cmx {
 
 namespace {
-
-constexpr int kSlabBytes = 128;     // K bytes per LDS slab and row
-constexpr int kChunks = kSlabBytes / 16;
-constexpr int kXcds = 8;
-
-// kEpiStoreBf16 / kEpiStoreFp16: 16-bit output whose rows and row pitch are multiples of eight elements (16-byte
-// stores, no per-element edge handling): small enough to sit inside a persistent kernel's tile loop.  Two epilogues, not one with a run-time switch: a second copy of the store loop inside the kernel costs
-// registers, and values spilled because of it are reloaded inside the scheduled loop, where the waits that the
-// compiler puts behind such reloads drain the operand loads in flight.
-// kEpiSwigluQuantAct: kEpiSwigluQuant that also writes the bf16 SwiGLU output (what the tests check the requantised
-// codes against).  A kernel of its own for the same reason: the extra output path costs the SwiGLU kernels
-// 30 registers, all of them spilled at the tile boundaries, 3 % of a launch, whether the output is asked for or not.
-enum Epilogue { kEpiStore = 0, kEpiSwigluQuant = 1, kEpiStoreBf16 = 2, kEpiI8DequantSwiglu = 3, kEpiStoreFp16 = 4, kEpiSwigluQuantAct = 5 };
-constexpr bool epi_is_lean_store(int epi) { return epi == kEpiStoreBf16 || epi == kEpiStoreFp16; }
-constexpr bool epi_is_swiglu_quant(int epi) { return epi == kEpiSwigluQuant || epi == kEpiSwigluQuantAct; }
-// epilogues whose weight tile pairs gate rows (first half of N) with their up partners (second half)
-constexpr bool epi_pairs_gate_up(int epi) { return epi_is_swiglu_quant(epi) || epi == kEpiI8DequantSwiglu; }
-// element "format" of the INT8 path inside the kernel templates (the public format codes are the MX ones)
-constexpr int kFmtI8 = 8;
-
-struct GemmParams {
-    const uint8_t* a;        // activations codes
-    const uint8_t* a_scale;
-    const uint8_t* w;        // weights codes [groups][n][ldw]
-    const uint8_t* w_scale;  // [groups][n][ld_ws]
-    void* c;
-    uint8_t* act_codes;
-    uint8_t* act_scales;
-    uint16_t* act_bf16;
-    const int32_t* row_off;     // [groups+1] (grouped) or null (dense)
-    const int32_t* tile_pref;   // [groups+1] prefix of m-tiles (grouped) or null
-    int32_t* tile_ctr;          // [8] per-XCD tile counters, zeroed before the launch (persistent grouped 4 x 1 kernels) or null
-    uint32_t lda, ld_as, ldw, ld_ws, ldc, ld_act, ld_acts;
-    uint32_t m, n, kbytes, kblocks;   // kblocks = K/32
-    uint32_t groups, w_tiles;
-    int out_type;
-    int scale_vec;   // scale rows are 4-byte aligned: one dword load per row and slab
-    int scale_vec16; // scale rows are 16-byte aligned: one 16-byte load per row fetches the scales of four slabs
-    int w_pretiled;  // w holds the weights in the tiled order of cmx_mx_pretile_weights (the weights-to-registers kernel)
-};
-
-__device__ __forceinline__ uint32_t swz(uint32_t row, uint32_t chunk) {
-    return chunk ^ ((row & 7u) ^ ((row >> 3) & 1u));
-}
-
-__device__ __forceinline__ v4f to_v4(const v16f& v, int q) {
-    v4f r = {v[4 * q], v[4 * q + 1], v[4 * q + 2], v[4 * q + 3]};
-    return r;
-}
 
 template <int FMT>
 __device__ __forceinline__ v16f mfma(v8i w, v8i a, v16f c, int opsel_tag, int sw, int sa);
@@ -124,127 +75,6 @@ __device__ __forceinline__ v16f mfma<kFmtI8>(v8i w, v8i a, v16f c, int, int, int
     acc = __builtin_amdgcn_mfma_i32_32x32x32_i8((v4i){w[0], w[1], w[2], w[3]}, (v4i){a[0], a[1], a[2], a[3]}, acc, 0, 0, 0);
     acc = __builtin_amdgcn_mfma_i32_32x32x32_i8((v4i){w[4], w[5], w[6], w[7]}, (v4i){a[4], a[5], a[6], a[7]}, acc, 0, 0, 0);
     return __builtin_bit_cast(v16f, acc);
-}
-
-// g / (1 + exp(-g)) * u with the hardware exponential and reciprocal (about 1 ulp each; the result is rounded
-// to bf16 right after)
-__device__ __forceinline__ float silu_mul(float g, float u) {
-    const float s = __builtin_amdgcn_rcpf(1.0f + __expf(-g));
-    return (g * s) * u;
-}
-
-struct Tile {
-    uint32_t g, mt, wt, row0, rows_valid;
-};
-
-// The group tables (row offsets, m-tile prefix) are written by gmm_prepare_kernel before the matmul kernel starts and
-// never change under it: reading them through the constant address space lets a wavefront-uniform lookup use scalar
-// loads, which wait on lgkmcnt and so do not drain the LDS-DMA loads a persistent kernel has in flight (a vector load
-// would: its s_waitcnt vmcnt covers everything issued before it).
-__device__ __forceinline__ int32_t table_at(const int32_t* t, uint32_t i) {
-    return ((const __attribute__((address_space(4))) int32_t*)t)[i];
-}
-
-// Tiles are numbered linearly: within a group m-tiles run fastest so that neighbours share a weight panel;
-// dense problems walk bands of four m-tiles across a run of weight tiles.
-template <int TM>
-__device__ __forceinline__ uint32_t count_m_tiles(const GemmParams& p) {
-    return p.row_off != nullptr ? (uint32_t)table_at(p.tile_pref, p.groups) : (p.m + TM - 1) / TM;
-}
-
-// Tile L of an XCD-aware order: linear ids congruent mod 8 run on one XCD; each XCD gets a contiguous run.
-// Returns the first tile of XCD x and the number of tiles it owns.
-__device__ __forceinline__ uint32_t xcd_run(uint32_t total_tiles, uint32_t x, uint32_t& count) {
-    const uint32_t base = total_tiles / kXcds, rem = total_tiles % kXcds;
-    count = base + (x < rem ? 1u : 0u);
-    return x * base + (x < rem ? x : rem);
-}
-
-// Persistent kernels that walk in fixed strides (no tile counter), with at least one full round of tiles: instead of
-// owning a contiguous run, the XCDs take turns at blocks of (workgroups per XCD) consecutive tiles, workgroup j of XCD x
-// walking tiles x * per + j, + grid, + 2 * grid, ...  The whole chip then works on one stretch of `grid` consecutive
-// tiles at a time -- two bands of m-tiles across all their weight tiles -- so an activation panel is wanted by four XCDs
-// and a weight panel by two at about the same time (the memory-side cache can serve the repeats), and every block of 32
-// tiles starts on a multiple of 32, where the contiguous runs cut across the bands.  Zipf-routed 16-expert problem: 16 %
-// fewer L2 misses, 1.7-3.3 % less time.  Problems of less than a round keep the contiguous runs, which spread few tiles
-// over all eight L2s.
-__device__ __forceinline__ void interleave_xcd_walk(uint32_t total_tiles, uint32_t& tile_id, uint32_t& stride, uint32_t& end) {
-    if (total_tiles < gridDim.x) return;
-    tile_id = (blockIdx.x % kXcds) * (gridDim.x / kXcds) + blockIdx.x / kXcds;
-    stride = gridDim.x;
-    end = total_tiles;
-}
-
-// One tile per workgroup (blockIdx.x < total_tiles).  Workgroups start in the order of their ids, ids congruent mod 8 on one
-// XCD.  Whole chunks of 256 tiles: the XCDs take blocks of 32 consecutive tiles of the chunk in turn, for the reason given
-// above (the INT8 operator on the 16-expert problem: 973-982 -> 942-945 us); the rest: a contiguous run per XCD.
-__device__ __forceinline__ uint32_t tile_of_workgroup(uint32_t total_tiles) {
-    constexpr uint32_t kChunk = 32 * kXcds;
-    const uint32_t bid = blockIdx.x, full = total_tiles / kChunk * kChunk;
-    if (bid < full) return bid / kChunk * kChunk + (bid % kXcds) * 32 + (bid % kChunk) / kXcds;
-    uint32_t count;
-    const uint32_t k = bid - full;
-    return full + xcd_run(total_tiles - full, k % kXcds, count) + k / kXcds;
-}
-
-// g_from: a group at or before the tile's (0, or the group of an earlier tile of an increasing sequence)
-template <int TM>
-__device__ __forceinline__ void decode_tile(const GemmParams& p, uint32_t m_tiles_all, uint32_t L, Tile& t, uint32_t g_from = 0) {
-    if (p.row_off != nullptr) {
-        // find g with tile_pref[g]*w_tiles <= L < tile_pref[g+1]*w_tiles.  A workgroup's next tile mostly lies in the
-        // same group or one of the next two: three independent loads settle that before the bisection's
-        // chain of dependent ones
-        const uint32_t G = p.groups;
-        uint32_t lo = g_from, hi = G;
-        const uint32_t i2 = lo + 2 < G ? lo + 2 : G, i3 = lo + 3 < G ? lo + 3 : G;
-        const uint32_t t1 = (uint32_t)table_at(p.tile_pref, lo + 1) * p.w_tiles, t2 = (uint32_t)table_at(p.tile_pref, i2) * p.w_tiles,
-                       t3 = (uint32_t)table_at(p.tile_pref, i3) * p.w_tiles;
-        if (t1 > L) hi = lo + 1;
-        else if (t2 > L) { lo += 1; hi = lo + 1; }
-        else if (t3 > L) { lo += 2; hi = lo + 1; }
-        else lo += 3;
-        while (hi - lo > 1) {
-            const uint32_t mid = (lo + hi) >> 1;
-            if ((uint32_t)table_at(p.tile_pref, mid) * p.w_tiles <= L) lo = mid; else hi = mid;
-        }
-        t.g = lo;
-        const uint32_t tp = (uint32_t)table_at(p.tile_pref, lo);
-        const uint32_t mtg = (uint32_t)table_at(p.tile_pref, lo + 1) - tp;
-        // bands of 8 m-tiles share a run of weight tiles (m fastest inside a band): the 32 tiles that an XCD
-        // works on at a time then touch 8 + 4 operand panels instead of mtg + 32/mtg
-        const uint32_t local = L - tp * p.w_tiles;
-        const uint32_t band = 8;
-        const uint32_t per_band = band * p.w_tiles;
-        const uint32_t b = local / per_band, within = local % per_band;
-        const uint32_t band_rows = (mtg - b * band) < band ? (mtg - b * band) : band;
-        t.mt = b * band + within % band_rows;
-        t.wt = within / band_rows;
-        const uint32_t r_begin = (uint32_t)table_at(p.row_off, lo), r_end = (uint32_t)table_at(p.row_off, lo + 1);
-        t.row0 = r_begin + t.mt * TM;
-        t.rows_valid = r_end - t.row0 < (uint32_t)TM ? r_end - t.row0 : (uint32_t)TM;
-    } else {
-        // bands of 4 m-tiles share a run of weight tiles
-        const uint32_t band = 4;
-        const uint32_t per_band = band * p.w_tiles;
-        const uint32_t b = L / per_band, within = L % per_band;
-        const uint32_t band_rows = (m_tiles_all - b * band) < band ? (m_tiles_all - b * band) : band;
-        t.g = 0;
-        t.mt = b * band + within % band_rows;
-        t.wt = within / band_rows;
-        t.row0 = t.mt * TM;
-        t.rows_valid = p.m - t.row0 < (uint32_t)TM ? p.m - t.row0 : (uint32_t)TM;
-    }
-}
-
-// One tile per workgroup: maps the workgroup id to (group, m-tile, weight tile).  Returns false for ids past
-// the last tile.
-template <int TM>
-__device__ __forceinline__ bool locate_tile(const GemmParams& p, Tile& t) {
-    const uint32_t m_tiles_all = count_m_tiles<TM>(p);
-    const uint32_t total_tiles = m_tiles_all * p.w_tiles;
-    if (blockIdx.x >= total_tiles) return false;
-    decode_tile<TM>(p, m_tiles_all, tile_of_workgroup(total_tiles), t);
-    return true;
 }
 
 // LDS/tile row of a wavefront's weight fragment f (gate fragments first, their up partners second)
@@ -1049,73 +879,6 @@ __global__ __launch_bounds__(256) void gmm_prepare_kernel(const int32_t* __restr
     }
 }
 
-// Launch state that belongs to a device, not to the process: the dynamic-LDS limit of a kernel has to be raised on
-// every device that runs it, and the CU count differs between devices.  One slot per device ordinal; the flags are
-// atomics so that concurrent first calls from several host threads are merely redundant.
-constexpr int kMaxDevices = 64;
-
-struct PerDeviceFlag {
-    std::atomic<bool> done[kMaxDevices];
-};
-
-int current_device_slot(int* dev_out) {
-    int dev = 0;
-    CMX_HIP(hipGetDevice(&dev));
-    CMX_REQUIRE(dev >= 0 && dev < kMaxDevices, "device ordinal out of range");
-    *dev_out = dev;
-    return CMX_OK;
-}
-
-// Every kernel that needs more dynamic LDS than the default limit is listed here at load time (one entry per
-// instantiation that a launch function names), so that cmx_init can raise all the limits up front and no first
-// call has to -- hipFuncSetAttribute is not allowed while a stream is being captured into a graph.
-struct LdsKernel {
-    const void* fn;
-    int bytes;
-    PerDeviceFlag* flag;
-};
-std::vector<LdsKernel>& lds_registry() {
-    static std::vector<LdsKernel> v;
-    return v;
-}
-template <auto KFN, size_t SMEM>
-struct LdsSetup {
-    static inline PerDeviceFlag flag{};
-    static inline const bool registered = (lds_registry().push_back({reinterpret_cast<const void*>(KFN), (int)SMEM, &flag}), true);
-};
-
-int allow_dynamic_lds(const void* kfn, int bytes, PerDeviceFlag& flag) {
-    int dev = 0;
-    int rc = current_device_slot(&dev);
-    if (rc != CMX_OK) return rc;
-    if (!flag.done[dev].load(std::memory_order_acquire)) {
-        CMX_HIP(hipFuncSetAttribute(kfn, hipFuncAttributeMaxDynamicSharedMemorySize, bytes));
-        flag.done[dev].store(true, std::memory_order_release);
-    }
-    return CMX_OK;
-}
-// raises the limit of KFN on the current device unless cmx_init or an earlier call has done so
-template <auto KFN, size_t SMEM>
-int allow_dynamic_lds() {
-    (void)LdsSetup<KFN, SMEM>::registered;
-    return allow_dynamic_lds(reinterpret_cast<const void*>(KFN), (int)SMEM, LdsSetup<KFN, SMEM>::flag);
-}
-
-int cu_count(int* out) {
-    static std::atomic<int> cus[kMaxDevices];
-    int dev = 0;
-    int rc = current_device_slot(&dev);
-    if (rc != CMX_OK) return rc;
-    int n = cus[dev].load(std::memory_order_acquire);
-    if (n == 0) {
-        CMX_HIP(hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev));
-        n = n > 0 ? n : 256;
-        cus[dev].store(n, std::memory_order_release);
-    }
-    *out = n;
-    return CMX_OK;
-}
-
 template <int FMT, int TW, int TM, int WW, int WM, int EPI, bool FAST>
 int launch_gemm_impl(const GemmParams& p, uint32_t max_m_tiles, hipStream_t s) {
     constexpr int kScaleDw = FMT == CMX_FMT_E2M1 ? 2 : 1;
@@ -1235,6 +998,46 @@ int g_pretiled_tile_rows = 0;          // 0 -> heuristic
 constexpr TileChoice g_force_tile = {0, 0, 0};
 constexpr int g_pretiled_tile_rows = 0;
 #endif
+
+#ifdef CMX_TEST_HOOKS
+KsplitTile g_force_ksplit = {0, 0, 0};
+#else
+constexpr KsplitTile g_force_ksplit = {0, 0, 0};
+#endif
+
+// Whether a problem goes to the split-K kernels (mx_gemm_ksplit.hip), and with which tile; fw == 0: no.  The choice depends
+// on sizes and element format only, so that every layout, pitch and output type of a problem gets the same sums.
+// Dense: the smallest tile that still leaves every CU at most one workgroup (time goes with the bytes a workgroup pulls
+// through its vector cache, and a second round costs as much as the first); past that 64 x 64 tiles, two workgroups of
+// four wavefronts on a CU, up to 1024 tiles.  Measured (us, E4M3, before = 256-row tiles): 16 x 4096 x 7168 44.7 -> 9.0,
+// 64 x 4096 x 7168 49.2 -> 10.8, 256 x 4096 x 7168 62.5 -> 18.0, 512 x 4096 x 7168 62.5 -> 28.1, 1024 x 4096 x 7168 (1024 tiles)
+// 63.0 -> 51.9, 2048 x 4096 x 7168 (2048 tiles) 63.4 against 99.3; 1000 x 1000 x 960 (no whole scale blocks) 37.6 -> 9.0.
+// Grouped: groups that average few rows stream their weights once whatever the tile; 64 x 64 tiles of four wavefronts
+// keep more of the stream in flight than the 256-row tiles (32 experts, K = 7168, N = 4096, GMM1, us): 4 rows per expert
+// 184 -> 142, 32 rows 189 -> 172, 64 rows 198 against 242; FP4 16 rows 113 -> 95, 64 rows 170 -> 140, 128 rows 202 against
+// 200; INT8 4 rows 223 -> 130, 32 rows 239 -> 171, 64 rows 235 against 237.
+int choose_ksplit(uint32_t m_hint, uint32_t n, int fmt, uint32_t kblocks, bool grouped, KsplitTile* out) {
+    *out = g_force_ksplit;
+    if (out->fw != 0 || g_force_tile.tw != 0 || g_pretiled_tile_rows != 0 || g_disable_dl) return CMX_OK;
+    const auto fits = [&](const KsplitTile& t) { return ksplit_lds_bytes(t, fmt, kblocks, false) <= kKsplitMaxLds; };
+    if (grouped) {
+        const KsplitTile t = {4, 4, 4};
+        if (m_hint <= (fmt == CMX_FMT_E2M1 ? 64u : 40u) && fits(t)) *out = t;
+        return CMX_OK;
+    }
+    int cus = 0;
+    if (int rc = cu_count(&cus); rc != CMX_OK) return rc;
+    const auto tiles = [&](const KsplitTile& t) { return (uint64_t)ceil_div(n, 16 * t.fw) * ceil_div(m_hint, 16 * t.fm); };
+    for (const KsplitTile& t : {KsplitTile{1, 1, 8}, KsplitTile{1, 2, 8}, KsplitTile{2, 1, 8}, KsplitTile{2, 2, 8}, KsplitTile{4, 1, 8},
+                                KsplitTile{2, 4, 8}, KsplitTile{4, 2, 8}, KsplitTile{4, 4, 8}})
+        if (tiles(t) <= (uint64_t)cus && fits(t)) {
+            *out = t;
+            return CMX_OK;
+        }
+    const KsplitTile t = {4, 4, 4};
+    if (tiles(t) <= 4 * (uint64_t)cus && fits(t)) *out = t;
+    return CMX_OK;
+}
 
 // waves: at 256 x 256 "4" and "5" select the hand-scheduled kernel in its 2 x 2 and 4 x 1 wavefront layouts
 // when the problem is eligible for it (8-bit elements, whole 512-byte K blocks).  2 x 2 reads a fifth less
@@ -1373,6 +1176,12 @@ extern "C" int cmx_debug_pretiled_tile_rows(int rows) {
     return CMX_OK;
 }
 
+// pin the split-K tile of every later matmul call (fw = 0 restores the heuristic)
+extern "C" int cmx_debug_force_ksplit(int fw, int fm, int waves) {
+    cmx::g_force_ksplit = {fw, fm, waves};
+    return CMX_OK;
+}
+
 // pin the tile shape and wavefront count of every later matmul call (tw = 0 restores the heuristic)
 extern "C" int cmx_debug_force_tile(int tw, int tm, int waves) {
     cmx::g_force_tile = (tw > 0 && tm > 0) ? cmx::TileChoice{tw, tm, waves > 0 ? waves : 4} : cmx::TileChoice{0, 0, 0};
@@ -1397,10 +1206,16 @@ extern "C" int cmx_mx_gemm(const uint8_t* a, uint32_t lda, const uint8_t* a_scal
     p.scale_vec = scales_dword_aligned(a_scale, ld_as, b_scale, ld_bs);
     p.scale_vec16 = scales_aligned16(a_scale, ld_as, b_scale, ld_bs);
     CMX_REQUIRE((uint64_t)n * ldb < (1ull << 32) && (uint64_t)lda * 256 < (1ull << 32), "operand tile exceeds 32-bit offsets");
+    hipStream_t s = static_cast<hipStream_t>(stream);
+    KsplitTile ks;
+    if (rc = choose_ksplit(m, n, fmt, p.kblocks, false, &ks); rc != CMX_OK) return rc;
+    if (ks.fw != 0) {
+        p.w_tiles = ceil_div(n, 16 * ks.fw);
+        return launch_ksplit(p, ks, fmt, kEpiStore, ceil_div(m, 16 * ks.fm), false, s);
+    }
     TileChoice t = choose_tile(m, n, fmt, false);
     p.w_tiles = ceil_div(n, t.tw);
     const uint32_t m_tiles = ceil_div(m, t.tm);
-    hipStream_t s = static_cast<hipStream_t>(stream);
     switch (fmt) {
         case CMX_FMT_E4M3: return dispatch_tile<CMX_FMT_E4M3, kEpiStore>(p, t, m_tiles, s);
         case CMX_FMT_E5M2: return dispatch_tile<CMX_FMT_E5M2, kEpiStore>(p, t, m_tiles, s);
@@ -1426,6 +1241,8 @@ int gmm_common(GemmParams& p, const int32_t* group_sizes, uint32_t groups, uint3
     if (p.w_pretiled)
         if (int rc = check_pretiled(p, fmt, swiglu); rc != CMX_OK) return rc;
     // average rows per group steers the tile height
+    KsplitTile ks;
+    if (int rc = choose_ksplit(ceil_div(m_total, groups), p.n, fmt, p.kblocks, true, &ks); rc != CMX_OK) return rc;
     TileChoice t = choose_tile(ceil_div(m_total, groups), p.n, fmt, true);
     // the weights-to-registers kernel, tiles drawn from the counters: 256 x 288 when the groups average less than four
     // tiles of rows (a group of 257 to 288 rows then takes one pass over its weights instead of two), else 256 x 256
@@ -1433,6 +1250,7 @@ int gmm_common(GemmParams& p, const int32_t* group_sizes, uint32_t groups, uint3
     int32_t* row_off = static_cast<int32_t*>(workspace);
     int32_t* tile_pref = row_off + (groups + 1);
     int32_t* tile_ctr = tile_pref + (groups + 1);
+    if (ks.fw) t = {16 * ks.fw, 16 * ks.fm, ks.waves};
     hipLaunchKernelGGL(gmm_prepare_kernel, dim3(1), dim3(256), 0, s, group_sizes, groups, (uint32_t)t.tm, m_total, row_off,
                        tile_pref, tile_ctr);
     CMX_LAUNCH_CHECK();
@@ -1445,6 +1263,8 @@ int gmm_common(GemmParams& p, const int32_t* group_sizes, uint32_t groups, uint3
     p.groups = groups;
     p.w_tiles = swiglu ? ceil_div(p.n / 2, t.tw / 2) : ceil_div(p.n, t.tw);
     const uint32_t max_m_tiles = m_total / t.tm + groups;
+    if (ks.fw) return launch_ksplit(p, ks, fmt, !swiglu ? kEpiStore : (p.act_bf16 != nullptr ? kEpiSwigluQuantAct : kEpiSwigluQuant), max_m_tiles,
+                                   ceil_div(m_total, groups) <= 32, s);
     if (p.w_pretiled) return t.tm == 288 ? launch_pretiled<288>(p, fmt, swiglu, max_m_tiles, s) : launch_pretiled<256>(p, fmt, swiglu, max_m_tiles, s);
     if (swiglu && p.act_bf16 != nullptr) return dispatch_tile<CMX_FMT_E4M3, kEpiSwigluQuantAct>(p, t, max_m_tiles, s);
     if (swiglu) return dispatch_tile<CMX_FMT_E4M3, kEpiSwigluQuant>(p, t, max_m_tiles, s);
@@ -1543,13 +1363,19 @@ extern "C" int cmx_int8_gmm_dequant_swiglu(const int8_t* a, uint32_t lda, const 
     int32_t* tile_pref = row_off + (groups + 1);
     int32_t* tile_ctr = tile_pref + (groups + 1);
     constexpr int kTile = 256;
-    hipLaunchKernelGGL(gmm_prepare_kernel, dim3(1), dim3(256), 0, s, group_sizes, groups, (uint32_t)kTile, m_total, row_off,
+    KsplitTile ks;
+    if (int rc = choose_ksplit(ceil_div(m_total, groups), n, kFmtI8, p.kblocks, true, &ks); rc != CMX_OK) return rc;
+    hipLaunchKernelGGL(gmm_prepare_kernel, dim3(1), dim3(256), 0, s, group_sizes, groups, (uint32_t)(ks.fw ? 16 * ks.fm : kTile), m_total, row_off,
                        tile_pref, tile_ctr);
     CMX_LAUNCH_CHECK();
     p.row_off = row_off;
     p.tile_pref = tile_pref;
     p.tile_ctr = tile_ctr;
     p.groups = groups;
+    if (ks.fw) {
+        p.w_tiles = ceil_div(n / 2, 8 * ks.fw);
+        return launch_ksplit(p, ks, kFmtI8, kEpiI8DequantSwiglu, m_total / (16 * ks.fm) + groups, ceil_div(m_total, groups) <= 32, s);
+    }
     p.w_tiles = ceil_div(n / 2, kTile / 2);
     // (hand-scheduled variants of this kernel were measured twice at 16 x 2048 x 7168 x 4096 and are not kept: two i8
     // MFMAs per step and accumulator in the 8-bit schedule 997 us, one per 32-K step in the 16-byte-fragment

@@ -1,0 +1,183 @@
+// What the block-scaled matmul kernels of all translation units share: the parameter block, the epilogue kinds, the mapping
+// of tile numbers to (group, m-tile, weight tile) and of workgroups to tile numbers.
+#pragma once
+
+#include "mx_common.h"
+
+namespace cmx {
+
+#if defined(__HIPCC__)
+
+constexpr int kSlabBytes = 128;     // K bytes per LDS slab and row
+constexpr int kChunks = kSlabBytes / 16;
+constexpr int kXcds = 8;
+
+// kEpiStoreBf16 / kEpiStoreFp16: 16-bit output whose rows and row pitch are multiples of eight elements (16-byte
+// stores, no per-element edge handling): small enough to sit inside a persistent kernel's tile loop.  Two epilogues, not one with a run-time switch: a second copy of the store loop inside the kernel costs
+// registers, and values spilled because of it are reloaded inside the scheduled loop, where the waits that the
+// compiler puts behind such reloads drain the operand loads in flight.
+// kEpiSwigluQuantAct: kEpiSwigluQuant that also writes the bf16 SwiGLU output (what the tests check the requantised
+// codes against).  A kernel of its own for the same reason: the extra output path costs the SwiGLU kernels
+// 30 registers, all of them spilled at the tile boundaries, 3 % of a launch, whether the output is asked for or not.
+enum Epilogue { kEpiStore = 0, kEpiSwigluQuant = 1, kEpiStoreBf16 = 2, kEpiI8DequantSwiglu = 3, kEpiStoreFp16 = 4, kEpiSwigluQuantAct = 5 };
+constexpr bool epi_is_lean_store(int epi) { return epi == kEpiStoreBf16 || epi == kEpiStoreFp16; }
+constexpr bool epi_is_swiglu_quant(int epi) { return epi == kEpiSwigluQuant || epi == kEpiSwigluQuantAct; }
+// epilogues whose weight tile pairs gate rows (first half of N) with their up partners (second half)
+constexpr bool epi_pairs_gate_up(int epi) { return epi_is_swiglu_quant(epi) || epi == kEpiI8DequantSwiglu; }
+// element "format" of the INT8 path inside the kernel templates (the public format codes are the MX ones)
+constexpr int kFmtI8 = 8;
+
+struct GemmParams {
+    const uint8_t* a;        // activations codes
+    const uint8_t* a_scale;
+    const uint8_t* w;        // weights codes [groups][n][ldw]
+    const uint8_t* w_scale;  // [groups][n][ld_ws]
+    void* c;
+    uint8_t* act_codes;
+    uint8_t* act_scales;
+    uint16_t* act_bf16;
+    const int32_t* row_off;     // [groups+1] (grouped) or null (dense)
+    const int32_t* tile_pref;   // [groups+1] prefix of m-tiles (grouped) or null
+    int32_t* tile_ctr;          // [8] per-XCD tile counters, zeroed before the launch (persistent grouped 4 x 1 kernels) or null
+    uint32_t lda, ld_as, ldw, ld_ws, ldc, ld_act, ld_acts;
+    uint32_t m, n, kbytes, kblocks;   // kblocks = K/32
+    uint32_t groups, w_tiles;
+    int out_type;
+    int scale_vec;   // scale rows are 4-byte aligned: one dword load per row and slab
+    int scale_vec16; // scale rows are 16-byte aligned: one 16-byte load per row fetches the scales of four slabs
+    int w_pretiled;  // w holds the weights in the tiled order of cmx_mx_pretile_weights (the weights-to-registers kernel)
+};
+
+__device__ __forceinline__ uint32_t swz(uint32_t row, uint32_t chunk) {
+    return chunk ^ ((row & 7u) ^ ((row >> 3) & 1u));
+}
+
+__device__ __forceinline__ v4f to_v4(const v16f& v, int q) {
+    v4f r = {v[4 * q], v[4 * q + 1], v[4 * q + 2], v[4 * q + 3]};
+    return r;
+}
+
+// g / (1 + exp(-g)) * u with the hardware exponential and reciprocal (about 1 ulp each; the result is rounded
+// to bf16 right after)
+__device__ __forceinline__ float silu_mul(float g, float u) {
+    const float s = __builtin_amdgcn_rcpf(1.0f + __expf(-g));
+    return (g * s) * u;
+}
+
+struct Tile {
+    uint32_t g, mt, wt, row0, rows_valid;
+};
+
+// The group tables (row offsets, m-tile prefix) are written by gmm_prepare_kernel before the matmul kernel starts and
+// never change under it: reading them through the constant address space lets a wavefront-uniform lookup use scalar
+// loads, which wait on lgkmcnt and so do not drain the LDS-DMA loads a persistent kernel has in flight (a vector load
+// would: its s_waitcnt vmcnt covers everything issued before it).
+__device__ __forceinline__ int32_t table_at(const int32_t* t, uint32_t i) {
+    return ((const __attribute__((address_space(4))) int32_t*)t)[i];
+}
+
+// Tiles are numbered linearly: within a group m-tiles run fastest so that neighbours share a weight panel;
+// dense problems walk bands of four m-tiles across a run of weight tiles.
+template <int TM>
+__device__ __forceinline__ uint32_t count_m_tiles(const GemmParams& p) {
+    return p.row_off != nullptr ? (uint32_t)table_at(p.tile_pref, p.groups) : (p.m + TM - 1) / TM;
+}
+
+// Tile L of an XCD-aware order: linear ids congruent mod 8 run on one XCD; each XCD gets a contiguous run.
+// Returns the first tile of XCD x and the number of tiles it owns.
+__device__ __forceinline__ uint32_t xcd_run(uint32_t total_tiles, uint32_t x, uint32_t& count) {
+    const uint32_t base = total_tiles / kXcds, rem = total_tiles % kXcds;
+    count = base + (x < rem ? 1u : 0u);
+    return x * base + (x < rem ? x : rem);
+}
+
+// Persistent kernels that walk in fixed strides (no tile counter), with at least one full round of tiles: instead of
+// owning a contiguous run, the XCDs take turns at blocks of (workgroups per XCD) consecutive tiles, workgroup j of XCD x
+// walking tiles x * per + j, + grid, + 2 * grid, ...  The whole chip then works on one stretch of `grid` consecutive
+// tiles at a time -- two bands of m-tiles across all their weight tiles -- so an activation panel is wanted by four XCDs
+// and a weight panel by two at about the same time (the memory-side cache can serve the repeats), and every block of 32
+// tiles starts on a multiple of 32, where the contiguous runs cut across the bands.  Zipf-routed 16-expert problem: 16 %
+// fewer L2 misses, 1.7-3.3 % less time.  Problems of less than a round keep the contiguous runs, which spread few tiles
+// over all eight L2s.
+__device__ __forceinline__ void interleave_xcd_walk(uint32_t total_tiles, uint32_t& tile_id, uint32_t& stride, uint32_t& end) {
+    if (total_tiles < gridDim.x) return;
+    tile_id = (blockIdx.x % kXcds) * (gridDim.x / kXcds) + blockIdx.x / kXcds;
+    stride = gridDim.x;
+    end = total_tiles;
+}
+
+// One tile per workgroup (blockIdx.x < total_tiles).  Workgroups start in the order of their ids, ids congruent mod 8 on one
+// XCD.  Whole chunks of 256 tiles: the XCDs take blocks of 32 consecutive tiles of the chunk in turn, for the reason given
+// above (the INT8 operator on the 16-expert problem: 973-982 -> 942-945 us); the rest: a contiguous run per XCD.
+__device__ __forceinline__ uint32_t tile_of_workgroup(uint32_t total_tiles) {
+    constexpr uint32_t kChunk = 32 * kXcds;
+    const uint32_t bid = blockIdx.x, full = total_tiles / kChunk * kChunk;
+    if (bid < full) return bid / kChunk * kChunk + (bid % kXcds) * 32 + (bid % kChunk) / kXcds;
+    uint32_t count;
+    const uint32_t k = bid - full;
+    return full + xcd_run(total_tiles - full, k % kXcds, count) + k / kXcds;
+}
+
+// g_from: a group at or before the tile's (0, or the group of an earlier tile of an increasing sequence)
+template <int TM>
+__device__ __forceinline__ void decode_tile(const GemmParams& p, uint32_t m_tiles_all, uint32_t L, Tile& t, uint32_t g_from = 0) {
+    if (p.row_off != nullptr) {
+        // find g with tile_pref[g]*w_tiles <= L < tile_pref[g+1]*w_tiles.  A workgroup's next tile mostly lies in the
+        // same group or one of the next two: three independent loads settle that before the bisection's
+        // chain of dependent ones
+        const uint32_t G = p.groups;
+        uint32_t lo = g_from, hi = G;
+        const uint32_t i2 = lo + 2 < G ? lo + 2 : G, i3 = lo + 3 < G ? lo + 3 : G;
+        const uint32_t t1 = (uint32_t)table_at(p.tile_pref, lo + 1) * p.w_tiles, t2 = (uint32_t)table_at(p.tile_pref, i2) * p.w_tiles,
+                       t3 = (uint32_t)table_at(p.tile_pref, i3) * p.w_tiles;
+        if (t1 > L) hi = lo + 1;
+        else if (t2 > L) { lo += 1; hi = lo + 1; }
+        else if (t3 > L) { lo += 2; hi = lo + 1; }
+        else lo += 3;
+        while (hi - lo > 1) {
+            const uint32_t mid = (lo + hi) >> 1;
+            if ((uint32_t)table_at(p.tile_pref, mid) * p.w_tiles <= L) lo = mid; else hi = mid;
+        }
+        t.g = lo;
+        const uint32_t tp = (uint32_t)table_at(p.tile_pref, lo);
+        const uint32_t mtg = (uint32_t)table_at(p.tile_pref, lo + 1) - tp;
+        // bands of 8 m-tiles share a run of weight tiles (m fastest inside a band): the 32 tiles that an XCD
+        // works on at a time then touch 8 + 4 operand panels instead of mtg + 32/mtg
+        const uint32_t local = L - tp * p.w_tiles;
+        const uint32_t band = 8;
+        const uint32_t per_band = band * p.w_tiles;
+        const uint32_t b = local / per_band, within = local % per_band;
+        const uint32_t band_rows = (mtg - b * band) < band ? (mtg - b * band) : band;
+        t.mt = b * band + within % band_rows;
+        t.wt = within / band_rows;
+        const uint32_t r_begin = (uint32_t)table_at(p.row_off, lo), r_end = (uint32_t)table_at(p.row_off, lo + 1);
+        t.row0 = r_begin + t.mt * TM;
+        t.rows_valid = r_end - t.row0 < (uint32_t)TM ? r_end - t.row0 : (uint32_t)TM;
+    } else {
+        // bands of 4 m-tiles share a run of weight tiles
+        const uint32_t band = 4;
+        const uint32_t per_band = band * p.w_tiles;
+        const uint32_t b = L / per_band, within = L % per_band;
+        const uint32_t band_rows = (m_tiles_all - b * band) < band ? (m_tiles_all - b * band) : band;
+        t.g = 0;
+        t.mt = b * band + within % band_rows;
+        t.wt = within / band_rows;
+        t.row0 = t.mt * TM;
+        t.rows_valid = p.m - t.row0 < (uint32_t)TM ? p.m - t.row0 : (uint32_t)TM;
+    }
+}
+
+// One tile per workgroup: maps the workgroup id to (group, m-tile, weight tile).  Returns false for ids past
+// the last tile.
+template <int TM>
+__device__ __forceinline__ bool locate_tile(const GemmParams& p, Tile& t) {
+    const uint32_t m_tiles_all = count_m_tiles<TM>(p);
+    const uint32_t total_tiles = m_tiles_all * p.w_tiles;
+    if (blockIdx.x >= total_tiles) return false;
+    decode_tile<TM>(p, m_tiles_all, tile_of_workgroup(total_tiles), t);
+    return true;
+}
+
+#endif  // __HIPCC__
+
+}  // namespace cmx

@@ -1,0 +1,542 @@
+// Block-scaled (and INT8) matmul for problems with few activation rows or few tiles: split over K inside the workgroup.
+//
+// A problem of a few rows reads every weight byte once and multiplies it a handful of times: what counts is how many
+// bytes are in flight on how many CUs, and tiles of 256 weight rows leave most of the chip without work (16 x 4096 x 7168:
+// sixteen workgroups).  Here a workgroup owns a small tile, 16 FW weight rows x 16 FM activation rows, and its NW wavefronts
+// split K between them: wavefront w multiplies the 128-byte K slabs w, w + NW, w + 2 NW, ... of the WHOLE tile, so
+//   * every operand byte of the tile is needed by exactly one wavefront: both operands go straight from memory into that
+//     wavefront's registers (buffer_load_dwordx4) through a ring of PD slabs, with no barrier and no wait for another
+//     wavefront in the K loop;
+//   * v_mfma_scale_f32_16x16x128_f8f6f4 takes, per lane group g = lane / 16, the bytes 16 g .. 16 g + 15 of a slab's first
+//     64 bytes in registers 0-3 and of its second 64 bytes in registers 4-7 (and the scale of the 32-block g), for the
+//     row lane % 16.  Loading row-major operands in that order costs the vector cache a visit per lane quad and row, twice
+//     the time of whole 128-byte lines (measured: 9.7 against 7.2 us at 16 x 4096 x 7168), so the lanes fetch whole lines, eight to a
+//     row, and a fragment changes places through 2 KiB of LDS that belong to the wavefront alone (its LDS accesses
+//     execute in order: nothing to wait for).  Pre-tiled weights are stored in the fragment order and need none of it;
+//   * the block scales of the tile, which are a byte per 32 elements in rows of their own, are fetched once, coalesced, for
+//     the whole of K into the LDS and read from there a byte per lane and fragment.
+// The NW partial sums meet in the LDS at the end and are added in the order of the wavefronts, so the result does not
+// depend on timing; it does depend on NW, and differs in the last bits from that of the kernels that walk K in one chain.
+// Every tile shape with the same NW gives the same bits, and so do row-major and pre-tiled weights.
+#include <type_traits>
+
+#include "mx_gemm_ksplit.h"
+#include "mx_launch.h"
+
+namespace cmx {
+
+namespace {
+
+typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
+
+constexpr int ks_scale_steps(int fmt) { return fmt == kFmtI8 ? 0 : (fmt == CMX_FMT_E2M1 ? 2 : 1); }   // scale dwords per row and slab
+// slabs in the register ring: what fits beside the accumulators, one slab of fragments in MFMA order, their scales and
+// addresses in 256 registers (two wavefronts per SIMD)
+constexpr int ks_ring(int fmt, int fw, int fm) {
+    const int room = 256 - 40 - 4 * fw * fm - (fw + fm) * (10 + 2 * ks_scale_steps(fmt));
+    const int n = room / ((fw + fm) * 8), most = fw + fm == 2 ? 8 : (fw + fm == 3 ? 5 : 4);
+    return n < 1 ? 1 : (n > most ? most : n);
+}
+// activation rows whose partial sums go through the LDS at a time (the NW partial tiles of all rows may exceed it)
+constexpr int ks_pass_frags(int fw, int fm, int nw) {
+    int n = fm;
+    while (n > 1 && nw * n * 16 * (16 * fw + 4) * 4 > 65536) n /= 2;
+    return n;
+}
+// exchange buffers of a wavefront (2 KiB, one fragment): four, used in turn
+constexpr int ks_exchange_bufs(int fw, int fm, bool tiled) { return (tiled ? 0 : fw) + fm < 4 ? (tiled ? 0 : fw) + fm : 4; }
+constexpr size_t ks_sum_bytes(int fw, int fm, int nw) { return (size_t)nw * ks_pass_frags(fw, fm, nw) * 16 * (16 * fw + 4) * 4; }
+// dwords of a scale row in the LDS: whole slabs, an odd count so that the sixteen rows of a fragment lie in different banks
+__host__ __device__ inline uint32_t ks_scale_pitch(int fmt, uint32_t kblocks) {
+    const uint32_t per = fmt == CMX_FMT_E2M1 ? 8 : 4;
+    return ((kblocks + per - 1) / per * per / 4) | 1u;
+}
+
+// acc += W-fragment x A-fragment over one 128-byte slab
+template <int FMT>
+__device__ __forceinline__ v4f ks_mfma(const v4i (&w)[2], const v4i (&a)[2], v4f c, const uint32_t (&sw)[2], const uint32_t (&sa)[2]) {
+    if constexpr (FMT == kFmtI8) {
+        v4i acc = __builtin_bit_cast(v4i, c);
+        acc = __builtin_amdgcn_mfma_i32_16x16x64_i8(w[0], a[0], acc, 0, 0, 0);
+        acc = __builtin_amdgcn_mfma_i32_16x16x64_i8(w[1], a[1], acc, 0, 0, 0);
+        return __builtin_bit_cast(v4f, acc);
+    } else if constexpr (FMT == CMX_FMT_E2M1) {
+        const v8i w0 = {w[0][0], w[0][1], w[0][2], w[0][3], 0, 0, 0, 0}, w1 = {w[1][0], w[1][1], w[1][2], w[1][3], 0, 0, 0, 0};
+        const v8i a0 = {a[0][0], a[0][1], a[0][2], a[0][3], 0, 0, 0, 0}, a1 = {a[1][0], a[1][1], a[1][2], a[1][3], 0, 0, 0, 0};
+        c = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(w0, a0, c, 4, 4, 0, (int)sw[0], 0, (int)sa[0]);
+        return __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(w1, a1, c, 4, 4, 0, (int)sw[1], 0, (int)sa[1]);
+    } else {
+        constexpr int kF = FMT == CMX_FMT_E5M2 ? 1 : 0;
+        const v8i w8 = {w[0][0], w[0][1], w[0][2], w[0][3], w[1][0], w[1][1], w[1][2], w[1][3]};
+        const v8i a8 = {a[0][0], a[0][1], a[0][2], a[0][3], a[1][0], a[1][1], a[1][2], a[1][3]};
+        return __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(w8, a8, c, kF, kF, 0, (int)sw[0], 0, (int)sa[0]);
+    }
+}
+
+// Sums of one output row, four consecutive columns (SwiGLU kinds: four gate columns and their up partners), to memory.
+template <int EPI, int TW>
+__device__ __forceinline__ void ks_store(const GemmParams& p, const Tile& tc, uint32_t mloc, uint32_t q, const v4f& v, const v4f& u) {
+    const bool mvalid = mloc < tc.rows_valid;
+    const size_t mrow = (size_t)(tc.row0 + (mvalid ? mloc : 0));
+    if constexpr (EPI == kEpiStore) {
+        const uint32_t ncol = tc.wt * TW + 4 * q;
+        if (!mvalid || ncol >= p.n) return;
+        const bool full = ncol + 4 <= p.n;
+        if (p.out_type == CMX_OUT_FP32) {
+            float* o = reinterpret_cast<float*>(p.c) + mrow * p.ldc + ncol;
+            if (full && (reinterpret_cast<uintptr_t>(o) & 15u) == 0) {
+                *reinterpret_cast<v4f*>(o) = v;
+            } else {
+                for (uint32_t i = 0; i < 4 && ncol + i < p.n; ++i) o[i] = v[i];
+            }
+        } else {
+            uint32_t h0, h1;
+            if (p.out_type == CMX_OUT_BF16) {
+                h0 = cvt_pk_bf16(v[0], v[1]);
+                h1 = cvt_pk_bf16(v[2], v[3]);
+            } else {
+                typedef _Float16 v2h __attribute__((ext_vector_type(2)));
+                h0 = __builtin_bit_cast(uint32_t, (v2h){(_Float16)v[0], (_Float16)v[1]});
+                h1 = __builtin_bit_cast(uint32_t, (v2h){(_Float16)v[2], (_Float16)v[3]});
+            }
+            uint16_t* o = reinterpret_cast<uint16_t*>(p.c) + mrow * p.ldc + ncol;
+            if (full && (reinterpret_cast<uintptr_t>(o) & 7u) == 0) {
+                *reinterpret_cast<uint2*>(o) = make_uint2(h0, h1);
+            } else {
+                const uint32_t h[2] = {h0, h1};
+                for (uint32_t i = 0; i < 4 && ncol + i < p.n; ++i) o[i] = (uint16_t)(h[i >> 1] >> (16 * (i & 1)));
+            }
+        }
+    } else if constexpr (EPI == kEpiI8DequantSwiglu) {
+        // INT32 sums -> fp32 * per-channel scale -> fp16 -> fp32 * per-token scale -> x0 * sigmoid(x0) * gate
+        const uint32_t half = p.n >> 1, ncol = tc.wt * (TW / 2) + 4 * q;
+        if (!mvalid || ncol >= half) return;                      // n is a multiple of 64: four columns are in or out together
+        const float* ch = reinterpret_cast<const float*>(p.w_scale) + (size_t)tc.g * p.n * p.ld_ws;
+        const float tsv = reinterpret_cast<const float*>(p.a_scale)[mrow];
+        const v4i ig = __builtin_bit_cast(v4i, v), iu = __builtin_bit_cast(v4i, u);
+        float y[4];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const float cg = ch[(size_t)(ncol + i) * p.ld_ws], cu = ch[(size_t)(half + ncol + i) * p.ld_ws];
+            const float x0 = __fmul_rn((float)(_Float16)__fmul_rn((float)ig[i], cg), tsv);
+            const float gate = __fmul_rn((float)(_Float16)__fmul_rn((float)iu[i], cu), tsv);
+            y[i] = __fmul_rn(__fmul_rn(x0, __builtin_amdgcn_rcpf(1.0f + __expf(-x0))), gate);
+        }
+        if (p.out_type == CMX_OUT_FP32) {
+            float* o = reinterpret_cast<float*>(p.c) + mrow * p.ldc + ncol;
+            if ((reinterpret_cast<uintptr_t>(o) & 15u) == 0) {
+                *reinterpret_cast<float4*>(o) = make_float4(y[0], y[1], y[2], y[3]);
+            } else {
+                for (uint32_t i = 0; i < 4; ++i) o[i] = y[i];
+            }
+        } else {
+            uint16_t h[4];
+#pragma unroll
+            for (int i = 0; i < 4; ++i)
+                h[i] = p.out_type == CMX_OUT_FP16 ? __builtin_bit_cast(uint16_t, (_Float16)y[i]) : (uint16_t)f32_to_bf16(y[i]);
+            uint16_t* o = reinterpret_cast<uint16_t*>(p.c) + mrow * p.ldc + ncol;
+            if ((reinterpret_cast<uintptr_t>(o) & 7u) == 0) {
+                *reinterpret_cast<uint2*>(o) = make_uint2(h[0] | ((uint32_t)h[1] << 16), h[2] | ((uint32_t)h[3] << 16));
+            } else {
+                for (uint32_t i = 0; i < 4; ++i) o[i] = h[i];
+            }
+        }
+    } else {
+        // SwiGLU on the bf16-rounded sums, bf16 again, then the MX block of 32 columns: eight neighbouring lanes hold it
+        static_assert(TW / 2 % 32 == 0, "whole MX blocks in a tile");
+        const uint32_t half = p.n >> 1, ncol = tc.wt * (TW / 2) + 4 * q;
+        uint32_t pk[2], m = 0;
+#pragma unroll
+        for (int j = 0; j < 2; ++j) {
+            const uint32_t g2 = cvt_pk_bf16(v[2 * j], v[2 * j + 1]), u2 = cvt_pk_bf16(u[2 * j], u[2 * j + 1]);
+            pk[j] = cvt_pk_bf16(silu_mul(__uint_as_float(g2 << 16), __uint_as_float(u2 << 16)),
+                                silu_mul(__uint_as_float(g2 & 0xFFFF0000u), __uint_as_float(u2 & 0xFFFF0000u)));
+            m = pk_max_u16(m, pk[j] & 0x7FFF7FFFu);
+        }
+        m = pk_max_u16(m, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)m, 0xB1, 0xF, 0xF, true));     // lane ^ 1
+        m = pk_max_u16(m, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)m, 0x4E, 0xF, 0xF, true));     // lane ^ 2
+        m = pk_max_u16(m, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)m, 0x141, 0xF, 0xF, true));    // the other quad of eight
+        const uint32_t amax = max(m & 0xFFFFu, m >> 16);
+        const int e = block_exp_from_bf16_amax(amax, kEmaxE4M3);
+        if (!mvalid || ncol >= half) return;
+        if constexpr (EPI == kEpiSwigluQuantAct) {
+            if (p.act_bf16) {
+                uint16_t* o = p.act_bf16 + mrow * half + ncol;
+#pragma unroll
+                for (int i = 0; i < 4; ++i) o[i] = (uint16_t)(pk[i >> 1] >> (16 * (i & 1)));
+            }
+        }
+        const uint32_t lim = (((uint32_t)(e + kEmaxE4M3 + 127) << 7) | 0x60u) * 0x10001u;
+        const float scale = __uint_as_float((uint32_t)(e + 127) << 23);
+        const uint32_t c0 = pk_min_u16(pk[0] & 0x7FFF7FFFu, lim) | (pk[0] & 0x80008000u);
+        const uint32_t c1 = pk_min_u16(pk[1] & 0x7FFF7FFFu, lim) | (pk[1] & 0x80008000u);
+        *reinterpret_cast<uint32_t*>(p.act_codes + mrow * p.ld_act + ncol) = cvt_scaled_pk4<CMX_FMT_E4M3>(c0, c1, scale);
+        if ((q & 7u) == 0) {
+            uint8_t* srow = p.act_scales + mrow * p.ld_acts;
+            const uint32_t blk = ncol >> 5, nblk = half >> 5;
+            srow[blk] = (uint8_t)(e + 127);
+            if (blk == nblk - 1 && (nblk & 1u)) srow[nblk] = 127;
+        }
+    }
+}
+
+// STREAM: weights are loaded non-temporal (one reader; a tile column has no other m-tile)
+template <int FMT, int FW, int FM, int NW, int EPI, bool TILED, bool STREAM>
+__device__ __forceinline__ void ks_tile(const GemmParams& p, const Tile& tc, uint8_t* smem) {
+    constexpr int NT = 64 * NW, TW = 16 * FW;
+    constexpr int kS = ks_scale_steps(FMT);
+    constexpr int kSA = kS ? kS : 1;
+    constexpr int PD = ks_ring(FMT, FW, FM);
+    constexpr int kRows = 16 * (FW + FM);
+    const uint32_t tid = threadIdx.x, lane = tid & 63u;
+    const uint32_t wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const uint32_t r = lane & 15u, g = lane >> 4;
+    const uint32_t half = p.n >> 1;
+
+    // global weight row of tile row t (rows past the matrix repeat the last one; masked at the store)
+    auto wrow_of = [&](uint32_t t) -> uint32_t {
+        if (epi_pairs_gate_up(EPI)) {
+            uint32_t rr = tc.wt * (TW / 2) + (t < TW / 2 ? t : t - TW / 2);
+            rr = rr < half ? rr : half - 1;
+            return t < TW / 2 ? rr : half + rr;
+        }
+        const uint32_t gr = tc.wt * TW + t;
+        return gr < p.n ? gr : p.n - 1;
+    };
+    auto arow_of = [&](uint32_t t) -> uint32_t { return t < tc.rows_valid ? t : tc.rows_valid - 1; };
+
+    // ---- scales of the tile: request -----------------------------------------------------------------------------------
+    const uint32_t pitch = ks_scale_pitch(FMT, p.kblocks);
+    uint32_t* const s_sc = reinterpret_cast<uint32_t*>(smem);
+    auto scale_row = [&](uint32_t t) -> const uint8_t* {
+        return t < (uint32_t)TW ? p.w_scale + ((size_t)tc.g * p.n + wrow_of(t)) * p.ld_ws
+                                : p.a_scale + (size_t)(tc.row0 + arow_of(t - TW)) * p.ld_as;
+    };
+    // 16-byte pieces when the rows allow it, numbered with the next power of two of pieces per row (no division)
+    constexpr int kBatch = 2048 / NT;                  // pieces per thread in flight together: 32 KiB per workgroup
+    const bool sc16 = kS && p.scale_vec16 && p.kblocks % 16 == 0;
+    const uint32_t pieces = p.kblocks / 16, shift = pieces > 1 ? 32 - __builtin_clz(pieces - 1) : 0;
+    const uint32_t total16 = kRows << shift;
+    u32x4 sreg[kBatch];
+    auto request16 = [&](uint32_t i0) {
+#pragma unroll
+        for (int b = 0; b < kBatch; ++b) {
+            const uint32_t i = i0 + b * NT + tid, t = i >> shift, q = i & ((1u << shift) - 1);
+            if (i < total16 && q < pieces) sreg[b] = *reinterpret_cast<const u32x4*>(scale_row(t) + q * 16);
+        }
+    };
+    auto deposit16 = [&](uint32_t i0) {
+#pragma unroll
+        for (int b = 0; b < kBatch; ++b) {
+            const uint32_t i = i0 + b * NT + tid, t = i >> shift, q = i & ((1u << shift) - 1);
+            if (i < total16 && q < pieces) {
+                uint32_t* d = s_sc + t * pitch + q * 4;
+#pragma unroll
+                for (int e = 0; e < 4; ++e) d[e] = sreg[b][e];
+            }
+        }
+    };
+    if (sc16) request16(0);
+
+    // ---- operand streams ---------------------------------------------------------------------------------------------
+    constexpr int kRsrcFlags = 0x00020000;
+    auto uniform_ptr = [](const uint8_t* q) -> uint8_t* {
+        const uint64_t v = reinterpret_cast<uint64_t>(q);
+        const uint32_t lo = __builtin_amdgcn_readfirstlane((uint32_t)v), hi = __builtin_amdgcn_readfirstlane((uint32_t)(v >> 32));
+        return reinterpret_cast<uint8_t*>(((uint64_t)hi << 32) | lo);
+    };
+    const uint8_t* wbase;
+    // row-major: load h of a fragment covers its rows 8 h .. 8 h + 7, lane -> row lane / 8, 16-byte chunk lane % 8
+    const uint32_t x_row = lane >> 3, x_chunk = lane & 7u;
+    uint32_t woff[FW][2], aoff[FM][2];
+    if constexpr (TILED) {
+        // [256-row tile][slab][wavefront block][step 0/1][fragment][half][lane half][32 rows][16 bytes]: the bytes
+        // 64 j + 16 g of a row's slab lie in step j, half g / 2, lane half g % 2
+        constexpr bool kPair = epi_pairs_gate_up(EPI);
+        const uint32_t row0 = kPair ? tc.wt * (TW / 2) : tc.wt * TW;
+        const uint32_t big = kPair ? row0 / 128 : row0 / 256;
+        const uint32_t w256 = kPair ? (half + 127) / 128 : (p.n + 255) / 256;
+        wbase = p.w + ((size_t)tc.g * w256 + big) * ((size_t)p.kbytes * 256);
+#pragma unroll
+        for (int f = 0; f < FW; ++f) {
+            uint32_t blk, frag, row;
+            if (kPair) {
+                const uint32_t q = (row0 + (f < FW / 2 ? f : f - FW / 2) * 16 + r) % 128;
+                blk = q / 32; frag = f < FW / 2 ? 0 : 1; row = q % 32;
+            } else {
+                const uint32_t q = (row0 + f * 16 + r) % 256;
+                blk = q / 64; frag = q / 32 % 2; row = q % 32;
+            }
+            woff[f][0] = blk * 8192 + frag * 2048 + (g >> 1) * 1024 + (g & 1u) * 512 + row * 16;
+            woff[f][1] = woff[f][0] + 4096;
+        }
+    } else {
+        wbase = p.w + (size_t)tc.g * p.n * p.ldw;
+#pragma unroll
+        for (int f = 0; f < FW; ++f)
+#pragma unroll
+            for (int h = 0; h < 2; ++h) woff[f][h] = wrow_of(f * 16 + 8 * h + x_row) * p.ldw + x_chunk * 16;
+    }
+#pragma unroll
+    for (int f = 0; f < FM; ++f)
+#pragma unroll
+        for (int h = 0; h < 2; ++h) aoff[f][h] = arow_of(f * 16 + 8 * h + x_row) * p.lda + x_chunk * 16;
+    const __amdgpu_buffer_rsrc_t w_rs = __builtin_amdgcn_make_buffer_rsrc(uniform_ptr(wbase), 0, -1, kRsrcFlags);
+    const __amdgpu_buffer_rsrc_t a_rs = __builtin_amdgcn_make_buffer_rsrc(uniform_ptr(p.a + (size_t)tc.row0 * p.lda), 0, -1, kRsrcFlags);
+    constexpr uint32_t kWSlab = TILED ? 256 * kSlabBytes : kSlabBytes;
+    constexpr int kWAux = STREAM ? 2 : 0;              // 2: non-temporal
+
+    v4i wf[PD][FW][2], af[PD][FM][2];
+    // Slab s of this wavefront into ring slot d; past the last slab every lane re-reads the operand's first bytes (one line,
+    // never used), so that the number of loads in flight does not depend on the length of K.
+    const uint32_t nslab = p.kbytes / kSlabBytes;
+    auto load_slot = [&](int d, uint32_t s) {
+        const bool in = s < nslab;
+        const uint32_t mask = in ? ~0u : 0u, sw = in ? s * kWSlab : 0u, sa = in ? s * kSlabBytes : 0u;
+#pragma unroll
+        for (int f = 0; f < FW; ++f)
+#pragma unroll
+            for (int h = 0; h < 2; ++h)
+                wf[d][f][h] = __builtin_bit_cast(v4i, __builtin_amdgcn_raw_buffer_load_b128(w_rs, (int)(woff[f][h] & mask), (int)sw, kWAux));
+#pragma unroll
+        for (int f = 0; f < FM; ++f)
+#pragma unroll
+            for (int h = 0; h < 2; ++h)
+                af[d][f][h] = __builtin_bit_cast(v4i, __builtin_amdgcn_raw_buffer_load_b128(a_rs, (int)(aoff[f][h] & mask), (int)sa, 0));
+    };
+#pragma unroll
+    for (int d = 0; d < PD; ++d) load_slot(d, wave + NW * d);
+
+    // ---- scales of the tile: deposit -----------------------------------------------------------------------------------
+    if constexpr (kS != 0) {
+        if (sc16) {
+            deposit16(0);
+            for (uint32_t i0 = kBatch * NT; i0 < total16; i0 += kBatch * NT) {
+                request16(i0);
+                deposit16(i0);
+            }
+        } else {
+            // dword by dword; a last slab in part is filled up with 1.0
+            const uint32_t sh = 32 - __builtin_clz(pitch - 1 | 1u);
+            for (uint32_t i = tid; i < ((uint32_t)kRows << sh); i += NT) {
+                const uint32_t t = i >> sh, q = i & ((1u << sh) - 1);
+                if (q >= pitch) continue;
+                const uint8_t* row = scale_row(t);
+                uint32_t v = 0x7F7F7F7Fu;
+                if (p.scale_vec && 4 * q + 4 <= p.kblocks) {
+                    v = *reinterpret_cast<const uint32_t*>(row + 4 * q);
+                } else {
+                    for (uint32_t b = 0; b < 4; ++b)
+                        if (4 * q + b < p.kblocks) v = (v & ~(0xFFu << (8 * b))) | ((uint32_t)row[4 * q + b] << (8 * b));
+                }
+                s_sc[t * pitch + q] = v;
+            }
+        }
+        __syncthreads();
+    }
+    const uint8_t* const sw_row = smem + r * pitch * 4 + g;
+    const uint8_t* const sa_row = smem + (TW + r) * pitch * 4 + g;
+
+    v4f acc[FW][FM];
+#pragma unroll
+    for (int i = 0; i < FW; ++i)
+#pragma unroll
+        for (int j = 0; j < FM; ++j) acc[i][j] = (v4f){0.f, 0.f, 0.f, 0.f};
+
+    // a fragment from the order of the loads (rows 8 h + lane / 8, chunk lane % 8) to that of the MFMA (row lane % 16, chunks
+    // lane / 16 and 4 + lane / 16); chunks XOR-swizzled by row: neither side meets bank conflicts
+    constexpr int kBufs = ks_exchange_bufs(FW, FM, TILED);
+    uint8_t* const xbuf = smem + kRows * pitch * 4 * (kS ? 1 : 0) + ((0u - kRows * pitch * 4 * (kS ? 1 : 0)) & 15u) + wave * (kBufs * 2048);
+    uint32_t xw[2], xr[2];
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+        xw[h] = (8 * h + x_row) * 128 + swz(8 * h + x_row, x_chunk) * 16;
+        xr[h] = r * 128 + swz(r, 4 * h + g) * 16;
+    }
+    auto exchange = [&](int buf, const v4i (&in)[2], v4i (&out)[2]) {
+        uint8_t* const b = xbuf + buf % kBufs * 2048;
+#pragma unroll
+        for (int h = 0; h < 2; ++h) *reinterpret_cast<v4i*>(b + xw[h]) = in[h];
+#pragma unroll
+        for (int h = 0; h < 2; ++h) out[h] = *reinterpret_cast<const v4i*>(b + xr[h]);
+    };
+    auto multiply = [&](const v4i (&wl)[FW][2], const v4i (&al)[FM][2], uint32_t s) {
+        v4i w[FW][2], a[FM][2];
+#pragma unroll
+        for (int f = 0; f < FM; ++f) exchange(f, al[f], a[f]);
+#pragma unroll
+        for (int f = 0; f < FW; ++f) {
+            if constexpr (TILED) {
+                w[f][0] = wl[f][0];
+                w[f][1] = wl[f][1];
+            } else {
+                exchange(FM + f, wl[f], w[f]);
+            }
+        }
+        uint32_t sw[FW][2] = {}, sa[FM][2] = {};
+#pragma unroll
+        for (int j = 0; j < kS; ++j) {
+#pragma unroll
+            for (int f = 0; f < FW; ++f) sw[f][j] = sw_row[f * 16 * pitch * 4 + s * (4 * kSA) + 4 * j];
+#pragma unroll
+            for (int f = 0; f < FM; ++f) sa[f][j] = sa_row[f * 16 * pitch * 4 + s * (4 * kSA) + 4 * j];
+        }
+#pragma unroll
+        for (int i = 0; i < FW; ++i)
+#pragma unroll
+            for (int j = 0; j < FM; ++j) acc[i][j] = ks_mfma<FMT>(w[i], a[j], acc[i][j], sw[i], sa[j]);
+    };
+
+    // ---- K loop --------------------------------------------------------------------------------------------------------
+    const uint32_t mine = nslab > wave ? (nslab - wave + NW - 1) / NW : 0u;          // slabs of this wavefront
+    uint32_t i = 0;
+    for (; i + PD < mine; i += PD) {
+#pragma unroll
+        for (int d = 0; d < PD; ++d) {
+            multiply(wf[d], af[d], wave + NW * (i + d));
+            load_slot(d, wave + NW * (i + PD + d));
+        }
+    }
+#pragma unroll
+    for (int d = 0; d < PD; ++d)
+        if (i + d < mine) multiply(wf[d], af[d], wave + NW * (i + d));
+    // K not a whole number of slabs: the rest, zeros past K
+    if constexpr (FMT != kFmtI8 && !TILED) {
+        if (p.kbytes % kSlabBytes != 0 && nslab % NW == wave) {
+#pragma unroll
+            for (int h = 0; h < 2; ++h) {
+                const bool in = nslab * kSlabBytes + x_chunk * 16 < p.kbytes;        // K is whole 16-byte pieces
+                const int kb = (int)(nslab * kSlabBytes);
+#pragma unroll
+                for (int f = 0; f < FW; ++f) {
+                    wf[0][f][h] = (v4i){0, 0, 0, 0};
+                    if (in) wf[0][f][h] = __builtin_bit_cast(v4i, __builtin_amdgcn_raw_buffer_load_b128(w_rs, (int)woff[f][h], kb, 0));
+                }
+#pragma unroll
+                for (int f = 0; f < FM; ++f) {
+                    af[0][f][h] = (v4i){0, 0, 0, 0};
+                    if (in) af[0][f][h] = __builtin_bit_cast(v4i, __builtin_amdgcn_raw_buffer_load_b128(a_rs, (int)aoff[f][h], kb, 0));
+                }
+            }
+            multiply(wf[0], af[0], nslab);
+        }
+    }
+
+    // ---- sum over the wavefronts, epilogue ------------------------------------------------------------------------------
+    // partial sums as [wavefront][row][column] with four floats between the rows
+    constexpr int kPass = ks_pass_frags(FW, FM, NW);
+    constexpr uint32_t kRowPitch = TW + 4, kPart = kPass * 16 * kRowPitch;
+    float* const sums = reinterpret_cast<float*>(smem);
+    constexpr uint32_t kQuads = epi_pairs_gate_up(EPI) ? TW / 8 : TW / 4;            // columns are written in fours
+#pragma unroll
+    for (int f0 = 0; f0 < FM; f0 += kPass) {
+        __syncthreads();                                                             // the scales (or the last pass's sums) have been read
+#pragma unroll
+        for (int j = 0; j < kPass; ++j)
+#pragma unroll
+            for (int f = 0; f < FW; ++f)
+                *reinterpret_cast<v4f*>(sums + wave * kPart + (j * 16 + r) * kRowPitch + f * 16 + 4 * g) = acc[f][f0 + j];
+        __syncthreads();
+        for (uint32_t it = tid; it < kPass * 16 * kQuads; it += NT) {
+            const uint32_t m = it / kQuads, q = it % kQuads;
+            auto total = [&](uint32_t col) -> v4f {
+                const float* s = sums + m * kRowPitch + col;
+                v4f v = *reinterpret_cast<const v4f*>(s);
+#pragma unroll
+                for (int w = 1; w < NW; ++w) {
+                    const v4f o = *reinterpret_cast<const v4f*>(s + w * kPart);
+                    if constexpr (FMT == kFmtI8) v = __builtin_bit_cast(v4f, __builtin_bit_cast(v4i, v) + __builtin_bit_cast(v4i, o));
+                    else v += o;
+                }
+                return v;
+            };
+            const v4f v = total(4 * q);
+            v4f u = v;
+            if constexpr (epi_pairs_gate_up(EPI)) u = total(TW / 2 + 4 * q);
+            ks_store<EPI, TW>(p, tc, f0 * 16 + m, q, v, u);
+        }
+    }
+}
+
+template <int FMT, int FW, int FM, int NW, int EPI, bool TILED, bool STREAM>
+__global__ __launch_bounds__(64 * NW, 2) void mx_gemm_ksplit_kernel(const GemmParams p) {
+    extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
+    Tile tc;
+    if (!locate_tile<16 * FM>(p, tc)) return;
+    tc.g = __builtin_amdgcn_readfirstlane(tc.g);
+    tc.wt = __builtin_amdgcn_readfirstlane(tc.wt);
+    tc.row0 = __builtin_amdgcn_readfirstlane(tc.row0);
+    tc.rows_valid = __builtin_amdgcn_readfirstlane(tc.rows_valid);
+    // a ragged tile does the work of the rows it has
+    if constexpr (FM >= 4) {
+        if (tc.rows_valid <= 16 * FM / 4) return ks_tile<FMT, FW, FM / 4, NW, EPI, TILED, STREAM>(p, tc, smem);
+    }
+    if constexpr (FM >= 2) {
+        if (tc.rows_valid <= 16 * FM / 2) return ks_tile<FMT, FW, FM / 2, NW, EPI, TILED, STREAM>(p, tc, smem);
+    }
+    ks_tile<FMT, FW, FM, NW, EPI, TILED, STREAM>(p, tc, smem);
+}
+
+template <int FMT, int FW, int FM, int NW, int EPI, bool TILED, bool STREAM>
+int launch_one(const GemmParams& p, uint32_t max_m_tiles, hipStream_t s) {
+    constexpr auto kfn = mx_gemm_ksplit_kernel<FMT, FW, FM, NW, EPI, TILED, STREAM>;
+    if (int rc = allow_dynamic_lds<kfn, kKsplitMaxLds>(); rc != CMX_OK) return rc;
+    const size_t smem = ksplit_lds_bytes({FW, FM, NW}, FMT, p.kblocks, TILED);
+    CMX_REQUIRE(smem <= kKsplitMaxLds, "split-K tile exceeds the LDS");
+    const uint64_t tiles = (uint64_t)max_m_tiles * p.w_tiles;
+    CMX_REQUIRE(tiles > 0 && tiles < (1ull << 31), "tile count out of range");
+    hipLaunchKernelGGL(kfn, dim3((uint32_t)tiles), dim3(64 * NW), smem, s, p);
+    CMX_LAUNCH_CHECK();
+    return CMX_OK;
+}
+
+// the tile shapes that exist for an element format and epilogue: one for grouped problems, all for dense ones
+template <int FMT, int EPI, bool TILED>
+int launch_shape(const GemmParams& p, const KsplitTile& t, uint32_t max_m_tiles, bool stream, hipStream_t s) {
+#define CMX_KS(FW_, FM_, NW_) if (t.fw == FW_ && t.fm == FM_ && t.waves == NW_) return launch_one<FMT, FW_, FM_, NW_, EPI, TILED, false>(p, max_m_tiles, s)
+    if (t.fw == 4 && t.fm == 4 && t.waves == 4) {
+        if (stream) return launch_one<FMT, 4, 4, 4, EPI, TILED, true>(p, max_m_tiles, s);
+        return launch_one<FMT, 4, 4, 4, EPI, TILED, false>(p, max_m_tiles, s);
+    }
+    if constexpr (EPI == kEpiStore && !TILED) {
+        CMX_KS(1, 1, 8);
+        CMX_KS(1, 2, 8);
+        CMX_KS(2, 1, 8);
+        CMX_KS(2, 2, 8);
+        CMX_KS(2, 4, 8);
+        CMX_KS(4, 1, 8);
+        CMX_KS(4, 2, 8);
+        CMX_KS(4, 4, 8);
+    }
+#undef CMX_KS
+    set_error("unsupported split-K tile");
+    return CMX_EINVAL;
+}
+
+}  // namespace
+
+size_t ksplit_lds_bytes(const KsplitTile& t, int fmt, uint32_t kblocks, bool tiled) {
+    const size_t scales = ks_scale_steps(fmt) ? round_up_sz((size_t)16 * (t.fw + t.fm) * ks_scale_pitch(fmt, kblocks) * 4, 16) : 0;
+    const size_t loop = scales + (size_t)t.waves * ks_exchange_bufs(t.fw, t.fm, tiled) * 2048;
+    const size_t sums = ks_sum_bytes(t.fw, t.fm, t.waves);
+    return loop > sums ? loop : sums;
+}
+
+int launch_ksplit(const GemmParams& p, const KsplitTile& t, int fmt, int epi, uint32_t max_m_tiles, bool stream, hipStream_t s) {
+    if (fmt == CMX_FMT_E4M3) {
+        if (epi == kEpiStore)
+            return p.w_pretiled ? launch_shape<CMX_FMT_E4M3, kEpiStore, true>(p, t, max_m_tiles, stream, s) : launch_shape<CMX_FMT_E4M3, kEpiStore, false>(p, t, max_m_tiles, stream, s);
+        if (epi == kEpiSwigluQuant)
+            return p.w_pretiled ? launch_shape<CMX_FMT_E4M3, kEpiSwigluQuant, true>(p, t, max_m_tiles, stream, s)
+                                : launch_shape<CMX_FMT_E4M3, kEpiSwigluQuant, false>(p, t, max_m_tiles, stream, s);
+        if (epi == kEpiSwigluQuantAct && !p.w_pretiled) return launch_shape<CMX_FMT_E4M3, kEpiSwigluQuantAct, false>(p, t, max_m_tiles, stream, s);
+    }
+    if (fmt == CMX_FMT_E5M2 && epi == kEpiStore)
+        return p.w_pretiled ? launch_shape<CMX_FMT_E5M2, kEpiStore, true>(p, t, max_m_tiles, stream, s) : launch_shape<CMX_FMT_E5M2, kEpiStore, false>(p, t, max_m_tiles, stream, s);
+    if (fmt == CMX_FMT_E2M1 && epi == kEpiStore) return launch_shape<CMX_FMT_E2M1, kEpiStore, false>(p, t, max_m_tiles, stream, s);
+    if (fmt == kFmtI8 && epi == kEpiI8DequantSwiglu) return launch_shape<kFmtI8, kEpiI8DequantSwiglu, false>(p, t, max_m_tiles, stream, s);
+    set_error("unsupported split-K problem");
+    return CMX_EINVAL;
+}
+
+}  // namespace cmx

@@ -44,6 +44,7 @@ _HOOKS = {
     "cmx_debug_force_tile": (_C.c_int, [_C.c_int] * 3),
     "cmx_debug_disable_streaming": (_C.c_int, [_C.c_int]),
     "cmx_debug_pretiled_tile_rows": (_C.c_int, [_C.c_int]),
+    "cmx_debug_force_ksplit": (_C.c_int, [_C.c_int] * 3),
 }
 _test_lib = None
 
@@ -73,6 +74,7 @@ class hooked_library:
         self.lib.cmx_debug_force_tile(0, 0, 0)
         self.lib.cmx_debug_disable_streaming(0)
         self.lib.cmx_debug_pretiled_tile_rows(0)
+        self.lib.cmx_debug_force_ksplit(0, 0, 0)
         _lib.activate(self.prev)
         return False
 
