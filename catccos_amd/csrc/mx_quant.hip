@@ -12,6 +12,8 @@ namespace cmx {
 
 namespace {
 
+typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
+
 constexpr int kUnroll = 4;
 constexpr int kThreads = 256;
 constexpr int kBlocksPerIter = kThreads / 4;   // MX blocks handled per unroll step by one workgroup
@@ -147,37 +149,77 @@ __global__ __launch_bounds__(kThreads) void mx_quant_kernel(const uint16_t* __re
     }
 }
 
-// ---- fast path: RNE 8-bit formats, cols % 32 == 0, 16-byte aligned rows ------------------------
+// ---- fast path: RNE 8-bit formats and E2M1, cols % 32 == 0, 16-byte aligned rows ------------------------
 // Same lane split (four lanes per block, one 16-byte load each) but laid out so that no lane ever
 // divides: a workgroup owns 64 consecutive blocks of four consecutive rows, one row per unroll step.
 // The arithmetic stays on packed 16-bit integers until the final cast: amax and the clamp to
 // +-max_normal * 2^e work on sign-cleared bf16 bit patterns (unsigned order == magnitude order), and
-// v_cvt_scalef32_pk_{fp8,bf8}_bf16 divides by 2^e and rounds to nearest even in one instruction.
+// v_cvt_scalef32_pk_{fp8,bf8,fp4}_bf16 divides by 2^e and rounds to nearest even in one instruction.
 // Each lane of a quad then stores the scale byte of one of the four rows.
+// E2M1 (bound: HBM, 2.53 bytes per element; the general kernel above, which compares every element with seven thresholds
+// in fp32, is bound by the VALU: 65536 x 7168 365 us there, 234 us here, 192 us with streaming loads).
+// STREAM: inputs that do not stay in the memory-side cache anyway (256 MiB, which the codes and the consumer's operands
+// share) are read non-temporal and leave it to those: from 96 MiB of input on.  65536 x 7168 to E2M1 234 -> 192 us, 8192 x
+// 7168 to E4M3 followed by its matmul 203 -> 197 us together; 4096 x 7168 (56 MiB), whose input is still cached, 15.5
+// against 16.7 us.
 constexpr int kFastRows = 4;
+constexpr uint64_t kStreamBytes = 96ull << 20;
 
-template <int FMT>
-__global__ __launch_bounds__(kThreads) void mx_quant_rne8_kernel(const uint8_t* __restrict__ x, uint32_t ld_x_bytes,
+// E2M1 under table rounding: ties go to the smaller magnitude, where the hardware cast takes the even code.  The two differ at
+// 0.75, 1.75 and 3.5 (times 2^e) alone, whose lower neighbours have odd codes: bf16 mantissas 0x40 and 0x60.  Taking one unit in
+// the last place off EVERY magnitude with such a mantissa sends those three down and changes no other result: 1.5 * 2^k
+// and 1.75 * 2^k are never less than a unit above any other tie, nor codes' midpoints from above.
+__device__ __forceinline__ uint32_t e2m1_ties_down(uint32_t a) {
+    const uint32_t t = pk_min_u16((a & 0x005F005Fu) ^ 0x00400040u, 0x00010001u);      // 0: such a mantissa, 1: another
+    return __builtin_bit_cast(uint32_t, (v2u16)(__builtin_bit_cast(v2u16, a) + __builtin_bit_cast(v2u16, t) - (v2u16){1, 1}));
+}
+
+// eight codes of E2M1 from sign-cleared bf16 pairs and their signs; table rounding has no negative zero
+template <bool LUT>
+__device__ __forceinline__ uint32_t e2m1_pack8(const uint32_t (&a)[4], const uint32_t (&d)[4], float scale) {
+    uint32_t w = 0;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        const uint32_t c = (LUT ? e2m1_ties_down(a[i]) : a[i]) | (d[i] & 0x80008000u);
+        const v2bf16 v = __builtin_bit_cast(v2bf16, c);
+        if (i == 0) w = __builtin_amdgcn_cvt_scalef32_pk_fp4_bf16(w, v, scale, 0);
+        if (i == 1) w = __builtin_amdgcn_cvt_scalef32_pk_fp4_bf16(w, v, scale, 1);
+        if (i == 2) w = __builtin_amdgcn_cvt_scalef32_pk_fp4_bf16(w, v, scale, 2);
+        if (i == 3) w = __builtin_amdgcn_cvt_scalef32_pk_fp4_bf16(w, v, scale, 3);
+    }
+    if (LUT) w &= 0x77777777u | ((((w << 1) | (w << 2) | (w << 3)) & 0x88888888u));
+    return w;
+}
+
+template <int FMT, bool LUT, bool STREAM>
+__global__ __launch_bounds__(kThreads) void mx_quant_fast_kernel(const uint8_t* __restrict__ x, uint32_t ld_x_bytes,
                                                                  uint8_t* __restrict__ codes, uint32_t ld_codes,
                                                                  uint8_t* __restrict__ scales, uint32_t ld_scales,
                                                                  uint32_t rows, uint32_t nb) {
-    constexpr int emax = FMT == CMX_FMT_E4M3 ? kEmaxE4M3 : kEmaxE5M2;
-    constexpr uint32_t lim_mant = FMT == CMX_FMT_E4M3 ? 0x60u : 0x60u;   // 448 = 1.75 * 2^8, 57344 = 1.75 * 2^15
+    constexpr bool kFp4 = FMT == CMX_FMT_E2M1;
+    static_assert(kFp4 || !LUT, "8-bit formats: nearest even only");
+    constexpr int emax = FMT == CMX_FMT_E4M3 ? kEmaxE4M3 : (FMT == CMX_FMT_E5M2 ? kEmaxE5M2 : kEmaxE2M1);
+    // mantissa of the largest magnitude: 448 = 1.75 * 2^8, 57344 = 1.75 * 2^15, 6 = 1.5 * 2^2
+    constexpr uint32_t lim_mant = kFp4 ? 0x40u : 0x60u;
     const uint32_t q = threadIdx.x & 3u;
     const uint32_t kb = blockIdx.x * kBlocksPerIter + (threadIdx.x >> 2);
     const uint32_t row0 = blockIdx.y * kFastRows;
     if (kb >= nb) return;                                  // whole quads leave together
     const uint32_t in_off = kb * 64u + q * 16u;            // bytes inside the row
-    const uint32_t out_off = kb * 32u + q * 8u;
+    const uint32_t out_off = kFp4 ? kb * 16u + q * 4u : kb * 32u + q * 8u;
 
     uint4 raw[kFastRows];
 #pragma unroll
     for (int u = 0; u < kFastRows; ++u) {
         const uint32_t row = row0 + u;
         raw[u] = make_uint4(0, 0, 0, 0);
-        if (row < rows) raw[u] = *reinterpret_cast<const uint4*>(x + (size_t)row * ld_x_bytes + in_off);
+        if (row < rows) {
+            const u32x4* src = reinterpret_cast<const u32x4*>(x + (size_t)row * ld_x_bytes + in_off);
+            const u32x4 v = STREAM ? __builtin_nontemporal_load(src) : *src;
+            raw[u] = make_uint4(v[0], v[1], v[2], v[3]);
+        }
     }
-    int my_e = 0;
+    uint32_t my_scale = 0;
 #pragma unroll
     for (int u = 0; u < kFastRows; ++u) {
         const uint32_t row = row0 + u;
@@ -190,22 +232,42 @@ __global__ __launch_bounds__(kThreads) void mx_quant_rne8_kernel(const uint8_t* 
         m = pk_max_u16(m, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)m, 0x4E, 0xF, 0xF, true));
         const uint32_t amax = max(m & 0xFFFFu, m >> 16);
         const int e = block_exp_from_bf16_amax(amax, emax);
-        // clamp magnitudes to max_normal * 2^e (bit pattern: exponent e + emax + 127, mantissa 1.75)
+        // clamp magnitudes to max_normal * 2^e (bit pattern: exponent e + emax + 127, mantissa above)
         const uint32_t lim = (((uint32_t)(e + emax + 127) << 7) | lim_mant) * 0x10001u;
         const float scale = __uint_as_float((uint32_t)(e + 127) << 23);
-        uint32_t c[4];
+        uint32_t sbyte = (uint32_t)(e + 127);
+        uint8_t* const o = codes + (size_t)row * ld_codes + out_off;
 #pragma unroll
-        for (int i = 0; i < 4; ++i) c[i] = pk_min_u16(a[i], lim) | (d[i] & 0x80008000u);
-        uint32_t w0 = cvt_scaled_pk4<FMT>(c[0], c[1], scale);
-        uint32_t w1 = cvt_scaled_pk4<FMT>(c[2], c[3], scale);
-        if (amax >= 0x7F80u) patch_nonfinite_fp8<FMT, false>(d, w0, w1);      // Inf / NaN in the block (rare)
-        if (row < rows) *reinterpret_cast<uint2*>(codes + (size_t)row * ld_codes + out_off) = make_uint2(w0, w1);
-        my_e = (int)q == u ? e : my_e;
+        for (int i = 0; i < 4; ++i) a[i] = pk_min_u16(a[i], lim);
+        if constexpr (kFp4) {
+            uint32_t w = e2m1_pack8<LUT>(a, d, scale);
+            if (amax >= 0x7F80u) {                         // Inf / NaN in the block (rare): scale 254, or 255 and codes 0
+                sbyte = amax > 0x7F80u ? 255u : 254u;
+                w = 0;
+                if (amax == 0x7F80u) {
+#pragma unroll
+                    for (int i = 0; i < 4; ++i) {
+                        w |= fp4_encode<FMT>(clamp_abs(ldexpf(__uint_as_float(d[i] << 16), -127), 6.0f), LUT) << (8 * i);
+                        w |= fp4_encode<FMT>(clamp_abs(ldexpf(__uint_as_float(d[i] & 0xFFFF0000u), -127), 6.0f), LUT) << (8 * i + 4);
+                    }
+                }
+            }
+            if (row < rows) *reinterpret_cast<uint32_t*>(o) = w;
+        } else {
+            uint32_t c[4];
+#pragma unroll
+            for (int i = 0; i < 4; ++i) c[i] = a[i] | (d[i] & 0x80008000u);
+            uint32_t w0 = cvt_scaled_pk4<FMT>(c[0], c[1], scale);
+            uint32_t w1 = cvt_scaled_pk4<FMT>(c[2], c[3], scale);
+            if (amax >= 0x7F80u) patch_nonfinite_fp8<FMT, false>(d, w0, w1);      // Inf / NaN in the block (rare)
+            if (row < rows) *reinterpret_cast<uint2*>(o) = make_uint2(w0, w1);
+        }
+        my_scale = (int)q == u ? sbyte : my_scale;
     }
     const uint32_t srow = row0 + q;
     if (srow < rows) {
         uint8_t* sp = scales + (size_t)srow * ld_scales;
-        sp[kb] = (uint8_t)(my_e + 127);
+        sp[kb] = (uint8_t)my_scale;
         if (kb == nb - 1 && (nb & 1u) && ld_scales > nb) sp[nb] = 127;       // pad the scale row to an even count with 1.0
     }
 }
@@ -283,17 +345,21 @@ extern "C" int cmx_mx_quant(const void* x, uint32_t ld_x, uint8_t* codes, uint32
     hipStream_t s = static_cast<hipStream_t>(stream);
     const uint16_t* xp = static_cast<const uint16_t*>(x);
     const bool lut = round_mode == CMX_ROUND_LUT;
-    const bool fast = !lut && !fp4 && cols % 32 == 0 && vec_in && vec_out &&
+    const bool fast = (fmt == CMX_FMT_E2M1 || (!lut && !fp4)) && cols % 32 == 0 && vec_in && vec_out &&
                       (uint64_t)ld_x * 2 < (1ull << 32) && ceil_div(rows, kFastRows) <= 65535u;
     if (fast) {
         dim3 fgrid(ceil_div(nb, kBlocksPerIter), ceil_div(rows, kFastRows));
         const uint8_t* xb = static_cast<const uint8_t*>(x);
-        if (fmt == CMX_FMT_E4M3)
-            hipLaunchKernelGGL((mx_quant_rne8_kernel<CMX_FMT_E4M3>), fgrid, dim3(kThreads), 0, s, xb, ld_x * 2, codes, ld_codes,
-                               scales, ld_scales, rows, nb);
-        else
-            hipLaunchKernelGGL((mx_quant_rne8_kernel<CMX_FMT_E5M2>), fgrid, dim3(kThreads), 0, s, xb, ld_x * 2, codes, ld_codes,
-                               scales, ld_scales, rows, nb);
+        const auto launch = [&](auto kernel) {
+            hipLaunchKernelGGL(kernel, fgrid, dim3(kThreads), 0, s, xb, ld_x * 2, codes, ld_codes, scales, ld_scales, rows, nb);
+        };
+        const bool stream = (uint64_t)rows * cols * 2 >= kStreamBytes;
+#define CMX_FAST(FMT_, LUT_) (stream ? launch(mx_quant_fast_kernel<FMT_, LUT_, true>) : launch(mx_quant_fast_kernel<FMT_, LUT_, false>))
+        if (fmt == CMX_FMT_E4M3) CMX_FAST(CMX_FMT_E4M3, false);
+        else if (fmt == CMX_FMT_E5M2) CMX_FAST(CMX_FMT_E5M2, false);
+        else if (lut) CMX_FAST(CMX_FMT_E2M1, true);
+        else CMX_FAST(CMX_FMT_E2M1, false);
+#undef CMX_FAST
         CMX_LAUNCH_CHECK();
         return CMX_OK;
     }

@@ -154,3 +154,42 @@ def test_bad_arguments_are_rejected():
     assert lib.cmx_mx_quant(None, 64, c.data_ptr(), 64, s.data_ptr(), 2, 4, 64, 0, 0, None) == -1
     assert b"pitch" in lib.cmx_last_error() or b"null" in lib.cmx_last_error()
     assert lib.cmx_mx_quant(x.data_ptr(), 64, c.data_ptr(), 64, s.data_ptr(), 2, 0, 64, 0, 0, None) == 0   # empty
+
+
+@pytest.mark.parametrize("mode", ["lut", "rne"])
+@pytest.mark.parametrize("fmt", ["E2M1", "E5M2", "E4M3"])
+def test_every_mantissa_next_to_every_block_maximum(fmt, mode):
+    """Whole 32-blocks on aligned rows (the packed kernel where it applies): block b's largest magnitude has the bits
+    0x3F80 | (b & 127) at exponent b >> 7, the other elements walk all patterns from eight binades below it upwards, both
+    signs, so that every rounding tie of the element formats occurs; plus blocks below 1e-12, an Inf and a NaN block.  Bytes equal to the oracle's."""
+    from catccos_amd import ops
+    tops = (np.array([1, 60, 120, 127, 140, 250])[:, None] << 7 | np.arange(0, 128, 7)[None, :]).reshape(-1).astype(np.uint32)
+    rows = []
+    for t in tops:
+        lo = max(0, int(t) - 8 * 128)
+        body = np.arange(lo, int(t) + 1, dtype=np.uint32)
+        body = np.resize(body, -(-len(body) // 31) * 31).reshape(-1, 31)
+        blk = np.concatenate([np.full((len(body), 1), t), body], axis=1)
+        blk[:, 1::2] |= 0x8000
+        rows.append(blk)
+    rows += [np.array([[0x7F80] + [0x3F80 + i for i in range(31)], [0x7FC1] + [0x3F80] * 31, [0] * 16 + [0x8000] * 16, [0x2B8C] + [0x8001] * 31])]
+    x = np.concatenate(rows).astype(np.uint16)
+    x = np.resize(x, (-(-len(x) // 7) * 7, 32)).reshape(7, -1)                    # 7 rows: a last group of rows in part
+    q, s = ops.mx_quant(bf16_dev(x), fmt, mode)
+    wq, ws = O.mx_quant_bf16(x, fmt, mode)
+    assert np.array_equal(host(s), ws)
+    assert np.array_equal(host(q), O.pack_fp4(wq) if fmt == "E2M1" else wq)
+
+
+@pytest.mark.parametrize("fmt", ["E4M3", "E5M2", "E2M1"])
+def test_large_inputs_are_quantised_like_their_halves(fmt):
+    """Inputs of 96 MiB and more are read non-temporal (another instantiation): same bytes as the two halves, which are not."""
+    from catccos_amd import ops
+    g = torch.Generator(device="cuda")
+    g.manual_seed(7)
+    x = torch.randn((7023, 7168), generator=g, device="cuda").to(torch.bfloat16)
+    assert x.numel() * 2 >= 96 << 20
+    q, s = ops.mx_quant(x, fmt)
+    for part in (slice(0, 3500), slice(3500, 7023)):
+        hq, hs = ops.mx_quant(x[part], fmt)
+        assert torch.equal(q[part], hq) and torch.equal(s[part], hs)
