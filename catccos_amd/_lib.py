@@ -63,6 +63,7 @@ SIGNATURES = {
     "cmx_moe_init_routing": (i32, [i32p, u32, u32, u32, i32p, i32p, i32p, vp, vp]),
     "cmx_packed_row_bytes": (u32, [u32]),
     "cmx_quant_scatter": (i32, [vp, u32, i32p, u8p, u32, u8p, u32, u32, u32, u32, vp]),
+    "cmx_quant_scatter_zeroed": (i32, [vp, u32, i32p, u8p, u32, u8p, u32, u32, u32, u32, vp]),
     "cmx_moe_token_unpermute": (i32, [vp, u32, u32, i32p, f32p, vp, u32, u32, u32, u32, vp]),
     "catccos_ascend950_symmetric_bytes": (u64, []),
     "catccos_ascend950_dispatch_ffn_combine_workspace_bytes": (sz, [u32, u32, u32, u32, u32, i32]),

@@ -5,6 +5,8 @@
 // exactly the order of a stable sort) -> scatter, where each chunk is owned by one wavefront that
 // ranks equal keys in lane order with ballots, so the result is the unique stable permutation with
 // no global atomics and no dependence on scheduling.
+#include <algorithm>
+
 #include "mx_common.h"
 
 namespace cmx {
@@ -292,6 +294,48 @@ __global__ __launch_bounds__(256) void quant_scatter_row_kernel(const uint16_t* 
     }
 }
 
+// Zeros for the output rows that no route is sent to.  A workgroup owns `per` rows (a multiple of 32, at most
+// kUnmappedRows): it reads all destinations, marks those of its rows in an LDS bitmap and clears the rows left over.
+// Bound: the read of the destinations from the L2, by at most 256 workgroups (routes * 4 bytes each).  It stands in for
+// a fill of the whole output before the scatter: 32768 x 7168 bytes of codes 36 us, this kernel 5 us.
+constexpr uint32_t kUnmappedRows = 65536, kUnmappedThreads = 1024;
+
+__global__ __launch_bounds__(kUnmappedThreads) void zero_unmapped_rows_kernel(const int32_t* __restrict__ src2sorted,
+                                                                              uint8_t* __restrict__ out_codes, uint32_t ld_out,
+                                                                              uint8_t* __restrict__ out_scales, uint32_t ld_outs,
+                                                                              uint32_t rows, uint32_t per, uint32_t nvec,
+                                                                              uint32_t scols) {
+    __shared__ uint32_t s_map[kUnmappedRows / 32];
+    const uint32_t r0 = blockIdx.x * per, n = min(per, rows - r0), words = (n + 31) / 32;
+    for (uint32_t i = threadIdx.x; i < words; i += kUnmappedThreads) s_map[i] = 0;
+    __syncthreads();
+    for (uint32_t i0 = 0; i0 < rows; i0 += 8 * kUnmappedThreads) {                   // one route per row
+        int32_t d[8];
+#pragma unroll
+        for (uint32_t j = 0; j < 8; ++j) {
+            const uint32_t i = i0 + j * kUnmappedThreads + threadIdx.x;
+            d[j] = i < rows ? src2sorted[i] : -1;
+        }
+#pragma unroll
+        for (uint32_t j = 0; j < 8; ++j) {
+            const uint32_t r = (uint32_t)d[j] - r0;                                  // dropped routes are negative: far above n
+            if (d[j] >= 0 && r < n) atomicOr(&s_map[r / 32], 1u << (r % 32));
+        }
+    }
+    __syncthreads();
+    const uint32_t lane = threadIdx.x & 63u;
+    for (uint32_t w = threadIdx.x / 64; w < words; w += kUnmappedThreads / 64) {
+        uint32_t miss = ~s_map[w];
+        if (w == words - 1 && n % 32 != 0) miss &= (1u << (n % 32)) - 1u;
+        while (miss != 0) {
+            const size_t row = r0 + w * 32 + (uint32_t)__builtin_ctz(miss);
+            miss &= miss - 1;
+            for (uint32_t v = lane; v < nvec; v += 64) *reinterpret_cast<uint4*>(out_codes + row * ld_out + v * 16) = make_uint4(0, 0, 0, 0);
+            for (uint32_t c = lane; c < scols; c += 64) out_scales[row * ld_outs + c] = 0;
+        }
+    }
+}
+
 // ---- weighted top-k combine -----------------------------------------------------------------------
 typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
 __device__ __forceinline__ uint4 load_stream16(const void* p) {
@@ -565,6 +609,22 @@ extern "C" int cmx_quant_scatter(const void* x, uint32_t ld_x, const int32_t* sr
     else
         hipLaunchKernelGGL((quant_scatter_kernel<false>), grid, dim3(256), 0, s, xp, ld_x, src2sorted, out_codes, ld_out,
                            out_scales, ld_outs, tokens, k, top_k, nb, total);
+    CMX_LAUNCH_CHECK();
+    return CMX_OK;
+}
+
+extern "C" int cmx_quant_scatter_zeroed(const void* x, uint32_t ld_x, const int32_t* src2sorted, uint8_t* out_codes,
+                                        uint32_t ld_out, uint8_t* out_scales, uint32_t ld_outs, uint32_t tokens, uint32_t k,
+                                        uint32_t top_k, cmx_stream_t stream) {
+    using namespace cmx;
+    const uint64_t rows = (uint64_t)tokens * top_k;
+    CMX_REQUIRE(rows < (1ull << 31), "tokens * top_k must stay below 2^31 routes");
+    int rc = cmx_quant_scatter(x, ld_x, src2sorted, out_codes, ld_out, out_scales, ld_outs, tokens, k, top_k, stream);
+    if (rc != CMX_OK || rows == 0 || k == 0) return rc;
+    const uint32_t per = std::min(kUnmappedRows, round_up(ceil_div((uint32_t)rows, 256u), 32u));
+    hipLaunchKernelGGL(zero_unmapped_rows_kernel, dim3(ceil_div((uint32_t)rows, per)), dim3(kUnmappedThreads), 0,
+                       static_cast<hipStream_t>(stream), src2sorted, out_codes, ld_out, out_scales, ld_outs, (uint32_t)rows, per,
+                       k / 16, scale_cols(k));
     CMX_LAUNCH_CHECK();
     return CMX_OK;
 }

@@ -274,7 +274,7 @@ def moe_init_routing(expert_idx: torch.Tensor, experts: int):
 
 def quant_scatter(x: torch.Tensor, src2sorted: torch.Tensor, top_k: int, packed: bool = False, out=None):
     """x bf16 [T, k] -> rows quantised once and written to their top_k destinations.
-    packed=False: (codes [T*topK, k], scales [T*topK, RoundUp2(k/32)]);
+    packed=False: (codes [T*topK, k], scales [T*topK, RoundUp2(k/32)]), zeros in rows that no route is sent to;
     packed=True: one buffer [T*topK, packed_row_bytes(k)] = codes | scales | pad (``out``: a caller's zeroed buffer
     of that shape)."""
     _need_cuda(x, src2sorted)
@@ -288,9 +288,9 @@ def quant_scatter(x: torch.Tensor, src2sorted: torch.Tensor, top_k: int, packed:
         _lib.check(lib.cmx_quant_scatter(_p(x), x.stride(0), _p(src2sorted), _p(buf), rb, buf.data_ptr() + k, rb, t, k,
                                          top_k, _stream()))
         return buf
-    codes = torch.zeros((rows, k), dtype=torch.uint8, device=x.device)
-    scales = torch.zeros((rows, scale_cols(k)), dtype=torch.uint8, device=x.device)
-    _lib.check(lib.cmx_quant_scatter(_p(x), x.stride(0), _p(src2sorted), _p(codes), k, _p(scales), scales.shape[1], t, k,
+    codes = torch.empty((rows, k), dtype=torch.uint8, device=x.device)
+    scales = torch.empty((rows, scale_cols(k)), dtype=torch.uint8, device=x.device)
+    _lib.check(lib.cmx_quant_scatter_zeroed(_p(x), x.stride(0), _p(src2sorted), _p(codes), k, _p(scales), scales.shape[1], t, k,
                                      top_k, _stream()))
     return codes, scales
 

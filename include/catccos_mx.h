@@ -321,6 +321,12 @@ uint32_t cmx_packed_row_bytes(uint32_t k);
 int cmx_quant_scatter(const void* x, uint32_t ld_x, const int32_t* src2sorted, uint8_t* out_codes, uint32_t ld_out,
                       uint8_t* out_scales, uint32_t ld_outs, uint32_t tokens, uint32_t k, uint32_t top_k,
                       cmx_stream_t stream);
+/* cmx_quant_scatter, after which the rows of out_codes (k bytes) and out_scales (RoundUp2(k/32) bytes) among the first
+ * tokens*top_k that no route is sent to hold zeros: what clearing both arrays beforehand gives, without the pass over
+ * them.  Destinations must be below tokens*top_k; tokens*top_k < 2^31. */
+int cmx_quant_scatter_zeroed(const void* x, uint32_t ld_x, const int32_t* src2sorted, uint8_t* out_codes, uint32_t ld_out,
+                             uint8_t* out_scales, uint32_t ld_outs, uint32_t tokens, uint32_t k, uint32_t top_k,
+                             cmx_stream_t stream);
 
 /* ------------------------------------------------------------------------------------------
  * Weighted top-k combine.  Replaces KernelMoeTokenUnpermute<bf16,int32,float,true>

@@ -143,3 +143,28 @@ def test_combine_ignores_out_of_range_rows():
     p = np.random.default_rng(3).random((4, 3)).astype(np.float32)
     out = host(ops.moe_token_unpermute(bf16_dev(y), dev(inv), dev(p)))
     assert np.array_equal(out, O.unpermute_combine(y, inv, p))
+
+
+@pytest.mark.parametrize("tokens,k,top_k", [(1, 32, 1), (40, 96, 3), (300, 512, 4), (9001, 64, 8)])
+@pytest.mark.parametrize("kept", [0.0, 0.5, 0.999, 1.0])
+def test_rows_without_a_route_are_zeros(tokens, k, top_k, kept):
+    """Routes dropped at random: the rows of the others as without drops, zeros elsewhere, in memory that held other values.
+    72008 rows: blocks of 288 rows, the last in part."""
+    from catccos_amd import ops
+    g = torch.Generator(device="cuda")
+    g.manual_seed(tokens + k)
+    rows = tokens * top_k
+    x = torch.randn((tokens, k), generator=g, device="cuda").to(torch.bfloat16)
+    dest = torch.randperm(rows, generator=g, device="cuda").to(torch.int32)
+    keep = torch.rand(rows, generator=g, device="cuda") < kept
+    full_codes, full_scales = ops.quant_scatter(x, dest, top_k)
+    reached = torch.zeros(rows, dtype=torch.bool, device="cuda")
+    reached[dest[keep].long()] = True
+    want_codes, want_scales = full_codes * reached[:, None], full_scales * reached[:, None]
+    poison = [torch.full_like(t, 171) for t in (full_codes, full_scales)]
+    del full_codes, full_scales, poison
+    codes, scales = ops.quant_scatter(x, torch.where(keep, dest, torch.full_like(dest, -1)), top_k)
+    assert torch.equal(codes, want_codes) and torch.equal(scales, want_scales)
+    wq, ws = O.mx_quant_bf16(host(x), "E4M3", "rne")
+    codes, scales = ops.quant_scatter(x, dest, top_k)
+    assert np.array_equal(host(codes)[host(dest)], np.repeat(wq, top_k, 0)) and np.array_equal(host(scales)[host(dest)], np.repeat(ws, top_k, 0))
