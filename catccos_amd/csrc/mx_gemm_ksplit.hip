@@ -212,17 +212,23 @@ __device__ __forceinline__ void ks_tile(const GemmParams& p, const Tile& tc, uin
         return t < (uint32_t)TW ? p.w_scale + ((size_t)tc.g * p.n + wrow_of(t)) * p.ld_ws
                                 : p.a_scale + (size_t)(tc.row0 + arow_of(t - TW)) * p.ld_as;
     };
-    // 16-byte pieces when the rows allow it, numbered with the next power of two of pieces per row (no division)
+    // Whole 16-byte pieces, numbered with the next power of two of pieces per row (no division), and behind them the up to
+    // 15 bytes of a row that is no whole number of pieces as four dwords (none reaches past the row: the last is read from its
+    // last four bytes and shifted; a last slab in part is filled up with 1.0).  Rows start at any byte (the pitch of 30 scales is 30): the pieces are read by unaligned loads.  All of it is
+    // requested before the operands and deposited behind their requests: one trip to memory.  (A dword at a time, each
+    // waited for, it was most of the kernel where K is no multiple of 512: see the rule's comment in mx_gemm.hip.)
     constexpr int kBatch = 2048 / NT;                  // pieces per thread in flight together: 32 KiB per workgroup
-    const bool sc16 = kS && p.scale_vec16 && p.kblocks % 16 == 0;
+    constexpr int kTail = (kRows * 4 + NT - 1) / NT;
     const uint32_t pieces = p.kblocks / 16, shift = pieces > 1 ? 32 - __builtin_clz(pieces - 1) : 0;
     const uint32_t total16 = kRows << shift;
+    const bool ragged = p.kblocks % 16 != 0;
     u32x4 sreg[kBatch];
+    uint32_t treg[kTail];
     auto request16 = [&](uint32_t i0) {
 #pragma unroll
         for (int b = 0; b < kBatch; ++b) {
             const uint32_t i = i0 + b * NT + tid, t = i >> shift, q = i & ((1u << shift) - 1);
-            if (i < total16 && q < pieces) sreg[b] = *reinterpret_cast<const u32x4*>(scale_row(t) + q * 16);
+            if (i < total16 && q < pieces) __builtin_memcpy(&sreg[b], scale_row(t) + q * 16, 16);
         }
     };
     auto deposit16 = [&](uint32_t i0) {
@@ -236,7 +242,16 @@ __device__ __forceinline__ void ks_tile(const GemmParams& p, const Tile& tc, uin
             }
         }
     };
-    if (sc16) request16(0);
+    if constexpr (kS != 0) {
+        request16(0);
+        if (ragged && p.kblocks >= 4) {
+#pragma unroll
+            for (int b = 0; b < kTail; ++b) {
+                const uint32_t i = b * NT + tid, at = 16 * pieces + 4 * (i & 3u);
+                if (i < kRows * 4) __builtin_memcpy(&treg[b], scale_row(i >> 2) + min(at, p.kblocks - 4), 4);
+            }
+        }
+    }
 
     // ---- operand streams ---------------------------------------------------------------------------------------------
     constexpr int kRsrcFlags = 0x00020000;
@@ -309,28 +324,27 @@ __device__ __forceinline__ void ks_tile(const GemmParams& p, const Tile& tc, uin
 
     // ---- scales of the tile: deposit -----------------------------------------------------------------------------------
     if constexpr (kS != 0) {
-        if (sc16) {
-            deposit16(0);
-            for (uint32_t i0 = kBatch * NT; i0 < total16; i0 += kBatch * NT) {
-                request16(i0);
-                deposit16(i0);
-            }
-        } else {
-            // dword by dword; a last slab in part is filled up with 1.0
-            const uint32_t sh = 32 - __builtin_clz(pitch - 1 | 1u);
-            for (uint32_t i = tid; i < ((uint32_t)kRows << sh); i += NT) {
-                const uint32_t t = i >> sh, q = i & ((1u << sh) - 1);
-                if (q >= pitch) continue;
-                const uint8_t* row = scale_row(t);
+        deposit16(0);
+        if (ragged) {
+#pragma unroll
+            for (int b = 0; b < kTail; ++b) {
+                const uint32_t i = b * NT + tid, q = 4 * pieces + (i & 3u);
+                if (i >= kRows * 4 || q >= pitch) continue;
                 uint32_t v = 0x7F7F7F7Fu;
-                if (p.scale_vec && 4 * q + 4 <= p.kblocks) {
-                    v = *reinterpret_cast<const uint32_t*>(row + 4 * q);
+                if (p.kblocks >= 4) {
+                    const uint32_t past = 4 * q - min(4 * q, p.kblocks - 4);          // bytes of the dword past the row
+                    if (past == 0) v = treg[b];
+                    else if (past < 4) v = (treg[b] >> (8 * past)) | (v << (32 - 8 * past));
                 } else {
-                    for (uint32_t b = 0; b < 4; ++b)
-                        if (4 * q + b < p.kblocks) v = (v & ~(0xFFu << (8 * b))) | ((uint32_t)row[4 * q + b] << (8 * b));
+                    const uint8_t* row = scale_row(i >> 2);
+                    for (uint32_t e = 0; 4 * q + e < p.kblocks; ++e) v = (v & ~(0xFFu << (8 * e))) | ((uint32_t)row[e] << (8 * e));
                 }
-                s_sc[t * pitch + q] = v;
+                s_sc[(i >> 2) * pitch + q] = v;
             }
+        }
+        for (uint32_t i0 = kBatch * NT; i0 < total16; i0 += kBatch * NT) {
+            request16(i0);
+            deposit16(i0);
         }
         __syncthreads();
     }

@@ -129,3 +129,33 @@ def test_grouped_int8(counts, out):
     # and the oracle twice (fp32, then fp16): they differ at exact ties
     gold = Q.gmm_dequant_swiglu(a, ts, b, ch, counts)
     assert np.allclose(got.float().cpu().numpy(), gold, rtol=2.0 ** -9 if out == "fp32" else 1e-2, atol=1e-6 if out == "fp32" else 1e-3)
+
+
+@pytest.mark.parametrize("shape", [(1, 1, 8), (4, 4, 8), (4, 4, 4)])
+@pytest.mark.parametrize("fmt,k", [("E4M3", 1952), ("E4M3", 8736), ("E2M1", 1952), ("E5M2", 496 * 32)])
+def test_scale_rows_at_any_byte_give_the_bits_of_aligned_ones(shape, fmt, k):
+    """61 scales (three 16-byte pieces and a tail of 13 bytes), 273 (more pieces than are in flight together, a tail of one)
+    and 496 (whole pieces) in rows of an odd pitch that start at an odd address: the result of the same scales in aligned
+    rows, and the oracle's."""
+    from catccos_amd import _lib, ops
+    hooks_lib().cmx_debug_force_ksplit(*shape)
+    rng = np.random.default_rng(k)
+    m, n, nb = 37, 45, k // 32
+    aq, asc = _mx(rng, m, k, fmt)
+    bq, bsc = _mx(rng, n, k, fmt)
+    pack = O.pack_fp4 if fmt == "E2M1" else (lambda x: x)
+    a, b, pitch = dev(pack(aq)), dev(pack(bq)), nb | 1
+    want = ops.mx_gemm(a, dev(asc), b, dev(bsc), k, fmt, "fp32")
+
+    def shifted(s):
+        buf = torch.full((1 + s.shape[0] * pitch,), 200, dtype=torch.uint8, device="cuda")
+        buf[1:].view(s.shape[0], pitch)[:, :nb] = dev(s)[:, :nb]
+        return buf[1:]
+    sa, sb, got = shifted(asc), shifted(bsc), torch.empty_like(want)
+    lib = _lib.load()
+    _lib.check(lib.cmx_mx_gemm(a.data_ptr(), a.shape[1], sa.data_ptr(), pitch, b.data_ptr(), b.shape[1], sb.data_ptr(), pitch, got.data_ptr(),
+                               n, m, n, k, ops.FMT[fmt], ops.OUT["fp32"], torch.cuda.current_stream().cuda_stream))
+    assert torch.equal(got, want)
+    gold = O.mx_dequant(aq, asc, fmt).astype(np.float64) @ O.mx_dequant(bq, bsc, fmt).astype(np.float64).T
+    bad, worst = close_bf16(host(got.to(torch.bfloat16)), gold)
+    assert bad == 0, (bad, worst)
