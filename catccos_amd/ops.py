@@ -19,7 +19,8 @@ _OUT_DTYPE = {"bf16": torch.bfloat16, "fp16": torch.float16, "fp32": torch.float
 
 
 def _stream():
-    return torch.cuda.current_stream().cuda_stream
+    # the handle of torch's current stream without a Stream object around it: 0.3 us of host time against 2.8, of 10 a call
+    return torch._C._cuda_getCurrentRawStream(torch.cuda.current_device())
 
 
 def _p(t: torch.Tensor):
