@@ -1005,13 +1005,30 @@ KsplitTile g_force_ksplit = {0, 0, 0};
 constexpr KsplitTile g_force_ksplit = {0, 0, 0};
 #endif
 
+// Dense 8-bit problems that 128 x 128 tiles of four wavefronts (mx_gemm_kernel) take: too many 64 x 64 tiles for the split-K
+// kernel to run in two rounds of a workgroup per CU, few enough 128 x 128 tiles for one, and K up to 2048: a tile of twice the
+// side pulls half the bytes per product through the vector cache, while a long K is better split between more wavefronts.
+// Measured (us, E4M3, 64 x 64 split-K -> 128 x 128): 1024 x 4096 at K = 512 12.4 -> 10.0, 1024 15.8 -> 12.2, 2048 22.3 -> 17.1,
+// 4096 33.8 against 33.1, 7168 55.2 against 52.2 (behind the pass that writes its weights, 62 against 64); 760 x 3072 x 2048 (576
+// 64 x 64 tiles) 18.7 -> 15.8, 640 x 4096 x 4096 (640) 28.4 against 33.0.
+bool takes_128_tile(uint32_t m, uint32_t n, int fmt, uint32_t kblocks, int cus) {
+    if (fmt == CMX_FMT_E2M1 || kblocks % 4 != 0 || kblocks > 64) return false;
+    const uint64_t t64 = (uint64_t)ceil_div(n, 64) * ceil_div(m, 64), t128 = (uint64_t)ceil_div(n, 128) * ceil_div(m, 128);
+    return t128 <= (uint64_t)cus && t64 > 2 * (uint64_t)cus;
+}
+
 // Whether a problem goes to the split-K kernels (mx_gemm_ksplit.hip), and with which tile; fw == 0: no.  The choice depends
 // on sizes and element format only, so that every layout, pitch and output type of a problem gets the same sums.
 // Dense: the smallest tile that still leaves every CU at most one workgroup (time goes with the bytes a workgroup pulls
 // through its vector cache, and a second round costs as much as the first); past that 64 x 64 tiles, two workgroups of
 // four wavefronts on a CU, up to 1024 tiles.  Measured (us, E4M3, before = 256-row tiles): 16 x 4096 x 7168 44.7 -> 9.0,
-// 64 x 4096 x 7168 49.2 -> 10.8, 256 x 4096 x 7168 62.5 -> 18.0, 512 x 4096 x 7168 62.5 -> 28.1, 1024 x 4096 x 7168 (1024 tiles)
-// 63.0 -> 51.9, 2048 x 4096 x 7168 (2048 tiles) 63.4 against 99.3; 1000 x 1000 x 960 (no whole scale blocks) 37.6 -> 9.0.
+// 64 x 4096 x 7168 49.2 -> 10.8, 256 x 4096 x 7168 62.5 -> 18.0, 512 x 4096 x 7168 62.5 -> 28.1, 640 x 4096 x 4096 (640
+// tiles) 38.7 -> 28.4, 2048 x 4096 x 7168 (2048 tiles) 63.4 against 99.3; 1000 x 1000 x 960 37.6 -> 7.7.  Scale rows that are no
+// whole 16-byte pieces or not aligned to them cost next to nothing (700 x 3000 x 1984, 62 scales a row: 36.0 with a dword
+// of scales at a time, 19.8 with pieces).
+// 8-bit problems whose K is no whole number of slabs are left to the register-staged 256-row kernel, slower by two to four
+// times than the streaming ones, so they stay here up to 2048 tiles (us, 256-row -> here): 2048 x 4096 x 6976 240 -> 117, 1536 x
+// 4096 x 3040 75 -> 47; 3000 x 5000 x 4064 (3713 tiles) 97 against 138, 8192 x 4096 x 7136 300 against 463.
 // Grouped: groups that average few rows stream their weights once whatever the tile; 64 x 64 tiles of four wavefronts
 // keep more of the stream in flight than the 256-row tiles (32 experts, K = 7168, N = 4096, GMM1, us): 4 rows per expert
 // 184 -> 142, 32 rows 189 -> 172, 64 rows 198 against 242; FP4 16 rows 113 -> 95, 64 rows 170 -> 140, 128 rows 202 against
@@ -1035,7 +1052,8 @@ int choose_ksplit(uint32_t m_hint, uint32_t n, int fmt, uint32_t kblocks, bool g
             return CMX_OK;
         }
     const KsplitTile t = {4, 4, 4};
-    if (tiles(t) <= 4 * (uint64_t)cus && fits(t)) *out = t;
+    const uint64_t per_cu = fmt != CMX_FMT_E2M1 && kblocks % 4 != 0 ? 8 : 4;
+    if (tiles(t) <= per_cu * cus && !takes_128_tile(m_hint, n, fmt, kblocks, cus) && fits(t)) *out = t;
     return CMX_OK;
 }
 
@@ -1213,7 +1231,10 @@ extern "C" int cmx_mx_gemm(const uint8_t* a, uint32_t lda, const uint8_t* a_scal
         p.w_tiles = ceil_div(n, 16 * ks.fw);
         return launch_ksplit(p, ks, fmt, kEpiStore, ceil_div(m, 16 * ks.fm), false, s);
     }
+    int cus = 0;
+    if (rc = cu_count(&cus); rc != CMX_OK) return rc;
     TileChoice t = choose_tile(m, n, fmt, false);
+    if (!g_force_tile.tw && !g_disable_dl && takes_128_tile(m, n, fmt, p.kblocks, cus)) t = {128, 128, 4};
     p.w_tiles = ceil_div(n, t.tw);
     const uint32_t m_tiles = ceil_div(m, t.tm);
     switch (fmt) {

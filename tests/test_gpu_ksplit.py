@@ -159,3 +159,16 @@ def test_scale_rows_at_any_byte_give_the_bits_of_aligned_ones(shape, fmt, k):
     gold = O.mx_dequant(aq, asc, fmt).astype(np.float64) @ O.mx_dequant(bq, bsc, fmt).astype(np.float64).T
     bad, worst = close_bf16(host(got.to(torch.bfloat16)), gold)
     assert bad == 0, (bad, worst)
+
+
+@pytest.mark.parametrize("m,n,k", [(1000, 4000, 512), (1024, 4104, 512), (1024, 4096, 2048), (1024, 4096, 2176), (2048, 4096, 96), (2049, 4096, 96), (520, 4000, 256)])
+def test_sizes_on_both_sides_of_the_dense_rules(m, n, k):
+    """256 and more 128 x 128 tiles; more than 2048 64 x 64 tiles where K is no whole number of slabs; the kernel that the
+    library chooses against the oracle."""
+    from catccos_amd import ops
+    rng = np.random.default_rng(m + n + k)
+    aq, asc = _mx(rng, m, k, "E4M3")
+    bq, bsc = _mx(rng, n, k, "E4M3")
+    gold = (O.mx_dequant(aq, asc).astype(np.float32) @ O.mx_dequant(bq, bsc).astype(np.float32).T)
+    bad, worst = close_bf16(host(ops.mx_gemm(dev(aq), dev(asc), dev(bq), dev(bsc), k)), gold)
+    assert bad == 0, (bad, worst)
