@@ -197,8 +197,8 @@ __device__ __forceinline__ void epilogue(const GemmParams& p, const Tile& tc, v1
 #pragma unroll
                     for (int i = 0; i < 4; ++i) {
                         const int r = 4 * q + i;
-                        const float x0 = __fmul_rn((float)(_Float16)__fmul_rn((float)ig[r], cg[i]), tsv);
-                        const float gate = __fmul_rn((float)(_Float16)__fmul_rn((float)iu[r], cu[i]), tsv);
+                        const float x0 = __fmul_rn(i8_dequant(ig[r], cg[i]), tsv);
+                        const float gate = __fmul_rn(i8_dequant(iu[r], cu[i]), tsv);
                         y[i] = __fmul_rn(__fmul_rn(x0, __builtin_amdgcn_rcpf(1.0f + __expf(-x0))), gate);
                     }
                     if (p.out_type == CMX_OUT_FP32) {
@@ -212,7 +212,7 @@ __device__ __forceinline__ void epilogue(const GemmParams& p, const Tile& tc, v1
                         uint16_t h[4];
 #pragma unroll
                         for (int i = 0; i < 4; ++i)
-                            h[i] = p.out_type == CMX_OUT_FP16 ? __builtin_bit_cast(uint16_t, (_Float16)y[i]) : (uint16_t)f32_to_bf16(y[i]);
+                            h[i] = p.out_type == CMX_OUT_FP16 ? __builtin_bit_cast(uint16_t, (_Float16)as_f32(y[i])) : (uint16_t)f32_to_bf16(y[i]);
                         uint16_t* o = reinterpret_cast<uint16_t*>(p.c) + mrow * p.ldc + ncol;
                         if (whole) {
                             *reinterpret_cast<uint2*>(o) = make_uint2(h[0] | ((uint32_t)h[1] << 16), h[2] | ((uint32_t)h[3] << 16));

@@ -64,6 +64,20 @@ __device__ __forceinline__ float silu_mul(float g, float u) {
     return (g * s) * u;
 }
 
+// v as the fp32 value it is written as.  (_Float16)(a * b) becomes one v_fma_mixlo_f16, which rounds the product to fp16
+// once, also where the product is written __fmul_rn: a whole fp16 step away from the two roundings where the fp32 product is
+// a tie between two fp16 values.  The empty asm makes the product a register of its own.
+__device__ __forceinline__ float as_f32(float v) {
+    asm("" : "+v"(v));
+    return v;
+}
+
+// INT8 path: fp16(fp32(sum) * channel scale), the two roundings of the reference's arithmetic
+// (examples/utils/gen_data_dispatch_gmm_dequant_swiglu.py:291-320), as fp32
+__device__ __forceinline__ float i8_dequant(int32_t sum, float channel_scale) {
+    return (float)(_Float16)as_f32(__fmul_rn((float)sum, channel_scale));
+}
+
 struct Tile {
     uint32_t g, mt, wt, row0, rows_valid;
 };

@@ -118,8 +118,8 @@ __device__ __forceinline__ void ks_store(const GemmParams& p, const Tile& tc, ui
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
             const float cg = ch[(size_t)(ncol + i) * p.ld_ws], cu = ch[(size_t)(half + ncol + i) * p.ld_ws];
-            const float x0 = __fmul_rn((float)(_Float16)__fmul_rn((float)ig[i], cg), tsv);
-            const float gate = __fmul_rn((float)(_Float16)__fmul_rn((float)iu[i], cu), tsv);
+            const float x0 = __fmul_rn(i8_dequant(ig[i], cg), tsv);
+            const float gate = __fmul_rn(i8_dequant(iu[i], cu), tsv);
             y[i] = __fmul_rn(__fmul_rn(x0, __builtin_amdgcn_rcpf(1.0f + __expf(-x0))), gate);
         }
         if (p.out_type == CMX_OUT_FP32) {
@@ -133,7 +133,7 @@ __device__ __forceinline__ void ks_store(const GemmParams& p, const Tile& tc, ui
             uint16_t h[4];
 #pragma unroll
             for (int i = 0; i < 4; ++i)
-                h[i] = p.out_type == CMX_OUT_FP16 ? __builtin_bit_cast(uint16_t, (_Float16)y[i]) : (uint16_t)f32_to_bf16(y[i]);
+                h[i] = p.out_type == CMX_OUT_FP16 ? __builtin_bit_cast(uint16_t, (_Float16)as_f32(y[i])) : (uint16_t)f32_to_bf16(y[i]);
             uint16_t* o = reinterpret_cast<uint16_t*>(p.c) + mrow * p.ldc + ncol;
             if ((reinterpret_cast<uintptr_t>(o) & 7u) == 0) {
                 *reinterpret_cast<uint2*>(o) = make_uint2(h[0] | ((uint32_t)h[1] << 16), h[2] | ((uint32_t)h[3] << 16));

@@ -95,6 +95,42 @@ def test_int32_sums_are_exact():
     assert np.array_equal(out[c[:, :32] == 0], np.zeros(np.count_nonzero(c[:, :32] == 0), dtype=np.float32))
 
 
+def _tie_products(rng, count):
+    """(whole numbers 1..127, fp32 scales) whose product rounds to fp32 exactly between two fp16 values without being there, and whose
+    two roundings (fp32, then fp16) give another fp16 value than one would."""
+    c, s = [], []
+    while len(c) < count:
+        i = rng.integers(3, 128, size=200000)
+        tie = (2048 + 2 * rng.integers(0, 1024, size=i.size) + 1).astype(np.float64) * 2.0 ** -12      # 11 bits and a half
+        f = (tie / i).astype(np.float32)
+        exact = i.astype(np.float64) * f                                                                # 7 + 24 bits: exact
+        hit = np.flatnonzero(exact.astype(np.float32).astype(np.float16) != exact.astype(np.float16))
+        c += list(i[hit])
+        s += list(f[hit])
+    return np.array(c[:count], dtype=np.int8), np.array(s[:count], dtype=np.float32)
+
+
+@pytest.mark.parametrize("rows", [1, 4, 300])           # the split-K kernel's smallest tiles, and the 256-row kernel
+@pytest.mark.parametrize("out", ["fp32", "fp16"])
+def test_products_that_round_to_a_tie_are_rounded_twice(rows, out):
+    """Every gate and up value is such a product: fp16(fp32(c * scale)) is a whole step (2^-10) from fp16(c * scale)."""
+    from catccos_amd import ops
+    n, k = 256, 128
+    c, ch = _tie_products(np.random.default_rng(rows), n)
+    a = np.zeros((rows, k), dtype=np.int8)
+    a[:, 3] = 1
+    b = np.zeros((1, k, n), dtype=np.int8)
+    b[0, 3] = c
+    ts = np.ones(rows, dtype=np.float32)
+    gold = Q.gmm_dequant_swiglu(a, ts, b, ch, [rows])
+    once = (c.astype(np.float64) * ch).astype(np.float16)
+    assert np.all(np.abs(once.astype(np.float64) / (c.astype(np.float32) * ch).astype(np.float16) - 1) > 2.0 ** -12)
+    got = host(ops.int8_gmm_dequant_swiglu(dev(a), dev(ts), dev(b), dev(ch), dev(np.array([rows], dtype=np.int32)), n, k, 0, out))
+    # fp32: the sigmoid's few ulp.  fp16: half a step of the result, and those ulp where they cross a tie
+    rtol = 1e-5 if out == "fp32" else 2.0 ** -11 + 1e-5
+    assert np.allclose(got.astype(np.float32), gold, rtol=rtol, atol=0), np.abs(got / gold - 1).max()
+
+
 def test_bad_arguments():
     from catccos_amd import _lib
     lib = _lib.load()

@@ -125,10 +125,9 @@ def test_grouped_int8(counts, out):
     hooks_lib().cmx_debug_force_ksplit(0, 0, 0)
     hooks_lib().cmx_debug_force_tile(256, 256, 8)
     assert torch.equal(got, ops.int8_gmm_dequant_swiglu(*args))
-    # and the oracle's values up to one step of the fp16 intermediate (2^-10), which the device rounds once from the product
-    # and the oracle twice (fp32, then fp16): they differ at exact ties
+    # and the oracle's: INT32 sums and the fp16 step are exact, the sigmoid is within a few ulp
     gold = Q.gmm_dequant_swiglu(a, ts, b, ch, counts)
-    assert np.allclose(got.float().cpu().numpy(), gold, rtol=2.0 ** -9 if out == "fp32" else 1e-2, atol=1e-6 if out == "fp32" else 1e-3)
+    assert np.allclose(got.float().cpu().numpy(), gold, rtol=1e-5 if out == "fp32" else 1e-2, atol=1e-7 if out == "fp32" else 1e-3)
 
 
 @pytest.mark.parametrize("shape", [(1, 1, 8), (4, 4, 8), (4, 4, 4)])
