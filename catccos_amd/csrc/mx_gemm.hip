@@ -810,11 +810,13 @@ __global__ __launch_bounds__(64 * WW * WM) void mx_gemm_dl_kernel(const GemmPara
 // groups; the 256 partial sums are scanned in LDS, first for the rows, then for the m-tiles.
 // Group sizes live on the device, so the host cannot check them: negative sizes count as zero and rows past
 // m_total (the rows the caller's buffers hold) are cut off here, so that no tile ever points outside them.
+// small_rows != 0: groups of 1 .. small_rows rows are one m-tile each of small_pref and none of tile_pref.
 __global__ __launch_bounds__(256) void gmm_prepare_kernel(const int32_t* __restrict__ sizes, uint32_t groups, uint32_t tile_m,
-                                                           uint32_t m_total, int32_t* __restrict__ row_off,
-                                                           int32_t* __restrict__ tile_pref, int32_t* __restrict__ tile_ctr) {
+                                                           uint32_t m_total, uint32_t small_rows, int32_t* __restrict__ row_off,
+                                                           int32_t* __restrict__ tile_pref, int32_t* __restrict__ small_pref,
+                                                           int32_t* __restrict__ tile_ctr) {
     __shared__ unsigned long long part_r[256];
-    __shared__ int32_t part_t[256];
+    __shared__ int32_t part_t[256], part_s[256];
     if (threadIdx.x < kXcds) tile_ctr[threadIdx.x] = 0;
     const uint32_t per = (groups + 255) / 256;
     const uint32_t lo = threadIdx.x * per < groups ? threadIdx.x * per : groups;
@@ -853,29 +855,39 @@ __global__ __launch_bounds__(256) void gmm_prepare_kernel(const int32_t* __restr
         const unsigned long long e = before + c < m_total ? before + c : m_total;
         return (uint32_t)(e - b);
     };
+    auto is_small = [&](uint32_t rows) -> bool { return rows != 0 && rows <= small_rows; };
     r = r_base;
-    int32_t t = 0;
+    int32_t t = 0, sm = 0;
     for (uint32_t i = lo; i < hi; ++i) {
         const unsigned long long c = size_of(i);
-        t += (int32_t)((clipped(r, c) + tile_m - 1) / tile_m);
+        const uint32_t rows = clipped(r, c);
+        if (is_small(rows)) ++sm;
+        else t += (int32_t)((rows + tile_m - 1) / tile_m);
         r += c;
     }
     part_t[threadIdx.x] = t;
+    part_s[threadIdx.x] = sm;
     __syncthreads();
     scan256(part_t);
+    if (small_rows != 0) scan256(part_s);
     r = r_base;
     t = threadIdx.x ? part_t[threadIdx.x - 1] : 0;
+    sm = threadIdx.x ? part_s[threadIdx.x - 1] : 0;
     for (uint32_t i = lo; i < hi; ++i) {
         const unsigned long long c = size_of(i);
+        const uint32_t rows = clipped(r, c);
         row_off[i] = (int32_t)(r < m_total ? r : m_total);
         tile_pref[i] = t;
-        t += (int32_t)((clipped(r, c) + tile_m - 1) / tile_m);
+        if (small_rows != 0) small_pref[i] = sm;
+        if (is_small(rows)) ++sm;
+        else t += (int32_t)((rows + tile_m - 1) / tile_m);
         r += c;
     }
     if (threadIdx.x == 255) {
         const unsigned long long all = part_r[255];
         row_off[groups] = (int32_t)(all < m_total ? all : m_total);
         tile_pref[groups] = part_t[255];
+        if (small_rows != 0) small_pref[groups] = part_s[255];
     }
 }
 
@@ -1029,22 +1041,13 @@ bool takes_128_tile(uint32_t m, uint32_t n, int fmt, uint32_t kblocks, int cus) 
 // 8-bit problems whose K is no whole number of slabs are left to the register-staged 256-row kernel, slower by two to four
 // times than the streaming ones, so they stay here up to 2048 tiles (us, 256-row -> here): 2048 x 4096 x 6976 240 -> 117, 1536 x
 // 4096 x 3040 75 -> 47; 3000 x 5000 x 4064 (3713 tiles) 97 against 138, 8192 x 4096 x 7136 300 against 463.
-// Grouped: groups that average few rows stream their weights once whatever the tile; 64 x 64 tiles of four wavefronts
-// keep more of the stream in flight than the 256-row tiles (32 experts, K = 7168, N = 4096, GMM1, us): 4 rows per expert
-// 184 -> 142, 32 rows 189 -> 172, 64 rows 198 against 242; FP4 16 rows 113 -> 95, 64 rows 170 -> 140, 128 rows 202 against
-// 200; INT8 4 rows 223 -> 130, 32 rows 239 -> 171, 64 rows 235 against 237.
-int choose_ksplit(uint32_t m_hint, uint32_t n, int fmt, uint32_t kblocks, bool grouped, KsplitTile* out) {
+int choose_ksplit(uint32_t m, uint32_t n, int fmt, uint32_t kblocks, KsplitTile* out) {
     *out = g_force_ksplit;
-    if (out->fw != 0 || g_force_tile.tw != 0 || g_pretiled_tile_rows != 0 || g_disable_dl) return CMX_OK;
+    if (out->fw != 0 || g_force_tile.tw != 0 || g_disable_dl) return CMX_OK;
     const auto fits = [&](const KsplitTile& t) { return ksplit_lds_bytes(t, fmt, kblocks, false) <= kKsplitMaxLds; };
-    if (grouped) {
-        const KsplitTile t = {4, 4, 4};
-        if (m_hint <= (fmt == CMX_FMT_E2M1 ? 64u : 40u) && fits(t)) *out = t;
-        return CMX_OK;
-    }
     int cus = 0;
     if (int rc = cu_count(&cus); rc != CMX_OK) return rc;
-    const auto tiles = [&](const KsplitTile& t) { return (uint64_t)ceil_div(n, 16 * t.fw) * ceil_div(m_hint, 16 * t.fm); };
+    const auto tiles = [&](const KsplitTile& t) { return (uint64_t)ceil_div(n, 16 * t.fw) * ceil_div(m, 16 * t.fm); };
     for (const KsplitTile& t : {KsplitTile{1, 1, 8}, KsplitTile{1, 2, 8}, KsplitTile{2, 1, 8}, KsplitTile{2, 2, 8}, KsplitTile{4, 1, 8},
                                 KsplitTile{2, 4, 8}, KsplitTile{4, 2, 8}, KsplitTile{4, 4, 8}})
         if (tiles(t) <= (uint64_t)cus && fits(t)) {
@@ -1053,7 +1056,50 @@ int choose_ksplit(uint32_t m_hint, uint32_t n, int fmt, uint32_t kblocks, bool g
         }
     const KsplitTile t = {4, 4, 4};
     const uint64_t per_cu = fmt != CMX_FMT_E2M1 && kblocks % 4 != 0 ? 8 : 4;
-    if (tiles(t) <= per_cu * cus && !takes_128_tile(m_hint, n, fmt, kblocks, cus) && fits(t)) *out = t;
+    if (tiles(t) <= per_cu * cus && !takes_128_tile(m, n, fmt, kblocks, cus) && fits(t)) *out = t;
+    return CMX_OK;
+}
+
+// Grouped problems on the split-K kernels: their tile (fw == 0: none of the groups), and the largest group that they take
+// (0: groups of any size).
+struct GroupedKsplit {
+    KsplitTile tile;
+    uint32_t small_rows;
+};
+constexpr uint32_t kSmallGroupRows = 64;               // one m-tile of the 64 x 64 tile
+
+// Groups that average few rows stream their weights once whatever the tile; 64 x 64 tiles of four wavefronts keep more of
+// the stream in flight than the 256-row tiles.  An average says little about the groups, though, and a group of many
+// m-tiles of 64 rows reads its weights as many times.  So beyond two 64 x 64 tiles per CU (up to there the split-K kernel is the
+// faster one also where all rows are one group's) the groups are told apart on the device: those of one m-tile go to the
+// split-K kernel, the others, in a second launch, to the 256-row kernel that the average selects.
+// Measured (us, K = 7168, N = 4096, 256 experts unless noted; 256-row kernels alone / split-K alone / both by size):
+//   rows per expert               E4M3 SwiGLU         pre-tiled           INT8
+//   8 each                        1397  1077  1080    1254  1106  1107    1674  1102  1106
+//   40 each                       1458  1407  1304    1308  1326  1175    1760  1422  1422
+//   32 on average, random         1444  1219  1214    1279  1137  1138    1748  1315  1313
+//   32 on average, Zipf           1526  1494  1352    1357  1414  1195    1814  1512  1264
+//   8192 rows on 8 experts         304   567   308     209   531   216     228   554   233
+//   2048 rows on 2 experts          72   143    75      89   127    95      80   139    85
+//   32 experts, 512 rows on 1       57    42   (42)     83    36   (36)     77    42   (42)
+//   32 experts, 1024 rows on 4      59    82    61      86    78    89      76    81    78
+// The empty one of the two launches costs 2-6 us.  A limit of 32 or 40 rows instead of 64: 1360 or 1308 against 1214 (random), 1349 or
+// 1298 against 1352 (Zipf).  8-bit problems whose K is no whole number of slabs go by size only past the 2048 tiles up to which the
+// split-K kernel beats the register-staged one (choose_ksplit).  The averages up to which this pays (us, 32 experts, the
+// two sides): 40 rows 191 -> 169, INT8 221 -> 188; above, the 256-row kernel at 44 to 64 rows: 191 to 195, INT8 231 to 236.
+// FP4: split-K alone is the faster side at every one of these distributions (8192 rows on 8 experts 359 -> 298, Zipf 1062 -> 927, 32
+// experts at 64 rows 129 -> 108, at 128 rows 202 against 200).
+int choose_grouped_ksplit(uint32_t m_total, uint32_t groups, uint32_t n, int fmt, uint32_t kblocks, GroupedKsplit* out) {
+    *out = {g_force_ksplit, 0};
+    if (out->tile.fw != 0 || g_force_tile.tw != 0 || g_pretiled_tile_rows != 0 || g_disable_dl) return CMX_OK;
+    const KsplitTile t = {4, 4, 4};
+    if (ceil_div(m_total, groups) > (fmt == CMX_FMT_E2M1 ? 64u : 40u) || ksplit_lds_bytes(t, fmt, kblocks, false) > kKsplitMaxLds) return CMX_OK;
+    out->tile = t;
+    if (fmt == CMX_FMT_E2M1) return CMX_OK;
+    int cus = 0;
+    if (int rc = cu_count(&cus); rc != CMX_OK) return rc;
+    const uint64_t per_cu = kblocks % 4 != 0 ? 8 : 2;
+    if ((uint64_t)ceil_div(n, 64) * ceil_div(m_total, 64) > per_cu * cus && m_total > kSmallGroupRows) out->small_rows = kSmallGroupRows;
     return CMX_OK;
 }
 
@@ -1226,7 +1272,7 @@ extern "C" int cmx_mx_gemm(const uint8_t* a, uint32_t lda, const uint8_t* a_scal
     CMX_REQUIRE((uint64_t)n * ldb < (1ull << 32) && (uint64_t)lda * 256 < (1ull << 32), "operand tile exceeds 32-bit offsets");
     hipStream_t s = static_cast<hipStream_t>(stream);
     KsplitTile ks;
-    if (rc = choose_ksplit(m, n, fmt, p.kblocks, false, &ks); rc != CMX_OK) return rc;
+    if (rc = choose_ksplit(m, n, fmt, p.kblocks, &ks); rc != CMX_OK) return rc;
     if (ks.fw != 0) {
         p.w_tiles = ceil_div(n, 16 * ks.fw);
         return launch_ksplit(p, ks, fmt, kEpiStore, ceil_div(m, 16 * ks.fm), false, s);
@@ -1245,12 +1291,49 @@ extern "C" int cmx_mx_gemm(const uint8_t* a, uint32_t lda, const uint8_t* a_scal
 }
 
 extern "C" size_t cmx_mx_gmm_workspace_bytes(uint32_t groups) {
-    // row offsets, m-tile prefix, per-XCD tile counters
-    return cmx::round_up_sz((2 * (size_t)(groups + 1) + 8) * sizeof(int32_t), 256);
+    // row offsets, m-tile prefixes of the larger and of the small groups, per-XCD tile counters
+    return cmx::round_up_sz((3 * (size_t)(groups + 1) + 8) * sizeof(int32_t), 256);
 }
 
 namespace cmx {
 namespace {
+// The schedule metadata of a grouped problem in its workspace.
+struct GroupTables {
+    int32_t *row_off, *tile_pref, *small_pref, *tile_ctr;
+    GroupTables(void* workspace, uint32_t groups)
+        : row_off(static_cast<int32_t*>(workspace)), tile_pref(row_off + (groups + 1)), small_pref(tile_pref + (groups + 1)),
+          tile_ctr(small_pref + (groups + 1)) {}
+};
+
+// Fills the tables for m-tiles of tile_m rows (of the groups past ks.small_rows) and sets the parameters that refer to them.
+int prepare_groups(GemmParams& p, const GroupTables& g, const int32_t* group_sizes, uint32_t groups, uint32_t m_total, uint32_t tile_m,
+                   uint32_t small_rows, hipStream_t s) {
+    hipLaunchKernelGGL(gmm_prepare_kernel, dim3(1), dim3(256), 0, s, group_sizes, groups, tile_m, m_total, small_rows, g.row_off, g.tile_pref,
+                       g.small_pref, g.tile_ctr);
+    CMX_LAUNCH_CHECK();
+    p.row_off = g.row_off;
+    p.tile_pref = g.tile_pref;
+    p.tile_ctr = g.tile_ctr;
+    p.groups = groups;
+    return CMX_OK;
+}
+
+// The split-K launch of a grouped problem: all groups, or those of at most ks.small_rows rows, which are one m-tile each and
+// read their weights once.
+int launch_grouped_ksplit(GemmParams p, const GroupTables& g, const GroupedKsplit& ks, int fmt, int epi, uint32_t m_total, hipStream_t s) {
+    p.w_tiles = epi_pairs_gate_up(epi) ? ceil_div(p.n / 2, 8 * ks.tile.fw) : ceil_div(p.n, 16 * ks.tile.fw);
+    if (ks.small_rows == 0)
+        return launch_ksplit(p, ks.tile, fmt, epi, m_total / (16 * ks.tile.fm) + p.groups, ceil_div(m_total, p.groups) <= 32, s);
+    p.tile_pref = g.small_pref;
+    return launch_ksplit(p, ks.tile, fmt, epi, p.groups < m_total ? p.groups : m_total, true, s);
+}
+
+// most m-tiles of tile_m rows that groups of more than small_rows rows can have
+uint32_t max_group_tiles(uint32_t m_total, uint32_t groups, uint32_t tile_m, uint32_t small_rows) {
+    const uint32_t n = m_total / (small_rows + 1);
+    return m_total / tile_m + (n < groups ? n : groups);
+}
+
 int gmm_common(GemmParams& p, const int32_t* group_sizes, uint32_t groups, uint32_t m_total, void* workspace, int fmt,
                bool swiglu, hipStream_t s) {
     CMX_REQUIRE(group_sizes && workspace, "null pointer");
@@ -1261,31 +1344,26 @@ int gmm_common(GemmParams& p, const int32_t* group_sizes, uint32_t groups, uint3
     CMX_REQUIRE((reinterpret_cast<uintptr_t>(workspace) & 3u) == 0, "workspace must be 4-byte aligned");
     if (p.w_pretiled)
         if (int rc = check_pretiled(p, fmt, swiglu); rc != CMX_OK) return rc;
+    GroupedKsplit ks;
+    if (int rc = choose_grouped_ksplit(m_total, groups, p.n, fmt, p.kblocks, &ks); rc != CMX_OK) return rc;
     // average rows per group steers the tile height
-    KsplitTile ks;
-    if (int rc = choose_ksplit(ceil_div(m_total, groups), p.n, fmt, p.kblocks, true, &ks); rc != CMX_OK) return rc;
     TileChoice t = choose_tile(ceil_div(m_total, groups), p.n, fmt, true);
     // the weights-to-registers kernel, tiles drawn from the counters: 256 x 288 when the groups average less than four
     // tiles of rows (a group of 257 to 288 rows then takes one pass over its weights instead of two), else 256 x 256
     if (p.w_pretiled) t = {256, g_pretiled_tile_rows ? g_pretiled_tile_rows : (ceil_div(m_total, groups) < 1024 ? 288 : 256), 5};
-    int32_t* row_off = static_cast<int32_t*>(workspace);
-    int32_t* tile_pref = row_off + (groups + 1);
-    int32_t* tile_ctr = tile_pref + (groups + 1);
-    if (ks.fw) t = {16 * ks.fw, 16 * ks.fm, ks.waves};
-    hipLaunchKernelGGL(gmm_prepare_kernel, dim3(1), dim3(256), 0, s, group_sizes, groups, (uint32_t)t.tm, m_total, row_off,
-                       tile_pref, tile_ctr);
-    CMX_LAUNCH_CHECK();
-    p.row_off = row_off;
-    p.tile_pref = tile_pref;
+    const bool all_ksplit = ks.tile.fw != 0 && ks.small_rows == 0;
+    const GroupTables tables(workspace, groups);
+    if (int rc = prepare_groups(p, tables, group_sizes, groups, m_total, all_ksplit ? 16 * ks.tile.fm : t.tm, ks.small_rows, s); rc != CMX_OK) return rc;
+    if (ks.tile.fw != 0) {
+        const int epi = !swiglu ? kEpiStore : (p.act_bf16 != nullptr ? kEpiSwigluQuantAct : kEpiSwigluQuant);
+        if (int rc = launch_grouped_ksplit(p, tables, ks, fmt, epi, m_total, s); rc != CMX_OK || all_ksplit) return rc;
+    }
     // The persistent kernels draw their next tile from a per-XCD counter when tiles differ in cost (4 x 1 wavefronts skip
     // the MFMAs of absent rows).  With 2 x 2 wavefronts every tile costs the same, so those kernels walk their XCD's run in
     // fixed strides instead: no atomic whose result has to be waited for with everything else in flight.
-    p.tile_ctr = t.waves == 4 ? nullptr : tile_ctr;
-    p.groups = groups;
+    if (t.waves == 4) p.tile_ctr = nullptr;
     p.w_tiles = swiglu ? ceil_div(p.n / 2, t.tw / 2) : ceil_div(p.n, t.tw);
-    const uint32_t max_m_tiles = m_total / t.tm + groups;
-    if (ks.fw) return launch_ksplit(p, ks, fmt, !swiglu ? kEpiStore : (p.act_bf16 != nullptr ? kEpiSwigluQuantAct : kEpiSwigluQuant), max_m_tiles,
-                                   ceil_div(m_total, groups) <= 32, s);
+    const uint32_t max_m_tiles = max_group_tiles(m_total, groups, t.tm, ks.small_rows);
     if (p.w_pretiled) return t.tm == 288 ? launch_pretiled<288>(p, fmt, swiglu, max_m_tiles, s) : launch_pretiled<256>(p, fmt, swiglu, max_m_tiles, s);
     if (swiglu && p.act_bf16 != nullptr) return dispatch_tile<CMX_FMT_E4M3, kEpiSwigluQuantAct>(p, t, max_m_tiles, s);
     if (swiglu) return dispatch_tile<CMX_FMT_E4M3, kEpiSwigluQuant>(p, t, max_m_tiles, s);
@@ -1380,28 +1458,19 @@ extern "C" int cmx_int8_gmm_dequant_swiglu(const int8_t* a, uint32_t lda, const 
     p.lda = lda; p.ld_as = 0; p.ldw = k; p.ld_ws = channel_scale_stride; p.ldc = ld_out;
     p.m = m_total; p.n = n; p.kbytes = k; p.kblocks = k / 32; p.out_type = out_type;
     p.scale_vec = 1;
-    int32_t* row_off = reinterpret_cast<int32_t*>(ws);
-    int32_t* tile_pref = row_off + (groups + 1);
-    int32_t* tile_ctr = tile_pref + (groups + 1);
     constexpr int kTile = 256;
-    KsplitTile ks;
-    if (int rc = choose_ksplit(ceil_div(m_total, groups), n, kFmtI8, p.kblocks, true, &ks); rc != CMX_OK) return rc;
-    hipLaunchKernelGGL(gmm_prepare_kernel, dim3(1), dim3(256), 0, s, group_sizes, groups, (uint32_t)(ks.fw ? 16 * ks.fm : kTile), m_total, row_off,
-                       tile_pref, tile_ctr);
-    CMX_LAUNCH_CHECK();
-    p.row_off = row_off;
-    p.tile_pref = tile_pref;
-    p.tile_ctr = tile_ctr;
-    p.groups = groups;
-    if (ks.fw) {
-        p.w_tiles = ceil_div(n / 2, 8 * ks.fw);
-        return launch_ksplit(p, ks, kFmtI8, kEpiI8DequantSwiglu, m_total / (16 * ks.fm) + groups, ceil_div(m_total, groups) <= 32, s);
-    }
+    GroupedKsplit ks;
+    if (int rc = choose_grouped_ksplit(m_total, groups, n, kFmtI8, p.kblocks, &ks); rc != CMX_OK) return rc;
+    const bool all_ksplit = ks.tile.fw != 0 && ks.small_rows == 0;
+    const GroupTables tables(ws, groups);
+    if (int rc = prepare_groups(p, tables, group_sizes, groups, m_total, all_ksplit ? 16 * ks.tile.fm : kTile, ks.small_rows, s); rc != CMX_OK) return rc;
+    if (ks.tile.fw != 0)
+        if (int rc = launch_grouped_ksplit(p, tables, ks, kFmtI8, kEpiI8DequantSwiglu, m_total, s); rc != CMX_OK || all_ksplit) return rc;
     p.w_tiles = ceil_div(n / 2, kTile / 2);
     // (hand-scheduled variants of this kernel were measured twice at 16 x 2048 x 7168 x 4096 and are not kept: two i8
     // MFMAs per step and accumulator in the 8-bit schedule 997 us, one per 32-K step in the 16-byte-fragment
     // schedule shared with FP4, one tile per workgroup, 994-1000 us, against 967-975 us for this one)
-    return launch_gemm_dl<kFmtI8, kTile, kTile, 2, 4, kEpiI8DequantSwiglu>(p, m_total / kTile + groups, s);
+    return launch_gemm_dl<kFmtI8, kTile, kTile, 2, 4, kEpiI8DequantSwiglu>(p, max_group_tiles(m_total, groups, kTile, ks.small_rows), s);
 }
 
 namespace cmx {
@@ -1430,12 +1499,12 @@ int gmm_swiglu_quant(const uint8_t* a, uint32_t lda, const uint8_t* a_scale, uin
     return gmm_common(p, group_sizes, groups, m_total, workspace, CMX_FMT_E4M3, true, static_cast<hipStream_t>(stream));
 }
 
-// Schedule metadata of the allocation-free entry point (row offsets, m-tile prefix, per-XCD tile counters of up to
+// Schedule metadata of the allocation-free entry point (row offsets, m-tile prefixes, per-XCD tile counters of up to
 // kStaticGroups groups): a fixed array in device memory instead of a caller's workspace.  Every device that runs
 // the library holds its own copy; its address on a device comes from hipGetSymbolAddress with that device current
 // (the array's name is only a host-side handle).
 constexpr uint32_t kStaticGroups = 4096;
-constexpr size_t kStaticScratchBytes = (2 * ((size_t)kStaticGroups + 1) + 8) * sizeof(int32_t);
+constexpr size_t kStaticScratchBytes = (3 * ((size_t)kStaticGroups + 1) + 8) * sizeof(int32_t);
 static __device__ __align__(256) unsigned char scratch[(kStaticScratchBytes + 255) / 256 * 256];
 
 int static_scratch(void** out) {

@@ -159,7 +159,7 @@ int cmx_mx_gmm_swiglu_quant(const uint8_t* a, uint32_t lda, const uint8_t* a_sca
 /* cmx_mx_gmm_swiglu_quant without a workspace argument and without any allocation: no counterpart in the
  * reference; it is for callers that cannot allocate device memory (code under HIP graph capture, tight serving
  * loops, harnesses that forbid it).  The tile schedule metadata lives in a fixed array inside the library's device
- * image (33 KiB per device, held until the process ends), which admits at most cmx_mx_gmm_noalloc_max_groups()
+ * image (49 KiB per device, held until the process ends), which admits at most cmx_mx_gmm_noalloc_max_groups()
  * = 4096 groups; more are rejected with CMX_EINVAL.  All calls on one device share that array: calls that overlap
  * on one device (different streams) race on it; calls on one stream do not.  Same results as
  * cmx_mx_gmm_swiglu_quant.  Under stream capture call cmx_init() beforehand. */

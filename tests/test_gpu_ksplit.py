@@ -171,3 +171,63 @@ def test_sizes_on_both_sides_of_the_dense_rules(m, n, k):
     gold = (O.mx_dequant(aq, asc).astype(np.float32) @ O.mx_dequant(bq, bsc).astype(np.float32).T)
     bad, worst = close_bf16(host(ops.mx_gemm(dev(aq), dev(asc), dev(bq), dev(bsc), k)), gold)
     assert bad == 0, (bad, worst)
+
+
+SKEWED = [1300, 0, 64, 65, 1, 700, 33, 63] + [0] * 55 + [66]
+
+
+@pytest.mark.parametrize("cut", [0, 5])
+def test_skewed_groups_take_the_kernel_of_their_size(cut):
+    """64 groups that average 36 rows, 576 and more tiles of 64 x 64: the groups of at most 64 rows have the bits of the split-K
+    kernel (four partial sums), the others those of the 256-row kernel (one chain over K), on row-major and on pre-tiled
+    weights.  cut: the operands hold five rows less than the groups ask for, which makes the last group one of 61."""
+    from catccos_amd import _lib, ops
+    h = hooks_lib()
+    rng = np.random.default_rng(11 + cut)
+    n, k, e = 1024, 512, len(SKEWED)
+    m = sum(SKEWED) - cut
+    counts = SKEWED[:-1] + [SKEWED[-1] - cut]
+    small = np.repeat([0 < c <= 64 for c in counts], counts)
+    small = torch.from_numpy(small).cuda()
+    aq, asc = _mx(rng, m, k, "E4M3")
+    wq, ws = _mx(rng, e * n, k, "E4M3", 1 / np.sqrt(k))
+    # block scales over 2^16: with equal ones the sums are short enough to be exact in any order
+    asc = (asc + rng.integers(-8, 9, asc.shape)).astype(np.uint8)
+    wq, ws = wq.reshape(e, n, k), ws.reshape(e, n, -1)
+    a, a_s, w, w_s, cnt = dev(aq), dev(asc), dev(wq), dev(ws), dev(np.array(SKEWED, dtype=np.int32))
+
+    def store(weights=w, out="fp32"):
+        return ops.mx_gmm(a, a_s, weights, w_s, cnt, k, "E4M3", out)
+
+    def swiglu(weights=w):
+        return torch.cat(ops.mx_gmm_swiglu_quant(a, a_s, weights, w_s, cnt, k)[:2], dim=1)
+
+    ai = torch.randint(-127, 128, (m, k), dtype=torch.int8, device="cuda")
+    wi = torch.randint(-127, 128, (e, n, k), dtype=torch.int8, device="cuda")
+    channel, token = torch.rand(e * n, device="cuda") * 1e-3, torch.rand(m, device="cuda")
+
+    def int8():
+        return ops.int8_gmm_dequant_swiglu(ai, token, wi, channel, cnt, n, k, 1)
+
+    calls = (store, swiglu, int8)
+    chosen = [f() for f in calls]
+    h.cmx_debug_force_ksplit(4, 4, 4)
+    split = [f() for f in calls]
+    h.cmx_debug_force_ksplit(0, 0, 0)
+    h.cmx_debug_force_tile(256, 128, 5)
+    chain = [f() for f in calls[:2]]
+    h.cmx_debug_force_tile(0, 0, 0)
+    assert float((split[0] != chain[0]).any(dim=1).float().mean()) > 0.9      # the two sides can be told apart
+    for got, s, c in zip(chosen, split, chain):
+        assert torch.equal(got[small], s[small])
+        assert torch.equal(got[~small], c[~small])
+    assert torch.equal(chosen[2], split[2])                                   # whole-number sums: the same on both
+    assert torch.equal(swiglu(ops.pretile_weights(w, True)), chosen[1])
+    assert torch.equal(store(ops.pretile_weights(w, False), "bf16"), store(out="bf16"))
+    codes, scales = torch.zeros((m, n // 2), dtype=torch.uint8, device="cuda"), torch.zeros((m, n // 64), dtype=torch.uint8, device="cuda")
+    _lib.check(h.cmx_mx_gmm_swiglu_quant_noalloc(a.data_ptr(), k, a_s.data_ptr(), a_s.shape[1], w.data_ptr(), w_s.data_ptr(), codes.data_ptr(),
+                                                 n // 2, scales.data_ptr(), n // 64, None, cnt.data_ptr(), e, m, n, k,
+                                                 torch.cuda.current_stream().cuda_stream))
+    assert torch.equal(torch.cat((codes, scales), dim=1), chosen[1])
+    gold = O.mx_gmm_f32(aq, asc, wq, ws, counts)
+    assert np.linalg.norm(host(chosen[0]) - gold) < 1e-3 * np.linalg.norm(gold)       # products keep 2^-13 of the largest of eight
