@@ -18,9 +18,15 @@ OUT = {"bf16": 0, "fp16": 1, "fp32": 2}
 _OUT_DTYPE = {"bf16": torch.bfloat16, "fp16": torch.float16, "fp32": torch.float32}
 
 
+# not a public function of torch, so it may be missing
+_raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)
+
+
 def _stream():
     # the handle of torch's current stream without a Stream object around it: 0.3 us of host time against 2.8, of 10 a call
-    return torch._C._cuda_getCurrentRawStream(torch.cuda.current_device())
+    if _raw_stream is not None:
+        return _raw_stream(torch.cuda.current_device())
+    return torch.cuda.current_stream().cuda_stream
 
 
 def _p(t: torch.Tensor):
