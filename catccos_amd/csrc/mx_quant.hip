@@ -158,12 +158,16 @@ __global__ __launch_bounds__(kThreads) void mx_quant_kernel(const uint16_t* __re
 // Each lane of a quad then stores the scale byte of one of the four rows.
 // E2M1 (bound: HBM, 2.53 bytes per element; the general kernel above, which compares every element with seven thresholds
 // in fp32, is bound by the VALU: 65536 x 7168 365 us there, 234 us here, 192 us with streaming loads).
-// STREAM: inputs that do not stay in the memory-side cache anyway (256 MiB, which the codes and the consumer's operands
-// share) are read non-temporal and leave it to those: from 96 MiB of input on.  65536 x 7168 to E2M1 234 -> 192 us, 8192 x
-// 7168 to E4M3 followed by its matmul 203 -> 197 us together; 4096 x 7168 (56 MiB), whose input is still cached, 15.5
-// against 16.7 us.
+// STREAM: non-temporal reads, which leave the memory-side cache (256 MiB) to the codes and to the consumer's operands: from 96 MiB
+// of input on, as long as the codes fit that cache.  Measured (us, rows x 7168 to E4M3, cached -> streaming loads):
+//   with the matmul behind it (N = 4096), three inputs and weights in turn: 56 MiB 104.9 -> 103.8, 84 MiB 191.0 -> 187.6, 98 MiB
+//   194.2 -> 191.6, 112 MiB 202.7 -> 200.9, 140 MiB 285.8 -> 282.3, 224 MiB 396.0 -> 393.8; one input again and again, which the
+//   cache holds: 56 MiB 104.7 -> 106.0, 84 MiB 185.8 -> 188.2, 112 MiB 197.3 -> 200.3, 168 MiB equal, 224 MiB 395.2 -> 393.0;
+//   alone, another input in each call: 56 MiB 16.3 -> 16.6, 112 MiB 30.2 -> 31.2, 140 MiB 36.8 -> 38.0, 168 MiB 43.8 -> 44.4, 182 MiB
+//   48.2 -> 47.9, 224 MiB 64.4 -> 57.9, 448 MiB (codes 224 MiB) 135 -> 113, 672 MiB 205 -> 204, 896 MiB 276 -> 283, 1344 MiB 416 -> 442.
+// E2M1, whose codes are half as large: 112 MiB equal, 224 MiB 53.3 -> 48.8, 896 MiB (codes 224 MiB) 230 -> 189, 1344 MiB equal.
 constexpr int kFastRows = 4;
-constexpr uint64_t kStreamBytes = 96ull << 20;
+constexpr uint64_t kStreamBytes = 96ull << 20, kStreamCodeBytes = 256ull << 20;
 
 // E2M1 under table rounding: ties go to the smaller magnitude, where the hardware cast takes the even code.  The two differ at
 // 0.75, 1.75 and 3.5 (times 2^e) alone, whose lower neighbours have odd codes: bf16 mantissas 0x40 and 0x60.  Taking one unit in
@@ -353,7 +357,8 @@ extern "C" int cmx_mx_quant(const void* x, uint32_t ld_x, uint8_t* codes, uint32
         const auto launch = [&](auto kernel) {
             hipLaunchKernelGGL(kernel, fgrid, dim3(kThreads), 0, s, xb, ld_x * 2, codes, ld_codes, scales, ld_scales, rows, nb);
         };
-        const bool stream = (uint64_t)rows * cols * 2 >= kStreamBytes;
+        const uint64_t elems = (uint64_t)rows * cols;
+        const bool stream = elems * 2 >= kStreamBytes && (fp4 ? elems / 2 : elems) <= kStreamCodeBytes;
 #define CMX_FAST(FMT_, LUT_) (stream ? launch(mx_quant_fast_kernel<FMT_, LUT_, true>) : launch(mx_quant_fast_kernel<FMT_, LUT_, false>))
         if (fmt == CMX_FMT_E4M3) CMX_FAST(CMX_FMT_E4M3, false);
         else if (fmt == CMX_FMT_E5M2) CMX_FAST(CMX_FMT_E5M2, false);
