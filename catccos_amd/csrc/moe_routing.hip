@@ -296,8 +296,9 @@ __global__ __launch_bounds__(256) void quant_scatter_row_kernel(const uint16_t* 
 
 // Zeros for the output rows that no route is sent to.  A workgroup owns `per` rows (a multiple of 32, at most
 // kUnmappedRows): it reads all destinations, marks those of its rows in an LDS bitmap and clears the rows left over.
-// Bound: the read of the destinations from the L2, by at most 256 workgroups (routes * 4 bytes each).  It stands in for
-// a fill of the whole output before the scatter: 32768 x 7168 bytes of codes 36 us, this kernel 6 us.
+// Bound: the read of the destinations from the L2 (routes * 4 bytes) by every workgroup, of which there are 256, or more where
+// 256 times kUnmappedRows rows (16.7 million) are not enough.  It stands in for a fill of the whole output before the
+// scatter: 32768 x 7168 bytes of codes 36 us, this kernel 6 us.
 constexpr uint32_t kUnmappedRows = 65536, kUnmappedThreads = 1024;
 
 __global__ __launch_bounds__(kUnmappedThreads) void zero_unmapped_rows_kernel(const int32_t* __restrict__ src2sorted,

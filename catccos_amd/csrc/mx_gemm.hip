@@ -1012,10 +1012,15 @@ constexpr int g_pretiled_tile_rows = 0;
 #endif
 
 #ifdef CMX_TEST_HOOKS
-KsplitTile g_force_ksplit = {0, 0, 0};
+KsplitTile g_force_ksplit = {0, 0, 0};   // fw == 0 -> heuristic, fw < 0 -> never
 #else
 constexpr KsplitTile g_force_ksplit = {0, 0, 0};
 #endif
+// whether the test build takes the choice of a split-K tile away from the heuristic, and with what
+bool ksplit_is_forced(KsplitTile* out) {
+    *out = g_force_ksplit.fw > 0 ? g_force_ksplit : KsplitTile{0, 0, 0};
+    return g_force_ksplit.fw != 0 || g_force_tile.tw != 0 || g_disable_dl;
+}
 
 // Dense 8-bit problems that 128 x 128 tiles of four wavefronts (mx_gemm_kernel) take: too many 64 x 64 tiles for the split-K
 // kernel to run in two rounds of a workgroup per CU, few enough 128 x 128 tiles for one, and K up to 2048: a tile of twice the
@@ -1023,6 +1028,9 @@ constexpr KsplitTile g_force_ksplit = {0, 0, 0};
 // Measured (us, E4M3, 64 x 64 split-K -> 128 x 128): 1024 x 4096 at K = 512 12.4 -> 10.0, 1024 15.8 -> 12.2, 2048 22.3 -> 17.1,
 // 4096 33.8 against 33.1, 7168 55.2 against 52.2 (behind the pass that writes its weights, 62 against 64); 760 x 3072 x 2048 (576
 // 64 x 64 tiles) 18.7 -> 15.8, 640 x 4096 x 4096 (640) 28.4 against 33.0.
+// The alignment of the scale rows does not enter, because it must not change the sums; rows that are not dword-aligned run the 128 x
+// 128 tile on the register-staged kernel with its byte loads: 1024 x 4096 x 2048 18.5 aligned, 32.0 not (256-row tiles 24.6 and 61.4; 64
+// x 64 split-K would take 23.9 and 23.1).
 bool takes_128_tile(uint32_t m, uint32_t n, int fmt, uint32_t kblocks, int cus) {
     if (fmt == CMX_FMT_E2M1 || kblocks % 4 != 0 || kblocks > 64) return false;
     const uint64_t t64 = (uint64_t)ceil_div(n, 64) * ceil_div(m, 64), t128 = (uint64_t)ceil_div(n, 128) * ceil_div(m, 128);
@@ -1030,7 +1038,7 @@ bool takes_128_tile(uint32_t m, uint32_t n, int fmt, uint32_t kblocks, int cus) 
 }
 
 // Whether a problem goes to the split-K kernels (mx_gemm_ksplit.hip), and with which tile; fw == 0: no.  The choice depends
-// on sizes and element format only, so that every layout, pitch and output type of a problem gets the same sums.
+// on sizes, element format and the number of CUs only, so that every layout, pitch and output type of a problem gets the same sums.
 // Dense: the smallest tile that still leaves every CU at most one workgroup (time goes with the bytes a workgroup pulls
 // through its vector cache, and a second round costs as much as the first); past that 64 x 64 tiles, two workgroups of
 // four wavefronts on a CU, up to 1024 tiles.  Measured (us, E4M3, before = 256-row tiles): 16 x 4096 x 7168 44.7 -> 9.0,
@@ -1042,8 +1050,7 @@ bool takes_128_tile(uint32_t m, uint32_t n, int fmt, uint32_t kblocks, int cus) 
 // times than the streaming ones, so they stay here up to 2048 tiles (us, 256-row -> here): 2048 x 4096 x 6976 240 -> 117, 1536 x
 // 4096 x 3040 75 -> 47; 3000 x 5000 x 4064 (3713 tiles) 97 against 138, 8192 x 4096 x 7136 300 against 463.
 int choose_ksplit(uint32_t m, uint32_t n, int fmt, uint32_t kblocks, KsplitTile* out) {
-    *out = g_force_ksplit;
-    if (out->fw != 0 || g_force_tile.tw != 0 || g_disable_dl) return CMX_OK;
+    if (ksplit_is_forced(out)) return CMX_OK;
     const auto fits = [&](const KsplitTile& t) { return ksplit_lds_bytes(t, fmt, kblocks, false) <= kKsplitMaxLds; };
     int cus = 0;
     if (int rc = cu_count(&cus); rc != CMX_OK) return rc;
@@ -1090,8 +1097,8 @@ constexpr uint32_t kSmallGroupRows = 64;               // one m-tile of the 64 x
 // FP4: split-K alone is the faster side at every one of these distributions (8192 rows on 8 experts 359 -> 298, Zipf 1062 -> 927, 32
 // experts at 64 rows 129 -> 108, at 128 rows 202 against 200).
 int choose_grouped_ksplit(uint32_t m_total, uint32_t groups, uint32_t n, int fmt, uint32_t kblocks, GroupedKsplit* out) {
-    *out = {g_force_ksplit, 0};
-    if (out->tile.fw != 0 || g_force_tile.tw != 0 || g_pretiled_tile_rows != 0 || g_disable_dl) return CMX_OK;
+    out->small_rows = 0;
+    if (ksplit_is_forced(&out->tile) || g_pretiled_tile_rows != 0) return CMX_OK;
     const KsplitTile t = {4, 4, 4};
     if (ceil_div(m_total, groups) > (fmt == CMX_FMT_E2M1 ? 64u : 40u) || ksplit_lds_bytes(t, fmt, kblocks, false) > kKsplitMaxLds) return CMX_OK;
     out->tile = t;
@@ -1115,6 +1122,7 @@ TileChoice choose_tile(uint32_t m_hint, uint32_t n, int fmt, bool grouped) {
     if (g_force_tile.tw) return g_force_tile;
     // short problems stream their weights once: the three-slot 256 x 128 kernel keeps two slabs in flight
     if (m_hint <= 128 && fmt != CMX_FMT_E2M1) return {256, 128, 5};
+    // (FP4, and of that what the split-K kernels leave: dense problems of more than 1024 of their tiles, rows of scales beyond the LDS)
     if (m_hint <= 64) return {256, 64, 4};
     if (m_hint <= 128) return {256, 128, 8};
     return {256, 256, grouped && m_hint < 512 ? 5 : 4};
@@ -1240,7 +1248,7 @@ extern "C" int cmx_debug_pretiled_tile_rows(int rows) {
     return CMX_OK;
 }
 
-// pin the split-K tile of every later matmul call (fw = 0 restores the heuristic)
+// pin the split-K tile of every later matmul call (fw = 0 restores the heuristic, fw < 0 keeps every problem off those kernels)
 extern "C" int cmx_debug_force_ksplit(int fw, int fm, int waves) {
     cmx::g_force_ksplit = {fw, fm, waves};
     return CMX_OK;

@@ -5,18 +5,20 @@
 // sixteen workgroups).  Here a workgroup owns a small tile, 16 FW weight rows x 16 FM activation rows, and its NW wavefronts
 // split K between them: wavefront w multiplies the 128-byte K slabs w, w + NW, w + 2 NW, ... of the WHOLE tile, so
 //   * every operand byte of the tile is needed by exactly one wavefront: both operands go straight from memory into that
-//     wavefront's registers (buffer_load_dwordx4) through a ring of PD slabs, with no barrier and no wait for another
-//     wavefront in the K loop;
+//     wavefront's registers (buffer_load_dwordx4) through a ring of PD slabs (eight for a tile of 16 x 16, one for a full 64 x
+//     64: what the registers hold), with no barrier and no wait for another wavefront in the K loop;
 //   * v_mfma_scale_f32_16x16x128_f8f6f4 takes, per lane group g = lane / 16, the bytes 16 g .. 16 g + 15 of a slab's first
 //     64 bytes in registers 0-3 and of its second 64 bytes in registers 4-7 (and the scale of the 32-block g), for the
-//     row lane % 16.  Loading row-major operands in that order costs the vector cache a visit per lane quad and row, twice
-//     the time of whole 128-byte lines (measured: 9.7 against 7.2 us at 16 x 4096 x 7168), so the lanes fetch whole lines, eight to a
-//     row, and a fragment changes places through 2 KiB of LDS that belong to the wavefront alone (its LDS accesses
-//     execute in order: nothing to wait for).  Pre-tiled weights are stored in the fragment order and need none of it;
+//     row lane % 16.  Loading row-major operands in that order costs the vector cache a visit per lane quad and row, a third
+//     more time than whole 128-byte lines (16 x 4096 x 7168, operands in the memory-side cache: 9.7 against 7.2 us), so the lanes
+//     fetch whole lines, eight to a row, and a fragment changes places through 2 KiB of LDS that belong to the wavefront alone
+//     (its LDS accesses execute in order: nothing to wait for).  Pre-tiled weights are stored in the fragment order and need none of it;
 //   * the block scales of the tile, which are a byte per 32 elements in rows of their own, are fetched once, coalesced, for
 //     the whole of K into the LDS and read from there a byte per lane and fragment.
 // The NW partial sums meet in the LDS at the end and are added in the order of the wavefronts, so the result does not
-// depend on timing; it does depend on NW, and differs in the last bits from that of the kernels that walk K in one chain.
+// depend on timing; it does depend on NW, and where the fp32 additions round it differs in the last bits from that of the
+// kernels that walk K in one chain.  (The error against 64-bit sums is the same on both: 6.3e-5 to 6.7e-5 of the 2-norm at K = 512 to
+// 7168, E4M3, normal data with outliers; it comes from the matrix cores, which keep 2^-13 of the largest of eight products.)
 // Every tile shape with the same NW gives the same bits, and so do row-major and pre-tiled weights.
 #include <type_traits>
 
@@ -31,7 +33,9 @@ typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
 
 constexpr int ks_scale_steps(int fmt) { return fmt == kFmtI8 ? 0 : (fmt == CMX_FMT_E2M1 ? 2 : 1); }   // scale dwords per row and slab
 // slabs in the register ring: what fits beside the accumulators, one slab of fragments in MFMA order, their scales and
-// addresses in 256 registers (two wavefronts per SIMD)
+// addresses in 256 registers (two wavefronts per SIMD).  The scale pieces in flight before the K loop (sreg, treg: up to 32
+// registers at 8 wavefronts) are not counted; by the compiler's report they cost 16 x 16 tiles 3-4 spilled registers and 16 x 32
+// tiles 7 (FP4 12), stored and reloaded before the loop, and no other tile more than one.
 constexpr int ks_ring(int fmt, int fw, int fm) {
     const int room = 256 - 40 - 4 * fw * fm - (fw + fm) * (10 + 2 * ks_scale_steps(fmt));
     const int n = room / ((fw + fm) * 8), most = fw + fm == 2 ? 8 : (fw + fm == 3 ? 5 : 4);
