@@ -1072,41 +1072,50 @@ int choose_ksplit(uint32_t m, uint32_t n, int fmt, uint32_t kblocks, KsplitTile*
 struct GroupedKsplit {
     KsplitTile tile;
     uint32_t small_rows;
+    KsplitWeights weights;
 };
 constexpr uint32_t kSmallGroupRows = 64;               // one m-tile of the 64 x 64 tile
 
 // Groups that average few rows stream their weights once whatever the tile; 64 x 64 tiles of four wavefronts keep more of
 // the stream in flight than the 256-row tiles.  An average says little about the groups, though, and a group of many
-// m-tiles of 64 rows reads its weights as many times.  So beyond two 64 x 64 tiles per CU (up to there the split-K kernel is the
+// m-tiles of 64 rows reads its weights as many times.  So beyond four 64 x 64 tiles per CU (up to there the split-K kernel is the
 // faster one also where all rows are one group's) the groups are told apart on the device: those of one m-tile go to the
 // split-K kernel, the others, in a second launch, to the 256-row kernel that the average selects.
-// Measured (us, K = 7168, N = 4096, 256 experts unless noted; 256-row kernels alone / split-K alone / both by size):
+// Measured (us, K = 7168, N = 4096, 256 experts unless noted; 256-row kernels alone / split-K alone, weights streamed where the average
+// is at most 32 / this rule):
 //   rows per expert               E4M3 SwiGLU         pre-tiled           INT8
-//   8 each                        1397  1077  1080    1254  1106  1107    1674  1102  1106
-//   40 each                       1458  1407  1304    1308  1326  1175    1760  1422  1422
-//   32 on average, random         1444  1219  1214    1279  1137  1138    1748  1315  1313
-//   32 on average, Zipf           1526  1494  1352    1357  1414  1195    1814  1512  1264
-//   8192 rows on 8 experts         304   567   308     209   531   216     228   554   233
-//   2048 rows on 2 experts          72   143    75      89   127    95      80   139    85
-//   32 experts, 512 rows on 1       57    42   (42)     83    36   (36)     77    42   (42)
-//   32 experts, 1024 rows on 4      59    82    61      86    78    89      76    81    78
+//   8 each                        1402  1082  1081    1251  1102  1105    1728  1104  1106
+//   40 each                       1464  1413  1265    1316  1329  1180    1762  1427  1398
+//   32 on average, random         1448  1220  1207    1281  1140  1145    1723  1317  1299
+//   32 on average, Zipf           1535  1505  1355    1369  1409  1210    1795  1520  1274
+//   8192 rows on 8 experts         305   565   314     206   530   210     223   561   227
+//   2048 rows on 2 experts          73   144    76      90   128    95      83   140    89
+//   32 experts, 512 rows on 1       57    42    40      84    37    36      77    40    39
+//   32 experts, 1024 rows on 4      59    82    55      85    78    50      75    79    54
+//   32 experts, 1280 rows on 4      56    69    59      91    60    92      78    66    81
 // The empty one of the two launches costs 2-6 us.  A limit of 32 or 40 rows instead of 64: 1360 or 1308 against 1214 (random), 1349 or
 // 1298 against 1352 (Zipf).  8-bit problems whose K is no whole number of slabs go by size only past the 2048 tiles up to which the
-// split-K kernel beats the register-staged one (choose_ksplit).  The averages up to which this pays (us, 32 experts, the
-// two sides): 40 rows 191 -> 169, INT8 221 -> 188; above, the 256-row kernel at 44 to 64 rows: 191 to 195, INT8 231 to 236.
-// FP4: split-K alone is the faster side at every one of these distributions (8192 rows on 8 experts 359 -> 298, Zipf 1062 -> 927, 32
-// experts at 64 rows 129 -> 108, at 128 rows 202 against 200).
+// split-K kernel beats the register-staged one (choose_ksplit).  Row-major and pre-tiled weights go by one rule, because they
+// promise the same bits.
+// The averages up to which this pays (32 experts, rows each; 256-row -> split-K): 36 rows E4M3 190 -> 164, pre-tiled 177 -> 162, INT8 220 ->
+// 178; 40 rows 191 -> 165, 178 -> 165, 221 -> 186; with cached weights 48 rows 193 -> 181, 176 against 181, 241 -> 184; 64 rows 197 ->
+// 195, 177 against 191, 234 -> 194: from there on it is the pre-tiled kernel that would lose.
+// FP4: split-K alone is the faster side at every one of these distributions (8192 rows on 8 experts 358 -> 257, Zipf 1063 -> 802, 32
+// experts at 64 rows 129 -> 107, at 128 rows 202 against 200), so it takes all groups in one launch.
+// Weights are streamed without a look at the group where all groups are one m-tile, and in small problems of few rows on
+// average, where the look would cost more (32 tokens of 256 experts 1101 -> 1110) than the rare larger group loses.
 int choose_grouped_ksplit(uint32_t m_total, uint32_t groups, uint32_t n, int fmt, uint32_t kblocks, GroupedKsplit* out) {
     out->small_rows = 0;
+    out->weights = KsplitWeights::kByGroup;
     if (ksplit_is_forced(&out->tile) || g_pretiled_tile_rows != 0) return CMX_OK;
     const KsplitTile t = {4, 4, 4};
     if (ceil_div(m_total, groups) > (fmt == CMX_FMT_E2M1 ? 64u : 40u) || ksplit_lds_bytes(t, fmt, kblocks, false) > kKsplitMaxLds) return CMX_OK;
     out->tile = t;
-    if (fmt == CMX_FMT_E2M1) return CMX_OK;
     int cus = 0;
     if (int rc = cu_count(&cus); rc != CMX_OK) return rc;
-    const uint64_t per_cu = kblocks % 4 != 0 ? 8 : 2;
-    if ((uint64_t)ceil_div(n, 64) * ceil_div(m_total, 64) > per_cu * cus && m_total > kSmallGroupRows) out->small_rows = kSmallGroupRows;
+    const uint64_t tiles = (uint64_t)ceil_div(n, 64) * ceil_div(m_total, 64), per_cu = kblocks % 4 != 0 ? 8 : 4;
+    if (fmt != CMX_FMT_E2M1 && tiles > per_cu * cus && m_total > kSmallGroupRows) out->small_rows = kSmallGroupRows;
+    if (out->small_rows != 0 || (tiles <= 2 * (uint64_t)cus && ceil_div(m_total, groups) <= 32)) out->weights = KsplitWeights::kStreamed;
     return CMX_OK;
 }
 
@@ -1283,7 +1292,7 @@ extern "C" int cmx_mx_gemm(const uint8_t* a, uint32_t lda, const uint8_t* a_scal
     if (rc = choose_ksplit(m, n, fmt, p.kblocks, &ks); rc != CMX_OK) return rc;
     if (ks.fw != 0) {
         p.w_tiles = ceil_div(n, 16 * ks.fw);
-        return launch_ksplit(p, ks, fmt, kEpiStore, ceil_div(m, 16 * ks.fm), false, s);
+        return launch_ksplit(p, ks, fmt, kEpiStore, ceil_div(m, 16 * ks.fm), KsplitWeights::kCached, s);
     }
     int cus = 0;
     if (rc = cu_count(&cus); rc != CMX_OK) return rc;
@@ -1331,9 +1340,9 @@ int prepare_groups(GemmParams& p, const GroupTables& g, const int32_t* group_siz
 int launch_grouped_ksplit(GemmParams p, const GroupTables& g, const GroupedKsplit& ks, int fmt, int epi, uint32_t m_total, hipStream_t s) {
     p.w_tiles = epi_pairs_gate_up(epi) ? ceil_div(p.n / 2, 8 * ks.tile.fw) : ceil_div(p.n, 16 * ks.tile.fw);
     if (ks.small_rows == 0)
-        return launch_ksplit(p, ks.tile, fmt, epi, m_total / (16 * ks.tile.fm) + p.groups, ceil_div(m_total, p.groups) <= 32, s);
+        return launch_ksplit(p, ks.tile, fmt, epi, m_total / (16 * ks.tile.fm) + p.groups, ks.weights, s);
     p.tile_pref = g.small_pref;
-    return launch_ksplit(p, ks.tile, fmt, epi, p.groups < m_total ? p.groups : m_total, true, s);
+    return launch_ksplit(p, ks.tile, fmt, epi, p.groups < m_total ? p.groups : m_total, ks.weights, s);
 }
 
 // most m-tiles of tile_m rows that groups of more than small_rows rows can have

@@ -80,6 +80,7 @@ __device__ __forceinline__ float i8_dequant(int32_t sum, float channel_scale) {
 
 struct Tile {
     uint32_t g, mt, wt, row0, rows_valid;
+    uint32_t rows_left;      // rows of the group (or problem) from row0 on
 };
 
 // The group tables (row offsets, m-tile prefix) are written by gmm_prepare_kernel before the matmul kernel starts and
@@ -166,7 +167,8 @@ __device__ __forceinline__ void decode_tile(const GemmParams& p, uint32_t m_tile
         t.wt = within / band_rows;
         const uint32_t r_begin = (uint32_t)table_at(p.row_off, lo), r_end = (uint32_t)table_at(p.row_off, lo + 1);
         t.row0 = r_begin + t.mt * TM;
-        t.rows_valid = r_end - t.row0 < (uint32_t)TM ? r_end - t.row0 : (uint32_t)TM;
+        t.rows_left = r_end - t.row0;
+        t.rows_valid = t.rows_left < (uint32_t)TM ? t.rows_left : (uint32_t)TM;
     } else {
         // bands of 4 m-tiles share a run of weight tiles
         const uint32_t band = 4;
@@ -177,7 +179,8 @@ __device__ __forceinline__ void decode_tile(const GemmParams& p, uint32_t m_tile
         t.mt = b * band + within % band_rows;
         t.wt = within / band_rows;
         t.row0 = t.mt * TM;
-        t.rows_valid = p.m - t.row0 < (uint32_t)TM ? p.m - t.row0 : (uint32_t)TM;
+        t.rows_left = p.m - t.row0;
+        t.rows_valid = t.rows_left < (uint32_t)TM ? t.rows_left : (uint32_t)TM;
     }
 }
 

@@ -15,11 +15,15 @@ struct KsplitTile {
 constexpr size_t kKsplitMaxLds = 160 * 1024;
 size_t ksplit_lds_bytes(const KsplitTile& t, int fmt, uint32_t kblocks, bool tiled);
 
+// How the weights are read.  kStreamed: non-temporal, for weights with one reader, which leaves the L2 to the activation rows (32
+// experts x 4 / 16 / 32 rows, K = 7168, N = 4096: 142 / 145 / 152 us with it, 160 / 162 / 172 without).  kCached: for weights that the
+// next m-tile reads again.  kByGroup: each group as its size asks for (32 experts, 1024 rows on one of them: streamed 76, by group 55; 256
+// experts x 8 rows, where all are streamed either way, pre-tiled 1101 and 1112: twice the code).
+enum class KsplitWeights { kCached, kStreamed, kByGroup };
+
 // p as for the other kernels, with w_tiles counted in tiles of 16 * t.fw weight rows (8 * t.fw output columns for epilogues
-// that pair gate and up) and, for grouped problems, group tables made for m-tiles of 16 * t.fm rows.
-// stream: load the weights non-temporal (grouped problems whose groups mostly fit one m-tile: each weight byte has one reader,
-// and the hint keeps the activation rows in the L2.  32 experts x 4 / 16 rows, K = 7168, N = 4096: 142 / 145 us with it, 160 /
-// 162 us without; 64 rows, where a second m-tile reads the weights again, 244 against 242 us).
-int launch_ksplit(const GemmParams& p, const KsplitTile& t, int fmt, int epi, uint32_t max_m_tiles, bool stream, hipStream_t s);
+// that pair gate and up) and, for grouped problems, group tables made for m-tiles of 16 * t.fm rows.  Dense problems read their
+// weights cached; `loads` is for grouped ones.
+int launch_ksplit(const GemmParams& p, const KsplitTile& t, int fmt, int epi, uint32_t max_m_tiles, KsplitWeights loads, hipStream_t s);
 
 }  // namespace cmx

@@ -184,7 +184,7 @@ __device__ __forceinline__ void ks_store(const GemmParams& p, const Tile& tc, ui
     }
 }
 
-// STREAM: weights are loaded non-temporal (one reader; a tile column has no other m-tile)
+// STREAM: weights are loaded non-temporal (KsplitWeights)
 template <int FMT, int FW, int FM, int NW, int EPI, bool TILED, bool STREAM>
 __device__ __forceinline__ void ks_tile(const GemmParams& p, const Tile& tc, uint8_t* smem) {
     constexpr int NT = 64 * NW, TW = 16 * FW;
@@ -481,16 +481,9 @@ __device__ __forceinline__ void ks_tile(const GemmParams& p, const Tile& tc, uin
     }
 }
 
+// a ragged tile does the work of the rows it has
 template <int FMT, int FW, int FM, int NW, int EPI, bool TILED, bool STREAM>
-__global__ __launch_bounds__(64 * NW, 2) void mx_gemm_ksplit_kernel(const GemmParams p) {
-    extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
-    Tile tc;
-    if (!locate_tile<16 * FM>(p, tc)) return;
-    tc.g = __builtin_amdgcn_readfirstlane(tc.g);
-    tc.wt = __builtin_amdgcn_readfirstlane(tc.wt);
-    tc.row0 = __builtin_amdgcn_readfirstlane(tc.row0);
-    tc.rows_valid = __builtin_amdgcn_readfirstlane(tc.rows_valid);
-    // a ragged tile does the work of the rows it has
+__device__ __forceinline__ void ks_rows(const GemmParams& p, const Tile& tc, uint8_t* smem) {
     if constexpr (FM >= 4) {
         if (tc.rows_valid <= 16 * FM / 4) return ks_tile<FMT, FW, FM / 4, NW, EPI, TILED, STREAM>(p, tc, smem);
     }
@@ -500,9 +493,25 @@ __global__ __launch_bounds__(64 * NW, 2) void mx_gemm_ksplit_kernel(const GemmPa
     ks_tile<FMT, FW, FM, NW, EPI, TILED, STREAM>(p, tc, smem);
 }
 
-template <int FMT, int FW, int FM, int NW, int EPI, bool TILED, bool STREAM>
+template <int FMT, int FW, int FM, int NW, int EPI, bool TILED, KsplitWeights LOADS>
+__global__ __launch_bounds__(64 * NW, 2) void mx_gemm_ksplit_kernel(const GemmParams p) {
+    extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
+    Tile tc;
+    if (!locate_tile<16 * FM>(p, tc)) return;
+    tc.g = __builtin_amdgcn_readfirstlane(tc.g);
+    tc.wt = __builtin_amdgcn_readfirstlane(tc.wt);
+    tc.row0 = __builtin_amdgcn_readfirstlane(tc.row0);
+    tc.rows_valid = __builtin_amdgcn_readfirstlane(tc.rows_valid);
+    if constexpr (LOADS == KsplitWeights::kByGroup) {
+        if (__builtin_amdgcn_readfirstlane(tc.mt != 0 || tc.rows_left > 16u * FM))
+            return ks_rows<FMT, FW, FM, NW, EPI, TILED, false>(p, tc, smem);
+    }
+    ks_rows<FMT, FW, FM, NW, EPI, TILED, LOADS != KsplitWeights::kCached>(p, tc, smem);
+}
+
+template <int FMT, int FW, int FM, int NW, int EPI, bool TILED, KsplitWeights LOADS>
 int launch_one(const GemmParams& p, uint32_t max_m_tiles, hipStream_t s) {
-    constexpr auto kfn = mx_gemm_ksplit_kernel<FMT, FW, FM, NW, EPI, TILED, STREAM>;
+    constexpr auto kfn = mx_gemm_ksplit_kernel<FMT, FW, FM, NW, EPI, TILED, LOADS>;
     if (int rc = allow_dynamic_lds<kfn, kKsplitMaxLds>(); rc != CMX_OK) return rc;
     const size_t smem = ksplit_lds_bytes({FW, FM, NW}, FMT, p.kblocks, TILED);
     CMX_REQUIRE(smem <= kKsplitMaxLds, "split-K tile exceeds the LDS");
@@ -515,13 +524,14 @@ int launch_one(const GemmParams& p, uint32_t max_m_tiles, hipStream_t s) {
 
 // the tile shapes that exist for an element format and epilogue: one for grouped problems, all for dense ones
 template <int FMT, int EPI, bool TILED>
-int launch_shape(const GemmParams& p, const KsplitTile& t, uint32_t max_m_tiles, bool stream, hipStream_t s) {
-#define CMX_KS(FW_, FM_, NW_) if (t.fw == FW_ && t.fm == FM_ && t.waves == NW_) return launch_one<FMT, FW_, FM_, NW_, EPI, TILED, false>(p, max_m_tiles, s)
-    if (t.fw == 4 && t.fm == 4 && t.waves == 4) {
-        if (stream) return launch_one<FMT, 4, 4, 4, EPI, TILED, true>(p, max_m_tiles, s);
-        return launch_one<FMT, 4, 4, 4, EPI, TILED, false>(p, max_m_tiles, s);
+int launch_shape(const GemmParams& p, const KsplitTile& t, uint32_t max_m_tiles, KsplitWeights loads, hipStream_t s) {
+#define CMX_KS(FW_, FM_, NW_) if (t.fw == FW_ && t.fm == FM_ && t.waves == NW_) return launch_one<FMT, FW_, FM_, NW_, EPI, TILED, KsplitWeights::kCached>(p, max_m_tiles, s)
+    if (t.fw == 4 && t.fm == 4 && t.waves == 4 && p.row_off != nullptr) {
+        if (loads == KsplitWeights::kStreamed) return launch_one<FMT, 4, 4, 4, EPI, TILED, KsplitWeights::kStreamed>(p, max_m_tiles, s);
+        return launch_one<FMT, 4, 4, 4, EPI, TILED, KsplitWeights::kByGroup>(p, max_m_tiles, s);
     }
     if constexpr (EPI == kEpiStore && !TILED) {
+        CMX_KS(4, 4, 4);
         CMX_KS(1, 1, 8);
         CMX_KS(1, 2, 8);
         CMX_KS(2, 1, 8);
@@ -545,19 +555,19 @@ size_t ksplit_lds_bytes(const KsplitTile& t, int fmt, uint32_t kblocks, bool til
     return loop > sums ? loop : sums;
 }
 
-int launch_ksplit(const GemmParams& p, const KsplitTile& t, int fmt, int epi, uint32_t max_m_tiles, bool stream, hipStream_t s) {
+int launch_ksplit(const GemmParams& p, const KsplitTile& t, int fmt, int epi, uint32_t max_m_tiles, KsplitWeights loads, hipStream_t s) {
     if (fmt == CMX_FMT_E4M3) {
         if (epi == kEpiStore)
-            return p.w_pretiled ? launch_shape<CMX_FMT_E4M3, kEpiStore, true>(p, t, max_m_tiles, stream, s) : launch_shape<CMX_FMT_E4M3, kEpiStore, false>(p, t, max_m_tiles, stream, s);
+            return p.w_pretiled ? launch_shape<CMX_FMT_E4M3, kEpiStore, true>(p, t, max_m_tiles, loads, s) : launch_shape<CMX_FMT_E4M3, kEpiStore, false>(p, t, max_m_tiles, loads, s);
         if (epi == kEpiSwigluQuant)
-            return p.w_pretiled ? launch_shape<CMX_FMT_E4M3, kEpiSwigluQuant, true>(p, t, max_m_tiles, stream, s)
-                                : launch_shape<CMX_FMT_E4M3, kEpiSwigluQuant, false>(p, t, max_m_tiles, stream, s);
-        if (epi == kEpiSwigluQuantAct && !p.w_pretiled) return launch_shape<CMX_FMT_E4M3, kEpiSwigluQuantAct, false>(p, t, max_m_tiles, stream, s);
+            return p.w_pretiled ? launch_shape<CMX_FMT_E4M3, kEpiSwigluQuant, true>(p, t, max_m_tiles, loads, s)
+                                : launch_shape<CMX_FMT_E4M3, kEpiSwigluQuant, false>(p, t, max_m_tiles, loads, s);
+        if (epi == kEpiSwigluQuantAct && !p.w_pretiled) return launch_shape<CMX_FMT_E4M3, kEpiSwigluQuantAct, false>(p, t, max_m_tiles, loads, s);
     }
     if (fmt == CMX_FMT_E5M2 && epi == kEpiStore)
-        return p.w_pretiled ? launch_shape<CMX_FMT_E5M2, kEpiStore, true>(p, t, max_m_tiles, stream, s) : launch_shape<CMX_FMT_E5M2, kEpiStore, false>(p, t, max_m_tiles, stream, s);
-    if (fmt == CMX_FMT_E2M1 && epi == kEpiStore) return launch_shape<CMX_FMT_E2M1, kEpiStore, false>(p, t, max_m_tiles, stream, s);
-    if (fmt == kFmtI8 && epi == kEpiI8DequantSwiglu) return launch_shape<kFmtI8, kEpiI8DequantSwiglu, false>(p, t, max_m_tiles, stream, s);
+        return p.w_pretiled ? launch_shape<CMX_FMT_E5M2, kEpiStore, true>(p, t, max_m_tiles, loads, s) : launch_shape<CMX_FMT_E5M2, kEpiStore, false>(p, t, max_m_tiles, loads, s);
+    if (fmt == CMX_FMT_E2M1 && epi == kEpiStore) return launch_shape<CMX_FMT_E2M1, kEpiStore, false>(p, t, max_m_tiles, loads, s);
+    if (fmt == kFmtI8 && epi == kEpiI8DequantSwiglu) return launch_shape<kFmtI8, kEpiI8DequantSwiglu, false>(p, t, max_m_tiles, loads, s);
     set_error("unsupported split-K problem");
     return CMX_EINVAL;
 }

@@ -221,13 +221,13 @@ SKEWED = [1300, 0, 64, 65, 1, 700, 33, 63] + [0] * 55 + [66]
 
 @pytest.mark.parametrize("cut", [0, 5])
 def test_skewed_groups_take_the_kernel_of_their_size(cut):
-    """64 groups that average 36 rows, 576 and more tiles of 64 x 64: the groups of at most 64 rows have the bits of the split-K
+    """64 groups that average 36 rows, 1152 tiles of 64 x 64 where 1024 are the most for one launch: the groups of at most 64 rows have the bits of the split-K
     kernel (four partial sums), the others those of the 256-row kernel (one chain over K), on row-major and on pre-tiled
     weights.  cut: the operands hold five rows less than the groups ask for, which makes the last group one of 61."""
     from catccos_amd import _lib, ops
     h = hooks_lib()
     rng = np.random.default_rng(11 + cut)
-    n, k, e = 1024, 512, len(SKEWED)
+    n, k, e = 2048, 512, len(SKEWED)
     m = sum(SKEWED) - cut
     counts = SKEWED[:-1] + [SKEWED[-1] - cut]
     small = np.repeat([0 < c <= 64 for c in counts], counts)
