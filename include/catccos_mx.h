@@ -108,6 +108,9 @@ int cmx_mx_dequant(const uint8_t* codes, uint32_t ld_codes, const uint8_t* scale
  *   a  codes [m, k] (FP4: k/2 bytes), pitch lda bytes;  a_scale u8 [m, k/32], pitch ld_as bytes
  *   b  codes [n, k] (transposed weight), pitch ldb;     b_scale u8 [n, k/32], pitch ld_bs
  *   c  [m, n] of out_type, pitch ldc elements
+ * A row's fp32 sums depend on the operands, the sizes and the number of CUs of the device only.  They are not batch-invariant:
+ * with few rows or columns K is split between wavefronts, so the same row can differ in its last bits between calls
+ * with different m or n.
  * k must be a multiple of 32; operand rows 16-byte aligned.
  * ---------------------------------------------------------------------------------------- */
 int cmx_mx_gemm(const uint8_t* a, uint32_t lda, const uint8_t* a_scale, uint32_t ld_as, const uint8_t* b,
@@ -128,6 +131,8 @@ int cmx_mx_gemm(const uint8_t* a, uint32_t lda, const uint8_t* a_scale, uint32_t
  *   c            [m_total, n]
  *   workspace    >= cmx_mx_gmm_workspace_bytes(groups) bytes (tile schedule metadata)
  * Rows beyond sum(group_sizes) (up to m_total) are left untouched.
+ * As for the dense matmul the fp32 sums of a row can differ in their last bits between batches: they depend on m_total, groups
+ * and n, and on whether the row's group has more than 64 rows.  Row-major and pre-tiled weights give the same bits.
  * ---------------------------------------------------------------------------------------- */
 size_t cmx_mx_gmm_workspace_bytes(uint32_t groups);
 int cmx_mx_gmm(const uint8_t* a, uint32_t lda, const uint8_t* a_scale, uint32_t ld_as, const uint8_t* b,

@@ -162,17 +162,19 @@ def test_scale_rows_at_any_byte_give_the_bits_of_aligned_ones(shape, fmt, k):
 
 @pytest.mark.parametrize("fmt,out,m,n,k", [("E4M3", "bf16", *mnk) for mnk in ((1000, 4000, 512), (1024, 4104, 512), (1024, 4096, 2048), (1024, 4096, 2176),
                                                                                (2048, 4096, 96), (2049, 4096, 96), (520, 4000, 256))] +
-                         [("E5M2", "bf16", 1000, 4000, 512), ("E4M3", "fp16", 1000, 4000, 512), ("E5M2", "fp32", 1000, 4004, 512)])
+                         [("E5M2", "bf16", 1000, 4000, 512), ("E4M3", "fp16", 1000, 4000, 512), ("E5M2", "fp32", 1000, 4004, 512),
+                          ("E4M3", "fp32", 2100, 4104, 512), ("E4M3", "bf16", 2100, 4104, 1024), ("E2M1", "fp32", 2100, 4104, 512), ("E2M1", "bf16", 1000, 4104, 1024)])
 @pytest.mark.parametrize("aligned", [True, False])
 def test_sizes_on_both_sides_of_the_dense_rules(fmt, out, m, n, k, aligned):
-    """256 and more 128 x 128 tiles; more than 2048 64 x 64 tiles where K is no whole number of slabs; the kernel that the
+    """256 and more 128 x 128 tiles; more than 1024 64 x 64 tiles, 2048 where K is no whole number of slabs; the kernel that the
     library chooses against the oracle.  Scale rows at an odd pitch (which takes the 128 x 128 and 256-row tiles to the
     register-staged kernel) give the bits of aligned ones."""
     from catccos_amd import _lib, ops
     rng = np.random.default_rng(m + n + k)
     aq, asc = _mx(rng, m, k, fmt)
     bq, bsc = _mx(rng, n, k, fmt)
-    a, b = dev(aq), dev(bq)
+    pack = O.pack_fp4 if fmt == "E2M1" else (lambda x: x)
+    a, b = dev(pack(aq)), dev(pack(bq))
     if not aligned:
         asc = (asc + rng.integers(-8, 9, asc.shape)).astype(np.uint8)      # (with equal scales most sums are exact in any order)
     c = ops.mx_gemm(a, dev(asc), b, dev(bsc), k, fmt, out)
@@ -180,8 +182,8 @@ def test_sizes_on_both_sides_of_the_dense_rules(fmt, out, m, n, k, aligned):
         pitch = (k // 32) | 1
         sa, sb = dev(np.pad(asc[:, :k // 32], ((0, 0), (0, pitch - k // 32)))), dev(np.pad(bsc[:, :k // 32], ((0, 0), (0, pitch - k // 32))))
         got = torch.empty_like(c)
-        _lib.check(_lib.load().cmx_mx_gemm(a.data_ptr(), k, sa.data_ptr(), pitch, b.data_ptr(), k, sb.data_ptr(), pitch, got.data_ptr(), n, m, n, k,
-                                           ops.FMT[fmt], ops.OUT[out], torch.cuda.current_stream().cuda_stream))
+        _lib.check(_lib.load().cmx_mx_gemm(a.data_ptr(), a.shape[1], sa.data_ptr(), pitch, b.data_ptr(), b.shape[1], sb.data_ptr(), pitch, got.data_ptr(), n, m, n,
+                                           k, ops.FMT[fmt], ops.OUT[out], torch.cuda.current_stream().cuda_stream))
         assert torch.equal(got, c)
         return
     gold = (O.mx_dequant(aq, asc, fmt).astype(np.float32) @ O.mx_dequant(bq, bsc, fmt).astype(np.float32).T)
