@@ -24,6 +24,7 @@
 
 #include "mx_gemm_common.h"
 #include "mx_gemm_ksplit.h"
+#include "mx_gemm_ring.h"
 #include "mx_launch.h"
 
 namespace cmx {
@@ -1002,6 +1003,7 @@ int launch_gemm(const GemmParams& p, uint32_t max_m_tiles, hipStream_t s) {
 struct TileChoice {
     int tw, tm, waves;
 };
+constexpr int kForceRing = 6;          // `waves` of a pinned tile that stands for the ring kernel
 
 #ifdef CMX_TEST_HOOKS
 TileChoice g_force_tile = {0, 0, 0};   // tw == 0 -> heuristic
@@ -1022,19 +1024,41 @@ bool ksplit_is_forced(KsplitTile* out) {
     return g_force_ksplit.fw != 0 || g_force_tile.tw != 0 || g_disable_dl;
 }
 
-// Dense 8-bit problems that 128 x 128 tiles of four wavefronts (mx_gemm_kernel) take: too many 64 x 64 tiles for the split-K
-// kernel to run in two rounds of a workgroup per CU, few enough 128 x 128 tiles for one, and K up to 2048: a tile of twice the
-// side pulls half the bytes per product through the vector cache, while a long K is better split between more wavefronts.
-// Measured (us, E4M3, 64 x 64 split-K -> 128 x 128): 1024 x 4096 at K = 512 12.4 -> 10.0, 1024 15.8 -> 12.2, 2048 22.3 -> 17.1,
-// 4096 33.8 against 33.1, 7168 55.2 against 52.2 (behind the pass that writes its weights, 62 against 64); 760 x 3072 x 2048 (576
-// 64 x 64 tiles) 18.7 -> 15.8, 640 x 4096 x 4096 (640) 28.4 against 33.0.
-// The alignment of the scale rows does not enter, because it must not change the sums; rows that are not dword-aligned run the 128 x
-// 128 tile on the register-staged kernel with its byte loads: 1024 x 4096 x 2048 18.5 aligned, 32.0 not (256-row tiles 24.6 and 61.4; 64
-// x 64 split-K would take 23.9 and 23.1).
+// Dense 8-bit problems that 128 x 128 tiles of four wavefronts (mx_gemm_dl_kernel) take: K of 128, 256 or 384, too many 64 x 64 tiles
+// for the split-K kernel to run in two rounds of a workgroup per CU, few enough 128 x 128 tiles for one.  From K = 512 on it is the ring
+// kernel that takes these sizes (a row of scales shorter than 16 bytes goes to its LDS through registers: 1024 x 4096 x 256 9.0
+// here, 13.6 there).
+// The alignment of the scale rows does not enter, because it must not change the sums.
 bool takes_128_tile(uint32_t m, uint32_t n, int fmt, uint32_t kblocks, int cus) {
-    if (fmt == CMX_FMT_E2M1 || kblocks % 4 != 0 || kblocks > 64) return false;
+    if (fmt == CMX_FMT_E2M1 || kblocks % 4 != 0 || kblocks >= 16) return false;
     const uint64_t t64 = (uint64_t)ceil_div(n, 64) * ceil_div(m, 64), t128 = (uint64_t)ceil_div(n, 128) * ceil_div(m, 128);
     return t128 <= (uint64_t)cus && t64 > 2 * (uint64_t)cus;
+}
+
+// Dense 8-bit problems that the ring kernel (mx_gemm_ring.hip) takes, and the height of its tile (0: none): more 64 x 64 tiles than
+// the split-K kernel runs in two rounds of a workgroup per CU, and few enough tiles of 128 x 128, 192 or 256 for one round of
+// the ring kernel's.  Its sums are the 256-row kernels' (one chain over K), so the limit to those is a matter of time only; the limit
+// to split-K (whose sums differ in the last bits) goes by sizes alone.
+// Measured (us, E4M3, bf16 out, operands of three calls in turn; before -> ring, [K, N] = on weights stored [K, N], where
+// the other kernels need a pass of 9 (K = 4096) to 15 (7168) before them):
+//   n = 4096:      K = 512         1024            2048            4096            7168            3968 (no multiple of 512)
+//   m = 512    7.6 against 9.4  8.9   10.8     12.0   14.4     19.8   23.1     27.2   31.4     19.5   22.0       split-K stays
+//   700        9.5 ->  9.5     12.8 -> 11.3    18.1 -> 14.8    26.7 -> 24.0    40.3 -> 33.8    27.5 -> 22.8       128
+//   1024      10.0 ->  9.9     13.3 -> 11.8    19.0 -> 15.5    33.2 -> 25.3    50.4 -> 36.4    33.9 -> 23.8       128
+//   1280      11.7 against 11.8 15.7 -> 14.1   23.5 -> 18.6    38.9 -> 29.0    62.7 -> 44.0    51.3 -> 28.3       192
+//   1536      11.8 against 12.2 15.8 -> 14.7   24.4 -> 19.5    38.9 -> 30.7    62.3 -> 47.1    50.4 -> 30.6       192
+//   2048      12.1 against 14.9 16.3 against 18.0 24.1 against 24.9 39.7 -> 38.6 63.2 -> 59.8  52.0 -> 38.8       256
+//   2560      (two rounds)      16.6   24.8    25.3   33.9     43.2   57.4     70     86       54.3   55.6       256-row kernels
+//   2048, [K, N]  12 + 4 -> 16.7   16 + 5 -> 19.8  24 + 6 -> 26.9  40 + 9 -> 40.8  63 + 15 -> 62.4
+int ring_rows(uint32_t m, uint32_t n, int fmt, uint32_t kblocks, int cus, bool k_slow) {
+    if (fmt == CMX_FMT_E2M1 || kblocks % 4 != 0 || kblocks < 16) return 0;
+    if ((uint64_t)ceil_div(n, 64) * ceil_div(m, 64) <= 2 * (uint64_t)cus) return 0;
+    const auto one_round = [&](uint32_t tm) { return (uint64_t)ceil_div(n, kRingTileW) * ceil_div(m, tm) <= (uint64_t)cus; };
+    const bool slow_256 = k_slow || kblocks % 16 != 0;        // the 256-row kernels need a pass first, or are the streaming ones
+    if (one_round(128)) return 128;
+    if (one_round(192) && (slow_256 || kblocks >= 32)) return 192;
+    if (one_round(256) && (slow_256 || kblocks >= 128)) return 256;
+    return 0;
 }
 
 // Whether a problem goes to the split-K kernels (mx_gemm_ksplit.hip), and with which tile; fw == 0: no.  The choice depends
@@ -1063,7 +1087,7 @@ int choose_ksplit(uint32_t m, uint32_t n, int fmt, uint32_t kblocks, KsplitTile*
         }
     const KsplitTile t = {4, 4, 4};
     const uint64_t per_cu = fmt != CMX_FMT_E2M1 && kblocks % 4 != 0 ? 8 : 4;
-    if (tiles(t) <= per_cu * cus && !takes_128_tile(m, n, fmt, kblocks, cus) && fits(t)) *out = t;
+    if (tiles(t) <= per_cu * cus && !takes_128_tile(m, n, fmt, kblocks, cus) && ring_rows(m, n, fmt, kblocks, cus, false) == 0 && fits(t)) *out = t;
     return CMX_OK;
 }
 
@@ -1270,6 +1294,15 @@ extern "C" int cmx_debug_force_tile(int tw, int tm, int waves) {
 }
 #endif
 
+namespace cmx {
+namespace {
+int ring_gemm(GemmParams& p, int tm, int fmt, bool k_slow, hipStream_t s) {
+    p.w_tiles = ceil_div(p.n, kRingTileW);
+    return launch_ring(p, tm, fmt, k_slow, ceil_div(p.m, tm), s);
+}
+}  // namespace
+}  // namespace cmx
+
 extern "C" int cmx_mx_gemm(const uint8_t* a, uint32_t lda, const uint8_t* a_scale, uint32_t ld_as, const uint8_t* b,
                            uint32_t ldb, const uint8_t* b_scale, uint32_t ld_bs, void* c, uint32_t ldc, uint32_t m,
                            uint32_t n, uint32_t k, int fmt, int out_type, cmx_stream_t stream) {
@@ -1297,7 +1330,11 @@ extern "C" int cmx_mx_gemm(const uint8_t* a, uint32_t lda, const uint8_t* a_scal
     int cus = 0;
     if (rc = cu_count(&cus); rc != CMX_OK) return rc;
     TileChoice t = choose_tile(m, n, fmt, false);
-    if (!g_force_tile.tw && !g_disable_dl && takes_128_tile(m, n, fmt, p.kblocks, cus)) t = {128, 128, 4};
+    if (!g_force_tile.tw && !g_disable_dl) {
+        if (const int tm = ring_rows(m, n, fmt, p.kblocks, cus, false)) return ring_gemm(p, tm, fmt, false, s);
+        if (takes_128_tile(m, n, fmt, p.kblocks, cus)) t = {128, 128, 4};
+    }
+    if (t.waves == kForceRing) return ring_gemm(p, t.tm, fmt, false, s);
     p.w_tiles = ceil_div(n, t.tw);
     const uint32_t m_tiles = ceil_div(m, t.tm);
     switch (fmt) {
@@ -1305,6 +1342,33 @@ extern "C" int cmx_mx_gemm(const uint8_t* a, uint32_t lda, const uint8_t* a_scal
         case CMX_FMT_E5M2: return dispatch_tile<CMX_FMT_E5M2, kEpiStore>(p, t, m_tiles, s);
         default: return dispatch_tile<CMX_FMT_E2M1, kEpiStore>(p, t, m_tiles, s);
     }
+}
+
+// cmx_mx_gemm on weights stored [k, n] with scales [k / 64, n, 2], where a kernel reads them as they lie: `taken` says whether
+// one does (the caller has them rewritten otherwise).  The sums are those of the same problem on K-contiguous weights.
+int cmx::gemm_k_slow(const uint8_t* a, const uint8_t* a_scale, const uint8_t* b, const uint8_t* b_scale, void* c, uint32_t ldc, uint32_t m,
+                     uint32_t n, uint32_t k, int fmt, int out_type, hipStream_t s, bool* taken) {
+    *taken = false;
+    if (!(fmt == CMX_FMT_E4M3 || fmt == CMX_FMT_E5M2) || k % kSlabBytes != 0) return CMX_OK;
+    // 16-byte pieces of a row start at any dword; the matrix ends in a piece of its own
+    if (n % 4 != 0 || n < 16 || (reinterpret_cast<uintptr_t>(b) & 3u) != 0 || (uint64_t)k * n >= (1ull << 32)) return CMX_OK;
+    int cus = 0;
+    if (int rc = cu_count(&cus); rc != CMX_OK) return rc;
+    KsplitTile forced;
+    int tm = g_force_tile.waves == kForceRing ? g_force_tile.tm : (ksplit_is_forced(&forced) ? 0 : ring_rows(m, n, fmt, k / 32, cus, true));
+    if (tm == 0) return CMX_OK;
+    CMX_REQUIRE(a && a_scale && b && b_scale && aligned16(a), "operand rows must be 16-byte aligned");
+    CMX_REQUIRE(c && ldc >= n, "bad output");
+    CMX_REQUIRE(out_type == CMX_OUT_BF16 || out_type == CMX_OUT_FP16 || out_type == CMX_OUT_FP32, "unknown output type");
+    CMX_REQUIRE((uint64_t)k * 256 < (1ull << 32), "operand tile exceeds 32-bit offsets");
+    GemmParams p{};
+    p.a = a; p.a_scale = a_scale; p.w = b; p.w_scale = b_scale; p.c = c;
+    p.lda = k; p.ld_as = k / 32; p.ldw = n; p.ld_ws = 2 * n; p.ldc = ldc;
+    p.m = m; p.n = n; p.kbytes = k; p.kblocks = k / 32;
+    p.groups = 1; p.out_type = out_type;
+    p.scale_vec = scales_dword_aligned(a_scale, p.ld_as, b_scale, p.ld_ws);
+    *taken = true;
+    return ring_gemm(p, tm, fmt, true, s);
 }
 
 extern "C" size_t cmx_mx_gmm_workspace_bytes(uint32_t groups) {

@@ -16,6 +16,7 @@
 
 #include "catccos_mx.h"
 #include "mx_common.h"
+#include "mx_gemm_ring.h"
 
 namespace cmx {
 namespace {
@@ -401,7 +402,10 @@ extern "C" int cmx_mx_gemm_ex(const uint8_t* a, const uint8_t* a_scale, const ui
         a_scale = ws + L.a_scales;
     }
     if (!trans_b) {
-        int rc = normalise(b, b_scale, ws + L.b_codes, ws + L.b_scales, k, n, 1, fmt, s);
+        bool taken = false;
+        int rc = gemm_k_slow(a, a_scale, b, b_scale, c, ldc, m, n, k, fmt, out_type, s, &taken);
+        if (rc != CMX_OK || taken) return rc;
+        rc = normalise(b, b_scale, ws + L.b_codes, ws + L.b_scales, k, n, 1, fmt, s);
         if (rc != CMX_OK) return rc;
         b = ws + L.b_codes;
         b_scale = ws + L.b_scales;

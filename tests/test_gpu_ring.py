@@ -1,0 +1,84 @@
+"""The ring matmul kernel against the 256-row kernels, whose bits it promises (one chain over K), and the oracle: rows and columns that
+end inside a tile, fewer slabs than ring slots, more blocks of scales than their area holds, scale rows that are no whole number of
+16-byte pieces or start at any byte; weights stored [N, K] and [K, N]."""
+import numpy as np
+import pytest
+import torch
+
+from oracle import mx_oracle as O
+from tests.gpu_util import dev, hooked_library, hooks_lib
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(autouse=True)
+def _hooked():
+    with hooked_library():
+        yield
+
+
+def _operands(rng, m, n, k, fmt):
+    aq, asc = O.mx_quant(O.bf16_round(rng.standard_normal((m, k)).astype(np.float32)), fmt)
+    bq, bsc = O.mx_quant(O.bf16_round(rng.standard_normal((n, k)).astype(np.float32)), fmt)
+    # block scales over 2^16: with equal ones most sums are exact in any order
+    return aq, (asc[:, :k // 32] + rng.integers(-16, 1, (m, k // 32))).astype(np.uint8), bq, (bsc[:, :k // 32] + rng.integers(-8, 9, (n, k // 32))).astype(np.uint8)
+
+
+def _near(c, aq, asc, bq, bsc, fmt):
+    """2-norm: products keep 2^-13 of the largest of eight (below 1e-3 on any sum of them), a bf16 output adds half a step of 2^-8."""
+    gold = O.mx_dequant(aq, asc, fmt).astype(np.float32) @ O.mx_dequant(bq, bsc, fmt).astype(np.float32).T
+    got = c.float().cpu().numpy().astype(np.float64)
+    assert np.linalg.norm(got - gold) < 4e-3 * np.linalg.norm(gold)
+
+
+@pytest.mark.parametrize("tm", [128, 192, 256])
+@pytest.mark.parametrize("fmt,out,m,n,k", [("E4M3", "fp32", 1, 16, 128), ("E5M2", "fp32", 129, 132, 256), ("E4M3", "bf16", 260, 148, 640),
+                                           ("E4M3", "fp32", 191, 300, 2176), ("E5M2", "fp16", 130, 264, 1024), ("E4M3", "fp32", 66, 20, 9344)])
+def test_bits_of_the_256_row_kernels_on_both_weight_layouts(tm, fmt, out, m, n, k):
+    from catccos_amd import ops
+    rng = np.random.default_rng(m + n + k)
+    aq, asc, bq, bsc = _operands(rng, m, n, k, fmt)
+    a, a_s, b, b_s = dev(aq), dev(asc), dev(bq), dev(bsc)
+    fb, fbs = O.to_file_layout(bq, bsc, True)
+    h = hooks_lib()
+    h.cmx_debug_force_tile(256, 256, 8)
+    want = ops.mx_gemm(a, a_s, b, b_s, k, fmt, out)
+    h.cmx_debug_force_tile(128, tm, 6)
+    assert torch.equal(ops.mx_gemm(a, a_s, b, b_s, k, fmt, out), want)
+    assert torch.equal(ops.mx_gemm_ex(a, a_s, dev(fb), dev(fbs), m, n, k, fmt, out, 0, 0), want)
+    _near(want, aq, asc, bq, bsc, fmt)
+
+
+@pytest.mark.parametrize("tm", [128, 192, 256])
+@pytest.mark.parametrize("k", [384, 1152, 8832])
+def test_scale_rows_at_any_byte(tm, k):
+    """An odd pitch and an odd start; an output pitch wider than n keeps its rest."""
+    from catccos_amd import _lib, ops
+    rng = np.random.default_rng(k)
+    m, n, pitch = 70, 45, k // 32 | 1
+    aq, asc, bq, bsc = _operands(rng, m, n, k, "E4M3")
+    a, b = dev(aq), dev(bq)
+    hooks_lib().cmx_debug_force_tile(128, tm, 6)
+    want = ops.mx_gemm(a, dev(asc), b, dev(bsc), k, "E4M3", "fp32")
+
+    def shifted(s):
+        buf = torch.full((1 + s.shape[0] * pitch,), 200, dtype=torch.uint8, device="cuda")
+        buf[1:].view(s.shape[0], pitch)[:, :k // 32] = dev(s)
+        return buf[1:]
+    sa, sb, got = shifted(asc), shifted(bsc), torch.full((m, n + 3), 7.0, device="cuda")
+    _lib.check(_lib.load().cmx_mx_gemm(a.data_ptr(), k, sa.data_ptr(), pitch, b.data_ptr(), k, sb.data_ptr(), pitch, got.data_ptr(), n + 3, m, n, k,
+                                       ops.FMT["E4M3"], ops.OUT["fp32"], torch.cuda.current_stream().cuda_stream))
+    assert torch.equal(got[:, :n], want) and bool((got[:, n:] == 7.0).all())
+
+
+@pytest.mark.parametrize("m,n,k", [(700, 3008, 512), (1030, 4100, 640), (1300, 4096, 1024), (1700, 4092, 512), (1700, 4090, 512), (700, 3008, 576)])
+def test_chosen_kernels_give_one_result_for_both_weight_layouts(m, n, k):
+    """Sizes of one round of each ring tile, and beside them what has the weights rewritten: columns no multiple of four, K no whole
+    number of slabs."""
+    from catccos_amd import ops
+    rng = np.random.default_rng(m + n + k)
+    aq, asc, bq, bsc = _operands(rng, m, n, k, "E4M3")
+    fb, fbs = O.to_file_layout(bq, bsc, True)
+    want = ops.mx_gemm(dev(aq), dev(asc), dev(bq), dev(bsc), k)
+    assert torch.equal(ops.mx_gemm_ex(dev(aq), dev(asc), dev(fb), dev(fbs), m, n, k, trans_b=0), want)
+    _near(want, aq, asc, bq, bsc, "E4M3")
