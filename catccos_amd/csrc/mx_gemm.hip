@@ -1075,7 +1075,7 @@ int ring_rows(uint32_t m, uint32_t n, int fmt, uint32_t kblocks, int cus, bool k
 // 4096 x 3040 75 -> 47; 3000 x 5000 x 4064 (3713 tiles) 97 against 138, 8192 x 4096 x 7136 300 against 463.
 int choose_ksplit(uint32_t m, uint32_t n, int fmt, uint32_t kblocks, KsplitTile* out) {
     if (ksplit_is_forced(out)) return CMX_OK;
-    const auto fits = [&](const KsplitTile& t) { return ksplit_lds_bytes(t, fmt, kblocks, false) <= kKsplitMaxLds; };
+    const auto fits = [&](const KsplitTile& t) { return ksplit_lds_bytes(t, fmt, kblocks) <= kKsplitMaxLds; };
     int cus = 0;
     if (int rc = cu_count(&cus); rc != CMX_OK) return rc;
     const auto tiles = [&](const KsplitTile& t) { return (uint64_t)ceil_div(n, 16 * t.fw) * ceil_div(m, 16 * t.fm); };
@@ -1133,7 +1133,7 @@ int choose_grouped_ksplit(uint32_t m_total, uint32_t groups, uint32_t n, int fmt
     out->weights = KsplitWeights::kByGroup;
     if (ksplit_is_forced(&out->tile) || g_pretiled_tile_rows != 0) return CMX_OK;
     const KsplitTile t = {4, 4, 4};
-    if (ceil_div(m_total, groups) > (fmt == CMX_FMT_E2M1 ? 64u : 40u) || ksplit_lds_bytes(t, fmt, kblocks, false) > kKsplitMaxLds) return CMX_OK;
+    if (ceil_div(m_total, groups) > (fmt == CMX_FMT_E2M1 ? 64u : 40u) || ksplit_lds_bytes(t, fmt, kblocks) > kKsplitMaxLds) return CMX_OK;
     out->tile = t;
     int cus = 0;
     if (int rc = cu_count(&cus); rc != CMX_OK) return rc;
@@ -1344,6 +1344,20 @@ extern "C" int cmx_mx_gemm(const uint8_t* a, uint32_t lda, const uint8_t* a_scal
     }
 }
 
+namespace cmx {
+namespace {
+// Split-K problems on weights stored [k, n]: a tile of 64 columns takes half a line from each of its K rows, 128 a slab where K-contiguous
+// rows take 64 lines, and its time goes with K; the pass that rewrites the weights costs a launch and goes with k * n.  Measured (us,
+// with the pass -> as they lie): 16 x 4096 x 7168 26.3 -> 19.2, 64 28.5 -> 18.3, 256 36.1 -> 23.5, 512 46.7 -> 33.9; 16 x 8192 x 512 9.6 -> 5.1;
+// 16 x 7168 x 2048 16.4 -> 9.3; 64 x 2052 x 2048 13.1 -> 8.4; 64 x 512 x 4096 11.1 -> 8.3; 64 x 2048 x 8192 22.0 -> 16.3; but 64 x 1024 x 8192 13.0
+// against 17.3, 64 x 512 x 8192 13.4 against 17.3, 700 x 1536 x 8192 37 against 46.
+bool k_slow_pays(uint32_t n, uint32_t k) {
+    KsplitTile t;
+    return k <= 4096 || (uint64_t)n * k >= (16u << 20) || ksplit_is_forced(&t);
+}
+}  // namespace
+}  // namespace cmx
+
 // cmx_mx_gemm on weights stored [k, n] with scales [k / 64, n, 2], where a kernel reads them as they lie: `taken` says whether
 // one does (the caller has them rewritten otherwise).  The sums are those of the same problem on K-contiguous weights.
 int cmx::gemm_k_slow(const uint8_t* a, const uint8_t* a_scale, const uint8_t* b, const uint8_t* b_scale, void* c, uint32_t ldc, uint32_t m,
@@ -1354,9 +1368,16 @@ int cmx::gemm_k_slow(const uint8_t* a, const uint8_t* a_scale, const uint8_t* b,
     if (n % 4 != 0 || n < 16 || (reinterpret_cast<uintptr_t>(b) & 3u) != 0 || (uint64_t)k * n >= (1ull << 32)) return CMX_OK;
     int cus = 0;
     if (int rc = cu_count(&cus); rc != CMX_OK) return rc;
-    KsplitTile forced;
-    int tm = g_force_tile.waves == kForceRing ? g_force_tile.tm : (ksplit_is_forced(&forced) ? 0 : ring_rows(m, n, fmt, k / 32, cus, true));
-    if (tm == 0) return CMX_OK;
+    // the kernel that the same problem gets on K-contiguous weights: split-K, or one whose sums the ring kernel gives
+    KsplitTile ks;
+    if (int rc = choose_ksplit(m, n, fmt, k / 32, &ks); rc != CMX_OK) return rc;
+    int tm = 0;
+    if (ks.fw != 0) {
+        if (!k_slow_pays(n, k) || !ksplit_k_slow_tile(&ks, m, n, fmt, k / 32, cus)) return CMX_OK;
+    } else {
+        tm = g_force_tile.waves == kForceRing ? g_force_tile.tm : (g_force_tile.tw || g_disable_dl ? 0 : ring_rows(m, n, fmt, k / 32, cus, true));
+        if (tm == 0) return CMX_OK;
+    }
     CMX_REQUIRE(a && a_scale && b && b_scale && aligned16(a), "operand rows must be 16-byte aligned");
     CMX_REQUIRE(c && ldc >= n, "bad output");
     CMX_REQUIRE(out_type == CMX_OUT_BF16 || out_type == CMX_OUT_FP16 || out_type == CMX_OUT_FP32, "unknown output type");
@@ -1368,7 +1389,9 @@ int cmx::gemm_k_slow(const uint8_t* a, const uint8_t* a_scale, const uint8_t* b,
     p.groups = 1; p.out_type = out_type;
     p.scale_vec = scales_dword_aligned(a_scale, p.ld_as, b_scale, p.ld_ws);
     *taken = true;
-    return ring_gemm(p, tm, fmt, true, s);
+    if (tm != 0) return ring_gemm(p, tm, fmt, true, s);
+    p.w_tiles = ceil_div(n, 64);
+    return launch_ksplit_k_slow(p, ks, fmt, ceil_div(m, 16 * ks.fm), s);
 }
 
 extern "C" size_t cmx_mx_gmm_workspace_bytes(uint32_t groups) {

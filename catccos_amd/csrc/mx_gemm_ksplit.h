@@ -13,7 +13,7 @@ struct KsplitTile {
 // LDS bytes the kernel needs for a tile of a problem (scale rows of the whole tile and the exchange buffers, or the partial
 // sums), and the most it may ask for.
 constexpr size_t kKsplitMaxLds = 160 * 1024;
-size_t ksplit_lds_bytes(const KsplitTile& t, int fmt, uint32_t kblocks, bool tiled);
+size_t ksplit_lds_bytes(const KsplitTile& t, int fmt, uint32_t kblocks, int layout = 0);
 
 // How the weights are read.  kStreamed: non-temporal, for weights with one reader, which leaves the L2 to the activation rows (32
 // experts x 4 / 16 / 32 rows, K = 7168, N = 4096: 142 / 145 / 152 us with it, 160 / 162 / 172 without).  kCached: for weights that the
@@ -25,5 +25,12 @@ enum class KsplitWeights { kCached, kStreamed, kByGroup };
 // that pair gate and up) and, for grouped problems, group tables made for m-tiles of 16 * t.fm rows.  Dense problems read their
 // weights cached; `loads` is for grouped ones.
 int launch_ksplit(const GemmParams& p, const KsplitTile& t, int fmt, int epi, uint32_t max_m_tiles, KsplitWeights loads, hipStream_t s);
+
+
+// Weights stored [K][ldw] with scales [K / 64][n][2] at a pitch of ld_ws bytes (dense, 8-bit formats, K whole slabs, n a multiple of 4
+// and at least 16, p.w dword-aligned, K * ldw below 2^32): tiles of 64 columns with the wavefronts, and so the bits, of the tile that
+// the same problem gets on K-contiguous weights.  Turns *t into such a tile; false where its scales do not fit the LDS.
+bool ksplit_k_slow_tile(KsplitTile* t, uint32_t m, uint32_t n, int fmt, uint32_t kblocks, int cus);
+int launch_ksplit_k_slow(const GemmParams& p, const KsplitTile& t, int fmt, uint32_t max_m_tiles, hipStream_t s);
 
 }  // namespace cmx

@@ -13,6 +13,10 @@
 //     more time than whole 128-byte lines (16 x 4096 x 7168, operands in the memory-side cache: 9.7 against 7.2 us), so the lanes
 //     fetch whole lines, eight to a row, and a fragment changes places through 2 KiB of LDS that belong to the wavefront alone
 //     (its LDS accesses execute in order: nothing to wait for).  Pre-tiled weights are stored in the fragment order and need none of it;
+//   * weights stored [K, N] (kKSlow) are fetched as they lie, 64 columns of 128 K positions a slab, and turned on the way out of the
+//     exchange by ds_read_b64_tr_b8.  A K row of the tile is half a line, so the vector cache serves 128 + 16 FM visits a slab instead
+//     of 64 + 16 FM and bounds the kernel (16 x 4096 x 7168: 64 workgroups, 19 us, where K-contiguous weights take 9.3 on 256); a pass that
+//     rewrites the weights first brings that to 26;
 //   * the block scales of the tile, which are a byte per 32 elements in rows of their own, are fetched once, coalesced, for
 //     the whole of K into the LDS and read from there a byte per lane and fragment.
 // The NW partial sums meet in the LDS at the end and are added in the order of the wavefronts, so the result does not
@@ -32,6 +36,9 @@ namespace {
 
 typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
 
+// how the weights lie in memory: rows of K; tiled by cmx_mx_pretile_weights; rows of N (K the slow axis)
+enum WeightLayout { kRowMajor = 0, kTiled = 1, kKSlow = 2 };
+
 constexpr int ks_scale_steps(int fmt) { return fmt == kFmtI8 ? 0 : (fmt == CMX_FMT_E2M1 ? 2 : 1); }   // scale dwords per row and slab
 // slabs in the register ring: what fits beside the accumulators, one slab of fragments in MFMA order, their scales and
 // addresses in 256 registers (two wavefronts per SIMD).  The scale pieces in flight before the K loop (sreg, treg: up to 32
@@ -48,8 +55,13 @@ constexpr int ks_pass_frags(int fw, int fm, int nw) {
     while (n > 1 && nw * n * 16 * (16 * fw + 4) * 4 > 65536) n /= 2;
     return n;
 }
-// exchange buffers of a wavefront (2 KiB, one fragment): four, used in turn
-constexpr int ks_exchange_bufs(int fw, int fm, bool tiled) { return (tiled ? 0 : fw) + fm < 4 ? (tiled ? 0 : fw) + fm : 4; }
+// exchange buffers of a wavefront (2 KiB, one fragment): four, used in turn; K-slow weights change places a whole slab at a time, in
+// four more, and leave two to the activations
+constexpr int ks_exchange_bufs(int fw, int fm, int layout) {
+    if (layout == kKSlow) return fw + (fm < 2 ? fm : 2);
+    const int n = (layout == kTiled ? 0 : fw) + fm;
+    return n < 4 ? n : 4;
+}
 constexpr size_t ks_sum_bytes(int fw, int fm, int nw) { return (size_t)nw * ks_pass_frags(fw, fm, nw) * 16 * (16 * fw + 4) * 4; }
 // dwords of a scale row in the LDS: whole slabs, an odd count so that the sixteen rows of a fragment lie in different banks
 __host__ __device__ inline uint32_t ks_scale_pitch(int fmt, uint32_t kblocks) {
@@ -79,13 +91,15 @@ __device__ __forceinline__ v4f ks_mfma(const v4i (&w)[2], const v4i (&a)[2], v4f
 }
 
 // STREAM: weights are loaded non-temporal (KsplitWeights)
-template <int FMT, int FW, int FM, int NW, int EPI, bool TILED, bool STREAM>
+template <int FMT, int FW, int FM, int NW, int EPI, int LAYOUT, bool STREAM>
 __device__ __forceinline__ void ks_tile(const GemmParams& p, const Tile& tc, uint8_t* smem) {
     constexpr int NT = 64 * NW, TW = 16 * FW;
     constexpr int kS = ks_scale_steps(FMT);
     constexpr int kSA = kS ? kS : 1;
     constexpr int PD = ks_ring(FMT, FW, FM);
-    constexpr int kRows = 16 * (FW + FM);
+    constexpr bool TILED = LAYOUT == kTiled, KSLOW = LAYOUT == kKSlow;
+    constexpr int kScaleW = KSLOW ? 0 : TW, kRows = kScaleW + 16 * FM;            // rows of scales: weights (unless K-slow), activations
+    static_assert(!KSLOW || (FW == 4 && kS == 1 && EPI == kEpiStore), "K-slow weights: 64 columns, 8-bit formats");
     const uint32_t tid = threadIdx.x, lane = tid & 63u;
     const uint32_t wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const uint32_t r = lane & 15u, g = lane >> 4;
@@ -104,12 +118,19 @@ __device__ __forceinline__ void ks_tile(const GemmParams& p, const Tile& tc, uin
     };
     auto arow_of = [&](uint32_t t) -> uint32_t { return t < tc.rows_valid ? t : tc.rows_valid - 1; };
 
+    // K-slow: first column of the tile's 16-column chunk c; one that the matrix ends inside of is moved back to end with it, one past
+    // the end repeats the last
+    auto wcol_of = [&](uint32_t c) -> uint32_t {
+        const uint32_t col = tc.wt * TW + 16 * c;
+        return col + 16 <= p.n ? col : p.n - 16;
+    };
+
     // ---- scales of the tile: request -----------------------------------------------------------------------------------
     const uint32_t pitch = ks_scale_pitch(FMT, p.kblocks);
     uint32_t* const s_sc = reinterpret_cast<uint32_t*>(smem);
     auto scale_row = [&](uint32_t t) -> const uint8_t* {
-        return t < (uint32_t)TW ? p.w_scale + ((size_t)tc.g * p.n + wrow_of(t)) * p.ld_ws
-                                : p.a_scale + (size_t)(tc.row0 + arow_of(t - TW)) * p.ld_as;
+        return t < (uint32_t)kScaleW ? p.w_scale + ((size_t)tc.g * p.n + wrow_of(t)) * p.ld_ws
+                                     : p.a_scale + (size_t)(tc.row0 + arow_of(t - kScaleW)) * p.ld_as;
     };
     // Whole 16-byte pieces, numbered with the next power of two of pieces per row (no division), and behind them the up to
     // 15 bytes of a row that is no whole number of pieces as four dwords (none reaches past the row: the last is read from its
@@ -141,6 +162,26 @@ __device__ __forceinline__ void ks_tile(const GemmParams& p, const Tile& tc, uin
             }
         }
     };
+    // K-slow weights: pairs of scales [K / 64][64 columns] behind the rows, in pieces of eight columns
+    uint8_t* const s_pairs = smem + kRows * pitch * 4 + ((0u - kRows * pitch * 4) & 15u);
+    const uint32_t pair_pieces = KSLOW ? p.kblocks / 2 * 8 : 0;
+    constexpr int kPairBatch = KSLOW ? 1024 / NT : 1;          // K = 8192 in flight together
+    u32x4 preg[kPairBatch];
+    auto request_pairs = [&](uint32_t i0) {
+#pragma unroll
+        for (int b = 0; b < kPairBatch; ++b) {
+            const uint32_t i = i0 + b * NT + tid;
+            if (i < pair_pieces) __builtin_memcpy(&preg[b], p.w_scale + (size_t)(i / 8) * p.ld_ws + 2 * (wcol_of(i % 8 / 2) + i % 2 * 8), 16);
+        }
+    };
+    auto deposit_pairs = [&](uint32_t i0) {
+#pragma unroll
+        for (int b = 0; b < kPairBatch; ++b) {
+            const uint32_t i = i0 + b * NT + tid;
+            if (i < pair_pieces) *reinterpret_cast<u32x4*>(s_pairs + i * 16) = preg[b];
+        }
+    };
+    if constexpr (KSLOW) request_pairs(0);
     if constexpr (kS != 0) {
         request16(0);
         if (ragged && p.kblocks >= 4) {
@@ -184,6 +225,13 @@ __device__ __forceinline__ void ks_tile(const GemmParams& p, const Tile& tc, uin
             woff[f][0] = blk * 8192 + frag * 2048 + (g >> 1) * 1024 + (g & 1u) * 512 + row * 16;
             woff[f][1] = woff[f][0] + 4096;
         }
+    } else if constexpr (KSLOW) {
+        // load 2 f + h: 16 K rows of 64 bytes, lane -> row lane / 4, columns 16 (lane % 4) ..
+        wbase = p.w;
+#pragma unroll
+        for (int f = 0; f < FW; ++f)
+#pragma unroll
+            for (int h = 0; h < 2; ++h) woff[f][h] = (32 * f + 16 * h + (lane >> 2)) * p.ldw + wcol_of(lane & 3u);
     } else {
         wbase = p.w + (size_t)tc.g * p.n * p.ldw;
 #pragma unroll
@@ -197,7 +245,7 @@ __device__ __forceinline__ void ks_tile(const GemmParams& p, const Tile& tc, uin
         for (int h = 0; h < 2; ++h) aoff[f][h] = arow_of(f * 16 + 8 * h + x_row) * p.lda + x_chunk * 16;
     const __amdgpu_buffer_rsrc_t w_rs = __builtin_amdgcn_make_buffer_rsrc(uniform_ptr(wbase), 0, -1, kRsrcFlags);
     const __amdgpu_buffer_rsrc_t a_rs = __builtin_amdgcn_make_buffer_rsrc(uniform_ptr(p.a + (size_t)tc.row0 * p.lda), 0, -1, kRsrcFlags);
-    constexpr uint32_t kWSlab = TILED ? 256 * kSlabBytes : kSlabBytes;
+    const uint32_t kWSlab = TILED ? 256 * kSlabBytes : (KSLOW ? kSlabBytes * p.ldw : kSlabBytes);
     constexpr int kWAux = STREAM ? 2 : 0;              // 2: non-temporal
 
     v4i wf[PD][FW][2], af[PD][FM][2];
@@ -222,6 +270,13 @@ __device__ __forceinline__ void ks_tile(const GemmParams& p, const Tile& tc, uin
     for (int d = 0; d < PD; ++d) load_slot(d, wave + NW * d);
 
     // ---- scales of the tile: deposit -----------------------------------------------------------------------------------
+    if constexpr (KSLOW) {
+        deposit_pairs(0);
+        for (uint32_t i0 = kPairBatch * NT; i0 < pair_pieces; i0 += kPairBatch * NT) {
+            request_pairs(i0);
+            deposit_pairs(i0);
+        }
+    }
     if constexpr (kS != 0) {
         deposit16(0);
         if (ragged) {
@@ -248,7 +303,8 @@ __device__ __forceinline__ void ks_tile(const GemmParams& p, const Tile& tc, uin
         __syncthreads();
     }
     const uint8_t* const sw_row = smem + r * pitch * 4 + g;
-    const uint8_t* const sa_row = smem + (TW + r) * pitch * 4 + g;
+    const uint8_t* const sa_row = smem + (kScaleW + r) * pitch * 4 + g;
+    const uint8_t* const sp_col = s_pairs + (g >> 1) * 128 + r * 2 + (g & 1u);
 
     v4f acc[FW][FM];
 #pragma unroll
@@ -258,8 +314,8 @@ __device__ __forceinline__ void ks_tile(const GemmParams& p, const Tile& tc, uin
 
     // a fragment from the order of the loads (rows 8 h + lane / 8, chunk lane % 8) to that of the MFMA (row lane % 16, chunks
     // lane / 16 and 4 + lane / 16); chunks XOR-swizzled by row: neither side meets bank conflicts
-    constexpr int kBufs = ks_exchange_bufs(FW, FM, TILED);
-    uint8_t* const xbuf = smem + kRows * pitch * 4 * (kS ? 1 : 0) + ((0u - kRows * pitch * 4 * (kS ? 1 : 0)) & 15u) + wave * (kBufs * 2048);
+    constexpr int kBufs = ks_exchange_bufs(FW, FM, LAYOUT), kWBufs = KSLOW ? FW : 0;
+    uint8_t* const xbuf = (kS ? s_pairs : smem) + pair_pieces * 16 + wave * (kBufs * 2048);
     uint32_t xw[2], xr[2];
 #pragma unroll
     for (int h = 0; h < 2; ++h) {
@@ -272,18 +328,47 @@ __device__ __forceinline__ void ks_tile(const GemmParams& p, const Tile& tc, uin
         asm("" : "+v"(xw[h]), "+v"(xr[h]));
     }
     auto exchange = [&](int buf, const v4i (&in)[2], v4i (&out)[2]) {
-        uint8_t* const b = xbuf + buf % kBufs * 2048;
+        uint8_t* const b = xbuf + (kWBufs + buf % (kBufs - kWBufs)) * 2048;
 #pragma unroll
         for (int h = 0; h < 2; ++h) *reinterpret_cast<v4i*>(b + xw[h]) = in[h];
 #pragma unroll
         for (int h = 0; h < 2; ++h) out[h] = *reinterpret_cast<const v4i*>(b + xr[h]);
     };
+    // K-slow: a slab as [128 K][64 columns], the 16-column pieces of a row XOR-swizzled; a fragment (column lane % 16, K 16 (lane / 16) ..
+    // and 64 + 16 (lane / 16) ..) by four transposing reads: lanes 16 i .. 16 i + 15 read eight K rows x 16 columns, two lanes to a row,
+    // and each gets the eight K values of its column.  Neither side meets bank conflicts.
+    auto kslow_piece = [](uint32_t k, uint32_t c) -> uint32_t { return k * 64 + (c ^ ((k >> 2 & 1u) | (k >> 3 & 2u))) * 16; };
+    uint32_t kw = kslow_piece(lane >> 2, lane & 3u), kr[2];
+#pragma unroll
+    for (int j = 0; j < 2; ++j) kr[j] = kslow_piece(16 * g + 8 * j + (r >> 1), 0) + (r & 1u) * 8;
+    asm("" : "+v"(kw), "+v"(kr[0]), "+v"(kr[1]));                                // as for xw and xr
+    typedef __attribute__((address_space(3))) v2i* lds_v2i;
+    auto exchange_kslow = [&](const v4i (&in)[FW][2], v4i (&out)[FW][2]) {
+#pragma unroll
+        for (int f = 0; f < FW; ++f)
+#pragma unroll
+            for (int h = 0; h < 2; ++h)
+                // (rows 16 apart from load to load: the swizzle's second bit changes with h)
+                *reinterpret_cast<v4i*>(xbuf + (2 * f + h) * 1024 + (kw ^ (h ? 32u : 0u))) = in[f][h];
+#pragma unroll
+        for (int f = 0; f < FW; ++f)
+#pragma unroll
+            for (int h = 0; h < 2; ++h)
+#pragma unroll
+                for (int j = 0; j < 2; ++j) {
+                    const uint8_t* at = xbuf + 4096 * h + (kr[j] ^ (16u * f));
+                    const v2i v = __builtin_amdgcn_ds_read_tr8_b64_v2i32((lds_v2i)(uintptr_t)(__attribute__((address_space(3))) const uint8_t*)at);
+                    out[f][h][2 * j] = v[0];
+                    out[f][h][2 * j + 1] = v[1];
+                }
+    };
     auto multiply = [&](const v4i (&wl)[FW][2], const v4i (&al)[FM][2], uint32_t s) {
         v4i w[FW][2], a[FM][2];
 #pragma unroll
         for (int f = 0; f < FM; ++f) exchange(f, al[f], a[f]);
+        if constexpr (KSLOW) exchange_kslow(wl, w);
 #pragma unroll
-        for (int f = 0; f < FW; ++f) {
+        for (int f = 0; f < FW && !KSLOW; ++f) {
             if constexpr (TILED) {
                 w[f][0] = wl[f][0];
                 w[f][1] = wl[f][1];
@@ -295,7 +380,7 @@ __device__ __forceinline__ void ks_tile(const GemmParams& p, const Tile& tc, uin
 #pragma unroll
         for (int j = 0; j < kS; ++j) {
 #pragma unroll
-            for (int f = 0; f < FW; ++f) sw[f][j] = sw_row[f * 16 * pitch * 4 + s * (4 * kSA) + 4 * j];
+            for (int f = 0; f < FW; ++f) sw[f][j] = KSLOW ? sp_col[s * 256 + f * 32] : sw_row[f * 16 * pitch * 4 + s * (4 * kSA) + 4 * j];
 #pragma unroll
             for (int f = 0; f < FM; ++f) sa[f][j] = sa_row[f * 16 * pitch * 4 + s * (4 * kSA) + 4 * j];
         }
@@ -319,7 +404,7 @@ __device__ __forceinline__ void ks_tile(const GemmParams& p, const Tile& tc, uin
     for (int d = 0; d < PD; ++d)
         if (i + d < mine) multiply(wf[d], af[d], wave + NW * (i + d));
     // K not a whole number of slabs: the rest, zeros past K
-    if constexpr (FMT != kFmtI8 && !TILED) {
+    if constexpr (FMT != kFmtI8 && LAYOUT == kRowMajor) {
         if (p.kbytes % kSlabBytes != 0 && nslab % NW == wave) {
 #pragma unroll
             for (int h = 0; h < 2; ++h) {
@@ -371,24 +456,26 @@ __device__ __forceinline__ void ks_tile(const GemmParams& p, const Tile& tc, uin
             const v4f v = total(4 * q);
             v4f u = v;
             if constexpr (epi_pairs_gate_up(EPI)) u = total(TW / 2 + 4 * q);
-            store_quad<EPI>(p, tc, f0 * 16 + m, tc.wt * (epi_pairs_gate_up(EPI) ? TW / 2 : TW) + 4 * q, v, u);
+            uint32_t ncol = tc.wt * (epi_pairs_gate_up(EPI) ? TW / 2 : TW) + 4 * q;
+            if constexpr (KSLOW) ncol = ncol / 16 * 16 < p.n ? wcol_of(q / 4) + q % 4 * 4 : p.n;
+            store_quad<EPI>(p, tc, f0 * 16 + m, ncol, v, u);
         }
     }
 }
 
 // a ragged tile does the work of the rows it has
-template <int FMT, int FW, int FM, int NW, int EPI, bool TILED, bool STREAM>
+template <int FMT, int FW, int FM, int NW, int EPI, int LAYOUT, bool STREAM>
 __device__ __forceinline__ void ks_rows(const GemmParams& p, const Tile& tc, uint8_t* smem) {
     if constexpr (FM >= 4) {
-        if (tc.rows_valid <= 16 * FM / 4) return ks_tile<FMT, FW, FM / 4, NW, EPI, TILED, STREAM>(p, tc, smem);
+        if (tc.rows_valid <= 16 * FM / 4) return ks_tile<FMT, FW, FM / 4, NW, EPI, LAYOUT, STREAM>(p, tc, smem);
     }
     if constexpr (FM >= 2) {
-        if (tc.rows_valid <= 16 * FM / 2) return ks_tile<FMT, FW, FM / 2, NW, EPI, TILED, STREAM>(p, tc, smem);
+        if (tc.rows_valid <= 16 * FM / 2) return ks_tile<FMT, FW, FM / 2, NW, EPI, LAYOUT, STREAM>(p, tc, smem);
     }
-    ks_tile<FMT, FW, FM, NW, EPI, TILED, STREAM>(p, tc, smem);
+    ks_tile<FMT, FW, FM, NW, EPI, LAYOUT, STREAM>(p, tc, smem);
 }
 
-template <int FMT, int FW, int FM, int NW, int EPI, bool TILED, KsplitWeights LOADS>
+template <int FMT, int FW, int FM, int NW, int EPI, int LAYOUT, KsplitWeights LOADS>
 __global__ __launch_bounds__(64 * NW, 2) void mx_gemm_ksplit_kernel(const GemmParams p) {
     extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
     Tile tc;
@@ -399,16 +486,16 @@ __global__ __launch_bounds__(64 * NW, 2) void mx_gemm_ksplit_kernel(const GemmPa
     tc.rows_valid = __builtin_amdgcn_readfirstlane(tc.rows_valid);
     if constexpr (LOADS == KsplitWeights::kByGroup) {
         if (__builtin_amdgcn_readfirstlane(tc.mt != 0 || tc.rows_left > 16u * FM))
-            return ks_rows<FMT, FW, FM, NW, EPI, TILED, false>(p, tc, smem);
+            return ks_rows<FMT, FW, FM, NW, EPI, LAYOUT, false>(p, tc, smem);
     }
-    ks_rows<FMT, FW, FM, NW, EPI, TILED, LOADS != KsplitWeights::kCached>(p, tc, smem);
+    ks_rows<FMT, FW, FM, NW, EPI, LAYOUT, LOADS != KsplitWeights::kCached>(p, tc, smem);
 }
 
-template <int FMT, int FW, int FM, int NW, int EPI, bool TILED, KsplitWeights LOADS>
+template <int FMT, int FW, int FM, int NW, int EPI, int LAYOUT, KsplitWeights LOADS>
 int launch_one(const GemmParams& p, uint32_t max_m_tiles, hipStream_t s) {
-    constexpr auto kfn = mx_gemm_ksplit_kernel<FMT, FW, FM, NW, EPI, TILED, LOADS>;
+    constexpr auto kfn = mx_gemm_ksplit_kernel<FMT, FW, FM, NW, EPI, LAYOUT, LOADS>;
     if (int rc = allow_dynamic_lds<kfn, kKsplitMaxLds>(); rc != CMX_OK) return rc;
-    const size_t smem = ksplit_lds_bytes({FW, FM, NW}, FMT, p.kblocks, TILED);
+    const size_t smem = ksplit_lds_bytes({FW, FM, NW}, FMT, p.kblocks, LAYOUT);
     CMX_REQUIRE(smem <= kKsplitMaxLds, "split-K tile exceeds the LDS");
     const uint64_t tiles = (uint64_t)max_m_tiles * p.w_tiles;
     CMX_REQUIRE(tiles > 0 && tiles < (1ull << 31), "tile count out of range");
@@ -418,14 +505,20 @@ int launch_one(const GemmParams& p, uint32_t max_m_tiles, hipStream_t s) {
 }
 
 // the tile shapes that exist for an element format and epilogue: one for grouped problems, all for dense ones
-template <int FMT, int EPI, bool TILED>
+template <int FMT, int EPI, int LAYOUT>
 int launch_shape(const GemmParams& p, const KsplitTile& t, uint32_t max_m_tiles, KsplitWeights loads, hipStream_t s) {
-#define CMX_KS(FW_, FM_, NW_) if (t.fw == FW_ && t.fm == FM_ && t.waves == NW_) return launch_one<FMT, FW_, FM_, NW_, EPI, TILED, KsplitWeights::kCached>(p, max_m_tiles, s)
-    if (t.fw == 4 && t.fm == 4 && t.waves == 4 && p.row_off != nullptr) {
-        if (loads == KsplitWeights::kStreamed) return launch_one<FMT, 4, 4, 4, EPI, TILED, KsplitWeights::kStreamed>(p, max_m_tiles, s);
-        return launch_one<FMT, 4, 4, 4, EPI, TILED, KsplitWeights::kByGroup>(p, max_m_tiles, s);
+#define CMX_KS(FW_, FM_, NW_) if (t.fw == FW_ && t.fm == FM_ && t.waves == NW_) return launch_one<FMT, FW_, FM_, NW_, EPI, LAYOUT, KsplitWeights::kCached>(p, max_m_tiles, s)
+    if constexpr (LAYOUT != kKSlow) if (t.fw == 4 && t.fm == 4 && t.waves == 4 && p.row_off != nullptr) {
+        if (loads == KsplitWeights::kStreamed) return launch_one<FMT, 4, 4, 4, EPI, LAYOUT, KsplitWeights::kStreamed>(p, max_m_tiles, s);
+        return launch_one<FMT, 4, 4, 4, EPI, LAYOUT, KsplitWeights::kByGroup>(p, max_m_tiles, s);
     }
-    if constexpr (EPI == kEpiStore && !TILED) {
+    if constexpr (LAYOUT == kKSlow) {
+        CMX_KS(4, 4, 4);
+        CMX_KS(4, 1, 8);
+        CMX_KS(4, 2, 8);
+        CMX_KS(4, 4, 8);
+    }
+    if constexpr (EPI == kEpiStore && LAYOUT == kRowMajor) {
         CMX_KS(4, 4, 4);
         CMX_KS(1, 1, 8);
         CMX_KS(1, 2, 8);
@@ -443,26 +536,45 @@ int launch_shape(const GemmParams& p, const KsplitTile& t, uint32_t max_m_tiles,
 
 }  // namespace
 
-size_t ksplit_lds_bytes(const KsplitTile& t, int fmt, uint32_t kblocks, bool tiled) {
-    const size_t scales = ks_scale_steps(fmt) ? round_up_sz((size_t)16 * (t.fw + t.fm) * ks_scale_pitch(fmt, kblocks) * 4, 16) : 0;
-    const size_t loop = scales + (size_t)t.waves * ks_exchange_bufs(t.fw, t.fm, tiled) * 2048;
+size_t ksplit_lds_bytes(const KsplitTile& t, int fmt, uint32_t kblocks, int layout) {
+    const size_t rows = layout == kKSlow ? 16 * t.fm : 16 * (t.fw + t.fm);
+    const size_t scales = ks_scale_steps(fmt) ? round_up_sz(rows * ks_scale_pitch(fmt, kblocks) * 4, 16) : 0;
+    const size_t pairs = layout == kKSlow ? (size_t)kblocks / 2 * 128 : 0;
+    const size_t loop = scales + pairs + (size_t)t.waves * ks_exchange_bufs(t.fw, t.fm, layout) * 2048;
     const size_t sums = ks_sum_bytes(t.fw, t.fm, t.waves);
     return loop > sums ? loop : sums;
+}
+
+bool ksplit_k_slow_tile(KsplitTile* t, uint32_t m, uint32_t n, int fmt, uint32_t kblocks, int cus) {
+    if (fmt == CMX_FMT_E2M1 || kblocks % 4 != 0) return false;
+    KsplitTile out = {4, 4, t->waves};
+    if (t->waves == 8) {
+        const auto tiles = [&](int fm) { return (uint64_t)ceil_div(n, 64) * ceil_div(m, 16 * fm); };
+        out.fm = tiles(1) <= (uint64_t)cus ? 1 : (tiles(2) <= (uint64_t)cus ? 2 : 4);
+    }
+    if (ksplit_lds_bytes(out, fmt, kblocks, kKSlow) > kKsplitMaxLds) return false;
+    *t = out;
+    return true;
+}
+
+int launch_ksplit_k_slow(const GemmParams& p, const KsplitTile& t, int fmt, uint32_t max_m_tiles, hipStream_t s) {
+    if (fmt == CMX_FMT_E5M2) return launch_shape<CMX_FMT_E5M2, kEpiStore, kKSlow>(p, t, max_m_tiles, KsplitWeights::kCached, s);
+    return launch_shape<CMX_FMT_E4M3, kEpiStore, kKSlow>(p, t, max_m_tiles, KsplitWeights::kCached, s);
 }
 
 int launch_ksplit(const GemmParams& p, const KsplitTile& t, int fmt, int epi, uint32_t max_m_tiles, KsplitWeights loads, hipStream_t s) {
     if (fmt == CMX_FMT_E4M3) {
         if (epi == kEpiStore)
-            return p.w_pretiled ? launch_shape<CMX_FMT_E4M3, kEpiStore, true>(p, t, max_m_tiles, loads, s) : launch_shape<CMX_FMT_E4M3, kEpiStore, false>(p, t, max_m_tiles, loads, s);
+            return p.w_pretiled ? launch_shape<CMX_FMT_E4M3, kEpiStore, kTiled>(p, t, max_m_tiles, loads, s) : launch_shape<CMX_FMT_E4M3, kEpiStore, kRowMajor>(p, t, max_m_tiles, loads, s);
         if (epi == kEpiSwigluQuant)
-            return p.w_pretiled ? launch_shape<CMX_FMT_E4M3, kEpiSwigluQuant, true>(p, t, max_m_tiles, loads, s)
-                                : launch_shape<CMX_FMT_E4M3, kEpiSwigluQuant, false>(p, t, max_m_tiles, loads, s);
-        if (epi == kEpiSwigluQuantAct && !p.w_pretiled) return launch_shape<CMX_FMT_E4M3, kEpiSwigluQuantAct, false>(p, t, max_m_tiles, loads, s);
+            return p.w_pretiled ? launch_shape<CMX_FMT_E4M3, kEpiSwigluQuant, kTiled>(p, t, max_m_tiles, loads, s)
+                                : launch_shape<CMX_FMT_E4M3, kEpiSwigluQuant, kRowMajor>(p, t, max_m_tiles, loads, s);
+        if (epi == kEpiSwigluQuantAct && !p.w_pretiled) return launch_shape<CMX_FMT_E4M3, kEpiSwigluQuantAct, kRowMajor>(p, t, max_m_tiles, loads, s);
     }
     if (fmt == CMX_FMT_E5M2 && epi == kEpiStore)
-        return p.w_pretiled ? launch_shape<CMX_FMT_E5M2, kEpiStore, true>(p, t, max_m_tiles, loads, s) : launch_shape<CMX_FMT_E5M2, kEpiStore, false>(p, t, max_m_tiles, loads, s);
-    if (fmt == CMX_FMT_E2M1 && epi == kEpiStore) return launch_shape<CMX_FMT_E2M1, kEpiStore, false>(p, t, max_m_tiles, loads, s);
-    if (fmt == kFmtI8 && epi == kEpiI8DequantSwiglu) return launch_shape<kFmtI8, kEpiI8DequantSwiglu, false>(p, t, max_m_tiles, loads, s);
+        return p.w_pretiled ? launch_shape<CMX_FMT_E5M2, kEpiStore, kTiled>(p, t, max_m_tiles, loads, s) : launch_shape<CMX_FMT_E5M2, kEpiStore, kRowMajor>(p, t, max_m_tiles, loads, s);
+    if (fmt == CMX_FMT_E2M1 && epi == kEpiStore) return launch_shape<CMX_FMT_E2M1, kEpiStore, kRowMajor>(p, t, max_m_tiles, loads, s);
+    if (fmt == kFmtI8 && epi == kEpiI8DequantSwiglu) return launch_shape<kFmtI8, kEpiI8DequantSwiglu, kRowMajor>(p, t, max_m_tiles, loads, s);
     set_error("unsupported split-K problem");
     return CMX_EINVAL;
 }

@@ -71,9 +71,25 @@ def test_scale_rows_at_any_byte(tm, k):
     assert torch.equal(got[:, :n], want) and bool((got[:, n:] == 7.0).all())
 
 
-@pytest.mark.parametrize("m,n,k", [(700, 3008, 512), (1030, 4100, 640), (1300, 4096, 1024), (1700, 4092, 512), (1700, 4090, 512), (700, 3008, 576)])
+@pytest.mark.parametrize("waves", [4, 8])
+@pytest.mark.parametrize("fmt,m,n,k", [("E4M3", 1, 16, 128), ("E5M2", 17, 68, 1152), ("E4M3", 65, 140, 2176), ("E4M3", 300, 1076, 640), ("E4M3", 280, 4100, 256),
+                                       ("E4M3", 37, 64, 10496)])
+def test_split_k_on_k_slow_weights_gives_the_bits_of_k_contiguous_ones(waves, fmt, m, n, k):
+    """Tiles of 64 columns x 16, 32 (300 x 1076) and 64 rows (280 x 4100, four wavefronts); more scales than are in flight together."""
+    from catccos_amd import ops
+    rng = np.random.default_rng(m + n + k)
+    aq, asc, bq, bsc = _operands(rng, m, n, k, fmt)
+    a, a_s = dev(aq), dev(asc)
+    fb, fbs = O.to_file_layout(bq, bsc, True)
+    hooks_lib().cmx_debug_force_ksplit(4, 4, waves)
+    want = ops.mx_gemm(a, a_s, dev(bq), dev(bsc), k, fmt, "fp32")
+    assert torch.equal(ops.mx_gemm_ex(a, a_s, dev(fb), dev(fbs), m, n, k, fmt, "fp32", 0, 0), want)
+    _near(want, aq, asc, bq, bsc, fmt)
+
+
+@pytest.mark.parametrize("m,n,k", [(33, 3008, 512), (5, 512, 4224), (400, 2500, 1024), (700, 3008, 512), (1030, 4100, 640), (1300, 4096, 1024), (1700, 4092, 512), (1700, 4090, 512), (700, 3008, 576)])
 def test_chosen_kernels_give_one_result_for_both_weight_layouts(m, n, k):
-    """Sizes of one round of each ring tile, and beside them what has the weights rewritten: columns no multiple of four, K no whole
+    """Sizes of the split-K tiles and of one round of each ring tile, and beside them what has the weights rewritten: columns no multiple of four, K no whole
     number of slabs."""
     from catccos_amd import ops
     rng = np.random.default_rng(m + n + k)
