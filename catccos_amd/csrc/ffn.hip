@@ -1,5 +1,6 @@
 // Single-device MoE FFN: routing sort -> fused quantise+scatter -> GMM1 (+SwiGLU +requant) ->
 // GMM2 -> weighted combine, chained on one stream with no host synchronisation.
+#include "group_tables.h"
 #include "mx_common.h"
 
 namespace cmx {
@@ -102,19 +103,23 @@ int ffn_chain(cmx_stream_t stream, const uint8_t* x, const uint8_t* expertIdx, c
     int rc = cmx_moe_init_routing(reinterpret_cast<const int32_t*>(expertIdx), m, topK, localExperts, sorted2src,
                                   src2sorted, counts, workspace + L.routing_scratch, stream);
     if (rc != CMX_OK) return rc;
+    // the group sizes are known from here on: the tables of both matmuls are filled beside the quantise + scatter stage, not in
+    // launches of their own in front of each (5 us)
+    hipStream_t s = static_cast<hipStream_t>(stream);
+    GroupTablesJob jobs[2];
+    rc = plan_group_tables(&jobs[0], counts, localExperts, rows, n, k, CMX_FMT_E4M3, pretiled, meta1);
+    if (rc != CMX_OK) return rc;
+    rc = plan_group_tables(&jobs[1], counts, localExperts, rows, k, n / 2, CMX_FMT_E4M3, pretiled, meta2);
+    if (rc != CMX_OK) return rc;
     const uint32_t ld_as = (uint32_t)L.a_scales_pitch;
-    rc = cmx_quant_scatter(x, k, src2sorted, a_codes, k, a_scales, ld_as, m, k, topK, stream);
+    rc = quant_scatter_with_tables(x, k, src2sorted, a_codes, k, a_scales, ld_as, m, k, topK, jobs, 2, s);
     if (rc != CMX_OK) return rc;
     const uint32_t ld_acts = scale_cols(n / 2);
-    rc = pretiled ? cmx_mx_gmm_swiglu_quant_pretiled(a_codes, k, a_scales, ld_as, w1, w1Scale, act_codes, n / 2, act_scales,
-                                                     ld_acts, nullptr, counts, localExperts, rows, n, k, meta1, stream)
-                  : cmx_mx_gmm_swiglu_quant(a_codes, k, a_scales, ld_as, w1, w1Scale, act_codes, n / 2, act_scales, ld_acts,
-                                            nullptr, counts, localExperts, rows, n, k, meta1, stream);
+    rc = gmm_swiglu_quant_prepared(a_codes, k, a_scales, ld_as, w1, w1Scale, act_codes, n / 2, act_scales, ld_acts, counts, localExperts, rows,
+                                   n, k, meta1, pretiled, s);
     if (rc != CMX_OK) return rc;
-    rc = pretiled ? cmx_mx_gmm_pretiled(act_codes, n / 2, act_scales, ld_acts, w2, w2Scale, y, k, counts, localExperts, rows, k,
-                                        n / 2, CMX_FMT_E4M3, CMX_OUT_BF16, meta2, stream)
-                  : cmx_mx_gmm(act_codes, n / 2, act_scales, ld_acts, w2, w2Scale, y, k, counts, localExperts, rows, k, n / 2,
-                               CMX_FMT_E4M3, CMX_OUT_BF16, meta2, stream);
+    rc = gmm_prepared(act_codes, n / 2, act_scales, ld_acts, w2, w2Scale, y, k, counts, localExperts, rows, k, n / 2, CMX_FMT_E4M3,
+                      CMX_OUT_BF16, meta2, pretiled, s);
     if (rc != CMX_OK) return rc;
     return cmx_moe_token_unpermute(y, k, rows, src2sorted, reinterpret_cast<const float*>(gateWeight), out, k, m, k,
                                    topK, stream);

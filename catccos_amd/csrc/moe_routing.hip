@@ -1,12 +1,14 @@
 // MoE routing on one device: stable counting sort of (expert, route) pairs, fused MX quantise +
 // scatter of the routed rows, and the weighted top-k combine.  All three are HBM-bound.
 //
-// Sort = histogram per 512-route chunk -> one-workgroup scan (expert-major, chunk-minor, which is
+// Sort, up to kSortRoutes routes and kSortExperts experts: one launch in which every workgroup counts all keys for itself (route_sort_kernel).
+// Beyond: histogram per 512-route chunk -> one-workgroup scan (expert-major, chunk-minor, which is
 // exactly the order of a stable sort) -> scatter, where each chunk is owned by one wavefront that
 // ranks equal keys in lane order with ballots, so the result is the unique stable permutation with
 // no global atomics and no dependence on scheduling.
 #include <algorithm>
 
+#include "group_tables.h"
 #include "mx_common.h"
 
 namespace cmx {
@@ -131,6 +133,79 @@ __global__ __launch_bounds__(64) void route_scatter_kernel(const int32_t* __rest
     }
 }
 
+// The whole sort in one launch.  Workgroup b owns routes 1024 b .. + 1024, one per thread.  It counts the keys of all routes in the LDS,
+// those before its own apart, so that no workgroup waits for another: position = rows of smaller experts + rows of this expert before
+// the workgroup + in the wavefronts before + in the lanes before (ballots), the unique stable permutation.
+// Bound by latency: launch, one pass over the keys (4 routes bytes from the L2 per workgroup, an LDS atomic each), one store.  In place of
+// three launches (histogram, one-workgroup scan over the chunks, scatter).
+constexpr uint32_t kSortThreads = 1024, kSortWaves = kSortThreads / 64, kSortExperts = 512, kSortRoutes = 131072;
+
+__global__ __launch_bounds__(kSortThreads) void route_sort_kernel(const int32_t* __restrict__ keys, uint32_t routes, uint32_t experts,
+                                                                   uint32_t key_bits, int32_t* __restrict__ sorted2src,
+                                                                   int32_t* __restrict__ src2sorted, int32_t* __restrict__ counts) {
+    extern __shared__ uint32_t sh[];
+    __shared__ uint32_t part[kSortWaves];
+    uint32_t* const before = sh;                     // [experts] keys of the routes before the workgroup's, then ...
+    uint32_t* const after = sh + experts;            // [experts] ... of its own and later ones
+    uint32_t* const in_wave = sh + 2 * experts;      // [wavefront][experts] keys of each wavefront, then where its rows start
+    const uint32_t tid = threadIdx.x, lane = tid & 63u, wave = tid >> 6;
+    const uint32_t base = blockIdx.x * kSortThreads, r = base + tid;
+    for (uint32_t i = tid; i < (2 + kSortWaves) * experts; i += kSortThreads) sh[i] = 0;
+    const int32_t raw = r < routes ? keys[r] : -1;
+    const bool live = raw >= 0 && (uint32_t)raw < experts;
+    const uint32_t k = live ? (uint32_t)raw : 0;
+    __syncthreads();
+    unsigned long long same = __ballot(live);
+    for (uint32_t b = 0; b < key_bits; ++b) {
+        const unsigned long long m = __ballot(live && ((k >> b) & 1));
+        same &= ((k >> b) & 1) ? m : ~m;
+    }
+    const uint32_t rank = __popcll(same & ((1ull << lane) - 1ull));
+    if (live && lane == 63u - (uint32_t)__clzll(same)) in_wave[wave * experts + k] = (uint32_t)__popcll(same);
+    for (uint32_t i0 = 0; i0 < routes; i0 += 8 * kSortThreads) {
+        int32_t v[8];
+#pragma unroll
+        for (uint32_t j = 0; j < 8; ++j) {
+            const uint32_t i = i0 + j * kSortThreads + tid;
+            v[j] = i < routes ? keys[i] : -1;
+        }
+#pragma unroll
+        for (uint32_t j = 0; j < 8; ++j) {
+            uint32_t* const to = i0 + j * kSortThreads < base ? before : after;          // whole workgroups of routes
+            if (v[j] >= 0 && (uint32_t)v[j] < experts) atomicAdd(&to[v[j]], 1u);
+        }
+    }
+    __syncthreads();
+    // exclusive scan over the experts, one per thread (experts <= kSortExperts < kSortThreads)
+    const uint32_t mine = tid < experts ? before[tid] + after[tid] : 0;
+    uint32_t sum = mine;
+#pragma unroll
+    for (int d = 1; d < 64; d <<= 1) {
+        const uint32_t u = __shfl_up(sum, d);
+        if (lane >= (uint32_t)d) sum += u;
+    }
+    if (lane == 63u) part[wave] = sum;
+    __syncthreads();
+    if (tid < experts) {
+        uint32_t run = sum - mine + before[tid];
+        for (uint32_t w = 0; w < wave; ++w) run += part[w];
+        for (uint32_t w = 0; w < kSortWaves; ++w) {
+            const uint32_t c = in_wave[w * experts + tid];
+            in_wave[w * experts + tid] = run;
+            run += c;
+        }
+        if (blockIdx.x == 0) counts[tid] = (int32_t)mine;
+    }
+    __syncthreads();
+    if (live) {
+        const uint32_t pos = in_wave[wave * experts + k] + rank;
+        sorted2src[pos] = (int32_t)r;
+        src2sorted[r] = (int32_t)pos;
+    } else if (r < routes) {
+        src2sorted[r] = -1;
+    }
+}
+
 // ---- fused quantise + scatter -------------------------------------------------------------------
 
 // Two lanes per MX block: each takes 16 elements with two 16-byte loads issued together, so a destination row is
@@ -218,6 +293,72 @@ __global__ __launch_bounds__(256) void quant_scatter_kernel(const uint16_t* __re
     }
 }
 
+// Zeros for the output rows that no route is sent to.  A workgroup owns `per` rows (a multiple of 32, at most
+// kUnmappedRows): it reads all destinations, marks those of its rows in an LDS bitmap and clears the rows left over.
+// Bound: the read of the destinations from the L2 (routes * 4 bytes) by every workgroup, of which there are 256, or more where
+// 256 times kUnmappedRows rows (16.7 million) are not enough.  It stands in for a fill of the whole output before the
+// scatter (32768 x 7168 bytes of codes 36 us) and runs beside the scatter, which writes the other rows (as a launch of its own behind it, 6
+// us, half of them the launch).
+constexpr uint32_t kUnmappedRows = 65536;
+
+struct ZeroJob {
+    uint32_t blocks;                 // workgroups of the launch that do this; 0: none
+    uint32_t rows, per, nvec, scols;
+};
+ZeroJob zero_job(uint32_t rows, uint32_t k) {
+    const uint32_t per = std::min(kUnmappedRows, round_up(ceil_div(rows, 256u), 32u));
+    return {ceil_div(rows, per), rows, per, k / 16, scale_cols(k)};
+}
+
+template <uint32_t THREADS>
+__device__ __forceinline__ void zero_unmapped_rows(const ZeroJob& z, uint32_t block, const int32_t* __restrict__ src2sorted,
+                                                   uint8_t* __restrict__ out_codes, uint32_t ld_out, uint8_t* __restrict__ out_scales,
+                                                   uint32_t ld_outs) {
+    __shared__ uint32_t s_map[kUnmappedRows / 32];
+    const uint32_t r0 = block * z.per, n = min(z.per, z.rows - r0), words = (n + 31) / 32;
+    for (uint32_t i = threadIdx.x; i < words; i += THREADS) s_map[i] = 0;
+    __syncthreads();
+    for (uint32_t i0 = 0; i0 < z.rows; i0 += 16 * THREADS) {                         // one route per row
+        int32_t d[16];
+#pragma unroll
+        for (uint32_t j = 0; j < 16; ++j) {
+            const uint32_t i = i0 + j * THREADS + threadIdx.x;
+            d[j] = i < z.rows ? src2sorted[i] : -1;
+        }
+#pragma unroll
+        for (uint32_t j = 0; j < 16; ++j) {
+            const uint32_t r = (uint32_t)d[j] - r0;                                  // dropped routes are negative: far above n
+            if (d[j] >= 0 && r < n) atomicOr(&s_map[r / 32], 1u << (r % 32));
+        }
+    }
+    __syncthreads();
+    const uint32_t lane = threadIdx.x & 63u;
+    for (uint32_t w = threadIdx.x / 64; w < words; w += THREADS / 64) {
+        uint32_t miss = ~s_map[w];
+        if (w == words - 1 && n % 32 != 0) miss &= (1u << (n % 32)) - 1u;
+        while (miss != 0) {
+            const size_t row = r0 + w * 32 + (uint32_t)__builtin_ctz(miss);
+            miss &= miss - 1;
+            for (uint32_t v = lane; v < z.nvec; v += 64) *reinterpret_cast<uint4*>(out_codes + row * ld_out + v * 16) = make_uint4(0, 0, 0, 0);
+            for (uint32_t c = lane; c < z.scols; c += 64) out_scales[row * ld_outs + c] = 0;
+        }
+    }
+}
+
+__global__ __launch_bounds__(256) void zero_unmapped_rows_kernel(const ZeroJob z, const int32_t* __restrict__ src2sorted,
+                                                                 uint8_t* __restrict__ out_codes, uint32_t ld_out,
+                                                                 uint8_t* __restrict__ out_scales, uint32_t ld_outs) {
+    zero_unmapped_rows<256>(z, blockIdx.x, src2sorted, out_codes, ld_out, out_scales, ld_outs);
+}
+
+// What the first workgroups of a quantise + scatter launch do beside it, having nothing to do with its rows: `tables` of them fill the
+// tables of a grouped matmul each, zero.blocks of them clear rows.
+struct ScatterExtras {
+    uint32_t tables;
+    GroupTablesJob job[kMaxTableJobs];
+    ZeroJob zero;
+};
+
 // One workgroup per token: the same two-lanes-per-block arithmetic in passes of 128 blocks, but the token's scale
 // bytes are collected in LDS and every destination gets them as one run of 16-byte stores covering `scale_run` bytes
 // (the scale row, its padding column and zeros up to a multiple of 16, or up to the whole pitch): with a pitch of a
@@ -226,9 +367,15 @@ __global__ __launch_bounds__(256) void quant_scatter_row_kernel(const uint16_t* 
                                                                  const int32_t* __restrict__ src2sorted,
                                                                  uint8_t* __restrict__ out_codes, uint32_t ld_out,
                                                                  uint8_t* __restrict__ out_scales, uint32_t ld_outs, uint32_t top_k,
-                                                                 uint32_t nb, uint32_t scale_run) {
+                                                                 uint32_t nb, uint32_t scale_run, const ScatterExtras ex) {
     __shared__ __attribute__((aligned(16))) uint8_t s_scale[1024 + 16];
-    const uint32_t row = blockIdx.x, h = threadIdx.x & 1u;
+    const uint32_t extras = ex.tables + ex.zero.blocks;
+    if (blockIdx.x < extras) {
+        if (blockIdx.x < ex.tables) fill_group_tables(ex.job[blockIdx.x]);
+        else zero_unmapped_rows<256>(ex.zero, blockIdx.x - ex.tables, src2sorted, out_codes, ld_out, out_scales, ld_outs);
+        return;
+    }
+    const uint32_t row = blockIdx.x - extras, h = threadIdx.x & 1u;
     const uint16_t* xrow = x + (size_t)row * ld_x;
     // zeros behind the scale bytes, 127 in the padding column of an odd count
     for (uint32_t i = nb + threadIdx.x; i < scale_run; i += 256) s_scale[i] = (i == nb && (nb & 1u)) ? 127 : 0;
@@ -290,49 +437,6 @@ __global__ __launch_bounds__(256) void quant_scatter_row_kernel(const uint16_t* 
             const uint32_t j = c / (scale_run / 16), q = c - j * (scale_run / 16);
             const int32_t d = j == 0 ? dst[0] : j == 1 ? dst[1] : j == 2 ? dst[2] : j == 3 ? dst[3] : j == 4 ? dst[4] : j == 5 ? dst[5] : j == 6 ? dst[6] : dst[7];
             if (d >= 0) *reinterpret_cast<uint4*>(out_scales + (size_t)d * ld_outs + q * 16) = *reinterpret_cast<const uint4*>(s_scale + q * 16);
-        }
-    }
-}
-
-// Zeros for the output rows that no route is sent to.  A workgroup owns `per` rows (a multiple of 32, at most
-// kUnmappedRows): it reads all destinations, marks those of its rows in an LDS bitmap and clears the rows left over.
-// Bound: the read of the destinations from the L2 (routes * 4 bytes) by every workgroup, of which there are 256, or more where
-// 256 times kUnmappedRows rows (16.7 million) are not enough.  It stands in for a fill of the whole output before the
-// scatter: 32768 x 7168 bytes of codes 36 us, this kernel 6 us.
-constexpr uint32_t kUnmappedRows = 65536, kUnmappedThreads = 1024;
-
-__global__ __launch_bounds__(kUnmappedThreads) void zero_unmapped_rows_kernel(const int32_t* __restrict__ src2sorted,
-                                                                              uint8_t* __restrict__ out_codes, uint32_t ld_out,
-                                                                              uint8_t* __restrict__ out_scales, uint32_t ld_outs,
-                                                                              uint32_t rows, uint32_t per, uint32_t nvec,
-                                                                              uint32_t scols) {
-    __shared__ uint32_t s_map[kUnmappedRows / 32];
-    const uint32_t r0 = blockIdx.x * per, n = min(per, rows - r0), words = (n + 31) / 32;
-    for (uint32_t i = threadIdx.x; i < words; i += kUnmappedThreads) s_map[i] = 0;
-    __syncthreads();
-    for (uint32_t i0 = 0; i0 < rows; i0 += 8 * kUnmappedThreads) {                   // one route per row
-        int32_t d[8];
-#pragma unroll
-        for (uint32_t j = 0; j < 8; ++j) {
-            const uint32_t i = i0 + j * kUnmappedThreads + threadIdx.x;
-            d[j] = i < rows ? src2sorted[i] : -1;
-        }
-#pragma unroll
-        for (uint32_t j = 0; j < 8; ++j) {
-            const uint32_t r = (uint32_t)d[j] - r0;                                  // dropped routes are negative: far above n
-            if (d[j] >= 0 && r < n) atomicOr(&s_map[r / 32], 1u << (r % 32));
-        }
-    }
-    __syncthreads();
-    const uint32_t lane = threadIdx.x & 63u;
-    for (uint32_t w = threadIdx.x / 64; w < words; w += kUnmappedThreads / 64) {
-        uint32_t miss = ~s_map[w];
-        if (w == words - 1 && n % 32 != 0) miss &= (1u << (n % 32)) - 1u;
-        while (miss != 0) {
-            const size_t row = r0 + w * 32 + (uint32_t)__builtin_ctz(miss);
-            miss &= miss - 1;
-            for (uint32_t v = lane; v < nvec; v += 64) *reinterpret_cast<uint4*>(out_codes + row * ld_out + v * 16) = make_uint4(0, 0, 0, 0);
-            for (uint32_t c = lane; c < scols; c += 64) out_scales[row * ld_outs + c] = 0;
         }
     }
 }
@@ -557,6 +661,12 @@ extern "C" int cmx_moe_init_routing(const int32_t* expert_idx, uint32_t tokens, 
     }
     uint32_t key_bits = 0;
     while ((1u << key_bits) < experts) ++key_bits;
+    if (routes <= kSortRoutes && experts <= kSortExperts) {
+        hipLaunchKernelGGL(route_sort_kernel, dim3(ceil_div(routes, kSortThreads)), dim3(kSortThreads),
+                           (2 + kSortWaves) * experts * sizeof(uint32_t), s, expert_idx, routes, experts, key_bits, sorted2src, src2sorted, counts);
+        CMX_LAUNCH_CHECK();
+        return CMX_OK;
+    }
     hipLaunchKernelGGL(route_hist_kernel, dim3(chunks), dim3(64), experts * sizeof(uint32_t), s, expert_idx, routes,
                        experts, hist);
     CMX_LAUNCH_CHECK();
@@ -571,10 +681,10 @@ extern "C" int cmx_moe_init_routing(const int32_t* expert_idx, uint32_t tokens, 
 
 extern "C" uint32_t cmx_packed_row_bytes(uint32_t k) { return cmx::round_up(k + cmx::scale_cols(k), 32); }
 
-extern "C" int cmx_quant_scatter(const void* x, uint32_t ld_x, const int32_t* src2sorted, uint8_t* out_codes,
-                                 uint32_t ld_out, uint8_t* out_scales, uint32_t ld_outs, uint32_t tokens, uint32_t k,
-                                 uint32_t top_k, cmx_stream_t stream) {
-    using namespace cmx;
+namespace cmx {
+namespace {
+int quant_scatter(const void* x, uint32_t ld_x, const int32_t* src2sorted, uint8_t* out_codes, uint32_t ld_out, uint8_t* out_scales,
+                  uint32_t ld_outs, uint32_t tokens, uint32_t k, uint32_t top_k, const ScatterExtras& ex, hipStream_t s) {
     CMX_REQUIRE(x && src2sorted && out_codes && out_scales, "null pointer");
     if (tokens == 0 || k == 0 || top_k == 0) return CMX_OK;
     CMX_REQUIRE(k % 32 == 0, "k must be a multiple of 32");
@@ -585,7 +695,6 @@ extern "C" int cmx_quant_scatter(const void* x, uint32_t ld_x, const int32_t* sr
     CMX_REQUIRE((uint64_t)tokens * nb < (1ull << 32), "too many blocks for one launch");
     const uint32_t total = tokens * nb;
     const uint16_t* xp = static_cast<const uint16_t*>(x);
-    hipStream_t s = static_cast<hipStream_t>(stream);
     // Scale rows that can be written in 16-byte pieces take the row-wise kernel: the row, its padding column and zeros
     // up to a multiple of 16 bytes (never beyond: in the packed wire row, whose scale bytes sit behind the codes of the
     // same row, round_up(scale_cols, 16) <= round_up(scale_cols, 32) = the bytes the row has left behind its codes).
@@ -597,11 +706,15 @@ extern "C" int cmx_quant_scatter(const void* x, uint32_t ld_x, const int32_t* sr
         const uintptr_t c0 = reinterpret_cast<uintptr_t>(out_codes), s0 = reinterpret_cast<uintptr_t>(out_scales);
         const bool disjoint = s0 >= c0 + dst_rows * ld_out || s0 + dst_rows * ld_outs <= c0;
         const uint32_t run = (disjoint && ld_outs == round_up(scale_cols(k), 128)) ? ld_outs : run16;
-        hipLaunchKernelGGL(quant_scatter_row_kernel, dim3(tokens), dim3(256), 0, s, xp, ld_x, src2sorted, out_codes, ld_out,
-                           out_scales, ld_outs, top_k, nb, run);
+        const uint64_t blocks = (uint64_t)tokens + ex.tables + ex.zero.blocks;
+        CMX_REQUIRE(blocks < (1ull << 32), "too many tokens for one launch");
+        hipLaunchKernelGGL(quant_scatter_row_kernel, dim3((uint32_t)blocks), dim3(256), 0, s, xp, ld_x, src2sorted, out_codes, ld_out,
+                           out_scales, ld_outs, top_k, nb, run, ex);
         CMX_LAUNCH_CHECK();
         return CMX_OK;
     }
+    for (uint32_t i = 0; i < ex.tables; ++i)
+        if (int rc = launch_group_tables(ex.job[i], s); rc != CMX_OK) return rc;
     const bool vec_scales = nb % 4 == 0 && ld_outs % 4 == 0 && (reinterpret_cast<uintptr_t>(out_scales) & 3u) == 0;
     const dim3 grid(ceil_div(total, 128));
     if (vec_scales)
@@ -611,7 +724,28 @@ extern "C" int cmx_quant_scatter(const void* x, uint32_t ld_x, const int32_t* sr
         hipLaunchKernelGGL((quant_scatter_kernel<false>), grid, dim3(256), 0, s, xp, ld_x, src2sorted, out_codes, ld_out,
                            out_scales, ld_outs, tokens, k, top_k, nb, total);
     CMX_LAUNCH_CHECK();
+    if (ex.zero.blocks != 0) {
+        hipLaunchKernelGGL(zero_unmapped_rows_kernel, dim3(ex.zero.blocks), dim3(256), 0, s, ex.zero, src2sorted, out_codes, ld_out, out_scales, ld_outs);
+        CMX_LAUNCH_CHECK();
+    }
     return CMX_OK;
+}
+}  // namespace
+
+int quant_scatter_with_tables(const void* x, uint32_t ld_x, const int32_t* src2sorted, uint8_t* out_codes, uint32_t ld_out, uint8_t* out_scales,
+                              uint32_t ld_outs, uint32_t tokens, uint32_t k, uint32_t top_k, const GroupTablesJob* job, int jobs, hipStream_t s) {
+    CMX_REQUIRE(jobs >= 0 && jobs <= kMaxTableJobs && tokens > 0 && k > 0 && top_k > 0, "bad jobs or an empty problem");
+    ScatterExtras ex{};
+    ex.tables = (uint32_t)jobs;
+    for (int i = 0; i < jobs; ++i) ex.job[i] = job[i];
+    return quant_scatter(x, ld_x, src2sorted, out_codes, ld_out, out_scales, ld_outs, tokens, k, top_k, ex, s);
+}
+}  // namespace cmx
+
+extern "C" int cmx_quant_scatter(const void* x, uint32_t ld_x, const int32_t* src2sorted, uint8_t* out_codes,
+                                 uint32_t ld_out, uint8_t* out_scales, uint32_t ld_outs, uint32_t tokens, uint32_t k,
+                                 uint32_t top_k, cmx_stream_t stream) {
+    return cmx::quant_scatter(x, ld_x, src2sorted, out_codes, ld_out, out_scales, ld_outs, tokens, k, top_k, {}, static_cast<hipStream_t>(stream));
 }
 
 extern "C" int cmx_quant_scatter_zeroed(const void* x, uint32_t ld_x, const int32_t* src2sorted, uint8_t* out_codes,
@@ -620,14 +754,9 @@ extern "C" int cmx_quant_scatter_zeroed(const void* x, uint32_t ld_x, const int3
     using namespace cmx;
     const uint64_t rows = (uint64_t)tokens * top_k;
     CMX_REQUIRE(rows < (1ull << 31), "tokens * top_k must stay below 2^31 routes");
-    int rc = cmx_quant_scatter(x, ld_x, src2sorted, out_codes, ld_out, out_scales, ld_outs, tokens, k, top_k, stream);
-    if (rc != CMX_OK || rows == 0 || k == 0) return rc;
-    const uint32_t per = std::min(kUnmappedRows, round_up(ceil_div((uint32_t)rows, 256u), 32u));
-    hipLaunchKernelGGL(zero_unmapped_rows_kernel, dim3(ceil_div((uint32_t)rows, per)), dim3(kUnmappedThreads), 0,
-                       static_cast<hipStream_t>(stream), src2sorted, out_codes, ld_out, out_scales, ld_outs, (uint32_t)rows, per,
-                       k / 16, scale_cols(k));
-    CMX_LAUNCH_CHECK();
-    return CMX_OK;
+    ScatterExtras ex{};
+    if (rows != 0 && k != 0) ex.zero = zero_job((uint32_t)rows, k);
+    return quant_scatter(x, ld_x, src2sorted, out_codes, ld_out, out_scales, ld_outs, tokens, k, top_k, ex, static_cast<hipStream_t>(stream));
 }
 
 extern "C" int cmx_int8_quant_scatter(const void* x, uint32_t ld_x, const int32_t* src2sorted, int8_t* codes,

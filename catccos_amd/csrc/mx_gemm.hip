@@ -22,6 +22,7 @@
 // weight panels in its own L2.
 #include <type_traits>
 
+#include "group_tables.h"
 #include "mx_gemm_common.h"
 #include "mx_gemm_ksplit.h"
 #include "mx_gemm_ring.h"
@@ -807,90 +808,7 @@ __global__ __launch_bounds__(64 * WW * WM) void mx_gemm_dl_kernel(const GemmPara
 #include "mx_gemm_wreg.h"
 #include "mx_gemm_pipe_fp4.h"
 
-// Row offsets and m-tile prefix of the groups (one workgroup of 256 threads): each thread owns a contiguous run of
-// groups; the 256 partial sums are scanned in LDS, first for the rows, then for the m-tiles.
-// Group sizes live on the device, so the host cannot check them: negative sizes count as zero and rows past
-// m_total (the rows the caller's buffers hold) are cut off here, so that no tile ever points outside them.
-// small_rows != 0: groups of 1 .. small_rows rows are one m-tile each of small_pref and none of tile_pref.
-__global__ __launch_bounds__(256) void gmm_prepare_kernel(const int32_t* __restrict__ sizes, uint32_t groups, uint32_t tile_m,
-                                                           uint32_t m_total, uint32_t small_rows, int32_t* __restrict__ row_off,
-                                                           int32_t* __restrict__ tile_pref, int32_t* __restrict__ small_pref,
-                                                           int32_t* __restrict__ tile_ctr) {
-    __shared__ unsigned long long part_r[256];
-    __shared__ int32_t part_t[256], part_s[256];
-    if (threadIdx.x < kXcds) tile_ctr[threadIdx.x] = 0;
-    const uint32_t per = (groups + 255) / 256;
-    const uint32_t lo = threadIdx.x * per < groups ? threadIdx.x * per : groups;
-    const uint32_t hi = lo + per < groups ? lo + per : groups;
-    auto size_of = [&](uint32_t i) -> unsigned long long {
-        const int32_t c = sizes[i];
-        return c > 0 ? (unsigned long long)c : 0ull;
-    };
-    // inclusive scan of part[0..255] in place: within each wavefront by lane shuffles, then the three wavefront totals
-    // before it added to every element (two barriers instead of sixteen)
-    auto scan256 = [&](auto* part) {
-        auto v = part[threadIdx.x];
-        const uint32_t lane = threadIdx.x & 63u, wave = threadIdx.x >> 6;
-#pragma unroll
-        for (int d = 1; d < 64; d <<= 1) {
-            const auto u = __shfl_up(v, d);
-            if (lane >= (uint32_t)d) v += u;
-        }
-        part[threadIdx.x] = v;
-        __syncthreads();
-        decltype(v) before = 0;
-        for (uint32_t w = 0; w < wave; ++w) before += part[64 * w + 63];
-        __syncthreads();
-        part[threadIdx.x] = v + before;
-        __syncthreads();
-    };
-    unsigned long long r = 0;
-    for (uint32_t i = lo; i < hi; ++i) r += size_of(i);
-    part_r[threadIdx.x] = r;
-    __syncthreads();
-    scan256(part_r);
-    const unsigned long long r_base = threadIdx.x ? part_r[threadIdx.x - 1] : 0ull;
-    // rows of group i that fit below m_total, given the rows before it
-    auto clipped = [&](unsigned long long before, unsigned long long c) -> uint32_t {
-        const unsigned long long b = before < m_total ? before : m_total;
-        const unsigned long long e = before + c < m_total ? before + c : m_total;
-        return (uint32_t)(e - b);
-    };
-    auto is_small = [&](uint32_t rows) -> bool { return rows != 0 && rows <= small_rows; };
-    r = r_base;
-    int32_t t = 0, sm = 0;
-    for (uint32_t i = lo; i < hi; ++i) {
-        const unsigned long long c = size_of(i);
-        const uint32_t rows = clipped(r, c);
-        if (is_small(rows)) ++sm;
-        else t += (int32_t)((rows + tile_m - 1) / tile_m);
-        r += c;
-    }
-    part_t[threadIdx.x] = t;
-    part_s[threadIdx.x] = sm;
-    __syncthreads();
-    scan256(part_t);
-    if (small_rows != 0) scan256(part_s);
-    r = r_base;
-    t = threadIdx.x ? part_t[threadIdx.x - 1] : 0;
-    sm = threadIdx.x ? part_s[threadIdx.x - 1] : 0;
-    for (uint32_t i = lo; i < hi; ++i) {
-        const unsigned long long c = size_of(i);
-        const uint32_t rows = clipped(r, c);
-        row_off[i] = (int32_t)(r < m_total ? r : m_total);
-        tile_pref[i] = t;
-        if (small_rows != 0) small_pref[i] = sm;
-        if (is_small(rows)) ++sm;
-        else t += (int32_t)((rows + tile_m - 1) / tile_m);
-        r += c;
-    }
-    if (threadIdx.x == 255) {
-        const unsigned long long all = part_r[255];
-        row_off[groups] = (int32_t)(all < m_total ? all : m_total);
-        tile_pref[groups] = part_t[255];
-        if (small_rows != 0) small_pref[groups] = part_s[255];
-    }
-}
+__global__ __launch_bounds__(256) void gmm_prepare_kernel(const GroupTablesJob job) { fill_group_tables(job); }
 
 template <int FMT, int TW, int TM, int WW, int WM, int EPI, bool FAST>
 int launch_gemm_impl(const GemmParams& p, uint32_t max_m_tiles, hipStream_t s) {
@@ -1409,16 +1327,19 @@ struct GroupTables {
           tile_ctr(small_pref + (groups + 1)) {}
 };
 
-// Fills the tables for m-tiles of tile_m rows (of the groups past ks.small_rows) and sets the parameters that refer to them.
-int prepare_groups(GemmParams& p, const GroupTables& g, const int32_t* group_sizes, uint32_t groups, uint32_t m_total, uint32_t tile_m,
-                   uint32_t small_rows, hipStream_t s) {
-    hipLaunchKernelGGL(gmm_prepare_kernel, dim3(1), dim3(256), 0, s, group_sizes, groups, tile_m, m_total, small_rows, g.row_off, g.tile_pref,
-                       g.small_pref, g.tile_ctr);
-    CMX_LAUNCH_CHECK();
-    p.row_off = g.row_off;
-    p.tile_pref = g.tile_pref;
-    p.tile_ctr = g.tile_ctr;
-    p.groups = groups;
+GroupTablesJob tables_job(const GroupTables& g, const int32_t* group_sizes, uint32_t groups, uint32_t m_total, uint32_t tile_m, uint32_t small_rows) {
+    return {group_sizes, groups, tile_m, m_total, small_rows, g.row_off, g.tile_pref, g.small_pref, g.tile_ctr};
+}
+
+// Fills the tables for m-tiles of tile_m rows (of the groups past ks.small_rows), unless an earlier launch has, and sets the parameters
+// that refer to them.
+int prepare_groups(GemmParams& p, const GroupTablesJob& job, bool filled, hipStream_t s) {
+    if (!filled)
+        if (int rc = launch_group_tables(job, s); rc != CMX_OK) return rc;
+    p.row_off = job.row_off;
+    p.tile_pref = job.tile_pref;
+    p.tile_ctr = job.tile_ctr;
+    p.groups = job.groups;
     return CMX_OK;
 }
 
@@ -1438,8 +1359,25 @@ uint32_t max_group_tiles(uint32_t m_total, uint32_t groups, uint32_t tile_m, uin
     return m_total / tile_m + (n < groups ? n : groups);
 }
 
+// Which kernels a grouped problem goes to, and the rows of their m-tiles.
+struct GroupPlan {
+    GroupedKsplit ks;
+    TileChoice t;
+    bool all_ksplit() const { return ks.tile.fw != 0 && ks.small_rows == 0; }
+    uint32_t tile_m() const { return all_ksplit() ? 16 * ks.tile.fm : t.tm; }
+};
+int plan_groups(GroupPlan* plan, uint32_t m_total, uint32_t groups, uint32_t n, int fmt, uint32_t kblocks, bool pretiled) {
+    if (int rc = choose_grouped_ksplit(m_total, groups, n, fmt, kblocks, &plan->ks); rc != CMX_OK) return rc;
+    // average rows per group steers the tile height
+    plan->t = choose_tile(ceil_div(m_total, groups), n, fmt, true);
+    // the weights-to-registers kernel, tiles drawn from the counters: 256 x 288 when the groups average less than four
+    // tiles of rows (a group of 257 to 288 rows then takes one pass over its weights instead of two), else 256 x 256
+    if (pretiled) plan->t = {256, g_pretiled_tile_rows ? g_pretiled_tile_rows : (ceil_div(m_total, groups) < 1024 ? 288 : 256), 5};
+    return CMX_OK;
+}
+
 int gmm_common(GemmParams& p, const int32_t* group_sizes, uint32_t groups, uint32_t m_total, void* workspace, int fmt,
-               bool swiglu, hipStream_t s) {
+               bool swiglu, bool tables_filled, hipStream_t s) {
     CMX_REQUIRE(group_sizes && workspace, "null pointer");
     CMX_REQUIRE(groups > 0 && groups <= 65536, "bad group count");
     CMX_REQUIRE(m_total < (1u << 31), "too many rows");
@@ -1448,16 +1386,13 @@ int gmm_common(GemmParams& p, const int32_t* group_sizes, uint32_t groups, uint3
     CMX_REQUIRE((reinterpret_cast<uintptr_t>(workspace) & 3u) == 0, "workspace must be 4-byte aligned");
     if (p.w_pretiled)
         if (int rc = check_pretiled(p, fmt, swiglu); rc != CMX_OK) return rc;
-    GroupedKsplit ks;
-    if (int rc = choose_grouped_ksplit(m_total, groups, p.n, fmt, p.kblocks, &ks); rc != CMX_OK) return rc;
-    // average rows per group steers the tile height
-    TileChoice t = choose_tile(ceil_div(m_total, groups), p.n, fmt, true);
-    // the weights-to-registers kernel, tiles drawn from the counters: 256 x 288 when the groups average less than four
-    // tiles of rows (a group of 257 to 288 rows then takes one pass over its weights instead of two), else 256 x 256
-    if (p.w_pretiled) t = {256, g_pretiled_tile_rows ? g_pretiled_tile_rows : (ceil_div(m_total, groups) < 1024 ? 288 : 256), 5};
-    const bool all_ksplit = ks.tile.fw != 0 && ks.small_rows == 0;
+    GroupPlan plan;
+    if (int rc = plan_groups(&plan, m_total, groups, p.n, fmt, p.kblocks, p.w_pretiled); rc != CMX_OK) return rc;
+    const GroupedKsplit& ks = plan.ks;
+    const TileChoice& t = plan.t;
+    const bool all_ksplit = plan.all_ksplit();
     const GroupTables tables(workspace, groups);
-    if (int rc = prepare_groups(p, tables, group_sizes, groups, m_total, all_ksplit ? 16 * ks.tile.fm : t.tm, ks.small_rows, s); rc != CMX_OK) return rc;
+    if (int rc = prepare_groups(p, tables_job(tables, group_sizes, groups, m_total, plan.tile_m(), ks.small_rows), tables_filled, s); rc != CMX_OK) return rc;
     if (ks.tile.fw != 0) {
         const int epi = !swiglu ? kEpiStore : (p.act_bf16 != nullptr ? kEpiSwigluQuantAct : kEpiSwigluQuant);
         if (int rc = launch_grouped_ksplit(p, tables, ks, fmt, epi, m_total, s); rc != CMX_OK || all_ksplit) return rc;
@@ -1484,7 +1419,7 @@ namespace cmx {
 namespace {
 int gmm_store(const uint8_t* a, uint32_t lda, const uint8_t* a_scale, uint32_t ld_as, const uint8_t* b, const uint8_t* b_scale,
               void* c, uint32_t ldc, const int32_t* group_sizes, uint32_t groups, uint32_t m_total, uint32_t n, uint32_t k,
-              int fmt, int out_type, void* workspace, bool pretiled, cmx_stream_t stream) {
+              int fmt, int out_type, void* workspace, bool pretiled, cmx_stream_t stream, bool tables_filled = false) {
     if (m_total == 0 || n == 0) return CMX_OK;
     const uint32_t kbytes = fmt == CMX_FMT_E2M1 ? k / 2 : k;
     // weight scale rows are as every producer writes them: padded to an even count (the quantizer, the
@@ -1501,7 +1436,7 @@ int gmm_store(const uint8_t* a, uint32_t lda, const uint8_t* a_scale, uint32_t l
     p.scale_vec = scales_dword_aligned(a_scale, ld_as, b_scale, ld_ws);
     p.scale_vec16 = scales_aligned16(a_scale, ld_as, b_scale, ld_ws);
     p.w_pretiled = pretiled ? 1 : 0;
-    return gmm_common(p, group_sizes, groups, m_total, workspace, fmt, false, static_cast<hipStream_t>(stream));
+    return gmm_common(p, group_sizes, groups, m_total, workspace, fmt, false, tables_filled, static_cast<hipStream_t>(stream));
 }
 }  // namespace
 }  // namespace cmx
@@ -1567,7 +1502,8 @@ extern "C" int cmx_int8_gmm_dequant_swiglu(const int8_t* a, uint32_t lda, const 
     if (int rc = choose_grouped_ksplit(m_total, groups, n, kFmtI8, p.kblocks, &ks); rc != CMX_OK) return rc;
     const bool all_ksplit = ks.tile.fw != 0 && ks.small_rows == 0;
     const GroupTables tables(ws, groups);
-    if (int rc = prepare_groups(p, tables, group_sizes, groups, m_total, all_ksplit ? 16 * ks.tile.fm : kTile, ks.small_rows, s); rc != CMX_OK) return rc;
+    const uint32_t tile_m = all_ksplit ? 16 * ks.tile.fm : kTile;
+    if (int rc = prepare_groups(p, tables_job(tables, group_sizes, groups, m_total, tile_m, ks.small_rows), false, s); rc != CMX_OK) return rc;
     if (ks.tile.fw != 0)
         if (int rc = launch_grouped_ksplit(p, tables, ks, kFmtI8, kEpiI8DequantSwiglu, m_total, s); rc != CMX_OK || all_ksplit) return rc;
     p.w_tiles = ceil_div(n / 2, kTile / 2);
@@ -1582,7 +1518,7 @@ namespace {
 int gmm_swiglu_quant(const uint8_t* a, uint32_t lda, const uint8_t* a_scale, uint32_t ld_as, const uint8_t* b,
                      const uint8_t* b_scale, uint8_t* act_codes, uint32_t ld_act, uint8_t* act_scales, uint32_t ld_acts,
                      void* act_bf16, const int32_t* group_sizes, uint32_t groups, uint32_t m_total, uint32_t n, uint32_t k,
-                     void* workspace, bool pretiled, cmx_stream_t stream) {
+                     void* workspace, bool pretiled, cmx_stream_t stream, bool tables_filled = false) {
     const uint32_t ld_ws = scale_cols(k);      // even-padded weight scale rows, as in cmx_mx_gmm
     int rc = check_operands(a, lda, a_scale, ld_as, b, k, b_scale, ld_ws, k, CMX_FMT_E4M3);
     if (rc != CMX_OK) return rc;
@@ -1600,7 +1536,7 @@ int gmm_swiglu_quant(const uint8_t* a, uint32_t lda, const uint8_t* a_scale, uin
     p.scale_vec = scales_dword_aligned(a_scale, ld_as, b_scale, ld_ws);
     p.scale_vec16 = scales_aligned16(a_scale, ld_as, b_scale, ld_ws);
     p.w_pretiled = pretiled ? 1 : 0;
-    return gmm_common(p, group_sizes, groups, m_total, workspace, CMX_FMT_E4M3, true, static_cast<hipStream_t>(stream));
+    return gmm_common(p, group_sizes, groups, m_total, workspace, CMX_FMT_E4M3, true, tables_filled, static_cast<hipStream_t>(stream));
 }
 
 // Schedule metadata of the allocation-free entry point (row offsets, m-tile prefixes, per-XCD tile counters of up to
@@ -1646,6 +1582,34 @@ extern "C" int cmx_mx_gmm_swiglu_quant_pretiled(const uint8_t* a, uint32_t lda, 
     if (m_total == 0 || n == 0) return CMX_OK;
     return cmx::gmm_swiglu_quant(a, lda, a_scale, ld_as, b_tiled, b_scale, act_codes, ld_act, act_scales, ld_acts,
                                  act_bf16, group_sizes, groups, m_total, n, k, workspace, true, stream);
+}
+
+int cmx::launch_group_tables(const GroupTablesJob& job, hipStream_t s) {
+    hipLaunchKernelGGL(gmm_prepare_kernel, dim3(1), dim3(256), 0, s, job);
+    CMX_LAUNCH_CHECK();
+    return CMX_OK;
+}
+
+int cmx::plan_group_tables(GroupTablesJob* job, const int32_t* group_sizes, uint32_t groups, uint32_t m_total, uint32_t n, uint32_t k, int fmt,
+                           bool pretiled, void* workspace) {
+    GroupPlan plan;
+    if (int rc = plan_groups(&plan, m_total, groups, n, fmt, k / 32, pretiled); rc != CMX_OK) return rc;
+    *job = tables_job(GroupTables(workspace, groups), group_sizes, groups, m_total, plan.tile_m(), plan.ks.small_rows);
+    return CMX_OK;
+}
+
+int cmx::gmm_swiglu_quant_prepared(const uint8_t* a, uint32_t lda, const uint8_t* a_scale, uint32_t ld_as, const uint8_t* b,
+                                   const uint8_t* b_scale, uint8_t* act_codes, uint32_t ld_act, uint8_t* act_scales, uint32_t ld_acts,
+                                   const int32_t* group_sizes, uint32_t groups, uint32_t m_total, uint32_t n, uint32_t k, void* workspace,
+                                   bool pretiled, hipStream_t s) {
+    return gmm_swiglu_quant(a, lda, a_scale, ld_as, b, b_scale, act_codes, ld_act, act_scales, ld_acts, nullptr, group_sizes, groups, m_total, n,
+                            k, workspace, pretiled, s, true);
+}
+
+int cmx::gmm_prepared(const uint8_t* a, uint32_t lda, const uint8_t* a_scale, uint32_t ld_as, const uint8_t* b, const uint8_t* b_scale, void* c,
+                      uint32_t ldc, const int32_t* group_sizes, uint32_t groups, uint32_t m_total, uint32_t n, uint32_t k, int fmt, int out_type,
+                      void* workspace, bool pretiled, hipStream_t s) {
+    return gmm_store(a, lda, a_scale, ld_as, b, b_scale, c, ldc, group_sizes, groups, m_total, n, k, fmt, out_type, workspace, pretiled, s, true);
 }
 
 extern "C" uint32_t cmx_mx_gmm_noalloc_max_groups(void) { return cmx::kStaticGroups; }

@@ -37,6 +37,21 @@ def test_sort_all_routes_to_one_expert_and_repeats():
     assert np.array_equal(host(s2s), O.moe_init_routing(bal, 16)[0])
 
 
+@pytest.mark.parametrize("routes,experts", [(63, 1), (1024, 512), (1025, 512), (1025, 513), (5000, 3), (131072, 64), (131073, 64)])
+def test_sort_at_the_edges_of_the_single_launch(routes, experts):
+    """Workgroups of 1024 routes, 512 experts and 131072 routes at most in one launch, three launches beyond; keys outside
+    0 .. experts - 1 are dropped on both sides."""
+    from catccos_amd import ops
+    keys = np.random.default_rng(routes).integers(-1, experts + 1, routes).astype(np.int32)
+    s2s, inv, counts = ops.moe_init_routing(dev(keys.reshape(-1, 1)), experts)
+    live = np.flatnonzero((keys >= 0) & (keys < experts))
+    order = live[np.argsort(keys[live], kind="stable")]
+    want = np.full(routes, -1, dtype=np.int32)
+    want[order] = np.arange(len(order))
+    assert np.array_equal(host(counts), np.bincount(keys[live], minlength=experts))
+    assert np.array_equal(host(s2s)[:len(order)], order) and np.array_equal(host(inv), want)
+
+
 @pytest.mark.parametrize("packed", [False, True])
 def test_quant_scatter_bit_exact(packed):
     from catccos_amd import ops
