@@ -107,9 +107,9 @@ int ffn_chain(cmx_stream_t stream, const uint8_t* x, const uint8_t* expertIdx, c
     // launches of their own in front of each (5 us)
     hipStream_t s = static_cast<hipStream_t>(stream);
     GroupTablesJob jobs[2];
-    rc = plan_group_tables(&jobs[0], counts, localExperts, rows, n, k, CMX_FMT_E4M3, pretiled, meta1);
+    rc = plan_group_tables(&jobs[0], counts, localExperts, rows, n, k, CMX_FMT_E4M3, true, pretiled, meta1);
     if (rc != CMX_OK) return rc;
-    rc = plan_group_tables(&jobs[1], counts, localExperts, rows, k, n / 2, CMX_FMT_E4M3, pretiled, meta2);
+    rc = plan_group_tables(&jobs[1], counts, localExperts, rows, k, n / 2, CMX_FMT_E4M3, false, pretiled, meta2);
     if (rc != CMX_OK) return rc;
     const uint32_t ld_as = (uint32_t)L.a_scales_pitch;
     rc = quant_scatter_with_tables(x, k, src2sorted, a_codes, k, a_scales, ld_as, m, k, topK, jobs, 2, s);

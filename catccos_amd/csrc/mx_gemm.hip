@@ -921,7 +921,7 @@ int launch_gemm(const GemmParams& p, uint32_t max_m_tiles, hipStream_t s) {
 struct TileChoice {
     int tw, tm, waves;
 };
-constexpr int kForceRing = 6;          // `waves` of a pinned tile that stands for the ring kernel
+constexpr int kRing = 6;               // `waves` of a tile of the ring kernel
 
 #ifdef CMX_TEST_HOOKS
 TileChoice g_force_tile = {0, 0, 0};   // tw == 0 -> heuristic
@@ -971,7 +971,7 @@ bool takes_128_tile(uint32_t m, uint32_t n, int fmt, uint32_t kblocks, int cus) 
 int ring_rows(uint32_t m, uint32_t n, int fmt, uint32_t kblocks, int cus, bool k_slow) {
     if (fmt == CMX_FMT_E2M1 || kblocks % 4 != 0 || kblocks < 16) return 0;
     if ((uint64_t)ceil_div(n, 64) * ceil_div(m, 64) <= 2 * (uint64_t)cus) return 0;
-    const auto one_round = [&](uint32_t tm) { return (uint64_t)ceil_div(n, kRingTileW) * ceil_div(m, tm) <= (uint64_t)cus; };
+    const auto one_round = [&](uint32_t tm) { return (uint64_t)ceil_div(n, 128) * ceil_div(m, tm) <= (uint64_t)cus; };
     const bool slow_256 = k_slow || kblocks % 16 != 0;        // the 256-row kernels need a pass first, or are the streaming ones
     if (one_round(128)) return 128;
     if (one_round(192) && (slow_256 || kblocks >= 32)) return 192;
@@ -1214,9 +1214,9 @@ extern "C" int cmx_debug_force_tile(int tw, int tm, int waves) {
 
 namespace cmx {
 namespace {
-int ring_gemm(GemmParams& p, int tm, int fmt, bool k_slow, hipStream_t s) {
-    p.w_tiles = ceil_div(p.n, kRingTileW);
-    return launch_ring(p, tm, fmt, k_slow, ceil_div(p.m, tm), s);
+int ring_gemm(GemmParams& p, const RingTile& t, int fmt, bool k_slow, hipStream_t s) {
+    p.w_tiles = ceil_div(p.n, t.tw);
+    return launch_ring(p, t, fmt, kEpiStore, k_slow, ceil_div(p.m, t.tm), s);
 }
 }  // namespace
 }  // namespace cmx
@@ -1249,10 +1249,10 @@ extern "C" int cmx_mx_gemm(const uint8_t* a, uint32_t lda, const uint8_t* a_scal
     if (rc = cu_count(&cus); rc != CMX_OK) return rc;
     TileChoice t = choose_tile(m, n, fmt, false);
     if (!g_force_tile.tw && !g_disable_dl) {
-        if (const int tm = ring_rows(m, n, fmt, p.kblocks, cus, false)) return ring_gemm(p, tm, fmt, false, s);
+        if (const int tm = ring_rows(m, n, fmt, p.kblocks, cus, false)) return ring_gemm(p, {128, tm}, fmt, false, s);
         if (takes_128_tile(m, n, fmt, p.kblocks, cus)) t = {128, 128, 4};
     }
-    if (t.waves == kForceRing) return ring_gemm(p, t.tm, fmt, false, s);
+    if (t.waves == kRing) return ring_gemm(p, {t.tw, t.tm}, fmt, false, s);
     p.w_tiles = ceil_div(n, t.tw);
     const uint32_t m_tiles = ceil_div(m, t.tm);
     switch (fmt) {
@@ -1293,7 +1293,7 @@ int cmx::gemm_k_slow(const uint8_t* a, const uint8_t* a_scale, const uint8_t* b,
     if (ks.fw != 0) {
         if (!k_slow_pays(n, k) || !ksplit_k_slow_tile(&ks, m, n, fmt, k / 32, cus)) return CMX_OK;
     } else {
-        tm = g_force_tile.waves == kForceRing ? g_force_tile.tm : (g_force_tile.tw || g_disable_dl ? 0 : ring_rows(m, n, fmt, k / 32, cus, true));
+        tm = g_force_tile.waves == kRing ? g_force_tile.tm : (g_force_tile.tw || g_disable_dl ? 0 : ring_rows(m, n, fmt, k / 32, cus, true));
         if (tm == 0) return CMX_OK;
     }
     CMX_REQUIRE(a && a_scale && b && b_scale && aligned16(a), "operand rows must be 16-byte aligned");
@@ -1307,7 +1307,7 @@ int cmx::gemm_k_slow(const uint8_t* a, const uint8_t* a_scale, const uint8_t* b,
     p.groups = 1; p.out_type = out_type;
     p.scale_vec = scales_dword_aligned(a_scale, p.ld_as, b_scale, p.ld_ws);
     *taken = true;
-    if (tm != 0) return ring_gemm(p, tm, fmt, true, s);
+    if (tm != 0) return ring_gemm(p, {128, tm}, fmt, true, s);
     p.w_tiles = ceil_div(n, 64);
     return launch_ksplit_k_slow(p, ks, fmt, ceil_div(m, 16 * ks.fm), s);
 }
@@ -1359,6 +1359,30 @@ uint32_t max_group_tiles(uint32_t m_total, uint32_t groups, uint32_t tile_m, uin
     return m_total / tile_m + (n < groups ? n : groups);
 }
 
+// Grouped 8-bit problems on row-major weights that the ring kernel takes from the 256-row kernels of choose_tile (same sums, so the line
+// is a matter of time).  128 x 128 where its tiles are one round of a workgroup per CU whatever the rows' distribution (a second round costs as
+// much as the first: 16 experts x 64 rows, Zipf, K = 2048, N = 2048, 320 tiles, 30 against 23); else 256 x 128 in the place of the three-slot
+// kernel of short groups, which pulls a dword of scales per row and slab; else 128 x 256 in one round.
+// Measured (us, before -> ring; SwiGLU + requant / 16-bit store; u: routes drawn uniformly, z: Zipf):
+//   128 x 128    8 experts x 64 rows u, K = 1024, N = 1024   14.6 -> 13.9 / 18.3 -> 13.7    x 200 z   22.1 -> 14.3 / 19.7 -> 14.5
+//                8 x 100 u, 4096, 2048                       35.7 -> 25.0 / 40.1 -> 25.4    16 x 64 z, 7168, 1024   56.8 -> 36.8 / 61.5 -> 36.7
+//   256 x 128    32 x 100 u, 7168, 4096                      206 -> 190 / 221 -> 204        32 x 128 z   320 -> 279 / 327 -> 284
+//                16 x 100 u, 2048, 2048                      23.4 against 24.0 / 28.2 -> 25.2, so not for SwiGLU at K below 3072 (at 1152
+//                22.6 against 24.2); 32 x 128 z, 4096, 1024 42.5 against 46.3 / 47.1 -> 47.1 is the most that this line loses
+//   128 x 256    8 x 200 u, 4096, 2048                       45.9 -> 34.5 / 43.1 -> 35.7    16 x 300 u, 7168, 1024   74 -> 57 / 69 -> 62
+//                8 x 500 u, 1024, 1024                       22.6 -> 18.6 / 20.0 against 19.9, so not for a store at K below 2048
+// Problems of more tiles stay on the persistent kernels (32 x 194 rows, 7168, 4096: 287 against 311 with 128 x 256).
+int ring_groups(TileChoice* t, uint32_t m_total, uint32_t groups, uint32_t n, int fmt, uint32_t kblocks, bool swiglu) {
+    if (fmt == CMX_FMT_E2M1 || kblocks % 4 != 0 || kblocks < 16) return CMX_OK;
+    int cus = 0;
+    if (int rc = cu_count(&cus); rc != CMX_OK) return rc;
+    const uint64_t w128 = ceil_div(n, 128);
+    if (w128 * (m_total / 128 + groups) <= (uint64_t)cus) *t = {128, 128, kRing};
+    else if (t->tm == 128 && (!swiglu || kblocks >= 96)) *t = {256, 128, kRing};
+    else if (t->tm == 256 && w128 * (m_total / 256 + groups * 3 / 4) <= (uint64_t)cus && (swiglu || kblocks >= 64)) *t = {128, 256, kRing};
+    return CMX_OK;
+}
+
 // Which kernels a grouped problem goes to, and the rows of their m-tiles.
 struct GroupPlan {
     GroupedKsplit ks;
@@ -1366,10 +1390,12 @@ struct GroupPlan {
     bool all_ksplit() const { return ks.tile.fw != 0 && ks.small_rows == 0; }
     uint32_t tile_m() const { return all_ksplit() ? 16 * ks.tile.fm : t.tm; }
 };
-int plan_groups(GroupPlan* plan, uint32_t m_total, uint32_t groups, uint32_t n, int fmt, uint32_t kblocks, bool pretiled) {
+int plan_groups(GroupPlan* plan, uint32_t m_total, uint32_t groups, uint32_t n, int fmt, uint32_t kblocks, bool swiglu, bool pretiled) {
     if (int rc = choose_grouped_ksplit(m_total, groups, n, fmt, kblocks, &plan->ks); rc != CMX_OK) return rc;
     // average rows per group steers the tile height
     plan->t = choose_tile(ceil_div(m_total, groups), n, fmt, true);
+    if (!pretiled && !g_force_tile.tw && !g_disable_dl)
+        if (int rc = ring_groups(&plan->t, m_total, groups, n, fmt, kblocks, swiglu); rc != CMX_OK) return rc;
     // the weights-to-registers kernel, tiles drawn from the counters: 256 x 288 when the groups average less than four
     // tiles of rows (a group of 257 to 288 rows then takes one pass over its weights instead of two), else 256 x 256
     if (pretiled) plan->t = {256, g_pretiled_tile_rows ? g_pretiled_tile_rows : (ceil_div(m_total, groups) < 1024 ? 288 : 256), 5};
@@ -1387,7 +1413,7 @@ int gmm_common(GemmParams& p, const int32_t* group_sizes, uint32_t groups, uint3
     if (p.w_pretiled)
         if (int rc = check_pretiled(p, fmt, swiglu); rc != CMX_OK) return rc;
     GroupPlan plan;
-    if (int rc = plan_groups(&plan, m_total, groups, p.n, fmt, p.kblocks, p.w_pretiled); rc != CMX_OK) return rc;
+    if (int rc = plan_groups(&plan, m_total, groups, p.n, fmt, p.kblocks, swiglu, p.w_pretiled); rc != CMX_OK) return rc;
     const GroupedKsplit& ks = plan.ks;
     const TileChoice& t = plan.t;
     const bool all_ksplit = plan.all_ksplit();
@@ -1404,6 +1430,8 @@ int gmm_common(GemmParams& p, const int32_t* group_sizes, uint32_t groups, uint3
     p.w_tiles = swiglu ? ceil_div(p.n / 2, t.tw / 2) : ceil_div(p.n, t.tw);
     const uint32_t max_m_tiles = max_group_tiles(m_total, groups, t.tm, ks.small_rows);
     if (p.w_pretiled) return t.tm == 288 ? launch_pretiled<288>(p, fmt, swiglu, max_m_tiles, s) : launch_pretiled<256>(p, fmt, swiglu, max_m_tiles, s);
+    if (t.waves == kRing)
+        return launch_ring(p, {t.tw, t.tm}, fmt, !swiglu ? kEpiStore : (p.act_bf16 != nullptr ? kEpiSwigluQuantAct : kEpiSwigluQuant), false, max_m_tiles, s);
     if (swiglu && p.act_bf16 != nullptr) return dispatch_tile<CMX_FMT_E4M3, kEpiSwigluQuantAct>(p, t, max_m_tiles, s);
     if (swiglu) return dispatch_tile<CMX_FMT_E4M3, kEpiSwigluQuant>(p, t, max_m_tiles, s);
     switch (fmt) {
@@ -1591,9 +1619,9 @@ int cmx::launch_group_tables(const GroupTablesJob& job, hipStream_t s) {
 }
 
 int cmx::plan_group_tables(GroupTablesJob* job, const int32_t* group_sizes, uint32_t groups, uint32_t m_total, uint32_t n, uint32_t k, int fmt,
-                           bool pretiled, void* workspace) {
+                           bool swiglu, bool pretiled, void* workspace) {
     GroupPlan plan;
-    if (int rc = plan_groups(&plan, m_total, groups, n, fmt, k / 32, pretiled); rc != CMX_OK) return rc;
+    if (int rc = plan_groups(&plan, m_total, groups, n, fmt, k / 32, swiglu, pretiled); rc != CMX_OK) return rc;
     *job = tables_job(GroupTables(workspace, groups), group_sizes, groups, m_total, plan.tile_m(), plan.ks.small_rows);
     return CMX_OK;
 }

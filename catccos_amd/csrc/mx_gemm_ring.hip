@@ -343,11 +343,16 @@ int launch_one(const GemmParams& p, uint32_t max_m_tiles, hipStream_t s) {
 }
 
 #ifndef RING_PROTO
-template <int FMT, bool KSLOW>
-int launch_shape(const GemmParams& p, int tm, uint32_t max_m_tiles, hipStream_t s) {
-    if (tm == 128) return launch_one<FMT, 128, 128, 2, 2, 3, 32, kEpiStore, KSLOW>(p, max_m_tiles, s);
-    if (tm == 192) return launch_one<FMT, 128, 192, 2, 2, 3, 16, kEpiStore, KSLOW>(p, max_m_tiles, s);
-    if (tm == 256) return launch_one<FMT, 128, 256, 2, 2, 3, 4, kEpiStore, KSLOW>(p, max_m_tiles, s);
+template <int FMT, int EPI, bool KSLOW>
+int launch_shape(const GemmParams& p, const RingTile& t, uint32_t max_m_tiles, hipStream_t s) {
+    if (t.tw == 128 && t.tm == 128) return launch_one<FMT, 128, 128, 2, 2, 3, 32, EPI, KSLOW>(p, max_m_tiles, s);
+    if (t.tw == 128 && t.tm == 256) return launch_one<FMT, 128, 256, 2, 2, 3, 4, EPI, KSLOW>(p, max_m_tiles, s);
+    if constexpr (EPI == kEpiStore) {
+        if (t.tw == 128 && t.tm == 192) return launch_one<FMT, 128, 192, 2, 2, 3, 16, EPI, KSLOW>(p, max_m_tiles, s);
+    }
+    if constexpr (!KSLOW) {
+        if (t.tw == 256 && t.tm == 128) return launch_one<FMT, 256, 128, 2, 2, 3, 4, EPI, KSLOW>(p, max_m_tiles, s);
+    }
     set_error("unsupported ring tile");
     return CMX_EINVAL;
 }
@@ -356,9 +361,13 @@ int launch_shape(const GemmParams& p, int tm, uint32_t max_m_tiles, hipStream_t 
 }  // namespace
 
 #ifndef RING_PROTO
-int launch_ring(const GemmParams& p, int tm, int fmt, bool k_slow, uint32_t max_m_tiles, hipStream_t s) {
-    if (fmt == CMX_FMT_E4M3) return k_slow ? launch_shape<CMX_FMT_E4M3, true>(p, tm, max_m_tiles, s) : launch_shape<CMX_FMT_E4M3, false>(p, tm, max_m_tiles, s);
-    if (fmt == CMX_FMT_E5M2) return k_slow ? launch_shape<CMX_FMT_E5M2, true>(p, tm, max_m_tiles, s) : launch_shape<CMX_FMT_E5M2, false>(p, tm, max_m_tiles, s);
+int launch_ring(const GemmParams& p, const RingTile& t, int fmt, int epi, bool k_slow, uint32_t max_m_tiles, hipStream_t s) {
+    if (fmt == CMX_FMT_E4M3 && epi == kEpiStore)
+        return k_slow ? launch_shape<CMX_FMT_E4M3, kEpiStore, true>(p, t, max_m_tiles, s) : launch_shape<CMX_FMT_E4M3, kEpiStore, false>(p, t, max_m_tiles, s);
+    if (fmt == CMX_FMT_E5M2 && epi == kEpiStore)
+        return k_slow ? launch_shape<CMX_FMT_E5M2, kEpiStore, true>(p, t, max_m_tiles, s) : launch_shape<CMX_FMT_E5M2, kEpiStore, false>(p, t, max_m_tiles, s);
+    if (fmt == CMX_FMT_E4M3 && epi == kEpiSwigluQuant && !k_slow) return launch_shape<CMX_FMT_E4M3, kEpiSwigluQuant, false>(p, t, max_m_tiles, s);
+    if (fmt == CMX_FMT_E4M3 && epi == kEpiSwigluQuantAct && !k_slow) return launch_shape<CMX_FMT_E4M3, kEpiSwigluQuantAct, false>(p, t, max_m_tiles, s);
     set_error("unsupported ring problem");
     return CMX_EINVAL;
 }

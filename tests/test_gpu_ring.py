@@ -98,3 +98,46 @@ def test_chosen_kernels_give_one_result_for_both_weight_layouts(m, n, k):
     want = ops.mx_gemm(dev(aq), dev(asc), dev(bq), dev(bsc), k)
     assert torch.equal(ops.mx_gemm_ex(dev(aq), dev(asc), dev(fb), dev(fbs), m, n, k, trans_b=0), want)
     _near(want, aq, asc, bq, bsc, "E4M3")
+
+
+@pytest.mark.parametrize("tile", [(128, 128), (128, 256), (256, 128)])
+@pytest.mark.parametrize("counts,n,k", [([1, 0, 127, 128, 129, 0, 257, 66], 320, 512), ([300, 2], 192, 1152), ([0, 5, 0], 64, 128)])
+def test_grouped_problems_give_the_bits_of_the_256_row_kernels(tile, counts, n, k):
+    """Groups that end at and beside a tile's last row, empty ones, gate and up halves that end inside a tile."""
+    from catccos_amd import ops
+    rng = np.random.default_rng(sum(counts) + n)
+    m, e = sum(counts), len(counts)
+    aq, asc, bq, bsc = _operands(rng, m, e * n, k, "E4M3")
+    a, a_s, w, w_s, cnt = dev(aq), dev(asc), dev(bq.reshape(e, n, k)), dev(bsc.reshape(e, n, -1)), dev(np.array(counts, dtype=np.int32))
+    h = hooks_lib()
+
+    def outputs():
+        c = torch.full((m + 2, n), 7.0, dtype=torch.bfloat16, device="cuda")
+        ops.mx_gmm(a, a_s, w, w_s, cnt, k, c=c)
+        return [*ops.mx_gmm_swiglu_quant(a, a_s, w, w_s, cnt, k, want_bf16=True), *ops.mx_gmm_swiglu_quant(a, a_s, w, w_s, cnt, k)[:2],
+                ops.mx_gmm(a, a_s, w, w_s, cnt, k, "E5M2", "fp32"), c]
+    h.cmx_debug_force_tile(256, 256, 8)
+    want = outputs()
+    h.cmx_debug_force_tile(*tile, 6)
+    for got, ref in zip(outputs(), want):
+        assert torch.equal(got.view(torch.uint8), ref.view(torch.uint8))
+    assert bool((want[-1][m:].float() == 7.0).all())
+
+
+@pytest.mark.parametrize("experts,avg,n,k", [(8, 100, 1024, 1024), (16, 100, 2048, 3072), (8, 200, 2048, 1024), (16, 100, 2048, 1024)])
+def test_chosen_grouped_kernels(experts, avg, n, k):
+    """Averages that take each of the ring tiles, and one that stays: the bits of the 256-row kernel either way."""
+    from catccos_amd import ops
+    rng = np.random.default_rng(avg)
+    counts = rng.multinomial(experts * avg, np.full(experts, 1 / experts)).astype(np.int32)
+    m = int(counts.sum())
+    aq, asc, bq, bsc = _operands(rng, m, 256, k, "E4M3")
+    w, w_s = dev(np.resize(bq, (experts, n, k))), dev(np.resize(bsc, (experts, n, k // 32)))
+    a, a_s, cnt = dev(aq), dev(asc), dev(counts)
+
+    def outputs():
+        return [*ops.mx_gmm_swiglu_quant(a, a_s, w, w_s, cnt, k)[:2], ops.mx_gmm(a, a_s, w, w_s, cnt, k)]
+    chosen = outputs()
+    hooks_lib().cmx_debug_force_tile(256, 256, 8)
+    for got, ref in zip(chosen, outputs()):
+        assert torch.equal(got, ref)
