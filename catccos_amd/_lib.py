@@ -110,11 +110,23 @@ def load() -> C.CDLL:
     return _lib
 
 
+_entries = None
+
+
+def entries() -> dict:
+    """name -> address of every entry point of the library that load() returns (what _native_call.run takes)."""
+    global _entries
+    if _entries is None:
+        lib = load()
+        _entries = {name: C.cast(getattr(lib, name), C.c_void_p).value for name in SIGNATURES}
+    return _entries
+
+
 def activate(lib) -> "C.CDLL | None":
     """Makes ``lib`` (a result of bind(), or None for the default) the library that load() returns; returns the
     previous one.  The test suite uses it to run the package's front end on the test build of the library."""
-    global _lib
-    prev, _lib = _lib, lib
+    global _lib, _entries
+    prev, _lib, _entries = _lib, lib, None
     return prev
 
 

@@ -1,4 +1,4 @@
-"""Builds libcatccos_mx.so (HIP kernels + C ABI) for gfx950 with hipcc.
+"""Builds libcatccos_mx.so (HIP kernels + C ABI) for gfx950 with hipcc, and the extension of the Python front end with g++.
 
 Usage: python -m catccos_amd.build [--verbose] [--jobs N]
 Objects go to catccos_amd/_build/, the library to catccos_amd/lib/.  Sources are
@@ -17,6 +17,8 @@ CSRC = os.path.join(HERE, "csrc")
 OBJ = os.path.join(HERE, "_build")
 LIBDIR = os.path.join(HERE, "lib")
 LIB = os.path.join(LIBDIR, "libcatccos_mx.so")
+NATIVE_SRC = os.path.join(CSRC, "native_call.cpp")
+NATIVE = os.path.join(HERE, "_native_call.so")
 
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 FLAGS = [
@@ -75,9 +77,28 @@ def _compile(src: str, verbose: bool) -> str:
     return obj
 
 
+def build_native(force: bool = False) -> str:
+    """The Python extension catccos_amd._native_call (host code only, against this interpreter's torch)."""
+    if not force and os.path.exists(NATIVE) and os.path.getmtime(NATIVE) >= os.path.getmtime(NATIVE_SRC):
+        return NATIVE
+    import sysconfig
+
+    import torch
+    t = os.path.dirname(torch.__file__)
+    cmd = ["g++", "-O2", "-std=c++17", "-fPIC", "-shared", f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}",
+           "-isystem", os.path.join(t, "include"), "-isystem", os.path.join(t, "include", "torch", "csrc", "api", "include"),
+           "-isystem", sysconfig.get_paths()["include"], NATIVE_SRC, "-o", NATIVE,
+           "-L" + os.path.join(t, "lib"), "-ltorch_python", "-ltorch", "-ltorch_cpu", "-lc10"]
+    r = subprocess.run(cmd, capture_output=True, text=True)
+    if r.returncode != 0:
+        raise RuntimeError(f"g++ failed on {NATIVE_SRC}:\n" + r.stdout + r.stderr)
+    return NATIVE
+
+
 def build(force: bool = False, verbose: bool = False, jobs: int = 4) -> str:
     os.makedirs(OBJ, exist_ok=True)
     os.makedirs(LIBDIR, exist_ok=True)
+    build_native(force)
     hm = _headers_mtime()
     todo, objs = [], []
     for s in sources():

@@ -1,7 +1,8 @@
 """Thin torch-tensor front end of the C ABI (device memory and streams only).
 
 Every function takes CUDA(=HIP) tensors, passes raw pointers to libcatccos_mx.so on
-torch's current stream and returns tensors.  bf16 data may be given as
+torch's current stream and returns tensors.  The calls of a layer allocate and call through _native_call; set-up and checking
+functions through ctypes.  bf16 data may be given as
 torch.bfloat16 or as int16/uint16 bit patterns.  No function here computes
 anything in torch.
 """
@@ -10,6 +11,13 @@ from __future__ import annotations
 import torch
 
 from . import _lib
+
+try:
+    from . import _native_call
+except ImportError as e:
+    raise ImportError(f"catccos_amd/_native_call.so: {e}; build it with `python -m catccos_amd.build`") from e
+
+_run, _empty = _native_call.run, _native_call.empty
 
 FMT = {"E4M3": 0, "E5M2": 1, "E2M1": 2, "E1M2": 3}
 _FP4 = ("E2M1", "E1M2")
@@ -20,17 +28,25 @@ _OUT_DTYPE = {"bf16": torch.bfloat16, "fp16": torch.float16, "fp32": torch.float
 
 # not a public function of torch, so it may be missing
 _raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)
+_device = getattr(torch._C, "_cuda_getDevice", None) or torch.cuda.current_device
 
 
 def _stream():
-    # the handle of torch's current stream without a Stream object around it: 0.3 us of host time against 2.8, of 10 a call
+    # the handle of torch's current stream without a Stream object around it: 0.2 us of host time against 2.8, of 5 a call
     if _raw_stream is not None:
-        return _raw_stream(torch.cuda.current_device())
+        return _raw_stream(_device())
     return torch.cuda.current_stream().cuda_stream
 
 
 def _p(t: torch.Tensor):
     return t.data_ptr() if t is not None else None
+
+
+def _launch(name, *args):
+    """The entry point `name` on these tensors (GPU tensors, or ValueError), integers and Nones, and torch's current stream."""
+    rc = _run(_lib.entries()[name], *args, _stream())
+    if rc != 0:
+        _lib.check(rc)
 
 
 def _need_cuda(*ts):
@@ -46,17 +62,17 @@ def scale_cols(cols: int) -> int:
 
 def mx_quant(x: torch.Tensor, fmt: str = "E4M3", mode: str | None = None):
     """x: bf16 [rows, cols] -> (codes u8 [rows, cols or cols/2], scales u8 [rows, RoundUp2(cols/32)])."""
-    _need_cuda(x)
-    assert x.dim() == 2 and x.element_size() == 2 and x.stride(1) == 1
+    assert x.dim() == 2 and x.element_size() == 2
     rows, cols = x.shape
+    pitch, step = x.stride()
+    assert step == 1
+    fp4 = fmt in _FP4
     if mode is None:
-        mode = "lut" if fmt in _FP4 else "rne"
-    ccols = (cols + 1) // 2 if fmt in _FP4 else cols
-    codes = torch.empty((rows, ccols), dtype=torch.uint8, device=x.device)
-    scales = torch.empty((rows, scale_cols(cols)), dtype=torch.uint8, device=x.device)
-    lib = _lib.load()
-    _lib.check(lib.cmx_mx_quant(_p(x), x.stride(0), _p(codes), ccols, _p(scales), scales.shape[1], rows, cols,
-                                FMT[fmt], ROUND[mode], _stream()))
+        mode = "lut" if fp4 else "rne"
+    ccols = (cols + 1) // 2 if fp4 else cols
+    scols = scale_cols(cols)
+    codes, scales = _empty(x, torch.uint8, rows, ccols), _empty(x, torch.uint8, rows, scols)
+    _launch("cmx_mx_quant", x, pitch, codes, ccols, scales, scols, rows, cols, FMT[fmt], ROUND[mode])
     return codes, scales
 
 
@@ -72,12 +88,10 @@ def mx_dequant(codes: torch.Tensor, scales: torch.Tensor, cols: int, fmt: str = 
 
 def mx_gemm(a, a_scale, b, b_scale, k: int, fmt: str = "E4M3", out: str = "bf16") -> torch.Tensor:
     """C[m,n] = deq(a)[m,k] . deq(b)[n,k]^T"""
-    _need_cuda(a, a_scale, b, b_scale)
-    m, n = a.shape[0], b.shape[0]
-    c = torch.empty((m, n), dtype=_OUT_DTYPE[out], device=a.device)
-    lib = _lib.load()
-    _lib.check(lib.cmx_mx_gemm(_p(a), a.stride(0), _p(a_scale), a_scale.stride(0), _p(b), b.stride(0), _p(b_scale),
-                               b_scale.stride(0), _p(c), n, m, n, k, FMT[fmt], OUT[out], _stream()))
+    m, n = a.size(0), b.size(0)
+    c = _empty(a, _OUT_DTYPE[out], m, n)
+    _launch("cmx_mx_gemm", a, a.stride(0), a_scale, a_scale.stride(0), b, b.stride(0), b_scale, b_scale.stride(0), c, n, m, n, k, FMT[fmt],
+            OUT[out])
     return c
 
 
@@ -112,14 +126,11 @@ def mx_gemm_ex(a, a_scale, b, b_scale, m: int, n: int, k: int, fmt: str = "E4M3"
                trans_b: int = 1) -> torch.Tensor:
     """Dense operands in the reference's file layouts: a [m, k] (trans_a = 1: [k, m], scales [k/64, m, 2]);
     b [n, k] (trans_b = 0: [k, n], scales [k/64, n, 2])."""
-    _need_cuda(a, a_scale, b, b_scale)
-    assert all(t.is_contiguous() for t in (a, a_scale, b, b_scale))
-    lib = _lib.load()
-    need = lib.cmx_mx_gemm_ex_workspace_bytes(m, n, k, trans_a, trans_b)
-    ws = torch.empty(max(need, 1), dtype=torch.uint8, device=a.device)
-    c = torch.empty((m, n), dtype=_OUT_DTYPE[out], device=a.device)
-    _lib.check(lib.cmx_mx_gemm_ex(_p(a), _p(a_scale), _p(b), _p(b_scale), _p(c), n, m, n, k, FMT[fmt], OUT[out], trans_a,
-                                  trans_b, _p(ws), _stream()))
+    assert a.is_contiguous() and a_scale.is_contiguous() and b.is_contiguous() and b_scale.is_contiguous()
+    need = _lib.load().cmx_mx_gemm_ex_workspace_bytes(m, n, k, trans_a, trans_b)
+    ws = _empty(a, torch.uint8, max(need, 1))
+    c = _empty(a, _OUT_DTYPE[out], m, n)
+    _launch("cmx_mx_gemm_ex", a, a_scale, b, b_scale, c, n, m, n, k, FMT[fmt], OUT[out], trans_a, trans_b, ws)
     return c
 
 
@@ -139,28 +150,25 @@ def mx_gmm_ex(a, a_scale, b, b_scale, group_sizes, n: int, k: int, fmt: str = "E
 
 def int8_quant_scatter(x: torch.Tensor, src2sorted, top_k: int = 1):
     """x bf16 [tokens, k] -> (codes int8 [tokens*top_k, k], scales fp32 [tokens*top_k]); row t goes to src2sorted[t*top_k + r]."""
-    _need_cuda(x, src2sorted)
-    assert x.dim() == 2 and x.element_size() == 2 and x.stride(1) == 1
+    assert x.dim() == 2 and x.element_size() == 2
     tokens, k = x.shape
-    codes = torch.empty((tokens * top_k, k), dtype=torch.int8, device=x.device)
-    scales = torch.empty((tokens * top_k,), dtype=torch.float32, device=x.device)
-    lib = _lib.load()
-    _lib.check(lib.cmx_int8_quant_scatter(_p(x), x.stride(0), _p(src2sorted), _p(codes), k, _p(scales), tokens, k, top_k, _stream()))
+    pitch, step = x.stride()
+    assert step == 1
+    codes, scales = _empty(x, torch.int8, tokens * top_k, k), _empty(x, torch.float32, tokens * top_k)
+    _launch("cmx_int8_quant_scatter", x, pitch, src2sorted, codes, k, scales, tokens, k, top_k)
     return codes, scales
 
 
 def int8_gmm_dequant_swiglu(a, token_scale, b, channel_scale, group_sizes, n: int, k: int, trans_b: int = 0,
                             out: str = "fp32", scale_stride: int = 1, c=None) -> torch.Tensor:
     """a int8 [rows, k]; b int8 [G, k, n] (trans_b = 0) or [G, n, k] (trans_b = 1); channel_scale fp32 [G*n*scale_stride]."""
-    _need_cuda(a, token_scale, b, channel_scale, group_sizes)
     assert a.is_contiguous() and b.is_contiguous() and group_sizes.dtype == torch.int32
-    rows, g = a.shape[0], b.shape[0]
-    lib = _lib.load()
-    ws = torch.empty(lib.cmx_int8_gmm_workspace_bytes(g, n, k, trans_b), dtype=torch.uint8, device=a.device)
+    rows, g = a.size(0), b.size(0)
+    ws = _empty(a, torch.uint8, _lib.load().cmx_int8_gmm_workspace_bytes(g, n, k, trans_b))
     if c is None:
         c = torch.zeros((rows, n // 2), dtype=_OUT_DTYPE[out], device=a.device)
-    _lib.check(lib.cmx_int8_gmm_dequant_swiglu(_p(a), k, _p(token_scale), _p(b), _p(channel_scale), scale_stride, _p(c),
-                                               c.stride(0), OUT[out], _p(group_sizes), g, rows, n, k, trans_b, _p(ws), _stream()))
+    _launch("cmx_int8_gmm_dequant_swiglu", a, k, token_scale, b, channel_scale, scale_stride, c, c.stride(0), OUT[out], group_sizes, g, rows, n, k,
+            trans_b, ws)
     return c
 
 
@@ -196,29 +204,26 @@ def pretile_weights(b: torch.Tensor, pair_gate_up: bool) -> PretiledWeights:
 
 
 def _weights(b, pair_gate_up: bool):
-    """(pointer, pretiled?) of a weight argument: a dense tensor or PretiledWeights of the matching kind."""
+    """(tensor, pretiled?) of a weight argument: a dense tensor or PretiledWeights of the matching kind."""
     if isinstance(b, PretiledWeights):
         assert b.pair_gate_up == pair_gate_up, "weights were pre-tiled for the other grouped matmul"
-        return _p(b.data), True
+        return b.data, True
     assert b.is_contiguous()
-    return _p(b), False
+    return b, False
 
 
 def mx_gmm(a, a_scale, b, b_scale, group_sizes, k: int, fmt: str = "E4M3", out: str = "bf16", c=None, workspace=None):
     """a [m_total, k], b [G, n, k] (dense tensor or PretiledWeights), group_sizes int32 [G] on device -> c [m_total, n]
     (rows past the groups untouched)."""
-    _need_cuda(a, a_scale, b_scale, group_sizes)
     assert b_scale.is_contiguous() and group_sizes.dtype == torch.int32
-    bp, tiled = _weights(b, False)
-    m, (g, n) = a.shape[0], b.shape[:2]
+    bd, tiled = _weights(b, False)
+    m, (g, n) = a.size(0), b.shape[:2]
     if c is None:
         c = torch.zeros((m, n), dtype=_OUT_DTYPE[out], device=a.device)
     if workspace is None:
         workspace = gmm_workspace(g, a.device)
-    lib = _lib.load()
-    fn = lib.cmx_mx_gmm_pretiled if tiled else lib.cmx_mx_gmm
-    _lib.check(fn(_p(a), a.stride(0), _p(a_scale), a_scale.stride(0), bp, _p(b_scale), _p(c), c.stride(0),
-                  _p(group_sizes), g, m, n, k, FMT[fmt], OUT[out], _p(workspace), _stream()))
+    _launch("cmx_mx_gmm_pretiled" if tiled else "cmx_mx_gmm", a, a.stride(0), a_scale, a_scale.stride(0), bd, b_scale, c, c.stride(0), group_sizes,
+            g, m, n, k, FMT[fmt], OUT[out], workspace)
     return c
 
 
@@ -226,10 +231,9 @@ def mx_gmm_swiglu_quant(a, a_scale, b, b_scale, group_sizes, k: int, want_bf16: 
                         outs=None):
     """GMM1 + SwiGLU + MX requant.  b [G, n, k] (gate rows then up rows; dense tensor or PretiledWeights).
     Returns (codes [m, n/2], scales, act_bf16|None)."""
-    _need_cuda(a, a_scale, b_scale, group_sizes)
     assert b_scale.is_contiguous() and group_sizes.dtype == torch.int32
-    bp, tiled = _weights(b, True)
-    m, (g, n) = a.shape[0], b.shape[:2]
+    bd, tiled = _weights(b, True)
+    m, (g, n) = a.size(0), b.shape[:2]
     half = n // 2
     if outs is None:
         codes = torch.zeros((m, half), dtype=torch.uint8, device=a.device)
@@ -239,10 +243,8 @@ def mx_gmm_swiglu_quant(a, a_scale, b, b_scale, group_sizes, k: int, want_bf16: 
     act = torch.zeros((m, half), dtype=torch.bfloat16, device=a.device) if want_bf16 else None
     if workspace is None:
         workspace = gmm_workspace(g, a.device)
-    lib = _lib.load()
-    fn = lib.cmx_mx_gmm_swiglu_quant_pretiled if tiled else lib.cmx_mx_gmm_swiglu_quant
-    _lib.check(fn(_p(a), a.stride(0), _p(a_scale), a_scale.stride(0), bp, _p(b_scale), _p(codes), codes.stride(0),
-                  _p(scales), scales.stride(0), _p(act), _p(group_sizes), g, m, n, k, _p(workspace), _stream()))
+    _launch("cmx_mx_gmm_swiglu_quant_pretiled" if tiled else "cmx_mx_gmm_swiglu_quant", a, a.stride(0), a_scale, a_scale.stride(0), bd, b_scale, codes,
+            codes.stride(0), scales, scales.stride(0), act, group_sizes, g, m, n, k, workspace)
     return codes, scales, act
 
 
@@ -265,17 +267,13 @@ def init() -> None:
 
 def moe_init_routing(expert_idx: torch.Tensor, experts: int):
     """expert_idx int32 [T, topK] -> (sorted2src, src2sorted, counts) int32."""
-    _need_cuda(expert_idx)
     assert expert_idx.dtype == torch.int32 and expert_idx.is_contiguous()
     t, top_k = expert_idx.shape
-    dev = expert_idx.device
-    s2s = torch.empty(t * top_k, dtype=torch.int32, device=dev)
-    inv = torch.empty(t * top_k, dtype=torch.int32, device=dev)
-    counts = torch.empty(experts, dtype=torch.int32, device=dev)
-    lib = _lib.load()
-    ws = torch.empty(lib.cmx_moe_routing_workspace_bytes(t * top_k, experts), dtype=torch.uint8, device=dev)
-    _lib.check(lib.cmx_moe_init_routing(_p(expert_idx), t, top_k, experts, _p(s2s), _p(inv), _p(counts), _p(ws),
-                                        _stream()))
+    routes = t * top_k
+    s2s, inv = _empty(expert_idx, torch.int32, routes), _empty(expert_idx, torch.int32, routes)
+    counts = _empty(expert_idx, torch.int32, experts)
+    ws = _empty(expert_idx, torch.uint8, _lib.load().cmx_moe_routing_workspace_bytes(routes, experts))
+    _launch("cmx_moe_init_routing", expert_idx, t, top_k, experts, s2s, inv, counts, ws)
     return s2s, inv, counts
 
 
@@ -295,10 +293,9 @@ def quant_scatter(x: torch.Tensor, src2sorted: torch.Tensor, top_k: int, packed:
         _lib.check(lib.cmx_quant_scatter(_p(x), x.stride(0), _p(src2sorted), _p(buf), rb, buf.data_ptr() + k, rb, t, k,
                                          top_k, _stream()))
         return buf
-    codes = torch.empty((rows, k), dtype=torch.uint8, device=x.device)
-    scales = torch.empty((rows, scale_cols(k)), dtype=torch.uint8, device=x.device)
-    _lib.check(lib.cmx_quant_scatter_zeroed(_p(x), x.stride(0), _p(src2sorted), _p(codes), k, _p(scales), scales.shape[1], t, k,
-                                     top_k, _stream()))
+    scols = scale_cols(k)
+    codes, scales = _empty(x, torch.uint8, rows, k), _empty(x, torch.uint8, rows, scols)
+    _launch("cmx_quant_scatter_zeroed", x, x.stride(0), src2sorted, codes, k, scales, scols, t, k, top_k)
     return codes, scales
 
 
@@ -337,20 +334,19 @@ def dispatch_ffn_combine(x, expert_idx, gate_weight, w1, w1_scale, w2, w2_scale,
     top_k = expert_idx.shape[1]
     for t in (x, expert_idx, gate_weight, w1_scale, w2_scale):
         assert t.is_contiguous()
-    w1p, tiled1 = _weights(w1, True)
-    w2p, tiled2 = _weights(w2, False)
+    w1d, tiled1 = _weights(w1, True)
+    w2d, tiled2 = _weights(w2, False)
     assert tiled1 == tiled2, "pre-tile both weight tensors or neither"
-    lib = _lib.load()
     if workspace is None:
-        workspace = torch.empty(ffn_workspace_bytes(m, k, n, e, top_k), dtype=torch.uint8, device=x.device)
+        workspace = _empty(x, torch.uint8, ffn_workspace_bytes(m, k, n, e, top_k))
     if out is None:
-        out = torch.empty((m, k), dtype=x.dtype, device=x.device)
+        out = _empty(x, x.dtype, m, k)
+    entries = _lib.entries()
     if tiled1:
-        _lib.check(lib.cmx_dispatch_ffn_combine_pretiled(
-            _stream(), _p(x), _p(expert_idx), _p(gate_weight), w1p, _p(w1_scale), w2p, _p(w2_scale), _p(out),
-            _p(workspace), m, k, n, e, top_k))
-        return out
-    _lib.check(lib.catccos_ascend950_dispatch_ffn_combine(
-        0, _stream(), 0, _p(x), _p(expert_idx), _p(gate_weight), w1p, _p(w1_scale), w2p, _p(w2_scale), _p(out),
-        _p(workspace), None, m, k, n, e, top_k, 1))
+        rc = _run(entries["cmx_dispatch_ffn_combine_pretiled"], _stream(), x, expert_idx, gate_weight, w1d, w1_scale, w2d, w2_scale, out, workspace,
+                  m, k, n, e, top_k)
+    else:
+        rc = _run(entries["catccos_ascend950_dispatch_ffn_combine"], 0, _stream(), 0, x, expert_idx, gate_weight, w1d, w1_scale, w2d, w2_scale, out,
+                  workspace, None, m, k, n, e, top_k, 1)
+    _lib.check(rc)
     return out

@@ -1,0 +1,63 @@
+"""catccos_amd._native_call: what reaches an entry point, and what is refused before it does."""
+import ctypes as C
+
+import pytest
+import torch
+
+from catccos_amd import _lib, _native_call, ops
+
+
+@pytest.mark.parametrize("n", [0, 6, 7, 24])
+def test_every_argument_arrives_in_its_place(n):
+    got = []
+    proto = C.CFUNCTYPE(C.c_int, *[C.c_uint64] * 24)
+
+    @proto
+    def callee(*args):
+        got.extend(args)
+        return -7
+    values = [2 ** 40 + i if i % 3 else (None if i % 2 else -1 - i) for i in range(n)]
+    assert _native_call.run(C.cast(callee, C.c_void_p).value, *values) == -7
+    want = [0 if v is None else v % 2 ** 64 for v in values]
+    assert got == want + [0] * (24 - n)
+
+
+def test_refusals():
+    x = torch.zeros(2, 32, dtype=torch.bfloat16)
+    address = _lib.entries()["cmx_version"]
+    for args in ((address, x),):
+        with pytest.raises(ValueError, match="expected a GPU tensor"):
+            _native_call.run(*args)
+    with pytest.raises(ValueError, match="expected a GPU tensor"):
+        _native_call.empty(x, torch.uint8, 2)
+    for call in (lambda: _native_call.run(), lambda: _native_call.run(address, *range(25)), lambda: _native_call.run(address, 1.5),
+                 lambda: _native_call.run(address, "x"), lambda: _native_call.empty(x, torch.uint8), lambda: _native_call.empty(1, torch.uint8, 2)):
+        with pytest.raises(TypeError):
+            call()
+    with pytest.raises(ValueError):
+        _native_call.run(0, 1)
+    for call in (lambda: ops.mx_quant(x), lambda: ops.mx_gemm(x, x, x, x, 32), lambda: ops.moe_init_routing(torch.zeros(2, 2, dtype=torch.int32), 4)):
+        with pytest.raises(ValueError, match="expected a GPU tensor"):
+            call()
+
+
+def test_entries_follow_the_active_library():
+    before = _lib.entries()
+    prev = _lib.activate(None)
+    try:
+        assert _lib.entries() is not before
+    finally:
+        _lib.activate(prev)
+    assert set(_lib.entries()) == set(_lib.SIGNATURES) and all(_lib.entries().values())
+
+
+@pytest.mark.gpu
+def test_outputs_and_errors_on_the_gpu():
+    x = torch.randn(3, 64, device="cuda").to(torch.bfloat16)
+    t = _native_call.empty(x, torch.float16, 2, 3, 4)
+    assert t.shape == (2, 3, 4) and t.dtype == torch.float16 and t.device == x.device and not t.requires_grad
+    assert _native_call.empty(x, torch.uint8, 0).numel() == 0
+    with pytest.raises(_lib.CmxError, match="k must be"):
+        ops.mx_gemm(x.view(torch.uint8), x.view(torch.uint8), x.view(torch.uint8), x.view(torch.uint8), 33)
+    with pytest.raises(ValueError, match="expected a GPU tensor"):
+        ops.mx_gemm(x.view(torch.uint8), x.view(torch.uint8), x.view(torch.uint8).cpu(), x.view(torch.uint8), 32)
