@@ -100,8 +100,8 @@ __device__ __forceinline__ void fill_group_tables(const GroupTablesJob& j) {
 #endif  // __HIPCC__
 
 // ---- a chain that fills the tables of its grouped matmuls in an earlier launch --------------------------------------------------------
-// What a grouped matmul on these sizes will ask of its tables (in `workspace`, as for the call itself), and the two matmuls of the FFN with
-// their tables filled.
+// What a grouped matmul on these sizes will ask of its tables (in `workspace`, as for the call itself), and the two matmuls of the
+// FFN with their tables filled.
 int plan_group_tables(GroupTablesJob* job, const int32_t* group_sizes, uint32_t groups, uint32_t m_total, uint32_t n, uint32_t k, int fmt,
                       bool swiglu, bool pretiled, void* workspace);
 int gmm_swiglu_quant_prepared(const uint8_t* a, uint32_t lda, const uint8_t* a_scale, uint32_t ld_as, const uint8_t* b, const uint8_t* b_scale,

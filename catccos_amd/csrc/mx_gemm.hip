@@ -1331,15 +1331,21 @@ GroupTablesJob tables_job(const GroupTables& g, const int32_t* group_sizes, uint
     return {group_sizes, groups, tile_m, m_total, small_rows, g.row_off, g.tile_pref, g.small_pref, g.tile_ctr};
 }
 
-// Fills the tables for m-tiles of tile_m rows (of the groups past ks.small_rows), unless an earlier launch has, and sets the parameters
-// that refer to them.
-int prepare_groups(GemmParams& p, const GroupTablesJob& job, bool filled, hipStream_t s) {
+// Sets the parameters that say where the groups lie: their sizes, where all kernels of the call locate their tiles by them, or the
+// tables for m-tiles of tile_m rows (of the groups past small_rows), filled here unless an earlier launch has.
+int prepare_groups(GemmParams& p, const GroupTablesJob& job, bool by_sizes, bool filled, hipStream_t s) {
+    p.small_rows = job.small_rows;
+    p.group_class = job.small_rows != 0 ? kLargeGroups : kAllGroups;
+    p.groups = job.groups;
+    if (by_sizes) {
+        p.sizes = job.sizes;
+        return CMX_OK;
+    }
     if (!filled)
         if (int rc = launch_group_tables(job, s); rc != CMX_OK) return rc;
     p.row_off = job.row_off;
     p.tile_pref = job.tile_pref;
     p.tile_ctr = job.tile_ctr;
-    p.groups = job.groups;
     return CMX_OK;
 }
 
@@ -1350,6 +1356,7 @@ int launch_grouped_ksplit(GemmParams p, const GroupTables& g, const GroupedKspli
     if (ks.small_rows == 0)
         return launch_ksplit(p, ks.tile, fmt, epi, m_total / (16 * ks.tile.fm) + p.groups, ks.weights, s);
     p.tile_pref = g.small_pref;
+    p.group_class = kSmallGroups;
     return launch_ksplit(p, ks.tile, fmt, epi, p.groups < m_total ? p.groups : m_total, ks.weights, s);
 }
 
@@ -1390,6 +1397,17 @@ struct GroupPlan {
     bool all_ksplit() const { return ks.tile.fw != 0 && ks.small_rows == 0; }
     uint32_t tile_m() const { return all_ksplit() ? 16 * ks.tile.fm : t.tm; }
 };
+
+// Whether kernels that take one tile per workgroup locate it by the sizes themselves.  A launch that fills tables first costs 5 us; a scan at
+// the start of a workgroup some 0.3 us more than the table reads, once for each round of workgroups: 32 experts x 16 rows of FP4, five
+// rounds of two workgroups per CU, 93.4 us with tables and 92.4 without; FFN of 32 tokens, 256 experts, where the tables cost no launch, 1119
+// with and 1053 against 1039 of another box without; INT8 of 2144 tiles, one per CU at a time, no difference.
+int tiles_by_sizes(bool* out, uint32_t groups, uint64_t max_tiles, uint32_t per_cu) {
+    int cus = 0;
+    if (int rc = cu_count(&cus); rc != CMX_OK) return rc;
+    *out = groups <= kInlineGroups && max_tiles <= 4 * (uint64_t)per_cu * cus;
+    return CMX_OK;
+}
 int plan_groups(GroupPlan* plan, uint32_t m_total, uint32_t groups, uint32_t n, int fmt, uint32_t kblocks, bool swiglu, bool pretiled) {
     if (int rc = choose_grouped_ksplit(m_total, groups, n, fmt, kblocks, &plan->ks); rc != CMX_OK) return rc;
     // average rows per group steers the tile height
@@ -1418,7 +1436,12 @@ int gmm_common(GemmParams& p, const int32_t* group_sizes, uint32_t groups, uint3
     const TileChoice& t = plan.t;
     const bool all_ksplit = plan.all_ksplit();
     const GroupTables tables(workspace, groups);
-    if (int rc = prepare_groups(p, tables_job(tables, group_sizes, groups, m_total, plan.tile_m(), ks.small_rows), tables_filled, s); rc != CMX_OK) return rc;
+    bool by_sizes = false;                                     // (the persistent kernels walk from tile to tile through tables)
+    if (!tables_filled && (all_ksplit || t.waves == kRing)) {
+        const uint64_t tiles = all_ksplit ? (uint64_t)(m_total / 64 + groups) * ceil_div(p.n, 64) : (uint64_t)(m_total / t.tm + groups) * ceil_div(p.n, t.tw);
+        if (int rc = tiles_by_sizes(&by_sizes, groups, tiles, all_ksplit ? 2 : 1); rc != CMX_OK) return rc;
+    }
+    if (int rc = prepare_groups(p, tables_job(tables, group_sizes, groups, m_total, plan.tile_m(), ks.small_rows), by_sizes, tables_filled, s); rc != CMX_OK) return rc;
     if (ks.tile.fw != 0) {
         const int epi = !swiglu ? kEpiStore : (p.act_bf16 != nullptr ? kEpiSwigluQuantAct : kEpiSwigluQuant);
         if (int rc = launch_grouped_ksplit(p, tables, ks, fmt, epi, m_total, s); rc != CMX_OK || all_ksplit) return rc;
@@ -1531,7 +1554,9 @@ extern "C" int cmx_int8_gmm_dequant_swiglu(const int8_t* a, uint32_t lda, const 
     const bool all_ksplit = ks.tile.fw != 0 && ks.small_rows == 0;
     const GroupTables tables(ws, groups);
     const uint32_t tile_m = all_ksplit ? 16 * ks.tile.fm : kTile;
-    if (int rc = prepare_groups(p, tables_job(tables, group_sizes, groups, m_total, tile_m, ks.small_rows), false, s); rc != CMX_OK) return rc;
+    bool by_sizes = false;                                     // (all its kernels take one tile per workgroup)
+    if (int rc = tiles_by_sizes(&by_sizes, groups, (uint64_t)(m_total / tile_m + groups) * ceil_div(n, all_ksplit ? 64 : kTile), all_ksplit ? 2 : 1); rc != CMX_OK) return rc;
+    if (int rc = prepare_groups(p, tables_job(tables, group_sizes, groups, m_total, tile_m, ks.small_rows), by_sizes, false, s); rc != CMX_OK) return rc;
     if (ks.tile.fw != 0)
         if (int rc = launch_grouped_ksplit(p, tables, ks, kFmtI8, kEpiI8DequantSwiglu, m_total, s); rc != CMX_OK || all_ksplit) return rc;
     p.w_tiles = ceil_div(n / 2, kTile / 2);

@@ -27,6 +27,10 @@ constexpr bool epi_pairs_gate_up(int epi) { return epi_is_swiglu_quant(epi) || e
 // element "format" of the INT8 path inside the kernel templates (the public format codes are the MX ones)
 constexpr int kFmtI8 = 8;
 
+// Groups of a grouped problem that a launch takes: all; those of 1 .. small_rows rows (one m-tile each); those of more.
+enum GroupClass { kAllGroups = 0, kSmallGroups = 1, kLargeGroups = 2 };
+constexpr uint32_t kInlineGroups = 256;
+
 struct GemmParams {
     const uint8_t* a;        // activations codes
     const uint8_t* a_scale;
@@ -38,6 +42,9 @@ struct GemmParams {
     uint16_t* act_bf16;
     const int32_t* row_off;     // [groups+1] (grouped) or null (dense)
     const int32_t* tile_pref;   // [groups+1] prefix of m-tiles (grouped) or null
+    const int32_t* sizes;       // [groups] rows of the groups, in the place of the two tables (at most kInlineGroups), or null
+    uint32_t small_rows;        // with `sizes`: the limit between ...
+    int group_class;            // ... the groups that this launch takes (GroupClass)
     int32_t* tile_ctr;          // [8] per-XCD tile counters, zeroed before the launch (persistent grouped 4 x 1 kernels) or null
     uint32_t lda, ld_as, ldw, ld_ws, ldc, ld_act, ld_acts;
     uint32_t m, n, kbytes, kblocks;   // kblocks = K/32
@@ -133,6 +140,25 @@ __device__ __forceinline__ uint32_t tile_of_workgroup(uint32_t total_tiles) {
     return full + xcd_run(total_tiles - full, k % kXcds, count) + k / kXcds;
 }
 
+// Tile L of group g, whose m-tiles are tp .. tp1 - 1 and whose rows r_begin .. r_end - 1.  Bands of 8 m-tiles share a run of weight tiles
+// (m fastest inside a band): the 32 tiles that an XCD works on at a time then touch 8 + 4 operand panels instead of mtg + 32/mtg
+template <int TM>
+__device__ __forceinline__ void place_in_group(const GemmParams& p, uint32_t g, uint32_t tp, uint32_t tp1, uint32_t r_begin, uint32_t r_end,
+                                               uint32_t L, Tile& t) {
+    t.g = g;
+    const uint32_t mtg = tp1 - tp;
+    const uint32_t local = L - tp * p.w_tiles;
+    const uint32_t band = 8;
+    const uint32_t per_band = band * p.w_tiles;
+    const uint32_t b = local / per_band, within = local % per_band;
+    const uint32_t band_rows = (mtg - b * band) < band ? (mtg - b * band) : band;
+    t.mt = b * band + within % band_rows;
+    t.wt = within / band_rows;
+    t.row0 = r_begin + t.mt * TM;
+    t.rows_left = r_end - t.row0;
+    t.rows_valid = t.rows_left < (uint32_t)TM ? t.rows_left : (uint32_t)TM;
+}
+
 // g_from: a group at or before the tile's (0, or the group of an earlier tile of an increasing sequence)
 template <int TM>
 __device__ __forceinline__ void decode_tile(const GemmParams& p, uint32_t m_tiles_all, uint32_t L, Tile& t, uint32_t g_from = 0) {
@@ -153,22 +179,8 @@ __device__ __forceinline__ void decode_tile(const GemmParams& p, uint32_t m_tile
             const uint32_t mid = (lo + hi) >> 1;
             if ((uint32_t)table_at(p.tile_pref, mid) * p.w_tiles <= L) lo = mid; else hi = mid;
         }
-        t.g = lo;
-        const uint32_t tp = (uint32_t)table_at(p.tile_pref, lo);
-        const uint32_t mtg = (uint32_t)table_at(p.tile_pref, lo + 1) - tp;
-        // bands of 8 m-tiles share a run of weight tiles (m fastest inside a band): the 32 tiles that an XCD
-        // works on at a time then touch 8 + 4 operand panels instead of mtg + 32/mtg
-        const uint32_t local = L - tp * p.w_tiles;
-        const uint32_t band = 8;
-        const uint32_t per_band = band * p.w_tiles;
-        const uint32_t b = local / per_band, within = local % per_band;
-        const uint32_t band_rows = (mtg - b * band) < band ? (mtg - b * band) : band;
-        t.mt = b * band + within % band_rows;
-        t.wt = within / band_rows;
-        const uint32_t r_begin = (uint32_t)table_at(p.row_off, lo), r_end = (uint32_t)table_at(p.row_off, lo + 1);
-        t.row0 = r_begin + t.mt * TM;
-        t.rows_left = r_end - t.row0;
-        t.rows_valid = t.rows_left < (uint32_t)TM ? t.rows_left : (uint32_t)TM;
+        place_in_group<TM>(p, lo, (uint32_t)table_at(p.tile_pref, lo), (uint32_t)table_at(p.tile_pref, lo + 1), (uint32_t)table_at(p.row_off, lo),
+                           (uint32_t)table_at(p.row_off, lo + 1), L, t);
     } else {
         // bands of 4 m-tiles share a run of weight tiles
         const uint32_t band = 4;
@@ -184,10 +196,67 @@ __device__ __forceinline__ void decode_tile(const GemmParams& p, uint32_t m_tile
     }
 }
 
+// op (neutral element 0) over lanes 0 .. l of the wavefront, in lane l
+template <class Op>
+__device__ __forceinline__ uint32_t wave_scan(uint32_t v, Op op) {
+    v = op(v, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x111, 0xF, 0xF, false));       // row_shr:1
+    v = op(v, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x112, 0xF, 0xF, false));
+    v = op(v, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x114, 0xF, 0xF, false));
+    v = op(v, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x118, 0xF, 0xF, false));
+    v = op(v, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x142, 0xA, 0xF, false));       // row_bcast:15
+    v = op(v, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x143, 0xC, 0xF, false));       // row_bcast:31
+    return v;
+}
+
+// The tile of this workgroup from the group sizes themselves: every wavefront scans them (four groups per lane), so that no launch has to
+// write tables first (5 us) and no chain of dependent table reads follows the start of every workgroup.  Sizes are clipped as in
+// fill_group_tables: negative ones count as zero, rows past m_total (p.m) do not exist (a sum that stops at m_total is associative).
+template <int TM>
+__device__ __forceinline__ bool locate_tile_by_sizes(const GemmParams& p, Tile& t) {
+    constexpr int kPer = kInlineGroups / 64;
+    const uint32_t lane = threadIdx.x & 63u, m = p.m;
+    const auto sat = [m](uint32_t a, uint32_t b) -> uint32_t { return min(a + b, m); };          // a, b <= m < 2^31
+    uint32_t c[kPer], sum = 0;
+#pragma unroll
+    for (int j = 0; j < kPer; ++j) {
+        const uint32_t i = kPer * lane + j;
+        const int32_t v = i < p.groups ? p.sizes[i] : 0;
+        c[j] = v > 0 ? min((uint32_t)v, m) : 0u;
+        sum = sat(sum, c[j]);
+    }
+    const uint32_t to = wave_scan(sum, sat);
+    uint32_t off[kPer + 1], tiles[kPer], all = 0;
+    off[0] = (uint32_t)__shfl_up((int)to, 1);
+    if (lane == 0) off[0] = 0;
+#pragma unroll
+    for (int j = 0; j < kPer; ++j) {
+        off[j + 1] = sat(off[j], c[j]);
+        const uint32_t rows = off[j + 1] - off[j], small = rows <= p.small_rows ? 1u : 0u;
+        const uint32_t whole = (rows + TM - 1) / TM;
+        tiles[j] = p.group_class == kAllGroups ? whole : (p.group_class == kSmallGroups ? (rows != 0 ? small : 0u) : (small ? 0u : whole));
+        all += tiles[j];
+    }
+    const uint32_t pref = wave_scan(all, [](uint32_t a, uint32_t b) -> uint32_t { return a + b; });
+    const uint32_t total = (uint32_t)__builtin_amdgcn_readlane((int)pref, 63) * p.w_tiles;
+    if (blockIdx.x >= total) return false;
+    const uint32_t L = tile_of_workgroup(total);
+    const int at = (int)__builtin_ctzll(__ballot(pref * p.w_tiles > L));                         // lane of the tile's group
+    uint32_t tp = (uint32_t)__builtin_amdgcn_readlane((int)(pref - all), at), g = kPer * at;
+#pragma unroll
+    for (int j = 0; j < kPer; ++j) {
+        const uint32_t n = (uint32_t)__builtin_amdgcn_readlane((int)tiles[j], at);
+        const uint32_t r0 = (uint32_t)__builtin_amdgcn_readlane((int)off[j], at), r1 = (uint32_t)__builtin_amdgcn_readlane((int)off[j + 1], at);
+        if (L >= tp * p.w_tiles && L < (tp + n) * p.w_tiles) place_in_group<TM>(p, g + j, tp, tp + n, r0, r1, L, t);
+        tp += n;
+    }
+    return true;
+}
+
 // One tile per workgroup: maps the workgroup id to (group, m-tile, weight tile).  Returns false for ids past
 // the last tile.
 template <int TM>
 __device__ __forceinline__ bool locate_tile(const GemmParams& p, Tile& t) {
+    if (p.sizes != nullptr) return locate_tile_by_sizes<TM>(p, t);
     const uint32_t m_tiles_all = count_m_tiles<TM>(p);
     const uint32_t total_tiles = m_tiles_all * p.w_tiles;
     if (blockIdx.x >= total_tiles) return false;

@@ -508,7 +508,7 @@ int launch_one(const GemmParams& p, uint32_t max_m_tiles, hipStream_t s) {
 template <int FMT, int EPI, int LAYOUT>
 int launch_shape(const GemmParams& p, const KsplitTile& t, uint32_t max_m_tiles, KsplitWeights loads, hipStream_t s) {
 #define CMX_KS(FW_, FM_, NW_) if (t.fw == FW_ && t.fm == FM_ && t.waves == NW_) return launch_one<FMT, FW_, FM_, NW_, EPI, LAYOUT, KsplitWeights::kCached>(p, max_m_tiles, s)
-    if constexpr (LAYOUT != kKSlow) if (t.fw == 4 && t.fm == 4 && t.waves == 4 && p.row_off != nullptr) {
+    if constexpr (LAYOUT != kKSlow) if (t.fw == 4 && t.fm == 4 && t.waves == 4 && (p.row_off != nullptr || p.sizes != nullptr)) {
         if (loads == KsplitWeights::kStreamed) return launch_one<FMT, 4, 4, 4, EPI, LAYOUT, KsplitWeights::kStreamed>(p, max_m_tiles, s);
         return launch_one<FMT, 4, 4, 4, EPI, LAYOUT, KsplitWeights::kByGroup>(p, max_m_tiles, s);
     }

@@ -141,3 +141,36 @@ def test_chosen_grouped_kernels(experts, avg, n, k):
     hooks_lib().cmx_debug_force_tile(256, 256, 8)
     for got, ref in zip(chosen, outputs()):
         assert torch.equal(got, ref)
+
+
+@pytest.mark.parametrize("kernel", ["ring", "split-K", "INT8"])
+@pytest.mark.parametrize("sizes,rows", [([5, -3, 0, 70, 1], 76), ([40, 2 ** 31 - 1, 2 ** 31 - 1, 9], 300), ([0, 0, 0], 10), ([1] * 256, 256),
+                                        ([3, 0, 66, 1] * 64, 4300), ([2 ** 31 - 1] * 256, 130)])
+def test_tiles_located_by_sizes_are_those_of_the_tables(kernel, sizes, rows):
+    """Up to 256 groups a launch reads the sizes themselves, more go through tables: empty groups behind the last one change
+    nothing.  Negative sizes count as zero, rows past the operand are cut off."""
+    from catccos_amd import ops
+    rng = np.random.default_rng(rows)
+    n, k, many = 64, 512, 300
+    aq, asc, bq, bsc = _operands(rng, rows, 4 * n, k, "E4M3")
+    a, a_s, w, w_s = dev(aq), dev(asc), dev(np.resize(bq, (many, n, k))), dev(np.resize(bsc, (many, n, k // 32)))
+    h = hooks_lib()
+    if kernel == "ring":
+        h.cmx_debug_force_tile(128, 128, 6)
+    else:
+        h.cmx_debug_force_ksplit(4, 4, 4)
+
+    def outputs(counts):
+        e = len(counts)
+        cnt = dev(np.array(counts, dtype=np.int32))
+        c = torch.full((rows, n), 7.0, dtype=torch.bfloat16, device="cuda")
+        if kernel == "INT8":
+            out = torch.zeros((rows, n // 2), device="cuda")
+            return ops.int8_gmm_dequant_swiglu(a.view(torch.int8), torch.ones(rows, device="cuda"), w[:e].view(torch.int8), torch.full((e * n,), 1e-5, device="cuda"),
+                                               cnt, n, k, 1, c=out)
+        return ops.mx_gmm(a, a_s, w[:e], w_s[:e], cnt, k, c=c)
+    got, want = outputs(sizes), outputs(sizes + [0] * (many - len(sizes)))
+    assert torch.equal(got, want)
+    if kernel == "ring":
+        done = min(sum(max(s, 0) for s in sizes), rows)
+        assert bool((got[done:].float() == 7.0).all()) and not bool((got[:done].float() == 7.0).all(dim=1).any())
