@@ -1379,13 +1379,17 @@ uint32_t max_group_tiles(uint32_t m_total, uint32_t groups, uint32_t tile_m, uin
 //   128 x 256    8 x 200 u, 4096, 2048                       45.9 -> 34.5 / 43.1 -> 35.7    16 x 300 u, 7168, 1024   74 -> 57 / 69 -> 62
 //                8 x 500 u, 1024, 1024                       22.6 -> 18.6 / 20.0 against 19.9, so not for a store at K below 2048
 // Problems of more tiles stay on the persistent kernels (32 x 194 rows, 7168, 4096: 287 against 311 with 128 x 256).
+// INT8, whose only other kernel has 256 x 256 tiles, one per workgroup (us, fp32 output):
+//   128 x 128    8 x 44 u, 4096, 2048 46.5 -> 21.6     8 x 200 u 47.7 -> 27.0     16 x 100 z, 7168, 1024 73.2 -> 34.8     16 x 44 u, 2048, 2048 29.7 -> 16.9
+//   256 x 128    32 x 44 u, 7168, 4096 222 -> 178       32 x 100 z 299 -> 232      32 x 100 z, 1152, 2048 46.3 -> 37.3
+//   128 x 256    16 x 200 u, 7168, 1024 71.8 -> 50.9; of more than a round 32 x 200 u, 7168, 4096 278 against 251, 16 x 2048 1077 against 1003
 int ring_groups(TileChoice* t, uint32_t m_total, uint32_t groups, uint32_t n, int fmt, uint32_t kblocks, bool swiglu) {
-    if (fmt == CMX_FMT_E2M1 || kblocks % 4 != 0 || kblocks < 16) return CMX_OK;
+    if (fmt == CMX_FMT_E2M1 || kblocks % 4 != 0 || (fmt != kFmtI8 && kblocks < 16)) return CMX_OK;
     int cus = 0;
     if (int rc = cu_count(&cus); rc != CMX_OK) return rc;
     const uint64_t w128 = ceil_div(n, 128);
     if (w128 * (m_total / 128 + groups) <= (uint64_t)cus) *t = {128, 128, kRing};
-    else if (t->tm == 128 && (!swiglu || kblocks >= 96)) *t = {256, 128, kRing};
+    else if (t->tm == 128 && (!swiglu || kblocks >= 96 || fmt == kFmtI8)) *t = {256, 128, kRing};
     else if (t->tm == 256 && w128 * (m_total / 256 + groups * 3 / 4) <= (uint64_t)cus && (swiglu || kblocks >= 64)) *t = {128, 256, kRing};
     return CMX_OK;
 }
@@ -1548,22 +1552,28 @@ extern "C" int cmx_int8_gmm_dequant_swiglu(const int8_t* a, uint32_t lda, const 
     p.lda = lda; p.ld_as = 0; p.ldw = k; p.ld_ws = channel_scale_stride; p.ldc = ld_out;
     p.m = m_total; p.n = n; p.kbytes = k; p.kblocks = k / 32; p.out_type = out_type;
     p.scale_vec = 1;
-    constexpr int kTile = 256;
     GroupedKsplit ks;
     if (int rc = choose_grouped_ksplit(m_total, groups, n, kFmtI8, p.kblocks, &ks); rc != CMX_OK) return rc;
     const bool all_ksplit = ks.tile.fw != 0 && ks.small_rows == 0;
+    TileChoice t = {256, ceil_div(m_total, groups) <= 128 ? 128 : 256, 8};
+    if (g_force_tile.waves == kRing) t = g_force_tile;
+    else if (!g_force_tile.tw && !g_disable_dl)
+        if (int rc = ring_groups(&t, m_total, groups, n, kFmtI8, p.kblocks, true); rc != CMX_OK) return rc;
+    if (t.waves != kRing) t.tm = 256;
     const GroupTables tables(ws, groups);
-    const uint32_t tile_m = all_ksplit ? 16 * ks.tile.fm : kTile;
+    const uint32_t tile_m = all_ksplit ? 16 * ks.tile.fm : t.tm;
     bool by_sizes = false;                                     // (all its kernels take one tile per workgroup)
-    if (int rc = tiles_by_sizes(&by_sizes, groups, (uint64_t)(m_total / tile_m + groups) * ceil_div(n, all_ksplit ? 64 : kTile), all_ksplit ? 2 : 1); rc != CMX_OK) return rc;
+    if (int rc = tiles_by_sizes(&by_sizes, groups, (uint64_t)(m_total / tile_m + groups) * ceil_div(n, all_ksplit ? 64 : t.tw), all_ksplit ? 2 : 1); rc != CMX_OK) return rc;
     if (int rc = prepare_groups(p, tables_job(tables, group_sizes, groups, m_total, tile_m, ks.small_rows), by_sizes, false, s); rc != CMX_OK) return rc;
     if (ks.tile.fw != 0)
         if (int rc = launch_grouped_ksplit(p, tables, ks, kFmtI8, kEpiI8DequantSwiglu, m_total, s); rc != CMX_OK || all_ksplit) return rc;
-    p.w_tiles = ceil_div(n / 2, kTile / 2);
+    p.w_tiles = ceil_div(n / 2, t.tw / 2);
+    const uint32_t max_m_tiles = max_group_tiles(m_total, groups, t.tm, ks.small_rows);
+    if (t.waves == kRing) return launch_ring(p, {t.tw, t.tm}, kFmtI8, kEpiI8DequantSwiglu, false, max_m_tiles, s);
     // (hand-scheduled variants of this kernel were measured twice at 16 x 2048 x 7168 x 4096 and are not kept: two i8
     // MFMAs per step and accumulator in the 8-bit schedule 997 us, one per 32-K step in the 16-byte-fragment
     // schedule shared with FP4, one tile per workgroup, 994-1000 us, against 967-975 us for this one)
-    return launch_gemm_dl<kFmtI8, kTile, kTile, 2, 4, kEpiI8DequantSwiglu>(p, max_group_tiles(m_total, groups, kTile, ks.small_rows), s);
+    return launch_gemm_dl<kFmtI8, 256, 256, 2, 4, kEpiI8DequantSwiglu>(p, max_m_tiles, s);
 }
 
 namespace cmx {

@@ -1,4 +1,5 @@
-// Block-scaled matmul for dense problems of one round of tiles: 128 weight rows x TM activation rows per workgroup of four wavefronts.
+// Block-scaled and INT8 matmul for problems of few or one round of tiles: TW weight rows x TM activation rows (128 x 128 to 256 x 128) per
+// workgroup of four wavefronts.
 //
 // What bounds it: a CU moves some 87 bytes per nanosecond from the L2 into its LDS (1.3-1.5 ns for a 128-byte line), whatever
 // waits for them, so a tile costs what its rows cost: 64 x 64 tiles of the split-K kernel pull a byte of operands for 64 flop,
@@ -29,6 +30,7 @@ namespace cmx {
 namespace {
 
 // SPAN: slabs whose scales one half of the scale area holds
+// (0: no scales, the INT8 kernels)
 constexpr int ring_scale_bytes(int tw, int tm, int span) { return 2 * (tw + tm) * 4 * span; }
 constexpr int ring_sum_bytes(int tw, int tm) { return tm * (tw + 4) * 4; }
 constexpr size_t ring_lds_bytes(int tw, int tm, int nslot, int span) {
@@ -55,6 +57,13 @@ __device__ __forceinline__ void ring_wait_barrier() {
 
 template <int FMT, int SEL>
 __device__ __forceinline__ v16f ring_mfma(const v8i& w, const v8i& a, const v16f& c, uint32_t sw, uint32_t sa) {
+    if constexpr (FMT == kFmtI8) {                                       // one 64-deep step on the halves of the same registers
+        typedef int v16i __attribute__((ext_vector_type(16)));
+        v16i acc = __builtin_bit_cast(v16i, c);
+        acc = __builtin_amdgcn_mfma_i32_32x32x32_i8((v4i){w[0], w[1], w[2], w[3]}, (v4i){a[0], a[1], a[2], a[3]}, acc, 0, 0, 0);
+        acc = __builtin_amdgcn_mfma_i32_32x32x32_i8((v4i){w[4], w[5], w[6], w[7]}, (v4i){a[4], a[5], a[6], a[7]}, acc, 0, 0, 0);
+        return __builtin_bit_cast(v16f, acc);
+    }
     constexpr int kF = FMT == CMX_FMT_E5M2 ? 1 : 0;
     return __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(w, a, c, kF, kF, SEL, (int)sw, SEL, (int)sa);
 }
@@ -65,6 +74,7 @@ __global__ __launch_bounds__(64 * WW * WM) void mx_gemm_ring_kernel(const GemmPa
     constexpr int kRows = TW + TM, kSlotBytes = kRows * kSlabBytes;
     constexpr int kTileLoads = kRows / (8 * NW), kWTileLoads = TW / (8 * NW);
     constexpr int kScaleBase = NSLOT * kSlotBytes, kScaleHalf = kRows * 4 * SPAN;
+    constexpr bool kScales = FMT != kFmtI8;
     constexpr int kPieces = SPAN / 4, kAllPieces = kRows * kPieces;     // 16-byte pieces of a row in a half; of all rows
     constexpr int kScaleLoads = (kAllPieces + NT - 1) / NT;
     constexpr int kEarly = kTileLoads / 2;                              // loads of a slab in the second step of the slab before, the rest in the first
@@ -72,7 +82,8 @@ __global__ __launch_bounds__(64 * WW * WM) void mx_gemm_ring_kernel(const GemmPa
     static_assert(TW % (8 * NW) == 0 && TM % (8 * NW) == 0 && TW % 64 == 0 && TM % 64 == 0 && FW >= 1 && FM >= 1, "tile shape");
     static_assert(!KSLOW || TW % 128 == 0, "whole 128-byte lines along n");
     static_assert(!epi_pairs_gate_up(EPI) || (!KSLOW && TW % 64 == 0), "gate and up rows");
-    static_assert((NSLOT - 1) * kTileLoads < 64 && TW * kPieces % 64 == 0 && TM * kPieces % 64 == 0 && (SPAN & (SPAN - 1)) == 0 && SPAN >= 4 && SPAN <= 32, "loads");
+    static_assert((NSLOT - 1) * kTileLoads < 64, "loads");
+    static_assert(kScales ? TW * kPieces % 64 == 0 && TM * kPieces % 64 == 0 && (SPAN & (SPAN - 1)) == 0 && SPAN >= 4 && SPAN <= 32 : SPAN == 0 && !KSLOW, "scales");
 
     extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
     const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) uint8_t*)smem;
@@ -111,6 +122,7 @@ __global__ __launch_bounds__(64 * WW * WM) void mx_gemm_ring_kernel(const GemmPa
     // every slab counts the same loads and the loop has no branch
     auto live_rsrc = [](const v4i& r, bool live) -> v4i { return (v4i){r[0], r[1], (int)uniform(live ? ~0u : 0u), r[3]}; };
     const v4i w_rs = make_rsrc(KSLOW ? p.w : p.w + (size_t)tc.g * p.n * p.ldw);
+    // (INT8: the scales are the epilogue's)
     const uint8_t* const w_scales = KSLOW ? p.w_scale : p.w_scale + (size_t)tc.g * p.n * p.ld_ws;
     const uint8_t* const a_scales = p.a_scale + (size_t)tc.row0 * p.ld_as;
     const v4i ws_rs = make_rsrc(w_scales);
@@ -143,34 +155,36 @@ __global__ __launch_bounds__(64 * WW * WM) void mx_gemm_ring_kernel(const GemmPa
     const bool whole_pieces = p.scale_vec && ndw >= 4;
     const uint32_t last_dw = whole_pieces ? ndw - 4 : ndw - 1;
     auto load_scales = [&](uint32_t b) {
-        const uint32_t half_at = kScaleBase + (b & 1u) * kScaleHalf;
-        auto address = [&](uint32_t piece, uint32_t d, bool of_w) -> uint32_t {
-            const uint32_t row = piece / kPieces;
-            if (KSLOW && of_w) {
-                const uint32_t k64 = 2 * SPAN * b + piece / (TW / 8), col = piece % (TW / 8) * 8 + 2 * d;
-                return (k64 < 2 * nslab ? k64 : 2 * nslab - 1) * p.ld_ws + 2 * (wcol_of(col / 16) + col % 16);
-            }
-            const uint32_t dw = SPAN * b + 4 * ((piece ^ (row / (64 / SPAN))) & (kPieces - 1)) + d;
-            const uint32_t at = 4 * (dw < last_dw ? dw : last_dw);               // past K: never used
-            return of_w ? wrow_of(row) * p.ld_ws + at : arow_of(row - TW) * p.ld_as + at;
-        };
-        constexpr uint32_t kWPieces = TW * kPieces;                              // the weights' come first; a load has one kind
-        if (whole_pieces) {
+        if constexpr (kScales) {
+            const uint32_t half_at = kScaleBase + (b & 1u) * kScaleHalf;
+            auto address = [&](uint32_t piece, uint32_t d, bool of_w) -> uint32_t {
+                const uint32_t row = piece / kPieces;
+                if (KSLOW && of_w) {
+                    const uint32_t k64 = 2 * SPAN * b + piece / (TW / 8), col = piece % (TW / 8) * 8 + 2 * d;
+                    return (k64 < 2 * nslab ? k64 : 2 * nslab - 1) * p.ld_ws + 2 * (wcol_of(col / 16) + col % 16);
+                }
+                const uint32_t dw = SPAN * b + 4 * ((piece ^ (row / (64 / SPAN))) & (kPieces - 1)) + d;
+                const uint32_t at = 4 * (dw < last_dw ? dw : last_dw);               // past K: never used
+                return of_w ? wrow_of(row) * p.ld_ws + at : arow_of(row - TW) * p.ld_as + at;
+            };
+            constexpr uint32_t kWPieces = TW * kPieces;                              // the weights' come first; a load has one kind
+            if (whole_pieces) {
 #pragma unroll
-            for (int i = 0; i < kScaleLoads; ++i) {
-                const uint32_t p0 = min((uint32_t)(NW * i + wave) * 64, (uint32_t)kAllPieces - 64);          // (a duplicate at most)
-                const bool of_w = p0 < kWPieces;
-                ring_dma16(lds0 + half_at + p0 * 16, address(p0 + lane, 0, of_w), of_w ? ws_rs : as_rs, 0);
-            }
-        } else {
-            // rows at any byte, or of less than a piece: through registers (the waits for them drain the ring, once in SPAN slabs)
+                for (int i = 0; i < kScaleLoads; ++i) {
+                    const uint32_t p0 = min((uint32_t)(NW * i + wave) * 64, (uint32_t)kAllPieces - 64);          // (a duplicate at most)
+                    const bool of_w = p0 < kWPieces;
+                    ring_dma16(lds0 + half_at + p0 * 16, address(p0 + lane, 0, of_w), of_w ? ws_rs : as_rs, 0);
+                }
+            } else {
+                // rows at any byte, or of less than a piece: through registers (the waits for them drain the ring, once in SPAN slabs)
 #pragma unroll 2
-            for (int i = 0; i < 4 * kScaleLoads; ++i) {
-                const uint32_t p0 = min((uint32_t)(NW * i + wave) * 16, (uint32_t)kAllPieces - 16);
-                const bool of_w = p0 < kWPieces;
-                uint32_t v;
-                __builtin_memcpy(&v, (of_w ? w_scales : a_scales) + address(p0 + lane / 4, lane & 3u, of_w), 4);
-                *reinterpret_cast<uint32_t*>(smem + half_at + p0 * 16 + lane * 4) = v;
+                for (int i = 0; i < 4 * kScaleLoads; ++i) {
+                    const uint32_t p0 = min((uint32_t)(NW * i + wave) * 16, (uint32_t)kAllPieces - 16);
+                    const bool of_w = p0 < kWPieces;
+                    uint32_t v;
+                    __builtin_memcpy(&v, (of_w ? w_scales : a_scales) + address(p0 + lane / 4, lane & 3u, of_w), 4);
+                    *reinterpret_cast<uint32_t*>(smem + half_at + p0 * 16 + lane * 4) = v;
+                }
             }
         }
     };
@@ -211,7 +225,7 @@ __global__ __launch_bounds__(64 * WW * WM) void mx_gemm_ring_kernel(const GemmPa
 #pragma unroll
             for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.0f;
     v8i wf[2][FW], af[2][FM];
-    uint32_t sw[FW], sa[FM], swn[FW], san[FM];
+    uint32_t sw[FW] = {}, sa[FM] = {}, swn[FW] = {}, san[FM] = {};
 
     const uint32_t a_row = wm * (TM / WM) + l32;                         // activation row of fragment 0
     // fragment `pos` in the order of first use by the MFMAs (weights outside, activations inside): W0 A0 A1 .. W1 W2 ..
@@ -223,8 +237,9 @@ __global__ __launch_bounds__(64 * WW * WM) void mx_gemm_ring_kernel(const GemmPa
         else wf[buf][f] = KSLOW ? read_frag_t(lds0 + slot * kSlotBytes, wfrag_row(f), h) : read_frag(st, wfrag_row(f) + l32, h);
     };
     // scale dword of slab s of fragment `pos` (0 .. FW - 1 weights, then activations), the lane's byte of step h at bits 16 h
-    const uint32_t sc_x = l32 / (64 / SPAN) & (kPieces - 1);
     auto read_scale = [&](uint32_t s, int pos) {
+        if constexpr (kScales) {
+        const uint32_t sc_x = l32 / (64 / SPAN) & (kPieces - 1);
         const uint8_t* at = smem + kScaleBase + (s / SPAN & 1u) * kScaleHalf;
         const uint32_t in_piece = whole_pieces && s >= (ndw & ~3u) ? s - last_dw : s % 4;
         const uint32_t in_row = ((s % SPAN / 4) ^ sc_x) * 16 + in_piece * 4;
@@ -235,6 +250,7 @@ __global__ __launch_bounds__(64 * WW * WM) void mx_gemm_ring_kernel(const GemmPa
             swn[pos] = q[0] | ((uint32_t)q[2 * TW] << 16);
         } else {
             swn[pos] = *reinterpret_cast<const uint32_t*>(at + in_row + (wfrag_row(pos) + l32) * (4 * SPAN));
+        }
         }
     };
     auto take_scales = [&]() {
@@ -288,7 +304,8 @@ __global__ __launch_bounds__(64 * WW * WM) void mx_gemm_ring_kernel(const GemmPa
         __builtin_amdgcn_sched_barrier(0);
         // block 1 of the scales behind the first slab; block b + 2 behind the last slab of block b, whose scales were read a slab
         // ago by all
-        if ((s == 0 && nslab > SPAN) || (s % SPAN == SPAN - 1 && s + SPAN + 1 < nslab)) load_scales(s == 0 ? 1 : s / SPAN + 2);
+        if constexpr (kScales)
+            if ((s == 0 && nslab > SPAN) || (s % SPAN == SPAN - 1 && s + SPAN + 1 < nslab)) load_scales(s == 0 ? 1 : s / SPAN + 2);
         const uint32_t next = slot + 1 < NSLOT ? slot + 1 : 0;
         step(c1{}, [&](int it) {
             if (it < kFrags) { read_one(next, 0, 0, it); read_scale(s + 1, it); }
@@ -368,6 +385,11 @@ int launch_ring(const GemmParams& p, const RingTile& t, int fmt, int epi, bool k
         return k_slow ? launch_shape<CMX_FMT_E5M2, kEpiStore, true>(p, t, max_m_tiles, s) : launch_shape<CMX_FMT_E5M2, kEpiStore, false>(p, t, max_m_tiles, s);
     if (fmt == CMX_FMT_E4M3 && epi == kEpiSwigluQuant && !k_slow) return launch_shape<CMX_FMT_E4M3, kEpiSwigluQuant, false>(p, t, max_m_tiles, s);
     if (fmt == CMX_FMT_E4M3 && epi == kEpiSwigluQuantAct && !k_slow) return launch_shape<CMX_FMT_E4M3, kEpiSwigluQuantAct, false>(p, t, max_m_tiles, s);
+    if (fmt == kFmtI8 && epi == kEpiI8DequantSwiglu && !k_slow) {
+        if (t.tw == 128 && t.tm == 128) return launch_one<kFmtI8, 128, 128, 2, 2, 4, 0, kEpiI8DequantSwiglu, false>(p, max_m_tiles, s);
+        if (t.tw == 128 && t.tm == 256) return launch_one<kFmtI8, 128, 256, 2, 2, 3, 0, kEpiI8DequantSwiglu, false>(p, max_m_tiles, s);
+        if (t.tw == 256 && t.tm == 128) return launch_one<kFmtI8, 256, 128, 2, 2, 3, 0, kEpiI8DequantSwiglu, false>(p, max_m_tiles, s);
+    }
     set_error("unsupported ring problem");
     return CMX_EINVAL;
 }

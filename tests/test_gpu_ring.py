@@ -143,6 +143,26 @@ def test_chosen_grouped_kernels(experts, avg, n, k):
         assert torch.equal(got, ref)
 
 
+@pytest.mark.parametrize("tile", [(128, 128), (128, 256), (256, 128)])
+@pytest.mark.parametrize("out", ["fp32", "bf16"])
+@pytest.mark.parametrize("counts,n,k", [([1, 0, 127, 128, 129, 0, 257, 66], 320, 512), ([300, 2], 192, 128), ([0, 5, 0], 64, 1152)])
+def test_grouped_int8_gives_the_bits_of_the_256_row_kernel(tile, out, counts, n, k):
+    """Whole-number sums and the same arithmetic behind them; fewer slabs than ring slots."""
+    from catccos_amd import ops
+    g = torch.Generator(device="cuda")
+    g.manual_seed(n + k)
+    m, e = sum(counts), len(counts)
+    a = torch.randint(-127, 128, (m, k), dtype=torch.int8, device="cuda", generator=g)
+    w = torch.randint(-127, 128, (e, n, k), dtype=torch.int8, device="cuda", generator=g)
+    channel, token = torch.rand(e * n, device="cuda", generator=g) * 1e-4, torch.rand(m, device="cuda", generator=g)
+    args = (a, token, w, channel, dev(np.array(counts, dtype=np.int32)), n, k, 1, out)
+    h = hooks_lib()
+    h.cmx_debug_force_tile(256, 256, 8)
+    want = ops.int8_gmm_dequant_swiglu(*args)
+    h.cmx_debug_force_tile(*tile, 6)
+    assert torch.equal(ops.int8_gmm_dequant_swiglu(*args), want)
+
+
 @pytest.mark.parametrize("kernel", ["ring", "split-K", "INT8"])
 @pytest.mark.parametrize("sizes,rows", [([5, -3, 0, 70, 1], 76), ([40, 2 ** 31 - 1, 2 ** 31 - 1, 9], 300), ([0, 0, 0], 10), ([1] * 256, 256),
                                         ([3, 0, 66, 1] * 64, 4300), ([2 ** 31 - 1] * 256, 130)])
