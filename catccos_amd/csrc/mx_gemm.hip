@@ -1366,8 +1366,8 @@ uint32_t max_group_tiles(uint32_t m_total, uint32_t groups, uint32_t tile_m, uin
     return m_total / tile_m + (n < groups ? n : groups);
 }
 
-// Grouped 8-bit problems on row-major weights that the ring kernel takes from the 256-row kernels of choose_tile (same sums, so the line
-// is a matter of time).  128 x 128 where its tiles are one round of a workgroup per CU whatever the rows' distribution (a second round costs as
+// Grouped problems on row-major weights that the ring kernel takes from the 256-row kernels of choose_tile (same sums, so the line is a
+// matter of time).  128 x 128 where its tiles are one round of a workgroup per CU whatever the rows' distribution (a second round costs as
 // much as the first: 16 experts x 64 rows, Zipf, K = 2048, N = 2048, 320 tiles, 30 against 23); else 256 x 128 in the place of the three-slot
 // kernel of short groups, which pulls a dword of scales per row and slab; else 128 x 256 in one round.
 // Measured (us, before -> ring; SwiGLU + requant / 16-bit store; u: routes drawn uniformly, z: Zipf):
@@ -1383,14 +1383,19 @@ uint32_t max_group_tiles(uint32_t m_total, uint32_t groups, uint32_t tile_m, uin
 //   128 x 128    8 x 44 u, 4096, 2048 46.5 -> 21.6     8 x 200 u 47.7 -> 27.0     16 x 100 z, 7168, 1024 73.2 -> 34.8     16 x 44 u, 2048, 2048 29.7 -> 16.9
 //   256 x 128    32 x 44 u, 7168, 4096 222 -> 178       32 x 100 z 299 -> 232      32 x 100 z, 1152, 2048 46.3 -> 37.3
 //   128 x 256    16 x 200 u, 7168, 1024 71.8 -> 50.9; of more than a round 32 x 200 u, 7168, 4096 278 against 251, 16 x 2048 1077 against 1003
+// FP4, whose other kernels past the split-K sizes have tiles of 256 x 128 and 256 x 256 (us, bf16 output):
+//   128 x 128    8 x 70 u, 4096, 2048 31.6 -> 15.9     8 x 200 u 36.0 -> 18.4     16 x 100 z, 7168, 1024 46.9 -> 24.1     8 x 70 u, 7168, 4096 49 -> 26
+//   256 x 128    32 x 70 u, 7168, 4096 144 -> 111       32 x 100 z 196 -> 141      32 x 100 z, 1280, 2048 29.9 -> 26.9
+//   128 x 256    8 x 200 u, 7168, 4096 56.7 -> 40.6; of more than a round 32 x 200 u, 7168, 4096 180 against 148
 int ring_groups(TileChoice* t, uint32_t m_total, uint32_t groups, uint32_t n, int fmt, uint32_t kblocks, bool swiglu) {
-    if (fmt == CMX_FMT_E2M1 || kblocks % 4 != 0 || (fmt != kFmtI8 && kblocks < 16)) return CMX_OK;
+    if (kblocks % (fmt == CMX_FMT_E2M1 ? 8 : 4) != 0 || (fmt != kFmtI8 && kblocks < 16)) return CMX_OK;
+    const bool eight_bit = fmt == CMX_FMT_E4M3 || fmt == CMX_FMT_E5M2;
     int cus = 0;
     if (int rc = cu_count(&cus); rc != CMX_OK) return rc;
     const uint64_t w128 = ceil_div(n, 128);
     if (w128 * (m_total / 128 + groups) <= (uint64_t)cus) *t = {128, 128, kRing};
-    else if (t->tm == 128 && (!swiglu || kblocks >= 96 || fmt == kFmtI8)) *t = {256, 128, kRing};
-    else if (t->tm == 256 && w128 * (m_total / 256 + groups * 3 / 4) <= (uint64_t)cus && (swiglu || kblocks >= 64)) *t = {128, 256, kRing};
+    else if (t->tm <= 128 && (!swiglu || kblocks >= 96 || !eight_bit)) *t = {256, 128, kRing};
+    else if (t->tm == 256 && w128 * (m_total / 256 + groups * 3 / 4) <= (uint64_t)cus && (swiglu || kblocks >= 64 || !eight_bit)) *t = {128, 256, kRing};
     return CMX_OK;
 }
 

@@ -1,4 +1,4 @@
-// Block-scaled and INT8 matmul for problems of few or one round of tiles: TW weight rows x TM activation rows (128 x 128 to 256 x 128) per
+// Block-scaled and INT8 matmul for problems of one round of tiles and for short groups: TW weight rows x TM activation rows (128 x 128 to 256 x 128) per
 // workgroup of four wavefronts.
 //
 // What bounds it: a CU moves some 87 bytes per nanosecond from the L2 into its LDS (1.3-1.5 ns for a 128-byte line), whatever
@@ -29,7 +29,7 @@ namespace cmx {
 
 namespace {
 
-// SPAN: slabs whose scales one half of the scale area holds
+// SPAN: scale dwords of a row that one half of the scale area holds
 // (0: no scales, the INT8 kernels)
 constexpr int ring_scale_bytes(int tw, int tm, int span) { return 2 * (tw + tm) * 4 * span; }
 constexpr int ring_sum_bytes(int tw, int tm) { return tm * (tw + 4) * 4; }
@@ -55,17 +55,23 @@ __device__ __forceinline__ void ring_wait_barrier() {
     asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(N) : "memory");
 }
 
-template <int FMT, int SEL>
-__device__ __forceinline__ v16f ring_mfma(const v8i& w, const v8i& a, const v16f& c, uint32_t sw, uint32_t sa) {
-    if constexpr (FMT == kFmtI8) {                                       // one 64-deep step on the halves of the same registers
+// MFMA j of a 64-byte step h: 8-bit formats one of 64 deep; FP4 two of 64 deep on the halves of the fragment registers, each with two scale
+// bytes of dword h; INT8 two of 32 deep (a sum of whole numbers does not care which lane holds which K position)
+constexpr int ring_subs(int fmt) { return fmt == CMX_FMT_E2M1 || fmt == kFmtI8 ? 2 : 1; }
+constexpr int ring_scale_dwords(int fmt) { return fmt == CMX_FMT_E2M1 ? 2 : 1; }             // per row and slab
+template <int FMT, int H, int J, int SD>
+__device__ __forceinline__ v16f ring_mfma(const v8i& w, const v8i& a, const v16f& c, const uint32_t (&sw)[SD], const uint32_t (&sa)[SD]) {
+    const v4i w4 = {w[4 * J], w[4 * J + 1], w[4 * J + 2], w[4 * J + 3]}, a4 = {a[4 * J], a[4 * J + 1], a[4 * J + 2], a[4 * J + 3]};
+    if constexpr (FMT == kFmtI8) {
         typedef int v16i __attribute__((ext_vector_type(16)));
-        v16i acc = __builtin_bit_cast(v16i, c);
-        acc = __builtin_amdgcn_mfma_i32_32x32x32_i8((v4i){w[0], w[1], w[2], w[3]}, (v4i){a[0], a[1], a[2], a[3]}, acc, 0, 0, 0);
-        acc = __builtin_amdgcn_mfma_i32_32x32x32_i8((v4i){w[4], w[5], w[6], w[7]}, (v4i){a[4], a[5], a[6], a[7]}, acc, 0, 0, 0);
-        return __builtin_bit_cast(v16f, acc);
+        return __builtin_bit_cast(v16f, __builtin_amdgcn_mfma_i32_32x32x32_i8(w4, a4, __builtin_bit_cast(v16i, c), 0, 0, 0));
+    } else if constexpr (FMT == CMX_FMT_E2M1) {
+        const v8i w8 = {w4[0], w4[1], w4[2], w4[3], 0, 0, 0, 0}, a8 = {a4[0], a4[1], a4[2], a4[3], 0, 0, 0, 0};
+        return __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(w8, a8, c, 4, 4, 2 * J, (int)sw[H], 2 * J, (int)sa[H]);
+    } else {
+        constexpr int kF = FMT == CMX_FMT_E5M2 ? 1 : 0;
+        return __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(w, a, c, kF, kF, 2 * H, (int)sw[0], 2 * H, (int)sa[0]);
     }
-    constexpr int kF = FMT == CMX_FMT_E5M2 ? 1 : 0;
-    return __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(w, a, c, kF, kF, SEL, (int)sw, SEL, (int)sa);
 }
 
 template <int FMT, int TW, int TM, int WW, int WM, int NSLOT, int SPAN, int EPI, bool KSLOW>
@@ -75,15 +81,16 @@ __global__ __launch_bounds__(64 * WW * WM) void mx_gemm_ring_kernel(const GemmPa
     constexpr int kTileLoads = kRows / (8 * NW), kWTileLoads = TW / (8 * NW);
     constexpr int kScaleBase = NSLOT * kSlotBytes, kScaleHalf = kRows * 4 * SPAN;
     constexpr bool kScales = FMT != kFmtI8;
+    constexpr int kSD = ring_scale_dwords(FMT), kSpanSlabs = kScales ? SPAN / kSD : 1;
     constexpr int kPieces = SPAN / 4, kAllPieces = kRows * kPieces;     // 16-byte pieces of a row in a half; of all rows
     constexpr int kScaleLoads = (kAllPieces + NT - 1) / NT;
     constexpr int kEarly = kTileLoads / 2;                              // loads of a slab in the second step of the slab before, the rest in the first
-    constexpr int kM = FW * FM, kFrags = FW + FM;                       // MFMAs and fragments per step
+    constexpr int kM = FW * FM, kSteps = kM * ring_subs(FMT), kFrags = FW + FM;                       // MFMAs and fragments per step
     static_assert(TW % (8 * NW) == 0 && TM % (8 * NW) == 0 && TW % 64 == 0 && TM % 64 == 0 && FW >= 1 && FM >= 1, "tile shape");
     static_assert(!KSLOW || TW % 128 == 0, "whole 128-byte lines along n");
     static_assert(!epi_pairs_gate_up(EPI) || (!KSLOW && TW % 64 == 0), "gate and up rows");
     static_assert((NSLOT - 1) * kTileLoads < 64, "loads");
-    static_assert(kScales ? TW * kPieces % 64 == 0 && TM * kPieces % 64 == 0 && (SPAN & (SPAN - 1)) == 0 && SPAN >= 4 && SPAN <= 32 : SPAN == 0 && !KSLOW, "scales");
+    static_assert(kScales ? TW * kPieces % 64 == 0 && TM * kPieces % 64 == 0 && (SPAN & (SPAN - 1)) == 0 && SPAN >= 4 && SPAN <= 32 && kSpanSlabs >= 2 && (!KSLOW || kSD == 1) : SPAN == 0 && !KSLOW, "scales");
 
     extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
     const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) uint8_t*)smem;
@@ -149,7 +156,7 @@ __global__ __launch_bounds__(64 * WW * WM) void mx_gemm_ring_kernel(const GemmPa
         if (i < kWTileLoads) ring_dma16(dst, goff[i], live_rsrc(w_rs, live), s * w_step);
         else ring_dma16(dst, goff[i], live_rsrc(a_rs, live), s * kSlabBytes);
     };
-    // Scales of block b (slabs SPAN b .. SPAN b + SPAN - 1) into half b % 2 of the scale area, in pieces of four dwords.
+    // Scales of block b (dwords SPAN b .. SPAN b + SPAN - 1 of a row, one a slab, FP4 two) into half b % 2 of the scale area, in pieces of four dwords.
     // K-contiguous rows: the pieces of a row change places by XOR so that the 32 rows of a fragment lie in different banks two by
     // two; a last piece in part is fetched from the row's last 16 bytes.  K-slow weights: [K / 64 within the block][column] pairs.
     const bool whole_pieces = p.scale_vec && ndw >= 4;
@@ -225,7 +232,7 @@ __global__ __launch_bounds__(64 * WW * WM) void mx_gemm_ring_kernel(const GemmPa
 #pragma unroll
             for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.0f;
     v8i wf[2][FW], af[2][FM];
-    uint32_t sw[FW] = {}, sa[FM] = {}, swn[FW] = {}, san[FM] = {};
+    uint32_t sw[FW][kSD] = {}, sa[FM][kSD] = {}, swn[FW][kSD] = {}, san[FM][kSD] = {};
 
     const uint32_t a_row = wm * (TM / WM) + l32;                         // activation row of fragment 0
     // fragment `pos` in the order of first use by the MFMAs (weights outside, activations inside): W0 A0 A1 .. W1 W2 ..
@@ -236,28 +243,36 @@ __global__ __launch_bounds__(64 * WW * WM) void mx_gemm_ring_kernel(const GemmPa
         if (!is_w) af[buf][f] = read_frag(st + TW * kSlabBytes, a_row + f * 32, h);
         else wf[buf][f] = KSLOW ? read_frag_t(lds0 + slot * kSlotBytes, wfrag_row(f), h) : read_frag(st, wfrag_row(f) + l32, h);
     };
-    // scale dword of slab s of fragment `pos` (0 .. FW - 1 weights, then activations), the lane's byte of step h at bits 16 h
+    // scale dwords of slab s of fragment `pos` (0 .. FW - 1 weights, then activations), the lane's byte of MFMA j (FP4) or step h at bits 16
+    const uint32_t sc_x = l32 * SPAN / 64 & (kPieces - 1);
     auto read_scale = [&](uint32_t s, int pos) {
         if constexpr (kScales) {
-        const uint32_t sc_x = l32 / (64 / SPAN) & (kPieces - 1);
-        const uint8_t* at = smem + kScaleBase + (s / SPAN & 1u) * kScaleHalf;
-        const uint32_t in_piece = whole_pieces && s >= (ndw & ~3u) ? s - last_dw : s % 4;
-        const uint32_t in_row = ((s % SPAN / 4) ^ sc_x) * 16 + in_piece * 4;
-        if (pos >= FW) {
-            san[pos - FW] = *reinterpret_cast<const uint32_t*>(at + TW * 4 * SPAN + in_row + (a_row + (pos - FW) * 32) * (4 * SPAN));
-        } else if (KSLOW) {
-            const uint8_t* q = at + s % SPAN * (4 * TW) + (wfrag_row(pos) + l32) * 2 + lh;
-            swn[pos] = q[0] | ((uint32_t)q[2 * TW] << 16);
-        } else {
-            swn[pos] = *reinterpret_cast<const uint32_t*>(at + in_row + (wfrag_row(pos) + l32) * (4 * SPAN));
-        }
+            const uint32_t d = kSD * s;
+            const uint8_t* at = smem + kScaleBase + (s / kSpanSlabs & 1u) * kScaleHalf;
+            const uint32_t in_piece = whole_pieces && d >= (ndw & ~3u) ? d - last_dw : d % 4;
+            const uint32_t in_row = ((d % SPAN / 4) ^ sc_x) * 16 + in_piece * 4;
+            if constexpr (KSLOW) {
+                if (pos < FW) {
+                    const uint8_t* q = at + s % SPAN * (4 * TW) + (wfrag_row(pos) + l32) * 2 + lh;
+                    swn[pos][0] = q[0] | ((uint32_t)q[2 * TW] << 16);
+                    return;
+                }
+            }
+#pragma unroll
+            for (int j = 0; j < kSD; ++j) {
+                if (pos >= FW) san[pos - FW][j] = *reinterpret_cast<const uint32_t*>(at + TW * 4 * SPAN + in_row + 4 * j + (a_row + (pos - FW) * 32) * (4 * SPAN));
+                else swn[pos][j] = *reinterpret_cast<const uint32_t*>(at + in_row + 4 * j + (wfrag_row(pos) + l32) * (4 * SPAN));
+            }
         }
     };
     auto take_scales = [&]() {
 #pragma unroll
-        for (int f = 0; f < FW; ++f) sw[f] = KSLOW ? swn[f] : swn[f] >> (8 * lh);
+        for (int j = 0; j < kSD; ++j) {
 #pragma unroll
-        for (int f = 0; f < FM; ++f) sa[f] = san[f] >> (8 * lh);
+            for (int f = 0; f < FW; ++f) sw[f][j] = KSLOW ? swn[f][j] : swn[f][j] >> (8 * lh);
+#pragma unroll
+            for (int f = 0; f < FM; ++f) sa[f][j] = san[f][j] >> (8 * lh);
+        }
     };
 
     // ---- K loop ----------------------------------------------------------------------------------------------------------
@@ -279,12 +294,13 @@ __global__ __launch_bounds__(64 * WW * WM) void mx_gemm_ring_kernel(const GemmPa
     auto step = [&](auto hc, auto&& items, auto n_items) {
         constexpr int h = decltype(hc)::value, n = decltype(n_items)::value;
 #pragma unroll
-        for (int x = 0; x < kM; ++x) {
-            const int i = x / FM, j = x % FM;
-            acc[i][j] = ring_mfma<FMT, 2 * h>(wf[h][i], af[h][j], acc[i][j], sw[i], sa[j]);
+        for (int x = 0; x < kSteps; ++x) {
+            const int i = x % kM / FM, j = x % FM;
+            if (x < kM) acc[i][j] = ring_mfma<FMT, h, 0>(wf[h][i], af[h][j], acc[i][j], sw[i], sa[j]);
+            else acc[i][j] = ring_mfma<FMT, h, 1>(wf[h][i], af[h][j], acc[i][j], sw[i], sa[j]);
             __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-            for (int it = x * n / kM; it < (x + 1) * n / kM; ++it) items(it);
+            for (int it = x * n / kSteps; it < (x + 1) * n / kSteps; ++it) items(it);
             __builtin_amdgcn_sched_barrier(0);
         }
         // (the sums are used here: otherwise the MFMAs sink below the barrier that follows)
@@ -305,7 +321,7 @@ __global__ __launch_bounds__(64 * WW * WM) void mx_gemm_ring_kernel(const GemmPa
         // block 1 of the scales behind the first slab; block b + 2 behind the last slab of block b, whose scales were read a slab
         // ago by all
         if constexpr (kScales)
-            if ((s == 0 && nslab > SPAN) || (s % SPAN == SPAN - 1 && s + SPAN + 1 < nslab)) load_scales(s == 0 ? 1 : s / SPAN + 2);
+            if ((s == 0 && nslab > kSpanSlabs) || (s % kSpanSlabs == kSpanSlabs - 1 && s + kSpanSlabs + 1 < nslab)) load_scales(s == 0 ? 1 : s / kSpanSlabs + 2);
         const uint32_t next = slot + 1 < NSLOT ? slot + 1 : 0;
         step(c1{}, [&](int it) {
             if (it < kFrags) { read_one(next, 0, 0, it); read_scale(s + 1, it); }
@@ -364,7 +380,7 @@ template <int FMT, int EPI, bool KSLOW>
 int launch_shape(const GemmParams& p, const RingTile& t, uint32_t max_m_tiles, hipStream_t s) {
     if (t.tw == 128 && t.tm == 128) return launch_one<FMT, 128, 128, 2, 2, 3, 32, EPI, KSLOW>(p, max_m_tiles, s);
     if (t.tw == 128 && t.tm == 256) return launch_one<FMT, 128, 256, 2, 2, 3, 4, EPI, KSLOW>(p, max_m_tiles, s);
-    if constexpr (EPI == kEpiStore) {
+    if constexpr (EPI == kEpiStore && FMT != CMX_FMT_E2M1) {
         if (t.tw == 128 && t.tm == 192) return launch_one<FMT, 128, 192, 2, 2, 3, 16, EPI, KSLOW>(p, max_m_tiles, s);
     }
     if constexpr (!KSLOW) {
@@ -385,6 +401,7 @@ int launch_ring(const GemmParams& p, const RingTile& t, int fmt, int epi, bool k
         return k_slow ? launch_shape<CMX_FMT_E5M2, kEpiStore, true>(p, t, max_m_tiles, s) : launch_shape<CMX_FMT_E5M2, kEpiStore, false>(p, t, max_m_tiles, s);
     if (fmt == CMX_FMT_E4M3 && epi == kEpiSwigluQuant && !k_slow) return launch_shape<CMX_FMT_E4M3, kEpiSwigluQuant, false>(p, t, max_m_tiles, s);
     if (fmt == CMX_FMT_E4M3 && epi == kEpiSwigluQuantAct && !k_slow) return launch_shape<CMX_FMT_E4M3, kEpiSwigluQuantAct, false>(p, t, max_m_tiles, s);
+    if (fmt == CMX_FMT_E2M1 && epi == kEpiStore && !k_slow) return launch_shape<CMX_FMT_E2M1, kEpiStore, false>(p, t, max_m_tiles, s);
     if (fmt == kFmtI8 && epi == kEpiI8DequantSwiglu && !k_slow) {
         if (t.tw == 128 && t.tm == 128) return launch_one<kFmtI8, 128, 128, 2, 2, 4, 0, kEpiI8DequantSwiglu, false>(p, max_m_tiles, s);
         if (t.tw == 128 && t.tm == 256) return launch_one<kFmtI8, 128, 256, 2, 2, 3, 0, kEpiI8DequantSwiglu, false>(p, max_m_tiles, s);

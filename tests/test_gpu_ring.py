@@ -145,6 +145,24 @@ def test_chosen_grouped_kernels(experts, avg, n, k):
 
 @pytest.mark.parametrize("tile", [(128, 128), (128, 256), (256, 128)])
 @pytest.mark.parametrize("out", ["fp32", "bf16"])
+@pytest.mark.parametrize("counts,n,k", [([1, 0, 127, 128, 129, 0, 257, 66], 320, 512), ([300, 2], 196, 1280), ([0, 5, 0], 64, 256), ([70], 130, 17664)])
+def test_grouped_fp4_gives_the_bits_of_the_256_row_kernel(tile, out, counts, n, k):
+    """Two dwords of scales a slab: a last piece of them in part (1280), more than their area holds (17664), less than a piece (256)."""
+    from catccos_amd import ops
+    rng = np.random.default_rng(sum(counts) + k)
+    m, e = sum(counts), len(counts)
+    aq, asc, bq, bsc = _operands(rng, m, e * n, k, "E2M1")
+    a, w = dev(O.pack_fp4(aq)), dev(O.pack_fp4(bq).reshape(e, n, k // 2))
+    args = (a, dev(asc), w, dev(bsc.reshape(e, n, -1)), dev(np.array(counts, dtype=np.int32)), k, "E2M1", out)
+    h = hooks_lib()
+    h.cmx_debug_force_tile(256, 256, 8)
+    want = ops.mx_gmm(*args)
+    h.cmx_debug_force_tile(*tile, 6)
+    assert torch.equal(ops.mx_gmm(*args), want)
+
+
+@pytest.mark.parametrize("tile", [(128, 128), (128, 256), (256, 128)])
+@pytest.mark.parametrize("out", ["fp32", "bf16"])
 @pytest.mark.parametrize("counts,n,k", [([1, 0, 127, 128, 129, 0, 257, 66], 320, 512), ([300, 2], 192, 128), ([0, 5, 0], 64, 1152)])
 def test_grouped_int8_gives_the_bits_of_the_256_row_kernel(tile, out, counts, n, k):
     """Whole-number sums and the same arithmetic behind them; fewer slabs than ring slots."""
