@@ -42,9 +42,6 @@ struct GemmParams {
     uint16_t* act_bf16;
     const int32_t* row_off;     // [groups+1] (grouped) or null (dense)
     const int32_t* tile_pref;   // [groups+1] prefix of m-tiles (grouped) or null
-    const int32_t* sizes;       // [groups] rows of the groups, in the place of the two tables (at most kInlineGroups), or null
-    uint32_t small_rows;        // with `sizes`: the limit between ...
-    int group_class;            // ... the groups that this launch takes (GroupClass)
     int32_t* tile_ctr;          // [8] per-XCD tile counters, zeroed before the launch (persistent grouped 4 x 1 kernels) or null
     uint32_t lda, ld_as, ldw, ld_ws, ldc, ld_act, ld_acts;
     uint32_t m, n, kbytes, kblocks;   // kblocks = K/32
@@ -53,6 +50,11 @@ struct GemmParams {
     int scale_vec;   // scale rows are 4-byte aligned: one dword load per row and slab
     int scale_vec16; // scale rows are 16-byte aligned: one 16-byte load per row fetches the scales of four slabs
     int w_pretiled;  // w holds the weights in the tiled order of cmx_mx_pretile_weights (the weights-to-registers kernel)
+    // (the last members: in front of the others they move the kernel arguments that the scheduled kernels keep in registers, and
+    // the weights-to-registers kernel of 256 rows then reloads a spilled value, and waits for all its loads, in every tile)
+    const int32_t* sizes;       // [groups] rows of the groups, in the place of row_off and tile_pref (at most kInlineGroups), or null
+    uint32_t small_rows;        // with `sizes`: the limit between ...
+    int group_class;            // ... the groups that this launch takes (GroupClass)
 };
 
 __device__ __forceinline__ uint32_t swz(uint32_t row, uint32_t chunk) {
