@@ -3,7 +3,7 @@
 // the launch 3.0, two torch.empty 3.4 and ctypes 0.5, where the kernel runs 3.3).  Here a tensor is 0.7 us and a call of 15 arguments 0.1:
 // quantizer 9.2 -> 5.8 us, dense matmul 7.8 -> 5.3; the two in turn at 16 x 4096 x 7168 17.0 -> 12.2, which is what their kernels take.
 //
-//   run(address, *args)              int(*)(...) at `address`: tensors by their data pointer, None as null, integers; ValueError for a tensor
+//   run(address, *args)              int(*)(...) at `address`: tensors by their data pointer, None as null, integers (anything with __index__); ValueError for a tensor
 //                                    that is not on the GPU.  Without the GIL, like a ctypes call.
 //   empty(like, dtype, size, ...)    torch.empty on the device of `like`, which is a GPU (ValueError)
 //
@@ -51,6 +51,9 @@ PyObject* run(PyObject*, PyObject* const* args, Py_ssize_t n) {
                 return nullptr;
             }
             v[i - 1] = reinterpret_cast<uint64_t>(t.data_ptr());
+        } else if (PyIndex_Check(o)) {                                   // numpy's integers
+            v[i - 1] = PyLong_AsUnsignedLongLongMask(o);
+            if (v[i - 1] == (uint64_t)-1 && PyErr_Occurred()) return nullptr;
         } else if (o != Py_None) {
             PyErr_Format(PyExc_TypeError, "argument %zd: a tensor, an integer or None, not %s", i, Py_TYPE(o)->tp_name);
             return nullptr;

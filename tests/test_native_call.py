@@ -1,6 +1,7 @@
 """catccos_amd._native_call: what reaches an entry point, and what is refused before it does."""
 import ctypes as C
 
+import numpy as np
 import pytest
 import torch
 
@@ -20,6 +21,19 @@ def test_every_argument_arrives_in_its_place(n):
     assert _native_call.run(C.cast(callee, C.c_void_p).value, *values) == -7
     want = [0 if v is None else v % 2 ** 64 for v in values]
     assert got == want + [0] * (24 - n)
+
+
+@pytest.mark.parametrize("value", [np.int64(2 ** 40 + 1), np.int32(-3), np.uint8(200), np.uint32(2 ** 32 - 1)], ids=lambda v: type(v).__name__)
+def test_numpy_integers_are_integers(value):
+    got = []
+    proto = C.CFUNCTYPE(C.c_int, *[C.c_uint64] * 24)
+
+    @proto
+    def callee(*args):
+        got.extend(args)
+        return 0
+    assert _native_call.run(C.cast(callee, C.c_void_p).value, 5, value, 6) == 0
+    assert got[:4] == [5, int(value) % 2 ** 64, 6, 0]
 
 
 def test_refusals():
