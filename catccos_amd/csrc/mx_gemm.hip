@@ -1409,12 +1409,12 @@ struct GroupPlan {
 
 // Whether kernels that take one tile per workgroup locate it by the sizes themselves.  A launch that fills tables first costs 5 us; a scan at
 // the start of a workgroup some 0.3 us more than the table reads, once for each round of workgroups: 32 experts x 16 rows of FP4, five
-// rounds of two workgroups per CU, 93.4 us with tables and 92.4 without; FFN of 32 tokens, 256 experts, where the tables cost no launch, 1119
-// with and 1053 against 1039 of another box without; INT8 of 2144 tiles, one per CU at a time, no difference.
+// rounds of two workgroups per CU, 93.4 us with tables and 92.4 without; INT8 of 2144 tiles, eight rounds of one per CU, no difference; FFN of
+// 32 tokens, 256 experts, where the tables cost no launch, 1119 with and 1053 against 1039 of another box without.  So up to six rounds.
 int tiles_by_sizes(bool* out, uint32_t groups, uint64_t max_tiles, uint32_t per_cu) {
     int cus = 0;
     if (int rc = cu_count(&cus); rc != CMX_OK) return rc;
-    *out = groups <= kInlineGroups && max_tiles <= 4 * (uint64_t)per_cu * cus;
+    *out = groups <= kInlineGroups && max_tiles <= 6 * (uint64_t)per_cu * cus;
     return CMX_OK;
 }
 int plan_groups(GroupPlan* plan, uint32_t m_total, uint32_t groups, uint32_t n, int fmt, uint32_t kblocks, bool swiglu, bool pretiled) {
