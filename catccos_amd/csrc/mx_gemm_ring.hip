@@ -375,7 +375,6 @@ int launch_one(const GemmParams& p, uint32_t max_m_tiles, hipStream_t s) {
     return CMX_OK;
 }
 
-#ifndef RING_PROTO
 template <int FMT, int EPI, bool KSLOW>
 int launch_shape(const GemmParams& p, const RingTile& t, uint32_t max_m_tiles, hipStream_t s) {
     if (t.tw == 128 && t.tm == 128) return launch_one<FMT, 128, 128, 2, 2, 3, 32, EPI, KSLOW>(p, max_m_tiles, s);
@@ -389,11 +388,9 @@ int launch_shape(const GemmParams& p, const RingTile& t, uint32_t max_m_tiles, h
     set_error("unsupported ring tile");
     return CMX_EINVAL;
 }
-#endif
 
 }  // namespace
 
-#ifndef RING_PROTO
 int launch_ring(const GemmParams& p, const RingTile& t, int fmt, int epi, bool k_slow, uint32_t max_m_tiles, hipStream_t s) {
     if (fmt == CMX_FMT_E4M3 && epi == kEpiStore)
         return k_slow ? launch_shape<CMX_FMT_E4M3, kEpiStore, true>(p, t, max_m_tiles, s) : launch_shape<CMX_FMT_E4M3, kEpiStore, false>(p, t, max_m_tiles, s);
@@ -410,6 +407,5 @@ int launch_ring(const GemmParams& p, const RingTile& t, int fmt, int epi, bool k
     set_error("unsupported ring problem");
     return CMX_EINVAL;
 }
-#endif
 
 }  // namespace cmx
