@@ -44,7 +44,12 @@ def _p(t: torch.Tensor):
 
 def _launch(name, *args):
     """The entry point `name` on these tensors (GPU tensors, or ValueError), integers and Nones, and torch's current stream."""
-    rc = _run(_lib.entries()[name], *args, _stream())
+    try:
+        stream = _stream()
+    except RuntimeError:                       # a process without a GPU has no stream; its tensors are refused as such
+        _need_cuda(*(t for t in args if isinstance(t, torch.Tensor)))
+        raise
+    rc = _run(_lib.entries()[name], *args, stream)
     if rc != 0:
         _lib.check(rc)
 

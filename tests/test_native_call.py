@@ -55,6 +55,27 @@ def test_refusals():
             call()
 
 
+def _host_calls():
+    """Calls whose every buffer is the caller's, on host tensors: nothing that they allocate is refused before the call itself."""
+    i32 = torch.zeros(2, dtype=torch.int32)
+    a, s = torch.zeros(4, 128, dtype=torch.uint8), torch.zeros(4, 4, dtype=torch.uint8)
+    b, bs = torch.zeros(2, 64, 128, dtype=torch.uint8), torch.zeros(2, 64, 4, dtype=torch.uint8)
+    work = torch.zeros(4096, dtype=torch.uint8)
+    return {"mx_gmm": lambda: ops.mx_gmm(a, s, b, bs, i32, 128, c=torch.zeros(4, 64, dtype=torch.bfloat16), workspace=work),
+            "mx_gmm, its own buffers": lambda: ops.mx_gmm(a, s, b, bs, i32, 128),
+            "mx_gmm_swiglu_quant": lambda: ops.mx_gmm_swiglu_quant(a, s, b, bs, i32, 128, workspace=work,
+                                                                   outs=(torch.zeros(4, 32, dtype=torch.uint8), torch.zeros(4, 2, dtype=torch.uint8))),
+            "int8_gmm_dequant_swiglu": lambda: ops.int8_gmm_dequant_swiglu(a.view(torch.int8), torch.zeros(4), b.view(torch.int8), torch.zeros(128), i32,
+                                                                           64, 128, 1, c=torch.zeros(4, 32))}
+
+
+@pytest.mark.parametrize("name", _host_calls())
+def test_host_tensors_are_refused_as_such(name):
+    # also in a process without a GPU, where asking for the current stream would fail first
+    with pytest.raises(ValueError, match="expected a GPU tensor"):
+        _host_calls()[name]()
+
+
 def test_entries_follow_the_active_library():
     before = _lib.entries()
     prev = _lib.activate(None)
