@@ -54,6 +54,12 @@ def _launch(name, *args):
         _lib.check(rc)
 
 
+def _brought(t):
+    """Weights, an output or a workspace that the caller brings, for _run: these may also lie in pinned host memory, which kernels reach by
+    its address (any other host tensor is passed on, and refused)."""
+    return t if isinstance(t, torch.Tensor) and (t.is_cuda or not t.is_pinned()) else t.data_ptr()
+
+
 def _need_cuda(*ts):
     for t in ts:
         if t is not None and not t.is_cuda:
@@ -172,7 +178,7 @@ def int8_gmm_dequant_swiglu(a, token_scale, b, channel_scale, group_sizes, n: in
     ws = _empty(a, torch.uint8, _lib.load().cmx_int8_gmm_workspace_bytes(g, n, k, trans_b))
     if c is None:
         c = torch.zeros((rows, n // 2), dtype=_OUT_DTYPE[out], device=a.device)
-    _launch("cmx_int8_gmm_dequant_swiglu", a, k, token_scale, b, channel_scale, scale_stride, c, c.stride(0), OUT[out], group_sizes, g, rows, n, k,
+    _launch("cmx_int8_gmm_dequant_swiglu", a, k, token_scale, b, channel_scale, scale_stride, _brought(c), c.stride(0), OUT[out], group_sizes, g, rows, n, k,
             trans_b, ws)
     return c
 
@@ -227,8 +233,8 @@ def mx_gmm(a, a_scale, b, b_scale, group_sizes, k: int, fmt: str = "E4M3", out: 
         c = torch.zeros((m, n), dtype=_OUT_DTYPE[out], device=a.device)
     if workspace is None:
         workspace = gmm_workspace(g, a.device)
-    _launch("cmx_mx_gmm_pretiled" if tiled else "cmx_mx_gmm", a, a.stride(0), a_scale, a_scale.stride(0), bd, b_scale, c, c.stride(0), group_sizes,
-            g, m, n, k, FMT[fmt], OUT[out], workspace)
+    _launch("cmx_mx_gmm_pretiled" if tiled else "cmx_mx_gmm", a, a.stride(0), a_scale, a_scale.stride(0), _brought(bd), b_scale, _brought(c),
+            c.stride(0), group_sizes, g, m, n, k, FMT[fmt], OUT[out], _brought(workspace))
     return c
 
 
@@ -248,8 +254,8 @@ def mx_gmm_swiglu_quant(a, a_scale, b, b_scale, group_sizes, k: int, want_bf16: 
     act = torch.zeros((m, half), dtype=torch.bfloat16, device=a.device) if want_bf16 else None
     if workspace is None:
         workspace = gmm_workspace(g, a.device)
-    _launch("cmx_mx_gmm_swiglu_quant_pretiled" if tiled else "cmx_mx_gmm_swiglu_quant", a, a.stride(0), a_scale, a_scale.stride(0), bd, b_scale, codes,
-            codes.stride(0), scales, scales.stride(0), act, group_sizes, g, m, n, k, workspace)
+    _launch("cmx_mx_gmm_swiglu_quant_pretiled" if tiled else "cmx_mx_gmm_swiglu_quant", a, a.stride(0), a_scale, a_scale.stride(0), _brought(bd),
+            b_scale, _brought(codes), codes.stride(0), _brought(scales), scales.stride(0), act, group_sizes, g, m, n, k, _brought(workspace))
     return codes, scales, act
 
 
@@ -346,12 +352,13 @@ def dispatch_ffn_combine(x, expert_idx, gate_weight, w1, w1_scale, w2, w2_scale,
         workspace = _empty(x, torch.uint8, ffn_workspace_bytes(m, k, n, e, top_k))
     if out is None:
         out = _empty(x, x.dtype, m, k)
+    w1d, w2d, out_at, workspace = _brought(w1d), _brought(w2d), _brought(out), _brought(workspace)
     entries = _lib.entries()
     if tiled1:
-        rc = _run(entries["cmx_dispatch_ffn_combine_pretiled"], _stream(), x, expert_idx, gate_weight, w1d, w1_scale, w2d, w2_scale, out, workspace,
+        rc = _run(entries["cmx_dispatch_ffn_combine_pretiled"], _stream(), x, expert_idx, gate_weight, w1d, w1_scale, w2d, w2_scale, out_at, workspace,
                   m, k, n, e, top_k)
     else:
-        rc = _run(entries["catccos_ascend950_dispatch_ffn_combine"], 0, _stream(), 0, x, expert_idx, gate_weight, w1d, w1_scale, w2d, w2_scale, out,
+        rc = _run(entries["catccos_ascend950_dispatch_ffn_combine"], 0, _stream(), 0, x, expert_idx, gate_weight, w1d, w1_scale, w2d, w2_scale, out_at,
                   workspace, None, m, k, n, e, top_k, 1)
     _lib.check(rc)
     return out

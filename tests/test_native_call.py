@@ -96,3 +96,38 @@ def test_outputs_and_errors_on_the_gpu():
         ops.mx_gemm(x.view(torch.uint8), x.view(torch.uint8), x.view(torch.uint8), x.view(torch.uint8), 33)
     with pytest.raises(ValueError, match="expected a GPU tensor"):
         ops.mx_gemm(x.view(torch.uint8), x.view(torch.uint8), x.view(torch.uint8).cpu(), x.view(torch.uint8), 32)
+
+
+@pytest.mark.gpu
+def test_buffers_that_the_caller_brings_may_be_pinned():
+    """Weights, outputs and workspaces in pinned host memory give the results that device buffers give (no kernel of these small problems uses
+    the workspace); other host memory, and inputs in host memory, are refused."""
+    gen = torch.Generator().manual_seed(3)
+    u8 = lambda *shape, hi=0x70: torch.randint(0, hi, shape, dtype=torch.uint8, generator=gen)
+    m, k, n, sizes = 96, 256, 128, torch.tensor([40, 0, 50], dtype=torch.int32).cuda()
+    a, s = u8(m, k).cuda(), (u8(m, 8, hi=8) + 120).cuda()
+    b, bs = u8(3, n, k), (u8(3, n, 8, hi=8) + 120).cuda()
+    work = ops.gmm_workspace(3, "cuda")
+    pinned = lambda *shape, dtype=torch.uint8: torch.zeros(shape, dtype=dtype, pin_memory=True)
+
+    want = ops.mx_gmm(a, s, b.cuda(), bs, sizes, k)
+    c = pinned(m, n, dtype=torch.bfloat16)
+    ops.mx_gmm(a, s, b.pin_memory(), bs, sizes, k, c=c, workspace=work)
+    codes, scales, _ = ops.mx_gmm_swiglu_quant(a, s, b.cuda(), bs, sizes, k)
+    outs = pinned(m, n // 2), pinned(m, 2)
+    ops.mx_gmm_swiglu_quant(a, s, b.pin_memory(), bs, sizes, k, workspace=pinned(work.numel()), outs=outs)
+    i8 = lambda t: t.view(torch.int8)
+    token, channel = torch.rand(m, generator=gen).cuda(), torch.rand(3 * n, generator=gen).cuda()
+    want8 = ops.int8_gmm_dequant_swiglu(i8(a), token, i8(b).cuda(), channel, sizes, n, k, 1)
+    c8 = pinned(m, n // 2, dtype=torch.float32)
+    ops.int8_gmm_dequant_swiglu(i8(a), token, i8(b).cuda(), channel, sizes, n, k, 1, c=c8)
+    torch.cuda.synchronize()
+    assert torch.equal(c, want.cpu()) and want.float().abs().max() > 0
+    assert torch.equal(outs[0], codes.cpu()) and torch.equal(outs[1], scales.cpu())
+    assert torch.equal(c8, want8.cpu())
+
+    for call in (lambda: ops.mx_gmm(a, s, b.cuda(), bs, sizes, k, c=torch.zeros(m, n, dtype=torch.bfloat16), workspace=work),
+                 lambda: ops.mx_gmm(a, s, b, bs, sizes, k), lambda: ops.mx_gmm(a, s.cpu().pin_memory(), b.cuda(), bs, sizes, k),
+                 lambda: ops.int8_gmm_dequant_swiglu(i8(a), token, i8(b).pin_memory(), channel, sizes, n, k, 1)):
+        with pytest.raises(ValueError, match="expected a GPU tensor"):
+            call()
