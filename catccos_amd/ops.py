@@ -8,6 +8,8 @@ anything in torch.
 """
 from __future__ import annotations
 
+from operator import index
+
 import torch
 
 from . import _lib
@@ -43,7 +45,8 @@ def _p(t: torch.Tensor):
 
 
 def _launch(name, *args):
-    """The entry point `name` on these tensors (GPU tensors, or ValueError), integers and Nones, and torch's current stream."""
+    """The entry point `name` on these tensors (GPU tensors, or ValueError), integers and Nones, and torch's current stream.  A whole number
+    that the caller gives goes through index() first: as a tensor of one element it would be passed by its address."""
     try:
         stream = _stream()
     except RuntimeError:                       # a process without a GPU has no stream; its tensors are refused as such
@@ -99,6 +102,7 @@ def mx_dequant(codes: torch.Tensor, scales: torch.Tensor, cols: int, fmt: str = 
 
 def mx_gemm(a, a_scale, b, b_scale, k: int, fmt: str = "E4M3", out: str = "bf16") -> torch.Tensor:
     """C[m,n] = deq(a)[m,k] . deq(b)[n,k]^T"""
+    k = index(k)
     m, n = a.size(0), b.size(0)
     c = _empty(a, _OUT_DTYPE[out], m, n)
     _launch("cmx_mx_gemm", a, a.stride(0), a_scale, a_scale.stride(0), b, b.stride(0), b_scale, b_scale.stride(0), c, n, m, n, k, FMT[fmt],
@@ -137,6 +141,7 @@ def mx_gemm_ex(a, a_scale, b, b_scale, m: int, n: int, k: int, fmt: str = "E4M3"
                trans_b: int = 1) -> torch.Tensor:
     """Dense operands in the reference's file layouts: a [m, k] (trans_a = 1: [k, m], scales [k/64, m, 2]);
     b [n, k] (trans_b = 0: [k, n], scales [k/64, n, 2])."""
+    m, n, k, trans_a, trans_b = index(m), index(n), index(k), index(trans_a), index(trans_b)
     assert a.is_contiguous() and a_scale.is_contiguous() and b.is_contiguous() and b_scale.is_contiguous()
     need = _lib.load().cmx_mx_gemm_ex_workspace_bytes(m, n, k, trans_a, trans_b)
     ws = _empty(a, torch.uint8, max(need, 1))
@@ -161,6 +166,7 @@ def mx_gmm_ex(a, a_scale, b, b_scale, group_sizes, n: int, k: int, fmt: str = "E
 
 def int8_quant_scatter(x: torch.Tensor, src2sorted, top_k: int = 1):
     """x bf16 [tokens, k] -> (codes int8 [tokens*top_k, k], scales fp32 [tokens*top_k]); row t goes to src2sorted[t*top_k + r]."""
+    top_k = index(top_k)
     assert x.dim() == 2 and x.element_size() == 2
     tokens, k = x.shape
     pitch, step = x.stride()
@@ -173,6 +179,7 @@ def int8_quant_scatter(x: torch.Tensor, src2sorted, top_k: int = 1):
 def int8_gmm_dequant_swiglu(a, token_scale, b, channel_scale, group_sizes, n: int, k: int, trans_b: int = 0,
                             out: str = "fp32", scale_stride: int = 1, c=None) -> torch.Tensor:
     """a int8 [rows, k]; b int8 [G, k, n] (trans_b = 0) or [G, n, k] (trans_b = 1); channel_scale fp32 [G*n*scale_stride]."""
+    n, k, trans_b, scale_stride = index(n), index(k), index(trans_b), index(scale_stride)
     assert a.is_contiguous() and b.is_contiguous() and group_sizes.dtype == torch.int32
     rows, g = a.size(0), b.size(0)
     ws = _empty(a, torch.uint8, _lib.load().cmx_int8_gmm_workspace_bytes(g, n, k, trans_b))
@@ -226,6 +233,7 @@ def _weights(b, pair_gate_up: bool):
 def mx_gmm(a, a_scale, b, b_scale, group_sizes, k: int, fmt: str = "E4M3", out: str = "bf16", c=None, workspace=None):
     """a [m_total, k], b [G, n, k] (dense tensor or PretiledWeights), group_sizes int32 [G] on device -> c [m_total, n]
     (rows past the groups untouched)."""
+    k = index(k)
     assert b_scale.is_contiguous() and group_sizes.dtype == torch.int32
     bd, tiled = _weights(b, False)
     m, (g, n) = a.size(0), b.shape[:2]
@@ -242,6 +250,7 @@ def mx_gmm_swiglu_quant(a, a_scale, b, b_scale, group_sizes, k: int, want_bf16: 
                         outs=None):
     """GMM1 + SwiGLU + MX requant.  b [G, n, k] (gate rows then up rows; dense tensor or PretiledWeights).
     Returns (codes [m, n/2], scales, act_bf16|None)."""
+    k = index(k)
     assert b_scale.is_contiguous() and group_sizes.dtype == torch.int32
     bd, tiled = _weights(b, True)
     m, (g, n) = a.size(0), b.shape[:2]
@@ -278,6 +287,7 @@ def init() -> None:
 
 def moe_init_routing(expert_idx: torch.Tensor, experts: int):
     """expert_idx int32 [T, topK] -> (sorted2src, src2sorted, counts) int32."""
+    experts = index(experts)
     assert expert_idx.dtype == torch.int32 and expert_idx.is_contiguous()
     t, top_k = expert_idx.shape
     routes = t * top_k
@@ -293,6 +303,7 @@ def quant_scatter(x: torch.Tensor, src2sorted: torch.Tensor, top_k: int, packed:
     packed=False: (codes [T*topK, k], scales [T*topK, RoundUp2(k/32)]), zeros in rows that no route is sent to;
     packed=True: one buffer [T*topK, packed_row_bytes(k)] = codes | scales | pad (``out``: a caller's zeroed buffer
     of that shape)."""
+    top_k = index(top_k)
     _need_cuda(x, src2sorted)
     t, k = x.shape
     rows = t * top_k

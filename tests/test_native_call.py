@@ -76,6 +76,33 @@ def test_host_tensors_are_refused_as_such(name):
         _host_calls()[name]()
 
 
+@pytest.mark.parametrize("name, call", [
+    ("cmx_mx_gemm", lambda x, i32, n: ops.mx_gemm(x, x, x, x, n(32))),
+    ("cmx_mx_gemm_ex", lambda x, i32, n: ops.mx_gemm_ex(x, x, x, x, n(2), n(3), n(64), trans_a=n(0), trans_b=n(1))),
+    ("cmx_int8_quant_scatter", lambda x, i32, n: ops.int8_quant_scatter(x, i32, n(4))),
+    ("cmx_int8_gmm_dequant_swiglu", lambda x, i32, n: ops.int8_gmm_dequant_swiglu(x, x, x, x, i32, n(64), n(128), n(1), scale_stride=n(5), c=x)),
+    ("cmx_mx_gmm", lambda x, i32, n: ops.mx_gmm(x, x, x, x, i32, n(32), c=x, workspace=x)),
+    ("cmx_mx_gmm_swiglu_quant", lambda x, i32, n: ops.mx_gmm_swiglu_quant(x, x, x, x, i32, n(32), outs=(x, x), workspace=x)),
+    ("cmx_moe_init_routing", lambda x, i32, n: ops.moe_init_routing(i32.view(1, 2), n(7))),
+    ("cmx_quant_scatter_zeroed", lambda x, i32, n: ops.quant_scatter(x, i32, n(4)))])
+def test_whole_numbers_as_tensors_of_one_element(monkeypatch, name, call):
+    """A size or flag given as a tensor of one element (which converts to an index) reaches the entry point as the number."""
+    seen = []
+
+    def run(address, *args):
+        seen.append([a for a in args if not isinstance(a, torch.Tensor)])
+        return 0
+    monkeypatch.setattr(ops, "_run", run)
+    monkeypatch.setattr(ops, "_empty", lambda like, dtype, *size: torch.empty(*(int(v) for v in size), dtype=dtype))
+    monkeypatch.setattr(ops, "_stream", lambda: 0)
+    monkeypatch.setattr(ops, "_need_cuda", lambda *ts: None)
+    monkeypatch.setattr(_lib, "entries", lambda: {name: 1})
+    x, i32 = torch.zeros(2, 32, dtype=torch.bfloat16), torch.zeros(2, dtype=torch.int32)
+    call(x, i32, int)
+    call(x, i32, torch.tensor)
+    assert seen[0] == seen[1] and len(seen) == 2, seen
+
+
 def test_entries_follow_the_active_library():
     before = _lib.entries()
     prev = _lib.activate(None)
