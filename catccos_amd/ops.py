@@ -14,12 +14,27 @@ import torch
 
 from . import _lib
 
-try:
-    from . import _native_call
-except ImportError as e:
-    raise ImportError(f"catccos_amd/_native_call.so: {e}; build it with `python -m catccos_amd.build`") from e
 
-_run, _empty = _native_call.run, _native_call.empty
+def _bind_native():
+    """Puts the functions of the extension in the place of the two below, at the first call as for the library: what needs no kernel
+    works without either."""
+    global _run, _empty
+    try:
+        from . import _native_call
+    except ImportError as e:
+        raise ImportError(f"catccos_amd/_native_call: {e}; build it with `python -m catccos_amd.build`") from e
+    _run, _empty = _native_call.run, _native_call.empty
+
+
+def _run(*args):
+    _bind_native()
+    return _run(*args)
+
+
+def _empty(*args):
+    _bind_native()
+    return _empty(*args)
+
 
 FMT = {"E4M3": 0, "E5M2": 1, "E2M1": 2, "E1M2": 3}
 _FP4 = ("E2M1", "E1M2")

@@ -1,5 +1,8 @@
 """catccos_amd._native_call: what reaches an entry point, and what is refused before it does."""
 import ctypes as C
+import os
+import subprocess
+import sys
 
 import numpy as np
 import pytest
@@ -74,6 +77,32 @@ def test_host_tensors_are_refused_as_such(name):
     # also in a process without a GPU, where asking for the current stream would fail first
     with pytest.raises(ValueError, match="expected a GPU tensor"):
         _host_calls()[name]()
+
+
+def test_the_front_end_imports_without_the_extension():
+    """The extension is asked for by the first call that needs it; its absence is an ImportError that says how to build it."""
+    code = """
+import sys
+sys.modules["catccos_amd._native_call"] = None              # an import of it fails
+import torch
+from catccos_amd import ops
+assert ops.scale_cols(96) == 4 and ops.ffn_workspace_bytes(1, 256, 512, 2, 1) > 0
+for _ in range(2):
+    try:
+        ops.mx_quant(torch.zeros(2, 32, dtype=torch.bfloat16))
+    except ImportError as e:
+        assert "python -m catccos_amd.build" in str(e)
+    else:
+        raise AssertionError("no ImportError")
+del sys.modules["catccos_amd._native_call"]                 # built in the meantime
+try:
+    ops.mx_quant(torch.zeros(2, 32, dtype=torch.bfloat16))
+except ValueError:
+    print("ok")
+"""
+    root = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+    r = subprocess.run([sys.executable, "-c", code], capture_output=True, text=True, cwd=root, timeout=110)
+    assert r.returncode == 0 and r.stdout.strip() == "ok", r.stderr
 
 
 @pytest.mark.parametrize("name, call", [
