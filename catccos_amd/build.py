@@ -9,6 +9,7 @@ from __future__ import annotations
 import os
 import subprocess
 import sys
+import sysconfig
 from concurrent.futures import ThreadPoolExecutor
 
 HERE = os.path.dirname(os.path.abspath(__file__))
@@ -18,7 +19,8 @@ OBJ = os.path.join(HERE, "_build")
 LIBDIR = os.path.join(HERE, "lib")
 LIB = os.path.join(LIBDIR, "libcatccos_mx.so")
 NATIVE_SRC = os.path.join(CSRC, "native_call.cpp")
-NATIVE = os.path.join(HERE, "_native_call.so")
+# the name carries the interpreter's ABI tag, so that another Python looks for an extension of its own
+NATIVE = os.path.join(HERE, "_native_call" + sysconfig.get_config_var("EXT_SUFFIX"))
 
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 FLAGS = [
@@ -78,20 +80,30 @@ def _compile(src: str, verbose: bool) -> str:
 
 
 def build_native(force: bool = False) -> str:
-    """The Python extension catccos_amd._native_call (host code only, against this interpreter's torch)."""
-    if not force and os.path.exists(NATIVE) and os.path.getmtime(NATIVE) >= os.path.getmtime(NATIVE_SRC):
-        return NATIVE
-    import sysconfig
-
+    """The Python extension catccos_amd._native_call (host code only, against this interpreter's torch).  It reads torch's structures, so
+    it is rebuilt when torch, Python or the command changes (the stamp beside the objects), not only for a newer source."""
     import torch
     t = os.path.dirname(torch.__file__)
     cmd = ["g++", "-O2", "-std=c++17", "-fPIC", "-shared", f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}",
+           f'-DCMX_TORCH_VERSION="{torch.__version__}"',
            "-isystem", os.path.join(t, "include"), "-isystem", os.path.join(t, "include", "torch", "csrc", "api", "include"),
-           "-isystem", sysconfig.get_paths()["include"], NATIVE_SRC, "-o", NATIVE,
+           "-isystem", sysconfig.get_paths()["include"], NATIVE_SRC,
            "-L" + os.path.join(t, "lib"), "-ltorch_python", "-ltorch", "-ltorch_cpu", "-lc10"]
-    r = subprocess.run(cmd, capture_output=True, text=True)
+    stamp, want = os.path.join(OBJ, "native_call.stamp"), "\n".join([sys.version, *cmd])
+    if (not force and os.path.exists(NATIVE) and os.path.getmtime(NATIVE) >= os.path.getmtime(NATIVE_SRC)
+            and os.path.exists(stamp) and open(stamp).read() == want):
+        return NATIVE
+    # to a file of its own, moved into place when it is whole: a build that is interrupted or runs twice leaves no part of one
+    tmp = f"{NATIVE}.{os.getpid()}"
+    r = subprocess.run([*cmd, "-o", tmp], capture_output=True, text=True)
     if r.returncode != 0:
+        if os.path.exists(tmp):
+            os.remove(tmp)
         raise RuntimeError(f"g++ failed on {NATIVE_SRC}:\n" + r.stdout + r.stderr)
+    os.replace(tmp, NATIVE)
+    os.makedirs(OBJ, exist_ok=True)
+    with open(stamp, "w") as f:
+        f.write(want)
     return NATIVE
 
 

@@ -105,4 +105,12 @@ PyModuleDef module = {PyModuleDef_HEAD_INIT, "_native_call", nullptr, -1, method
 
 }  // namespace
 
-PyMODINIT_FUNC PyInit__native_call() { return PyModule_Create(&module); }
+// torch_version: the torch whose structures this reads
+PyMODINIT_FUNC PyInit__native_call() {
+    PyObject* const m = PyModule_Create(&module);
+    if (m != nullptr && PyModule_AddStringConstant(m, "torch_version", CMX_TORCH_VERSION) != 0) {
+        Py_DECREF(m);
+        return nullptr;
+    }
+    return m;
+}

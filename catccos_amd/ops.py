@@ -21,6 +21,8 @@ def _bind_native():
     global _run, _empty
     try:
         from . import _native_call
+        if _native_call.torch_version != str(torch.__version__):
+            raise ImportError(f"built for torch {_native_call.torch_version}, not {torch.__version__}")
     except ImportError as e:
         raise ImportError(f"catccos_amd/_native_call: {e}; build it with `python -m catccos_amd.build`") from e
     _run, _empty = _native_call.run, _native_call.empty

@@ -105,6 +105,39 @@ except ValueError:
     assert r.returncode == 0 and r.stdout.strip() == "ok", r.stderr
 
 
+def test_the_extension_is_rebuilt_for_another_torch(monkeypatch, tmp_path):
+    """Newer than its source is not enough: a change of torch or of the command builds it again; a failed build leaves the old one alone."""
+    from catccos_amd import build
+    target, calls = tmp_path / "ext.so", []
+
+    def compiler(cmd, **kw):
+        calls.append(cmd)
+        out = cmd[cmd.index("-o") + 1]
+        with open(out, "w") as f:
+            f.write(f"build {len(calls)}")
+        return subprocess.CompletedProcess(cmd, 1 if len(calls) == 3 else 0, "", "error")
+    monkeypatch.setattr(build, "NATIVE", str(target))
+    monkeypatch.setattr(build, "OBJ", str(tmp_path / "obj"))
+    monkeypatch.setattr(build.subprocess, "run", compiler)
+    build.build_native()
+    build.build_native()
+    assert len(calls) == 1 and target.read_text() == "build 1"
+    monkeypatch.setattr(torch, "__version__", "0.0.0")
+    build.build_native()
+    build.build_native()
+    assert len(calls) == 2 and target.read_text() == "build 2"
+    with pytest.raises(RuntimeError, match="error"):
+        build.build_native(force=True)
+    assert target.read_text() == "build 2" and sorted(os.listdir(tmp_path)) == ["ext.so", "obj"]
+
+
+def test_an_extension_of_another_torch_is_refused(monkeypatch):
+    assert _native_call.torch_version == torch.__version__
+    monkeypatch.setattr(_native_call, "torch_version", "0.0.0")
+    with pytest.raises(ImportError, match="built for torch 0.0.0"):
+        ops._bind_native()
+
+
 @pytest.mark.parametrize("name, call", [
     ("cmx_mx_gemm", lambda x, i32, n: ops.mx_gemm(x, x, x, x, n(32))),
     ("cmx_mx_gemm_ex", lambda x, i32, n: ops.mx_gemm_ex(x, x, x, x, n(2), n(3), n(64), trans_a=n(0), trans_b=n(1))),
