@@ -683,6 +683,18 @@ extern "C" uint32_t cmx_packed_row_bytes(uint32_t k) { return cmx::round_up(k + 
 
 namespace cmx {
 namespace {
+// the extras of a quantise + scatter in launches of their own
+int launch_extras(const ScatterExtras& ex, const int32_t* src2sorted, uint8_t* out_codes, uint32_t ld_out, uint8_t* out_scales, uint32_t ld_outs,
+                  hipStream_t s) {
+    for (uint32_t i = 0; i < ex.tables; ++i)
+        if (int rc = launch_group_tables(ex.job[i], s); rc != CMX_OK) return rc;
+    if (ex.zero.blocks != 0) {
+        hipLaunchKernelGGL(zero_unmapped_rows_kernel, dim3(ex.zero.blocks), dim3(256), 0, s, ex.zero, src2sorted, out_codes, ld_out, out_scales, ld_outs);
+        CMX_LAUNCH_CHECK();
+    }
+    return CMX_OK;
+}
+
 int quant_scatter(const void* x, uint32_t ld_x, const int32_t* src2sorted, uint8_t* out_codes, uint32_t ld_out, uint8_t* out_scales,
                   uint32_t ld_outs, uint32_t tokens, uint32_t k, uint32_t top_k, const ScatterExtras& ex, hipStream_t s) {
     CMX_REQUIRE(x && src2sorted && out_codes && out_scales, "null pointer");
@@ -706,15 +718,14 @@ int quant_scatter(const void* x, uint32_t ld_x, const int32_t* src2sorted, uint8
         const uintptr_t c0 = reinterpret_cast<uintptr_t>(out_codes), s0 = reinterpret_cast<uintptr_t>(out_scales);
         const bool disjoint = s0 >= c0 + dst_rows * ld_out || s0 + dst_rows * ld_outs <= c0;
         const uint32_t run = (disjoint && ld_outs == round_up(scale_cols(k), 128)) ? ld_outs : run16;
+        // (a launch holds fewer than 2^32 threads: the last few token counts that fit leave no room for the extras)
         const uint64_t blocks = (uint64_t)tokens + ex.tables + ex.zero.blocks;
-        CMX_REQUIRE(blocks < (1ull << 32), "too many tokens for one launch");
-        hipLaunchKernelGGL(quant_scatter_row_kernel, dim3((uint32_t)blocks), dim3(256), 0, s, xp, ld_x, src2sorted, out_codes, ld_out,
-                           out_scales, ld_outs, top_k, nb, run, ex);
+        const bool beside = blocks * 256 < (1ull << 32);
+        hipLaunchKernelGGL(quant_scatter_row_kernel, dim3(beside ? (uint32_t)blocks : tokens), dim3(256), 0, s, xp, ld_x, src2sorted, out_codes, ld_out,
+                           out_scales, ld_outs, top_k, nb, run, beside ? ex : ScatterExtras{});
         CMX_LAUNCH_CHECK();
-        return CMX_OK;
+        return beside ? CMX_OK : launch_extras(ex, src2sorted, out_codes, ld_out, out_scales, ld_outs, s);
     }
-    for (uint32_t i = 0; i < ex.tables; ++i)
-        if (int rc = launch_group_tables(ex.job[i], s); rc != CMX_OK) return rc;
     const bool vec_scales = nb % 4 == 0 && ld_outs % 4 == 0 && (reinterpret_cast<uintptr_t>(out_scales) & 3u) == 0;
     const dim3 grid(ceil_div(total, 128));
     if (vec_scales)
@@ -724,11 +735,7 @@ int quant_scatter(const void* x, uint32_t ld_x, const int32_t* src2sorted, uint8
         hipLaunchKernelGGL((quant_scatter_kernel<false>), grid, dim3(256), 0, s, xp, ld_x, src2sorted, out_codes, ld_out,
                            out_scales, ld_outs, tokens, k, top_k, nb, total);
     CMX_LAUNCH_CHECK();
-    if (ex.zero.blocks != 0) {
-        hipLaunchKernelGGL(zero_unmapped_rows_kernel, dim3(ex.zero.blocks), dim3(256), 0, s, ex.zero, src2sorted, out_codes, ld_out, out_scales, ld_outs);
-        CMX_LAUNCH_CHECK();
-    }
-    return CMX_OK;
+    return launch_extras(ex, src2sorted, out_codes, ld_out, out_scales, ld_outs, s);
 }
 }  // namespace
 

@@ -124,6 +124,28 @@ def test_quant_scatter_skips_negative_destinations():
     assert np.all(got[3] == 0) and np.array_equal(got[2], q[1]) and np.array_equal(got[4], q[2])
 
 
+@pytest.mark.parametrize("tokens", [2 ** 24 - 258, 2 ** 24 - 1])
+def test_as_many_tokens_as_one_launch_holds(tokens):
+    """A workgroup of 256 threads per token and fewer than 2^32 threads in a launch: 2^24 - 1 tokens are taken, with and without room for the
+    workgroups that clear rows beside them."""
+    from catccos_amd import _lib, ops
+    k, pitch = 32, 16
+    g = torch.Generator(device="cuda")
+    g.manual_seed(tokens)
+    x = torch.randint(-2 ** 15, 2 ** 15, (tokens, k), generator=g, device="cuda", dtype=torch.int16).view(torch.bfloat16)
+    dest = torch.arange(tokens, device="cuda", dtype=torch.int32)
+    dropped = torch.tensor([0, 5, tokens // 2, tokens - 1], device="cuda")
+    dest[dropped] = -1
+    codes = torch.full((tokens, k), 171, dtype=torch.uint8, device="cuda")
+    scales = torch.full((tokens, pitch), 171, dtype=torch.uint8, device="cuda")
+    _lib.check(_lib.load().cmx_quant_scatter_zeroed(x.data_ptr(), k, dest.data_ptr(), codes.data_ptr(), k, scales.data_ptr(), pitch, tokens, k, 1,
+                                                    torch.cuda.current_stream().cuda_stream))
+    want_codes, want_scales = ops.mx_quant(x)
+    want_codes[dropped] = 0
+    want_scales[dropped] = 0
+    assert torch.equal(codes, want_codes) and torch.equal(scales[:, :2], want_scales)
+
+
 @pytest.mark.parametrize("tokens,hidden,top_k", [(5, 64, 1), (33, 7168, 8), (100, 520, 6), (64, 2048, 3), (9, 100, 9)])
 def test_combine_bit_exact(tokens, hidden, top_k):
     from catccos_amd import ops
