@@ -138,19 +138,40 @@ __global__ __launch_bounds__(64) void route_scatter_kernel(const int32_t* __rest
 // the workgroup + in the wavefronts before + in the lanes before (ballots), the unique stable permutation.
 // Bound by latency: launch, one pass over the keys (4 routes bytes from the L2 per workgroup, an LDS atomic each), one store.  In place of
 // three launches (histogram, one-workgroup scan over the chunks, scatter).
+// Lanes that add to one address take turns, so the counters come in `copies` (lane % copies picks one; an odd pitch puts the copies of a key
+// into different banks).  Measured (us, three launches / one counter per key / copies; the last sizes are the limits below):
+//    32768 routes,  16 experts   uniform 16.0  8.2  7.1    Zipf 16.0 12.7  7.1    all to one expert 15.9  30.8  6.8
+//    32768         256                   20.6  7.3  7.7         20.5 10.4  7.5                       20.3  31.2  8.0
+//   131072          16                   29.6 22.5 17.3         29.6 40.3 17.3                       29.5 113.3 17.1
+//   131072         512                   42.0 17.7 18.5         41.7 28.8 20.0                       41.4 114.1 33.6
 constexpr uint32_t kSortThreads = 1024, kSortWaves = kSortThreads / 64, kSortExperts = 512, kSortRoutes = 131072;
 
+constexpr uint32_t sort_pitch(uint32_t experts) { return experts | 1u; }
+constexpr size_t sort_lds_bytes(uint32_t experts, uint32_t copies) {
+    return (2 * (size_t)copies * sort_pitch(experts) + kSortWaves * experts) * sizeof(uint32_t);
+}
+// Copies of the counters.  Few experts meet on an address whatever the load, and get one for two lanes.  From 17 on it takes a skewed load, and
+// eight, whose clearing and adding up cost even loads 0.1 to 0.5 us (32 cost them up to 1.4: 131072 routes over 256 experts 17.0 with one,
+// 17.9 with 8, 18.6 with 32; all to one expert 113, 20.7, 17.6).  64 KiB of LDS hold four of 512 experts.  A workgroup that sees two keys per
+// thread does without.
+uint32_t sort_copies(uint32_t routes, uint32_t experts) {
+    uint32_t c = routes <= 2 * kSortThreads ? 1 : (experts <= 16 ? 32 : 8);
+    while (c > 1 && sort_lds_bytes(experts, c) > 65536 - 1024) c /= 2;
+    return c;
+}
+
 __global__ __launch_bounds__(kSortThreads) void route_sort_kernel(const int32_t* __restrict__ keys, uint32_t routes, uint32_t experts,
-                                                                   uint32_t key_bits, int32_t* __restrict__ sorted2src,
+                                                                   uint32_t key_bits, uint32_t copies, int32_t* __restrict__ sorted2src,
                                                                    int32_t* __restrict__ src2sorted, int32_t* __restrict__ counts) {
     extern __shared__ uint32_t sh[];
     __shared__ uint32_t part[kSortWaves];
-    uint32_t* const before = sh;                     // [experts] keys of the routes before the workgroup's, then ...
-    uint32_t* const after = sh + experts;            // [experts] ... of its own and later ones
-    uint32_t* const in_wave = sh + 2 * experts;      // [wavefront][experts] keys of each wavefront, then where its rows start
+    const uint32_t pitch = sort_pitch(experts), half = copies * pitch;
+    uint32_t* const before = sh;                     // [copy][pitch] keys of the routes before the workgroup's, then ([half ..])
+                                                     // of its own and later ones
+    uint32_t* const in_wave = sh + 2 * half;         // [wavefront][experts] keys of each wavefront, then where its rows start
     const uint32_t tid = threadIdx.x, lane = tid & 63u, wave = tid >> 6;
     const uint32_t base = blockIdx.x * kSortThreads, r = base + tid;
-    for (uint32_t i = tid; i < (2 + kSortWaves) * experts; i += kSortThreads) sh[i] = 0;
+    for (uint32_t i = tid; i < 2 * half + kSortWaves * experts; i += kSortThreads) sh[i] = 0;
     const int32_t raw = r < routes ? keys[r] : -1;
     const bool live = raw >= 0 && (uint32_t)raw < experts;
     const uint32_t k = live ? (uint32_t)raw : 0;
@@ -162,6 +183,7 @@ __global__ __launch_bounds__(kSortThreads) void route_sort_kernel(const int32_t*
     }
     const uint32_t rank = __popcll(same & ((1ull << lane) - 1ull));
     if (live && lane == 63u - (uint32_t)__clzll(same)) in_wave[wave * experts + k] = (uint32_t)__popcll(same);
+    uint32_t* const mine_before = before + (lane & (copies - 1)) * pitch;
     for (uint32_t i0 = 0; i0 < routes; i0 += 8 * kSortThreads) {
         int32_t v[8];
 #pragma unroll
@@ -171,13 +193,21 @@ __global__ __launch_bounds__(kSortThreads) void route_sort_kernel(const int32_t*
         }
 #pragma unroll
         for (uint32_t j = 0; j < 8; ++j) {
-            uint32_t* const to = i0 + j * kSortThreads < base ? before : after;          // whole workgroups of routes
+            uint32_t* const to = mine_before + (i0 + j * kSortThreads < base ? 0 : half);          // whole workgroups of routes
             if (v[j] >= 0 && (uint32_t)v[j] < experts) atomicAdd(&to[v[j]], 1u);
         }
     }
     __syncthreads();
     // exclusive scan over the experts, one per thread (experts <= kSortExperts < kSortThreads)
-    const uint32_t mine = tid < experts ? before[tid] + after[tid] : 0;
+    uint32_t rows_before = 0, mine = 0;
+    if (tid < experts) {
+#pragma unroll 4
+        for (uint32_t c = 0; c < copies; ++c) {
+            rows_before += before[c * pitch + tid];
+            mine += before[half + c * pitch + tid];
+        }
+        mine += rows_before;
+    }
     uint32_t sum = mine;
 #pragma unroll
     for (int d = 1; d < 64; d <<= 1) {
@@ -187,7 +217,7 @@ __global__ __launch_bounds__(kSortThreads) void route_sort_kernel(const int32_t*
     if (lane == 63u) part[wave] = sum;
     __syncthreads();
     if (tid < experts) {
-        uint32_t run = sum - mine + before[tid];
+        uint32_t run = sum - mine + rows_before;
         for (uint32_t w = 0; w < wave; ++w) run += part[w];
         for (uint32_t w = 0; w < kSortWaves; ++w) {
             const uint32_t c = in_wave[w * experts + tid];
@@ -662,8 +692,9 @@ extern "C" int cmx_moe_init_routing(const int32_t* expert_idx, uint32_t tokens, 
     uint32_t key_bits = 0;
     while ((1u << key_bits) < experts) ++key_bits;
     if (routes <= kSortRoutes && experts <= kSortExperts) {
+        const uint32_t copies = sort_copies(routes, experts);
         hipLaunchKernelGGL(route_sort_kernel, dim3(ceil_div(routes, kSortThreads)), dim3(kSortThreads),
-                           (2 + kSortWaves) * experts * sizeof(uint32_t), s, expert_idx, routes, experts, key_bits, sorted2src, src2sorted, counts);
+                           sort_lds_bytes(experts, copies), s, expert_idx, routes, experts, key_bits, copies, sorted2src, src2sorted, counts);
         CMX_LAUNCH_CHECK();
         return CMX_OK;
     }

@@ -52,6 +52,24 @@ def test_sort_at_the_edges_of_the_single_launch(routes, experts):
     assert np.array_equal(host(s2s)[:len(order)], order) and np.array_equal(host(inv), want)
 
 
+@pytest.mark.parametrize("routes", [2048, 2049, 9000])
+@pytest.mark.parametrize("experts", [1, 16, 17, 440, 512])
+@pytest.mark.parametrize("load", ["random", "one", "last"])
+def test_sort_with_copies_of_the_counters(routes, experts, load):
+    """One counter per key up to 2048 routes; beyond, 32 copies up to 16 experts, 8, and as many as the LDS holds (4 at 512 experts).  All
+    routes to one expert put every lane of a workgroup on one key."""
+    from catccos_amd import ops
+    keys = np.random.default_rng(routes + experts).integers(0, experts, routes).astype(np.int32)
+    if load != "random":
+        keys[:] = experts // 2 if load == "one" else experts - 1
+    s2s, inv, counts = ops.moe_init_routing(dev(keys.reshape(-1, 1)), experts)
+    order = np.argsort(keys, kind="stable")
+    want = np.empty(routes, dtype=np.int32)
+    want[order] = np.arange(routes)
+    assert np.array_equal(host(counts), np.bincount(keys, minlength=experts))
+    assert np.array_equal(host(s2s), order) and np.array_equal(host(inv), want)
+
+
 @pytest.mark.parametrize("packed", [False, True])
 def test_quant_scatter_bit_exact(packed):
     from catccos_amd import ops
