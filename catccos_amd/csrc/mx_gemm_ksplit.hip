@@ -479,7 +479,7 @@ template <int FMT, int FW, int FM, int NW, int EPI, int LAYOUT, KsplitWeights LO
 __global__ __launch_bounds__(64 * NW, 2) void mx_gemm_ksplit_kernel(const GemmParams p) {
     extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
     Tile tc;
-    if (!locate_tile<16 * FM>(p, tc)) return;
+    if (!locate_tile<16 * FM, LOADS == KsplitWeights::kCached>(p, tc)) return;
     tc.g = __builtin_amdgcn_readfirstlane(tc.g);
     tc.wt = __builtin_amdgcn_readfirstlane(tc.wt);
     tc.row0 = __builtin_amdgcn_readfirstlane(tc.row0);
@@ -508,10 +508,12 @@ int launch_one(const GemmParams& p, uint32_t max_m_tiles, hipStream_t s) {
 template <int FMT, int EPI, int LAYOUT>
 int launch_shape(const GemmParams& p, const KsplitTile& t, uint32_t max_m_tiles, KsplitWeights loads, hipStream_t s) {
 #define CMX_KS(FW_, FM_, NW_) if (t.fw == FW_ && t.fm == FM_ && t.waves == NW_) return launch_one<FMT, FW_, FM_, NW_, EPI, LAYOUT, KsplitWeights::kCached>(p, max_m_tiles, s)
-    if constexpr (LAYOUT != kKSlow) if (t.fw == 4 && t.fm == 4 && t.waves == 4 && (p.row_off != nullptr || p.sizes != nullptr)) {
+    const bool grouped = p.row_off != nullptr || p.sizes != nullptr;             // (kCached kernels know no groups)
+    if constexpr (LAYOUT != kKSlow) if (t.fw == 4 && t.fm == 4 && t.waves == 4 && grouped) {
         if (loads == KsplitWeights::kStreamed) return launch_one<FMT, 4, 4, 4, EPI, LAYOUT, KsplitWeights::kStreamed>(p, max_m_tiles, s);
         return launch_one<FMT, 4, 4, 4, EPI, LAYOUT, KsplitWeights::kByGroup>(p, max_m_tiles, s);
     }
+    CMX_REQUIRE(!grouped, "split-K tile of a grouped problem: 64 x 64 only");
     if constexpr (LAYOUT == kKSlow) {
         CMX_KS(4, 4, 4);
         CMX_KS(4, 1, 8);

@@ -108,6 +108,15 @@ def test_grouped_fp4(counts):
     assert np.allclose(host(c), gold, rtol=1e-5, atol=1e-4)
 
 
+def test_dense_tiles_refuse_groups():
+    """The kernels of dense problems have no code that looks for groups: a grouped problem on one of their tiles is an error of the host."""
+    from catccos_amd import _lib, ops
+    hooks_lib().cmx_debug_force_ksplit(1, 1, 8)
+    u8 = lambda *shape: torch.zeros(shape, dtype=torch.uint8, device="cuda")
+    with pytest.raises(_lib.CmxError, match="64 x 64 only"):
+        ops.mx_gmm(u8(32, 128), u8(32, 4), u8(2, 64, 128), u8(2, 64, 4), torch.tensor([16, 16], dtype=torch.int32, device="cuda"), 128)
+
+
 @pytest.mark.parametrize("counts", COUNTS)
 @pytest.mark.parametrize("out", ["fp32", "bf16"])
 def test_grouped_int8(counts, out):
