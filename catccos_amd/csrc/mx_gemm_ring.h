@@ -11,7 +11,7 @@ struct RingTile {
 };
 
 // p as for the other kernels, with w_tiles counted in tiles of t.tw weight rows (t.tw / 2 output columns for epilogues that pair gate and
-// up) and, for grouped problems, group tables made for m-tiles of t.tm rows; MX formats (scale rows of any alignment) and INT8, K whole
+// up) and, for grouped problems, group tables made for m-tiles of t.tm rows; MX formats (scale rows of any alignment and pitch) and INT8, K whole
 // 128-byte slabs.
 // k_slow: p.w is [K][ldw] and p.w_scale [K / 64][n][2] at a pitch of ld_ws bytes; dense, n a multiple of 4 and at least 16, p.w dword-aligned,
 // K * ldw below 2^32.

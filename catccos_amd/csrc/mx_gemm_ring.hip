@@ -164,15 +164,17 @@ __global__ __launch_bounds__(64 * WW * WM) void mx_gemm_ring_kernel(const GemmPa
     auto load_scales = [&](uint32_t b) {
         if constexpr (kScales) {
             const uint32_t half_at = kScaleBase + (b & 1u) * kScaleHalf;
-            auto address = [&](uint32_t piece, uint32_t d, bool of_w) -> uint32_t {
+            // in bytes, as a T: 32 bits do where the pieces are whole (launch_ring)
+            auto address = [&](auto as, uint32_t piece, uint32_t d, bool of_w) {
+                using T = decltype(as);
                 const uint32_t row = piece / kPieces;
                 if (KSLOW && of_w) {
                     const uint32_t k64 = 2 * SPAN * b + piece / (TW / 8), col = piece % (TW / 8) * 8 + 2 * d;
-                    return (k64 < 2 * nslab ? k64 : 2 * nslab - 1) * p.ld_ws + 2 * (wcol_of(col / 16) + col % 16);
+                    return (T)(k64 < 2 * nslab ? k64 : 2 * nslab - 1) * p.ld_ws + 2 * (wcol_of(col / 16) + col % 16);
                 }
                 const uint32_t dw = SPAN * b + 4 * ((piece ^ (row / (64 / SPAN))) & (kPieces - 1)) + d;
                 const uint32_t at = 4 * (dw < last_dw ? dw : last_dw);               // past K: never used
-                return of_w ? wrow_of(row) * p.ld_ws + at : arow_of(row - TW) * p.ld_as + at;
+                return of_w ? (T)wrow_of(row) * p.ld_ws + at : (T)arow_of(row - TW) * p.ld_as + at;
             };
             constexpr uint32_t kWPieces = TW * kPieces;                              // the weights' come first; a load has one kind
             if (whole_pieces) {
@@ -180,16 +182,16 @@ __global__ __launch_bounds__(64 * WW * WM) void mx_gemm_ring_kernel(const GemmPa
                 for (int i = 0; i < kScaleLoads; ++i) {
                     const uint32_t p0 = min((uint32_t)(NW * i + wave) * 64, (uint32_t)kAllPieces - 64);          // (a duplicate at most)
                     const bool of_w = p0 < kWPieces;
-                    ring_dma16(lds0 + half_at + p0 * 16, address(p0 + lane, 0, of_w), of_w ? ws_rs : as_rs, 0);
+                    ring_dma16(lds0 + half_at + p0 * 16, address(uint32_t{}, p0 + lane, 0, of_w), of_w ? ws_rs : as_rs, 0);
                 }
             } else {
-                // rows at any byte, or of less than a piece: through registers (the waits for them drain the ring, once in SPAN slabs)
+                // rows at any byte, of less than a piece, or further apart than 32 bits reach: through registers (the waits for them drain the ring, once in SPAN slabs)
 #pragma unroll 2
                 for (int i = 0; i < 4 * kScaleLoads; ++i) {
                     const uint32_t p0 = min((uint32_t)(NW * i + wave) * 16, (uint32_t)kAllPieces - 16);
                     const bool of_w = p0 < kWPieces;
                     uint32_t v;
-                    __builtin_memcpy(&v, (of_w ? w_scales : a_scales) + address(p0 + lane / 4, lane & 3u, of_w), 4);
+                    __builtin_memcpy(&v, (of_w ? w_scales : a_scales) + address(size_t{}, p0 + lane / 4, lane & 3u, of_w), 4);
                     *reinterpret_cast<uint32_t*>(smem + half_at + p0 * 16 + lane * 4) = v;
                 }
             }
@@ -391,7 +393,10 @@ int launch_shape(const GemmParams& p, const RingTile& t, uint32_t max_m_tiles, h
 
 }  // namespace
 
-int launch_ring(const GemmParams& p, const RingTile& t, int fmt, int epi, bool k_slow, uint32_t max_m_tiles, hipStream_t s) {
+int launch_ring(const GemmParams& params, const RingTile& t, int fmt, int epi, bool k_slow, uint32_t max_m_tiles, hipStream_t s) {
+    GemmParams p = params;
+    // The split-K kernels, which share the dense sizes with this one, take scale rows of any pitch.
+    if (!k_slow && ((uint64_t)p.n * p.ld_ws >= (1ull << 32) || (uint64_t)p.ld_as * t.tm >= (1ull << 32))) p.scale_vec = 0;
     if (fmt == CMX_FMT_E4M3 && epi == kEpiStore)
         return k_slow ? launch_shape<CMX_FMT_E4M3, kEpiStore, true>(p, t, max_m_tiles, s) : launch_shape<CMX_FMT_E4M3, kEpiStore, false>(p, t, max_m_tiles, s);
     if (fmt == CMX_FMT_E5M2 && epi == kEpiStore)

@@ -49,6 +49,20 @@ def test_bits_of_the_256_row_kernels_on_both_weight_layouts(tm, fmt, out, m, n, 
     _near(want, aq, asc, bq, bsc, fmt)
 
 
+@pytest.mark.parametrize("m,n,far", [(1100, 2048, "weights"), (128, 16448, "activations")])
+def test_scale_rows_further_apart_than_32_bits_reach(m, n, far):
+    """Default dispatch.  2048 weight rows of scales 4 MiB apart, 128 activation rows 64 MiB apart: byte offsets up to 2^33."""
+    from catccos_amd import ops
+    k, rng = 512, np.random.default_rng(m)
+    aq, asc, bq, bsc = _operands(rng, m, n, k, "E4M3")
+    a, a_s, b, b_s = dev(aq), dev(asc), dev(bq), dev(bsc)
+    want = ops.mx_gemm(a, a_s, b, b_s, k, "E4M3", "fp32")
+    near = b_s if far == "weights" else a_s
+    apart = torch.empty((near.shape[0], 2 ** 33 // near.shape[0]), dtype=torch.uint8, device="cuda")[:, :near.shape[1]]
+    apart.copy_(near)
+    assert torch.equal(ops.mx_gemm(a, a_s if far == "weights" else apart, b, apart if far == "weights" else b_s, k, "E4M3", "fp32"), want)
+
+
 @pytest.mark.parametrize("tm", [128, 192, 256])
 @pytest.mark.parametrize("k", [384, 1152, 8832])
 def test_scale_rows_at_any_byte(tm, k):
