@@ -25,7 +25,7 @@
 #include "group_tables.h"
 #include "mx_gemm_common.h"
 #include "mx_gemm_ksplit.h"
-#include "mx_gemm_ring.h"
+#include "mx_gemm_ring_tile.h"
 #include "mx_launch.h"
 
 namespace cmx {
@@ -586,7 +586,7 @@ typedef __attribute__((address_space(3))) void* lds_void_ptr;
 typedef const __attribute__((address_space(1))) void* global_void_ptr;
 
 template <int FMT, int TW, int TM, int WW, int WM, int EPI>
-__global__ __launch_bounds__(64 * WW * WM) void mx_gemm_dl_kernel(const GemmParams p) {
+__device__ __forceinline__ void dl_tile(const GemmParams& p, const Tile& tc) {
     constexpr int NW = WW * WM;                        // wavefronts: 4 (one per SIMD) or 8 (two per SIMD)
     static_assert(NW == 4 || NW == 8, "four or eight wavefronts per workgroup");
     constexpr bool kFp4 = FMT == CMX_FMT_E2M1;
@@ -616,8 +616,6 @@ __global__ __launch_bounds__(64 * WW * WM) void mx_gemm_dl_kernel(const GemmPara
     const uint32_t ww = wave % WW, wm = wave / WW;
     const uint32_t l32 = lane & 31u, lh = lane >> 5;
 
-    Tile tc;
-    if (!locate_tile<TM>(p, tc)) return;
     const uint32_t g = __builtin_amdgcn_readfirstlane(tc.g), wt = __builtin_amdgcn_readfirstlane(tc.wt);
     const uint32_t row0 = __builtin_amdgcn_readfirstlane(tc.row0);
     const uint32_t rows_valid = __builtin_amdgcn_readfirstlane(tc.rows_valid);
@@ -804,9 +802,59 @@ __global__ __launch_bounds__(64 * WW * WM) void mx_gemm_dl_kernel(const GemmPara
     epilogue<TW, TM, WW, WM, EPI, FW, FM>(p, tc, acc, ww, wm, lane);
 }
 
+template <int FMT, int TW, int TM, int WW, int WM, int EPI>
+__global__ __launch_bounds__(64 * WW * WM) void mx_gemm_dl_kernel(const GemmParams p) {
+    Tile tc;
+    if (!locate_tile<TM>(p, tc)) return;
+    dl_tile<FMT, TW, TM, WW, WM, EPI>(p, tc);
+}
+
 #include "mx_gemm_pipe.h"
 #include "mx_gemm_wreg.h"
 #include "mx_gemm_pipe_fp4.h"
+
+// INT8 groups of up to 128 rows on average (but one round of 128 x 128 tiles): 256 x 128 tiles of the ring kernel, or 256 x 256 ones.
+// What decides is the number of rounds, of a workgroup per CU, that each takes, and with it how the rows lie, which the host does not
+// know: a round of the ring's tiles is the shorter one by an eighth (K = 2048) to a quarter (K >= 4096), but where groups are a little longer
+// than 128 rows, or few of them hold all rows, it takes two for one.  So each workgroup counts both from the sizes.  Both sides
+// in one kernel (the ring takes four of its eight wavefronts): two launches, of which one finds nothing to do, cost 3-6 us more.  One scan of
+// the sizes for the count and the tile is no gain: the ring's loop then comes out slower (64 x 48 rows u, 7168, 2048 212 us against 183).
+// Measured (us, fp32 output, 256 x 256 alone / 256 x 128 alone / the choice; u: routes drawn uniformly, z: Zipf, c: all rows on four groups):
+//   K, N, groups x rows      u               z               c
+//   7168, 4096, 32 x 90      232 195 201     293 227 224      87 116  85
+//   7168, 4096, 32 x 112     240 250 240     306 233 231     104 122 105
+//   7168, 3072, 16 x 118     108  88  89     109 123 106      76  56  56
+//   4096, 4096, 32 x 90      157 148 151     186 156 156      57  81  54
+//   2048, 2048, 32 x 112      48  70  48      78  63  62      35  32  31
+//   1024, 4096, 32 x 72       59  53  55      70  60  63      27  42  25
+//   4096, 4096, 64 x 112     314 292 300     345 321 347     128 166 126     (8 rounds: a choice at the start of each)
+// (p.sizes; cus: workgroups that run at a time.)
+__device__ __forceinline__ bool short_tiles_pay(const GemmParams& p, uint32_t cus) {
+    uint32_t off[kGroupsPerLane + 1], n128 = 0, n256 = 0;
+    scan_group_rows(p, off);
+#pragma unroll
+    for (int j = 0; j < kGroupsPerLane; ++j) {
+        n128 += tiles_of_group(p, off[j + 1] - off[j], 128);
+        n256 += tiles_of_group(p, off[j + 1] - off[j], 256);
+    }
+    const auto add = [](uint32_t a, uint32_t b) -> uint32_t { return a + b; };
+    const uint32_t t128 = (uint32_t)__builtin_amdgcn_readlane((int)wave_scan(n128, add), 63) * p.w_tiles;
+    const uint32_t t256 = (uint32_t)__builtin_amdgcn_readlane((int)wave_scan(n256, add), 63) * p.w_tiles;
+    const uint32_t r128 = (t128 + cus - 1) / cus, r256 = (t256 + cus - 1) / cus;
+    return p.kblocks >= 128 ? 3 * r128 <= 4 * r256 : 7 * r128 <= 8 * r256;
+}
+constexpr size_t kI8ChoiceLds = 3 * (256 + 128) * kSlabBytes;           // the ring's slots; its sums and the two slots of the other are less
+static_assert(ring_lds_bytes(256, 128, 3, 0) <= kI8ChoiceLds && 2 * (256 + 256) * (kSlabBytes + 4) <= kI8ChoiceLds, "LDS");
+__global__ __launch_bounds__(512) void mx_gemm_i8_choice_kernel(const GemmParams p, const uint32_t cus) {
+    Tile tc;
+    if (__builtin_amdgcn_readfirstlane((int)short_tiles_pay(p, cus))) {
+        if (threadIdx.x >= 256 || !locate_tile_by_sizes<128>(p, tc)) return;
+        ring_tile<kFmtI8, 256, 128, 2, 2, 3, 0, kEpiI8DequantSwiglu, false>(p, tc);
+    } else {
+        if (!locate_tile_by_sizes<256>(p, tc)) return;
+        dl_tile<kFmtI8, 256, 256, 2, 4, kEpiI8DequantSwiglu>(p, tc);
+    }
+}
 
 __global__ __launch_bounds__(256) void gmm_prepare_kernel(const GroupTablesJob job) { fill_group_tables(job); }
 
@@ -832,6 +880,17 @@ int launch_gemm_dl(const GemmParams& p, uint32_t max_m_tiles, hipStream_t s) {
     const uint64_t tiles = (uint64_t)max_m_tiles * p.w_tiles;
     CMX_REQUIRE(tiles > 0 && tiles < (1ull << 31), "tile count out of range");
     hipLaunchKernelGGL(kfn, dim3((uint32_t)tiles), dim3(64 * WW * WM), smem, s, p);
+    CMX_LAUNCH_CHECK();
+    return CMX_OK;
+}
+
+int launch_i8_choice(const GemmParams& p, uint32_t max_m_tiles, hipStream_t s) {
+    if (int rc = allow_dynamic_lds<mx_gemm_i8_choice_kernel, kI8ChoiceLds>(); rc != CMX_OK) return rc;
+    const uint64_t tiles = (uint64_t)max_m_tiles * p.w_tiles;
+    CMX_REQUIRE(tiles > 0 && tiles < (1ull << 31), "tile count out of range");
+    int cus = 0;
+    if (int rc = cu_count(&cus); rc != CMX_OK) return rc;
+    hipLaunchKernelGGL(mx_gemm_i8_choice_kernel, dim3((uint32_t)tiles), dim3(512), kI8ChoiceLds, s, p, (uint32_t)cus);
     CMX_LAUNCH_CHECK();
     return CMX_OK;
 }
@@ -1035,6 +1094,9 @@ constexpr uint32_t kSmallGroupRows = 64;               // one m-tile of the 64 x
 //   32 experts, 512 rows on 1       57    42    40      84    37    36      77    40    39
 //   32 experts, 1024 rows on 4      59    82    55      85    78    50      75    79    54
 //   32 experts, 1280 rows on 4      56    69    59      91    60    92      78    66    81
+// (256-row kernel: the three-slot 256 x 128 kernel for E4M3 SwiGLU, 256 x 256 tiles for INT8.  Since ring_groups has put the ring's tiles in their
+// place the rule's column reads, E4M3 SwiGLU and INT8: 32 on average, Zipf 1315 and 1318; 8192 rows on 8 experts 256 and 226, 2048 on 2 69 and 85;
+// 32 experts, 512 rows on 1 37 and 37, 1024 on 4 53 and 50, 1280 on 4 53 and 60.)
 // The empty one of the two launches costs 2-6 us.  A limit of 32 or 40 rows instead of 64: 1360 or 1308 against 1214 (random), 1349 or
 // 1298 against 1352 (Zipf).  8-bit problems whose K is no whole number of slabs go by size only past the 2048 tiles up to which the
 // split-K kernel beats the register-staged one (choose_ksplit).  Row-major and pre-tiled weights go by one rule, because they
@@ -1375,13 +1437,16 @@ uint32_t max_group_tiles(uint32_t m_total, uint32_t groups, uint32_t tile_m, uin
 //                8 x 100 u, 4096, 2048                       35.7 -> 25.0 / 40.1 -> 25.4    16 x 64 z, 7168, 1024   56.8 -> 36.8 / 61.5 -> 36.7
 //   256 x 128    32 x 100 u, 7168, 4096                      206 -> 190 / 221 -> 204        32 x 128 z   320 -> 279 / 327 -> 284
 //                16 x 100 u, 2048, 2048                      23.4 against 24.0 / 28.2 -> 25.2, so not for SwiGLU at K below 3072 (at 1152
-//                22.6 against 24.2); 32 x 128 z, 4096, 1024 42.5 against 46.3 / 47.1 -> 47.1 is the most that this line loses
+//                22.6 against 24.2); 32 x 128 z, 4096, 1024 57.0 -> 48.6 / 47.1 -> 47.1.  The most that this line loses: 64 x 64 u, 3072, 1024 40.4
+//                against 42.3 with weights in the memory-side cache; store 64 x 40 u, 1024, 4096 74.8 against 78.3
 //   128 x 256    8 x 200 u, 4096, 2048                       45.9 -> 34.5 / 43.1 -> 35.7    16 x 300 u, 7168, 1024   74 -> 57 / 69 -> 62
 //                8 x 500 u, 1024, 1024                       22.6 -> 18.6 / 20.0 against 19.9, so not for a store at K below 2048
 // Problems of more tiles stay on the persistent kernels (32 x 194 rows, 7168, 4096: 287 against 311 with 128 x 256).
 // INT8, whose only other kernel has 256 x 256 tiles, one per workgroup (us, fp32 output):
 //   128 x 128    8 x 44 u, 4096, 2048 46.5 -> 21.6     8 x 200 u 47.7 -> 27.0     16 x 100 z, 7168, 1024 73.2 -> 34.8     16 x 44 u, 2048, 2048 29.7 -> 16.9
-//   256 x 128    32 x 44 u, 7168, 4096 222 -> 178       32 x 100 z 299 -> 232      32 x 100 z, 1152, 2048 46.3 -> 37.3
+//   256 x 128    32 x 44 u, 7168, 4096 222 -> 178       32 x 100 z 299 -> 232      32 x 100 z, 1152, 2048 46.3 -> 37.3: where the device chooses it
+//                (mx_gemm_i8_choice_kernel); not for more than 96 rows on average at K below 2048: 32 x 112, 1024, 4096 58 against 75 u, 73 against 71
+//                z, 28 against 47 on four groups, 64 x 100 112 against 111, 126 against 122, 53 against 87
 //   128 x 256    16 x 200 u, 7168, 1024 71.8 -> 50.9; of more than a round 32 x 200 u, 7168, 4096 278 against 251, 16 x 2048 1077 against 1003
 // FP4, whose other kernels past the split-K sizes have tiles of 256 x 128 and 256 x 256 (us, bf16 output):
 //   128 x 128    8 x 70 u, 4096, 2048 31.6 -> 15.9     8 x 200 u 36.0 -> 18.4     16 x 100 z, 7168, 1024 46.9 -> 24.1     8 x 70 u, 7168, 4096 49 -> 26
@@ -1394,7 +1459,7 @@ int ring_groups(TileChoice* t, uint32_t m_total, uint32_t groups, uint32_t n, in
     if (int rc = cu_count(&cus); rc != CMX_OK) return rc;
     const uint64_t w128 = ceil_div(n, 128);
     if (w128 * (m_total / 128 + groups) <= (uint64_t)cus) *t = {128, 128, kRing};
-    else if (t->tm <= 128 && (!swiglu || kblocks >= 96 || !eight_bit)) *t = {256, 128, kRing};
+    else if (t->tm <= 128 && (fmt == kFmtI8 ? kblocks >= 64 || ceil_div(m_total, groups) <= 96 : !swiglu || kblocks >= 96 || !eight_bit)) *t = {256, 128, kRing};
     else if (t->tm == 256 && w128 * (m_total / 256 + groups * 3 / 4) <= (uint64_t)cus && (swiglu || kblocks >= 64 || !eight_bit)) *t = {128, 256, kRing};
     return CMX_OK;
 }
@@ -1561,19 +1626,31 @@ extern "C" int cmx_int8_gmm_dequant_swiglu(const int8_t* a, uint32_t lda, const 
     if (int rc = choose_grouped_ksplit(m_total, groups, n, kFmtI8, p.kblocks, &ks); rc != CMX_OK) return rc;
     const bool all_ksplit = ks.tile.fw != 0 && ks.small_rows == 0;
     TileChoice t = {256, ceil_div(m_total, groups) <= 128 ? 128 : 256, 8};
+    bool choice = false;                                       // 128- or 256-row tiles: the device chooses by the sizes
     if (g_force_tile.waves == kRing) t = g_force_tile;
-    else if (!g_force_tile.tw && !g_disable_dl)
+    else if (!g_force_tile.tw && !g_disable_dl) {
         if (int rc = ring_groups(&t, m_total, groups, n, kFmtI8, p.kblocks, true); rc != CMX_OK) return rc;
+        choice = !all_ksplit && t.waves == kRing && t.tw == 256;
+    }
     if (t.waves != kRing) t.tm = 256;
+    // All kernels of the call take one tile per workgroup.  The choice goes by the sizes up to eight rounds; past them the 256 x 128 tiles lead
+    // on most loads (256 x 90 rows, 2048, 2048: 293 against 325 u, 330 against 369 z, 171 against 120 on four groups), but where the small groups
+    // go to the split-K kernel those that are left are large for their average (256 x 32, 7168, 4096, on eight groups 227 against 277).
+    bool by_sizes = false;
+    const uint64_t most = all_ksplit ? (uint64_t)(m_total / 64 + groups) * ceil_div(n, 64) : (uint64_t)(m_total / t.tm + groups) * ceil_div(n, t.tw);
+    if (int rc = tiles_by_sizes(&by_sizes, groups, choice && ks.small_rows == 0 ? most * 6 / 8 : most, all_ksplit ? 2 : 1); rc != CMX_OK) return rc;
+    if (choice && !by_sizes) {
+        choice = false;
+        if (ks.small_rows != 0) t = {256, 256, 8};
+    }
     const GroupTables tables(ws, groups);
     const uint32_t tile_m = all_ksplit ? 16 * ks.tile.fm : t.tm;
-    bool by_sizes = false;                                     // (all its kernels take one tile per workgroup)
-    if (int rc = tiles_by_sizes(&by_sizes, groups, (uint64_t)(m_total / tile_m + groups) * ceil_div(n, all_ksplit ? 64 : t.tw), all_ksplit ? 2 : 1); rc != CMX_OK) return rc;
     if (int rc = prepare_groups(p, tables_job(tables, group_sizes, groups, m_total, tile_m, ks.small_rows), by_sizes, false, s); rc != CMX_OK) return rc;
     if (ks.tile.fw != 0)
         if (int rc = launch_grouped_ksplit(p, tables, ks, kFmtI8, kEpiI8DequantSwiglu, m_total, s); rc != CMX_OK || all_ksplit) return rc;
     p.w_tiles = ceil_div(n / 2, t.tw / 2);
     const uint32_t max_m_tiles = max_group_tiles(m_total, groups, t.tm, ks.small_rows);
+    if (choice) return launch_i8_choice(p, max_m_tiles, s);
     if (t.waves == kRing) return launch_ring(p, {t.tw, t.tm}, kFmtI8, kEpiI8DequantSwiglu, false, max_m_tiles, s);
     // (hand-scheduled variants of this kernel were measured twice at 16 x 2048 x 7168 x 4096 and are not kept: two i8
     // MFMAs per step and accumulator in the 8-bit schedule 997 us, one per 32-K step in the 16-byte-fragment

@@ -218,29 +218,39 @@ __device__ __forceinline__ uint32_t wave_scan(uint32_t v, Op op) {
 // The tile of this workgroup from the group sizes themselves: every wavefront scans them (four groups per lane), so that no launch has to
 // write tables first (5 us) and no chain of dependent table reads follows the start of every workgroup.  Sizes are clipped as in
 // fill_group_tables: negative ones count as zero, rows past m_total (p.m) do not exist (a sum that stops at m_total is associative).
-template <int TM>
-__device__ __forceinline__ bool locate_tile_by_sizes(const GemmParams& p, Tile& t) {
-    constexpr int kPer = kInlineGroups / 64;
+constexpr int kGroupsPerLane = kInlineGroups / 64;
+// off[0 .. kGroupsPerLane]: where the rows of the lane's groups begin, and where the last of them ends
+__device__ __forceinline__ void scan_group_rows(const GemmParams& p, uint32_t (&off)[kGroupsPerLane + 1]) {
     const uint32_t lane = threadIdx.x & 63u, m = p.m;
     const auto sat = [m](uint32_t a, uint32_t b) -> uint32_t { return min(a + b, m); };          // a, b <= m < 2^31
-    uint32_t c[kPer], sum = 0;
+    uint32_t c[kGroupsPerLane], sum = 0;
 #pragma unroll
-    for (int j = 0; j < kPer; ++j) {
-        const uint32_t i = kPer * lane + j;
+    for (int j = 0; j < kGroupsPerLane; ++j) {
+        const uint32_t i = kGroupsPerLane * lane + j;
         const int32_t v = i < p.groups ? p.sizes[i] : 0;
         c[j] = v > 0 ? min((uint32_t)v, m) : 0u;
         sum = sat(sum, c[j]);
     }
     const uint32_t to = wave_scan(sum, sat);
-    uint32_t off[kPer + 1], tiles[kPer], all = 0;
     off[0] = (uint32_t)__shfl_up((int)to, 1);
     if (lane == 0) off[0] = 0;
 #pragma unroll
+    for (int j = 0; j < kGroupsPerLane; ++j) off[j + 1] = sat(off[j], c[j]);
+}
+// m-tiles of tm rows that the launch makes of a group
+__device__ __forceinline__ uint32_t tiles_of_group(const GemmParams& p, uint32_t rows, uint32_t tm) {
+    const uint32_t small = rows <= p.small_rows ? 1u : 0u, whole = (rows + tm - 1) / tm;
+    return p.group_class == kAllGroups ? whole : (p.group_class == kSmallGroups ? (rows != 0 ? small : 0u) : (small ? 0u : whole));
+}
+
+template <int TM>
+__device__ __forceinline__ bool locate_tile_by_sizes(const GemmParams& p, Tile& t) {
+    constexpr int kPer = kGroupsPerLane;
+    uint32_t off[kPer + 1], tiles[kPer], all = 0;
+    scan_group_rows(p, off);
+#pragma unroll
     for (int j = 0; j < kPer; ++j) {
-        off[j + 1] = sat(off[j], c[j]);
-        const uint32_t rows = off[j + 1] - off[j], small = rows <= p.small_rows ? 1u : 0u;
-        const uint32_t whole = (rows + TM - 1) / TM;
-        tiles[j] = p.group_class == kAllGroups ? whole : (p.group_class == kSmallGroups ? (rows != 0 ? small : 0u) : (small ? 0u : whole));
+        tiles[j] = tiles_of_group(p, off[j + 1] - off[j], TM);
         all += tiles[j];
     }
     const uint32_t pref = wave_scan(all, [](uint32_t a, uint32_t b) -> uint32_t { return a + b; });

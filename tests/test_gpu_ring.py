@@ -195,6 +195,32 @@ def test_grouped_int8_gives_the_bits_of_the_256_row_kernel(tile, out, counts, n,
     assert torch.equal(ops.int8_gmm_dequant_swiglu(*args), want)
 
 
+@pytest.mark.parametrize("counts,rows,n,k", [
+    ([110] * 20, 2200, 4096, 128),                                     # K < 2048, more than 96 rows each: 256 x 256 tiles without a choice
+    ([90] * 20, 1800, 4096, 128),                                      # the choice: two rounds of either, the ring's
+    ([1700, 0, 0, 90] + [3] * 16, 1838, 4096, 128),                    # two rounds of the ring's, one of the others'
+    ([100, 0, 130, 120] * 8, 2800, 2048, 2048),                        # the same by groups of a little more than 128 rows
+    ([2 ** 31 - 1, -4, 7, 2 ** 31 - 1] + [9] * 16, 1900, 4096, 128),   # sizes past the rows that there are, negative ones
+    ([128, 129] * 9, 2313, 3072, 4096),                                # K >= 4096
+    ([1100, 0, 64, 65, 1, 800, 33, 200] + [0] * 52, 2263, 4096, 128),  # small groups to split-K, the choice for the others
+    ([1, 200, 64, 65] * 64, 21120 - 9, 2048, 128),                     # more than eight rounds: tables, the ring's tiles
+    ([60, 70, 129, 5] * 75, 19800, 1024, 128)])                        # more groups than a scan takes: tables, the ring's tiles
+def test_chosen_int8_kernels(counts, rows, n, k):
+    """Whatever of the 256 x 128 and 256 x 256 tiles the host or the device takes: one result, that of the 256-row kernel alone."""
+    from catccos_amd import ops
+    g = torch.Generator(device="cuda")
+    g.manual_seed(rows)
+    e = len(counts)
+    a = torch.randint(-127, 128, (rows, k), dtype=torch.int8, device="cuda", generator=g)
+    w = torch.randint(-127, 128, (e, n, k), dtype=torch.int8, device="cuda", generator=g)
+    channel, token = torch.rand(e * n, device="cuda", generator=g) * 1e-4, torch.rand(rows, device="cuda", generator=g)
+    args = (a, token, w, channel, dev(np.array(counts, dtype=np.int32)), n, k, 1)
+    chosen = ops.int8_gmm_dequant_swiglu(*args)
+    hooks_lib().cmx_debug_force_ksplit(-1, 0, 0)
+    hooks_lib().cmx_debug_force_tile(256, 256, 8)
+    assert torch.equal(ops.int8_gmm_dequant_swiglu(*args), chosen) and chosen.abs().max() > 0
+
+
 @pytest.mark.parametrize("kernel", ["ring", "split-K", "INT8"])
 @pytest.mark.parametrize("sizes,rows", [([5, -3, 0, 70, 1], 76), ([40, 2 ** 31 - 1, 2 ** 31 - 1, 9], 300), ([0, 0, 0], 10), ([1] * 256, 256),
                                         ([3, 0, 66, 1] * 64, 4300), ([2 ** 31 - 1] * 256, 130)])
