@@ -1331,9 +1331,15 @@ namespace {
 // with the pass -> as they lie): 16 x 4096 x 7168 26.3 -> 19.2, 64 28.5 -> 18.3, 256 36.1 -> 23.5, 512 46.7 -> 33.9; 16 x 8192 x 512 9.6 -> 5.1;
 // 16 x 7168 x 2048 16.4 -> 9.3; 64 x 2052 x 2048 13.1 -> 8.4; 64 x 512 x 4096 11.1 -> 8.3; 64 x 2048 x 8192 22.0 -> 16.3; but 64 x 1024 x 8192 13.0
 // against 17.3, 64 x 512 x 8192 13.4 against 17.3, 700 x 1536 x 8192 37 against 46.
-bool k_slow_pays(uint32_t n, uint32_t k) {
+// `ks`: the tile on K-contiguous weights.  Two lines inside of that: tiles of 16 columns x 32 rows that fill three quarters of the CUs are hard to beat
+// behind a short pass (100 x 1024 at K = 3584 10.1 against 11.2, 4096 10.4 against 12.9, but 100 x 768 x 4096, 192 tiles, 11.9 -> 11.5), and past
+// K = 7168 the scales of a 64 x 64 tile leave room for one workgroup per CU instead of two (K = 8192, 700 x 2048 41.1 against 41.7,
+// 400 x 2560 40.8 against 45.4, 700 x 2816 45.5 -> 43.3, 700 x 4096 66 -> 39).
+bool k_slow_pays(uint32_t m, uint32_t n, uint32_t k, const KsplitTile& ks, int cus) {
     KsplitTile t;
-    return k <= 4096 || (uint64_t)n * k >= (16u << 20) || ksplit_is_forced(&t);
+    if (ksplit_is_forced(&t)) return true;
+    if (k <= 4096) return !(k > 3328 && ks.fw == 1 && ks.fm == 2 && (uint64_t)ceil_div(n, 16) * ceil_div(m, 32) * 4 > 3 * (uint64_t)cus);
+    return (uint64_t)n * k >= (k > 7168 && ks.waves == 4 ? 22u << 20 : 16u << 20);
 }
 }  // namespace
 }  // namespace cmx
@@ -1353,7 +1359,7 @@ int cmx::gemm_k_slow(const uint8_t* a, const uint8_t* a_scale, const uint8_t* b,
     if (int rc = choose_ksplit(m, n, fmt, k / 32, &ks); rc != CMX_OK) return rc;
     int tm = 0;
     if (ks.fw != 0) {
-        if (!k_slow_pays(n, k) || !ksplit_k_slow_tile(&ks, m, n, fmt, k / 32, cus)) return CMX_OK;
+        if (!k_slow_pays(m, n, k, ks, cus) || !ksplit_k_slow_tile(&ks, m, n, fmt, k / 32, cus)) return CMX_OK;
     } else {
         tm = g_force_tile.waves == kRing ? g_force_tile.tm : (g_force_tile.tw || g_disable_dl ? 0 : ring_rows(m, n, fmt, k / 32, cus, true));
         if (tm == 0) return CMX_OK;

@@ -138,6 +138,19 @@ def test_grouped_problems_give_the_bits_of_the_256_row_kernels(tile, counts, n, 
     assert bool((want[-1][m:].float() == 7.0).all())
 
 
+@pytest.mark.parametrize("m,n,k", [(100, 1024, 3328), (100, 1024, 3456), (100, 768, 4096), (65, 2560, 8192), (300, 2816, 8192), (300, 2752, 8192), (600, 2368, 7168)])
+def test_both_sides_of_the_k_slow_lines(m, n, k):
+    """Default dispatch of split-K problems, weights read as they lie or behind the pass: the bits of K-contiguous weights."""
+    from catccos_amd import ops
+    g = torch.Generator(device="cuda")
+    g.manual_seed(n)
+    codes = lambda *shape: torch.randint(0, 0x70, shape, dtype=torch.uint8, device="cuda", generator=g)
+    scales = lambda *shape: torch.randint(110, 125, shape, dtype=torch.uint8, device="cuda", generator=g)
+    a, a_s, b, b_s = codes(m, k), scales(m, k // 32), codes(n, k), scales(n, k // 32)
+    got = ops.mx_gemm_ex(a, a_s, b.t().contiguous(), b_s.view(n, k // 64, 2).permute(1, 0, 2).contiguous(), m, n, k, "E4M3", "fp32", trans_b=0)
+    assert torch.equal(got, ops.mx_gemm(a, a_s, b, b_s, k, "E4M3", "fp32"))
+
+
 @pytest.mark.parametrize("experts,avg,n,k", [(8, 100, 1024, 1024), (16, 100, 2048, 3072), (8, 200, 2048, 1024), (16, 100, 2048, 1024)])
 def test_chosen_grouped_kernels(experts, avg, n, k):
     """Averages that take each of the ring tiles, and one that stays: the bits of the 256-row kernel either way."""
