@@ -328,8 +328,10 @@ __global__ __launch_bounds__(256) void quant_scatter_kernel(const uint16_t* __re
 // Bound: the read of the destinations from the L2 (routes * 4 bytes) by every workgroup, of which there are 256, or more where
 // 256 times kUnmappedRows rows (16.7 million) are not enough.  It stands in for a fill of the whole output before the
 // scatter (32768 x 7168 bytes of codes 36 us) and runs beside the scatter, which writes the other rows (as a launch of its own behind it, 6
-// us, half of them the launch).
-constexpr uint32_t kUnmappedRows = 65536;
+// us, half of them the launch).  A launch of its own has the chip to itself and takes four times the threads, with half the
+// loads each (with the 256 and 16 of a workgroup beside the scatter, scatter and clearing of 28356 x 448, top 4, 52.7 against 28.7; of 4 x 192,
+// top 2, 4.3 against 3.5).
+constexpr uint32_t kUnmappedRows = 65536, kUnmappedThreads = 1024;
 
 struct ZeroJob {
     uint32_t blocks;                 // workgroups of the launch that do this; 0: none
@@ -340,7 +342,7 @@ ZeroJob zero_job(uint32_t rows, uint32_t k) {
     return {ceil_div(rows, per), rows, per, k / 16, scale_cols(k)};
 }
 
-template <uint32_t THREADS>
+template <uint32_t THREADS, uint32_t BATCH>
 __device__ __forceinline__ void zero_unmapped_rows(const ZeroJob& z, uint32_t block, const int32_t* __restrict__ src2sorted,
                                                    uint8_t* __restrict__ out_codes, uint32_t ld_out, uint8_t* __restrict__ out_scales,
                                                    uint32_t ld_outs) {
@@ -348,15 +350,15 @@ __device__ __forceinline__ void zero_unmapped_rows(const ZeroJob& z, uint32_t bl
     const uint32_t r0 = block * z.per, n = min(z.per, z.rows - r0), words = (n + 31) / 32;
     for (uint32_t i = threadIdx.x; i < words; i += THREADS) s_map[i] = 0;
     __syncthreads();
-    for (uint32_t i0 = 0; i0 < z.rows; i0 += 16 * THREADS) {                         // one route per row
-        int32_t d[16];
+    for (uint32_t i0 = 0; i0 < z.rows; i0 += BATCH * THREADS) {                         // one route per row
+        int32_t d[BATCH];
 #pragma unroll
-        for (uint32_t j = 0; j < 16; ++j) {
+        for (uint32_t j = 0; j < BATCH; ++j) {
             const uint32_t i = i0 + j * THREADS + threadIdx.x;
             d[j] = i < z.rows ? src2sorted[i] : -1;
         }
 #pragma unroll
-        for (uint32_t j = 0; j < 16; ++j) {
+        for (uint32_t j = 0; j < BATCH; ++j) {
             const uint32_t r = (uint32_t)d[j] - r0;                                  // dropped routes are negative: far above n
             if (d[j] >= 0 && r < n) atomicOr(&s_map[r / 32], 1u << (r % 32));
         }
@@ -375,10 +377,10 @@ __device__ __forceinline__ void zero_unmapped_rows(const ZeroJob& z, uint32_t bl
     }
 }
 
-__global__ __launch_bounds__(256) void zero_unmapped_rows_kernel(const ZeroJob z, const int32_t* __restrict__ src2sorted,
-                                                                 uint8_t* __restrict__ out_codes, uint32_t ld_out,
-                                                                 uint8_t* __restrict__ out_scales, uint32_t ld_outs) {
-    zero_unmapped_rows<256>(z, blockIdx.x, src2sorted, out_codes, ld_out, out_scales, ld_outs);
+__global__ __launch_bounds__(kUnmappedThreads) void zero_unmapped_rows_kernel(const ZeroJob z, const int32_t* __restrict__ src2sorted,
+                                                                              uint8_t* __restrict__ out_codes, uint32_t ld_out,
+                                                                              uint8_t* __restrict__ out_scales, uint32_t ld_outs) {
+    zero_unmapped_rows<kUnmappedThreads, 8>(z, blockIdx.x, src2sorted, out_codes, ld_out, out_scales, ld_outs);
 }
 
 // What the first workgroups of a quantise + scatter launch do beside it, having nothing to do with its rows: `tables` of them fill the
@@ -402,7 +404,7 @@ __global__ __launch_bounds__(256) void quant_scatter_row_kernel(const uint16_t* 
     const uint32_t extras = ex.tables + ex.zero.blocks;
     if (blockIdx.x < extras) {
         if (blockIdx.x < ex.tables) fill_group_tables(ex.job[blockIdx.x]);
-        else zero_unmapped_rows<256>(ex.zero, blockIdx.x - ex.tables, src2sorted, out_codes, ld_out, out_scales, ld_outs);
+        else zero_unmapped_rows<256, 16>(ex.zero, blockIdx.x - ex.tables, src2sorted, out_codes, ld_out, out_scales, ld_outs);
         return;
     }
     const uint32_t row = blockIdx.x - extras, h = threadIdx.x & 1u;
@@ -720,7 +722,7 @@ int launch_extras(const ScatterExtras& ex, const int32_t* src2sorted, uint8_t* o
     for (uint32_t i = 0; i < ex.tables; ++i)
         if (int rc = launch_group_tables(ex.job[i], s); rc != CMX_OK) return rc;
     if (ex.zero.blocks != 0) {
-        hipLaunchKernelGGL(zero_unmapped_rows_kernel, dim3(ex.zero.blocks), dim3(256), 0, s, ex.zero, src2sorted, out_codes, ld_out, out_scales, ld_outs);
+        hipLaunchKernelGGL(zero_unmapped_rows_kernel, dim3(ex.zero.blocks), dim3(kUnmappedThreads), 0, s, ex.zero, src2sorted, out_codes, ld_out, out_scales, ld_outs);
         CMX_LAUNCH_CHECK();
     }
     return CMX_OK;
