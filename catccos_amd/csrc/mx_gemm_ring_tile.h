@@ -318,6 +318,20 @@ __device__ __forceinline__ void ring_tile(const GemmParams& p, Tile tc) {
     // ---- epilogue: sums through the LDS, whole rows to memory ----------------------------------------------------------------
     constexpr uint32_t kPitch = TW + 4;
     float* const sums = reinterpret_cast<float*>(smem);
+    constexpr uint32_t kQuads = epi_pairs_gate_up(EPI) ? TW / 8 : TW / 4;
+    // INT8: a thread keeps its columns from row to row, so their scales and those of its rows are requested once and up front.  Between
+    // the stores, which the compiler cannot tell from them, every row would wait for nine loads of its own (256 x 128 tiles, us: 32 groups x 90
+    // rows, K = 128, N = 1024, one round, 16.6 -> 10.3; 256 x 48, four rounds, 43.2 -> 31.8, at K = 1024 81.1 -> 70.6).
+    constexpr int kTurns = EPI == kEpiI8DequantSwiglu ? TM * kQuads / NT : 1;
+    static_assert(NT % kQuads == 0 && TM * kQuads % NT == 0, "whole rows a turn");
+    v4f i8_g, i8_u;
+    float i8_t[kTurns];
+    if constexpr (EPI == kEpiI8DequantSwiglu) {
+        const uint32_t ncol = tc.wt * (TW / 2) + 4 * (tid % kQuads);
+        load_channel_scales(p, tc.g, ncol < half ? ncol : half - 4, i8_g, i8_u);
+#pragma unroll
+        for (int i = 0; i < kTurns; ++i) i8_t[i] = reinterpret_cast<const float*>(p.a_scale)[tc.row0 + arow_of((i * NT + tid) / kQuads)];
+    }
     __syncthreads();
 #pragma unroll
     for (int j = 0; j < FM; ++j)
@@ -327,7 +341,17 @@ __device__ __forceinline__ void ring_tile(const GemmParams& p, Tile tc) {
             for (int q = 0; q < 4; ++q)
                 *reinterpret_cast<v4f*>(sums + (wm * (TM / WM) + j * 32 + l32) * kPitch + wfrag_row(i) + 8 * q + 4 * lh) = to_v4(acc[i][j], q);
     __syncthreads();
-    constexpr uint32_t kQuads = epi_pairs_gate_up(EPI) ? TW / 8 : TW / 4;
+    if constexpr (EPI == kEpiI8DequantSwiglu) {
+        const uint32_t q = tid % kQuads, ncol = tc.wt * (TW / 2) + 4 * q;
+#pragma unroll
+        for (int i = 0; i < kTurns; ++i) {
+            const uint32_t m = (i * NT + tid) / kQuads;
+            if (m >= tc.rows_valid || ncol >= half) continue;
+            store_i8_quad(p, (size_t)(tc.row0 + m), ncol, *reinterpret_cast<const v4f*>(sums + m * kPitch + 4 * q),
+                          *reinterpret_cast<const v4f*>(sums + m * kPitch + TW / 2 + 4 * q), i8_g, i8_u, i8_t[i]);
+        }
+        return;
+    }
 #pragma unroll 4
     for (uint32_t it = tid; it < TM * kQuads; it += NT) {
         const uint32_t m = it / kQuads, q = it % kQuads;

@@ -7,6 +7,48 @@ namespace cmx {
 
 #if defined(__HIPCC__)
 
+// channel scales of four gate columns from ncol on and of their up partners (ncol + 4 <= n / 2)
+__device__ __forceinline__ void load_channel_scales(const GemmParams& p, uint32_t g, uint32_t ncol, v4f& cg, v4f& cu) {
+    const float* ch = reinterpret_cast<const float*>(p.w_scale) + (size_t)g * p.n * p.ld_ws;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        cg[i] = ch[(size_t)(ncol + i) * p.ld_ws];
+        cu[i] = ch[(size_t)((p.n >> 1) + ncol + i) * p.ld_ws];
+    }
+}
+
+// INT32 sums of four gate and up columns -> fp32 * per-channel scale -> fp16 -> fp32 * per-token scale -> x0 * sigmoid(x0) * gate
+__device__ __forceinline__ void store_i8_quad(const GemmParams& p, size_t mrow, uint32_t ncol, const v4f& v, const v4f& u, const v4f& cg,
+                                              const v4f& cu, float tsv) {
+    const v4i ig = __builtin_bit_cast(v4i, v), iu = __builtin_bit_cast(v4i, u);
+    float y[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        const float x0 = __fmul_rn(i8_dequant(ig[i], cg[i]), tsv);
+        const float gate = __fmul_rn(i8_dequant(iu[i], cu[i]), tsv);
+        y[i] = __fmul_rn(__fmul_rn(x0, __builtin_amdgcn_rcpf(1.0f + __expf(-x0))), gate);
+    }
+    if (p.out_type == CMX_OUT_FP32) {
+        float* o = reinterpret_cast<float*>(p.c) + mrow * p.ldc + ncol;
+        if ((reinterpret_cast<uintptr_t>(o) & 15u) == 0) {
+            *reinterpret_cast<float4*>(o) = make_float4(y[0], y[1], y[2], y[3]);
+        } else {
+            for (uint32_t i = 0; i < 4; ++i) o[i] = y[i];
+        }
+    } else {
+        uint16_t h[4];
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+            h[i] = p.out_type == CMX_OUT_FP16 ? __builtin_bit_cast(uint16_t, (_Float16)as_f32(y[i])) : (uint16_t)f32_to_bf16(y[i]);
+        uint16_t* o = reinterpret_cast<uint16_t*>(p.c) + mrow * p.ldc + ncol;
+        if ((reinterpret_cast<uintptr_t>(o) & 7u) == 0) {
+            *reinterpret_cast<uint2*>(o) = make_uint2(h[0] | ((uint32_t)h[1] << 16), h[2] | ((uint32_t)h[3] << 16));
+        } else {
+            for (uint32_t i = 0; i < 4; ++i) o[i] = h[i];
+        }
+    }
+}
+
 // Sums of one output row, four consecutive columns from ncol on (SwiGLU kinds: four gate columns and their up partners, ncol the
 // activation column), to memory.  SwiGLU + requant: eight neighbouring lanes hold the 32 columns of an MX block.
 template <int EPI>
@@ -42,39 +84,11 @@ __device__ __forceinline__ void store_quad(const GemmParams& p, const Tile& tc, 
             }
         }
     } else if constexpr (EPI == kEpiI8DequantSwiglu) {
-        // INT32 sums -> fp32 * per-channel scale -> fp16 -> fp32 * per-token scale -> x0 * sigmoid(x0) * gate
         const uint32_t half = p.n >> 1;
         if (!mvalid || ncol >= half) return;                      // n is a multiple of 64: four columns are in or out together
-        const float* ch = reinterpret_cast<const float*>(p.w_scale) + (size_t)tc.g * p.n * p.ld_ws;
-        const float tsv = reinterpret_cast<const float*>(p.a_scale)[mrow];
-        const v4i ig = __builtin_bit_cast(v4i, v), iu = __builtin_bit_cast(v4i, u);
-        float y[4];
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            const float cg = ch[(size_t)(ncol + i) * p.ld_ws], cu = ch[(size_t)(half + ncol + i) * p.ld_ws];
-            const float x0 = __fmul_rn(i8_dequant(ig[i], cg), tsv);
-            const float gate = __fmul_rn(i8_dequant(iu[i], cu), tsv);
-            y[i] = __fmul_rn(__fmul_rn(x0, __builtin_amdgcn_rcpf(1.0f + __expf(-x0))), gate);
-        }
-        if (p.out_type == CMX_OUT_FP32) {
-            float* o = reinterpret_cast<float*>(p.c) + mrow * p.ldc + ncol;
-            if ((reinterpret_cast<uintptr_t>(o) & 15u) == 0) {
-                *reinterpret_cast<float4*>(o) = make_float4(y[0], y[1], y[2], y[3]);
-            } else {
-                for (uint32_t i = 0; i < 4; ++i) o[i] = y[i];
-            }
-        } else {
-            uint16_t h[4];
-#pragma unroll
-            for (int i = 0; i < 4; ++i)
-                h[i] = p.out_type == CMX_OUT_FP16 ? __builtin_bit_cast(uint16_t, (_Float16)as_f32(y[i])) : (uint16_t)f32_to_bf16(y[i]);
-            uint16_t* o = reinterpret_cast<uint16_t*>(p.c) + mrow * p.ldc + ncol;
-            if ((reinterpret_cast<uintptr_t>(o) & 7u) == 0) {
-                *reinterpret_cast<uint2*>(o) = make_uint2(h[0] | ((uint32_t)h[1] << 16), h[2] | ((uint32_t)h[3] << 16));
-            } else {
-                for (uint32_t i = 0; i < 4; ++i) o[i] = h[i];
-            }
-        }
+        v4f cg, cu;
+        load_channel_scales(p, tc.g, ncol, cg, cu);
+        store_i8_quad(p, mrow, ncol, v, u, cg, cu, reinterpret_cast<const float*>(p.a_scale)[mrow]);
     } else {
         // SwiGLU on the bf16-rounded sums, bf16 again, then the MX block of 32 columns: eight neighbouring lanes hold it
         const uint32_t half = p.n >> 1;
