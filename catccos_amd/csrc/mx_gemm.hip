@@ -380,7 +380,7 @@ __global__ __launch_bounds__(64 * WW * WM) void mx_gemm_kernel(const GemmParams 
     const uint32_t ww = wave % WW, wm = wave / WW;
 
     Tile tc;
-    if (!locate_tile<TM>(p, tc)) return;
+    if (!locate_tile<TM, Locate::kTables>(p, tc)) return;
     const uint32_t g = tc.g, wt = tc.wt, row0 = tc.row0, rows_valid = tc.rows_valid;
 
     // ---- global -> LDS staging assignments -----------------------------------------------------
@@ -805,7 +805,7 @@ __device__ __forceinline__ void dl_tile(const GemmParams& p, const Tile& tc) {
 template <int FMT, int TW, int TM, int WW, int WM, int EPI>
 __global__ __launch_bounds__(64 * WW * WM) void mx_gemm_dl_kernel(const GemmParams p) {
     Tile tc;
-    if (!locate_tile<TM>(p, tc)) return;
+    if (!locate_tile<TM, FMT == kFmtI8 ? Locate::kAny : Locate::kTables>(p, tc)) return;
     dl_tile<FMT, TW, TM, WW, WM, EPI>(p, tc);
 }
 

@@ -475,11 +475,11 @@ __device__ __forceinline__ void ks_rows(const GemmParams& p, const Tile& tc, uin
     ks_tile<FMT, FW, FM, NW, EPI, LAYOUT, STREAM>(p, tc, smem);
 }
 
-template <int FMT, int FW, int FM, int NW, int EPI, int LAYOUT, KsplitWeights LOADS>
+template <int FMT, int FW, int FM, int NW, int EPI, int LAYOUT, KsplitWeights LOADS, Locate HOW>
 __global__ __launch_bounds__(64 * NW, 2) void mx_gemm_ksplit_kernel(const GemmParams p) {
     extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
     Tile tc;
-    if (!locate_tile<16 * FM, LOADS == KsplitWeights::kCached>(p, tc)) return;
+    if (!locate_tile<16 * FM, HOW>(p, tc)) return;
     tc.g = __builtin_amdgcn_readfirstlane(tc.g);
     tc.wt = __builtin_amdgcn_readfirstlane(tc.wt);
     tc.row0 = __builtin_amdgcn_readfirstlane(tc.row0);
@@ -491,9 +491,9 @@ __global__ __launch_bounds__(64 * NW, 2) void mx_gemm_ksplit_kernel(const GemmPa
     ks_rows<FMT, FW, FM, NW, EPI, LAYOUT, LOADS != KsplitWeights::kCached>(p, tc, smem);
 }
 
-template <int FMT, int FW, int FM, int NW, int EPI, int LAYOUT, KsplitWeights LOADS>
+template <int FMT, int FW, int FM, int NW, int EPI, int LAYOUT, KsplitWeights LOADS, Locate HOW>
 int launch_one(const GemmParams& p, uint32_t max_m_tiles, hipStream_t s) {
-    constexpr auto kfn = mx_gemm_ksplit_kernel<FMT, FW, FM, NW, EPI, LAYOUT, LOADS>;
+    constexpr auto kfn = mx_gemm_ksplit_kernel<FMT, FW, FM, NW, EPI, LAYOUT, LOADS, HOW>;
     if (int rc = allow_dynamic_lds<kfn, kKsplitMaxLds>(); rc != CMX_OK) return rc;
     const size_t smem = ksplit_lds_bytes({FW, FM, NW}, FMT, p.kblocks, LAYOUT);
     CMX_REQUIRE(smem <= kKsplitMaxLds, "split-K tile exceeds the LDS");
@@ -507,11 +507,13 @@ int launch_one(const GemmParams& p, uint32_t max_m_tiles, hipStream_t s) {
 // the tile shapes that exist for an element format and epilogue: one for grouped problems, all for dense ones
 template <int FMT, int EPI, int LAYOUT>
 int launch_shape(const GemmParams& p, const KsplitTile& t, uint32_t max_m_tiles, KsplitWeights loads, hipStream_t s) {
-#define CMX_KS(FW_, FM_, NW_) if (t.fw == FW_ && t.fm == FM_ && t.waves == NW_) return launch_one<FMT, FW_, FM_, NW_, EPI, LAYOUT, KsplitWeights::kCached>(p, max_m_tiles, s)
+#define CMX_KS(FW_, FM_, NW_) if (t.fw == FW_ && t.fm == FM_ && t.waves == NW_) return launch_one<FMT, FW_, FM_, NW_, EPI, LAYOUT, KsplitWeights::kCached, Locate::kDense>(p, max_m_tiles, s)
     const bool grouped = p.row_off != nullptr || p.sizes != nullptr;             // (kCached kernels know no groups)
+    constexpr KsplitWeights kS = KsplitWeights::kStreamed, kG = KsplitWeights::kByGroup;
     if constexpr (LAYOUT != kKSlow) if (t.fw == 4 && t.fm == 4 && t.waves == 4 && grouped) {
-        if (loads == KsplitWeights::kStreamed) return launch_one<FMT, 4, 4, 4, EPI, LAYOUT, KsplitWeights::kStreamed>(p, max_m_tiles, s);
-        return launch_one<FMT, 4, 4, 4, EPI, LAYOUT, KsplitWeights::kByGroup>(p, max_m_tiles, s);
+        if (p.sizes != nullptr)
+            return loads == kS ? launch_one<FMT, 4, 4, 4, EPI, LAYOUT, kS, Locate::kSizes>(p, max_m_tiles, s) : launch_one<FMT, 4, 4, 4, EPI, LAYOUT, kG, Locate::kSizes>(p, max_m_tiles, s);
+        return loads == kS ? launch_one<FMT, 4, 4, 4, EPI, LAYOUT, kS, Locate::kTables>(p, max_m_tiles, s) : launch_one<FMT, 4, 4, 4, EPI, LAYOUT, kG, Locate::kTables>(p, max_m_tiles, s);
     }
     CMX_REQUIRE(!grouped, "split-K tile of a grouped problem: 64 x 64 only");
     if constexpr (LAYOUT == kKSlow) {

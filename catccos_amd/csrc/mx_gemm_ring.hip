@@ -29,7 +29,7 @@ namespace {
 template <int FMT, int TW, int TM, int WW, int WM, int NSLOT, int SPAN, int EPI, bool KSLOW>
 __global__ __launch_bounds__(64 * WW * WM) void mx_gemm_ring_kernel(const GemmParams p) {
     Tile tc;
-    if (!locate_tile<TM>(p, tc)) return;
+    if (!locate_tile<TM, Locate::kAny>(p, tc)) return;
     ring_tile<FMT, TW, TM, WW, WM, NSLOT, SPAN, EPI, KSLOW>(p, tc);
 }
 
