@@ -2,6 +2,8 @@
 // launches of a chain can fill on the side.
 #pragma once
 
+#include <type_traits>
+
 #include "mx_gemm_common.h"
 
 namespace cmx {
@@ -20,9 +22,14 @@ struct GroupTablesJob {
 // Group sizes live on the device, so the host cannot check them: negative sizes count as zero and rows past
 // m_total (the rows the caller's buffers hold) are cut off here, so that no tile ever points outside them.
 // small_rows != 0: groups of 1 .. small_rows rows are one m-tile each of small_pref and none of tile_pref.
-__device__ __forceinline__ void fill_group_tables(const GroupTablesJob& j) {
+// With pick, the tables are for m-tiles of tile_m or of alt_tile_m rows: pick(m-tiles of the first height, of the second) says whether the
+// first, to every thread alike.
+struct NoPick {};
+template <class Pick = NoPick>
+__device__ __forceinline__ void fill_group_tables(const GroupTablesJob& j, uint32_t alt_tile_m = 0, Pick pick = {}) {
+    constexpr bool kPick = !std::is_same<Pick, NoPick>::value;
     __shared__ unsigned long long part_r[256];
-    __shared__ int32_t part_t[256], part_s[256];
+    __shared__ int32_t part_t[256], part_s[256], part_a[kPick ? 256 : 1];
     if (threadIdx.x < kXcds) j.tile_ctr[threadIdx.x] = 0;
     const uint32_t per = (j.groups + 255) / 256;
     const uint32_t lo = threadIdx.x * per < j.groups ? threadIdx.x * per : j.groups;
@@ -63,21 +70,33 @@ __device__ __forceinline__ void fill_group_tables(const GroupTablesJob& j) {
     };
     auto is_small = [&](uint32_t rows) -> bool { return rows != 0 && rows <= j.small_rows; };
     r = r_base;
-    int32_t t = 0, sm = 0;
+    int32_t t = 0, sm = 0, ta = 0;
     for (uint32_t i = lo; i < hi; ++i) {
         const unsigned long long c = size_of(i);
         const uint32_t rows = clipped(r, c);
         if (is_small(rows)) ++sm;
         else t += (int32_t)((rows + j.tile_m - 1) / j.tile_m);
+        if constexpr (kPick)
+            if (!is_small(rows)) ta += (int32_t)((rows + alt_tile_m - 1) / alt_tile_m);
         r += c;
     }
     part_t[threadIdx.x] = t;
     part_s[threadIdx.x] = sm;
+    if constexpr (kPick) part_a[threadIdx.x] = ta;
     __syncthreads();
     scan256(part_t);
     if (j.small_rows != 0) scan256(part_s);
+    const int32_t* tiles = part_t;
+    uint32_t tile_m = j.tile_m;
+    if constexpr (kPick) {
+        scan256(part_a);
+        if (!pick((uint32_t)part_t[255], (uint32_t)part_a[255])) {
+            tiles = part_a;
+            tile_m = alt_tile_m;
+        }
+    }
     r = r_base;
-    t = threadIdx.x ? part_t[threadIdx.x - 1] : 0;
+    t = threadIdx.x ? tiles[threadIdx.x - 1] : 0;
     sm = threadIdx.x ? part_s[threadIdx.x - 1] : 0;
     for (uint32_t i = lo; i < hi; ++i) {
         const unsigned long long c = size_of(i);
@@ -86,13 +105,13 @@ __device__ __forceinline__ void fill_group_tables(const GroupTablesJob& j) {
         j.tile_pref[i] = t;
         if (j.small_rows != 0) j.small_pref[i] = sm;
         if (is_small(rows)) ++sm;
-        else t += (int32_t)((rows + j.tile_m - 1) / j.tile_m);
+        else t += (int32_t)((rows + tile_m - 1) / tile_m);
         r += c;
     }
     if (threadIdx.x == 255) {
         const unsigned long long all = part_r[255];
         j.row_off[j.groups] = (int32_t)(all < j.m_total ? all : j.m_total);
-        j.tile_pref[j.groups] = part_t[255];
+        j.tile_pref[j.groups] = tiles[255];
         if (j.small_rows != 0) j.small_pref[j.groups] = part_s[255];
     }
 }

@@ -815,21 +815,26 @@ __global__ __launch_bounds__(64 * WW * WM) void mx_gemm_dl_kernel(const GemmPara
 
 // INT8 groups of up to 128 rows on average (but one round of 128 x 128 tiles): 256 x 128 tiles of the ring kernel, or 256 x 256 ones.
 // What decides is the number of rounds, of a workgroup per CU, that each takes, and with it how the rows lie, which the host does not
-// know: a round of the ring's tiles is the shorter one by an eighth (K = 2048) to a quarter (K >= 4096), but where groups are a little longer
-// than 128 rows, or few of them hold all rows, it takes two for one.  So each workgroup counts both from the sizes.  Both sides
-// in one kernel (the ring takes four of its eight wavefronts): two launches, of which one finds nothing to do, cost 3-6 us more.  One scan of
-// the sizes for the count and the tile is no gain: the ring's loop then comes out slower (64 x 48 rows u, 7168, 2048 212 us against 183).
+// know: a round of the ring's tiles takes 0.73 (K < 2048) to 0.62 of one of the others, but where groups are a little longer than 128 rows,
+// or few of them hold all rows, there are up to twice as many.  So the device counts both from the sizes: in every workgroup up to two
+// rounds, in the launch that fills the tables beyond (a count costs each tile 1 us).  A kernel for each side, the one that the choice
+// leaves out finding nothing to do (2 us): both in one kernel share its registers, and the ring's loop comes out slower by a quarter
+// (8 groups x 76 rows u, 7168, 3072 58.8 against 41.5).  Below K = 512 the launches cost more than is won (64 x 128 u, 128, 3072 42 -> 51).
 // Measured (us, fp32 output, 256 x 256 alone / 256 x 128 alone / the choice; u: routes drawn uniformly, z: Zipf, c: all rows on four groups):
 //   K, N, groups x rows      u               z               c
-//   7168, 4096, 32 x 90      232 195 201     293 227 224      87 116  85
-//   7168, 4096, 32 x 112     240 250 240     306 233 231     104 122 105
-//   7168, 3072, 16 x 118     108  88  89     109 123 106      76  56  56
-//   4096, 4096, 32 x 90      157 148 151     186 156 156      57  81  54
-//   2048, 2048, 32 x 112      48  70  48      78  63  62      35  32  31
-//   1024, 4096, 32 x 72       59  53  55      70  60  63      27  42  25
-//   4096, 4096, 64 x 112     314 292 300     345 321 347     128 166 126     (8 rounds: a choice at the start of each)
-// (p.sizes; cus: workgroups that run at a time.)
-__device__ __forceinline__ bool short_tiles_pay(const GemmParams& p, uint32_t cus) {
+//   7168, 3072, 64 x 100     335 279 285     394 333 339     180 157 162
+//   7168, 3072, 32 x 90      201 152 161     202 178 191      83  97  87
+//   4096, 3072, 64 x 128     229 226 234     263 236 240     117 134 119
+//   2048, 3072, 32 x 90       63  46  51      66  61  69      33  40  38
+//   2048, 1024, 256 x 48     156 125 129     164 126 134      37  42  43
+//   1024, 3072, 64 x 100      73  57  61      83  73  77      44  47  50
+//    512, 3072, 128 x 70     104  77  78     107  88  87      42  53  44
+// tiles of 128 and of 256 rows that a problem has; cus: workgroups that run at a time
+__device__ __forceinline__ bool short_tiles_pay(uint32_t t128, uint32_t t256, uint32_t cus, uint32_t kblocks) {
+    const uint32_t r128 = (t128 + cus - 1) / cus, r256 = (t256 + cus - 1) / cus;
+    return kblocks >= 64 ? 5 * r128 <= 8 * r256 : 8 * r128 <= 11 * r256;
+}
+__device__ __forceinline__ bool short_tiles_pay_by_sizes(const GemmParams& p, uint32_t cus) {
     uint32_t off[kGroupsPerLane + 1], n128 = 0, n256 = 0;
     scan_group_rows(p, off);
 #pragma unroll
@@ -838,22 +843,30 @@ __device__ __forceinline__ bool short_tiles_pay(const GemmParams& p, uint32_t cu
         n256 += tiles_of_group(p, off[j + 1] - off[j], 256);
     }
     const auto add = [](uint32_t a, uint32_t b) -> uint32_t { return a + b; };
-    const uint32_t t128 = (uint32_t)__builtin_amdgcn_readlane((int)wave_scan(n128, add), 63) * p.w_tiles;
-    const uint32_t t256 = (uint32_t)__builtin_amdgcn_readlane((int)wave_scan(n256, add), 63) * p.w_tiles;
-    const uint32_t r128 = (t128 + cus - 1) / cus, r256 = (t256 + cus - 1) / cus;
-    return p.kblocks >= 128 ? 3 * r128 <= 4 * r256 : 7 * r128 <= 8 * r256;
+    return short_tiles_pay((uint32_t)__builtin_amdgcn_readlane((int)wave_scan(n128, add), 63) * p.w_tiles,
+                           (uint32_t)__builtin_amdgcn_readlane((int)wave_scan(n256, add), 63) * p.w_tiles, cus, p.kblocks);
 }
-constexpr size_t kI8ChoiceLds = 3 * (256 + 128) * kSlabBytes;           // the ring's slots; its sums and the two slots of the other are less
-static_assert(ring_lds_bytes(256, 128, 3, 0) <= kI8ChoiceLds && 2 * (256 + 256) * (kSlabBytes + 4) <= kI8ChoiceLds, "LDS");
-__global__ __launch_bounds__(512) void mx_gemm_i8_choice_kernel(const GemmParams p, const uint32_t cus) {
+// One side of the choice, which is left at once where it falls on the other.  A workgroup goes on with further tiles, so that there are no
+// more of them than run at a time: leaving takes each 0.3 us (256 groups x 48 rows c, 512, 1024, a workgroup for each tile 33.9, so 26.3).
+// short_tiles: the choice, where tables of its m-tiles have been filled (i8_choice_prepare_kernel).
+template <bool SHORT>
+__global__ __launch_bounds__(SHORT ? 256 : 512) void mx_gemm_i8_choice_kernel(const GemmParams p, const uint32_t cus, const int32_t* const short_tiles) {
+    const bool pay = p.sizes != nullptr ? short_tiles_pay_by_sizes(p, cus) : table_at(short_tiles, 0) != 0;
+    if ((__builtin_amdgcn_readfirstlane((int)pay) != 0) != SHORT) return;
     Tile tc;
-    if (__builtin_amdgcn_readfirstlane((int)short_tiles_pay(p, cus))) {
-        if (threadIdx.x >= 256 || !locate_tile_by_sizes<128>(p, tc)) return;
-        ring_tile<kFmtI8, 256, 128, 2, 2, 3, 0, kEpiI8DequantSwiglu, false>(p, tc);
-    } else {
-        if (!locate_tile_by_sizes<256>(p, tc)) return;
-        dl_tile<kFmtI8, 256, 256, 2, 4, kEpiI8DequantSwiglu>(p, tc);
+    for (uint32_t id = blockIdx.x; locate_tile<SHORT ? 128 : 256, Locate::kAny>(p, tc, id); id += gridDim.x) {
+        if (id != blockIdx.x) __syncthreads();                 // the LDS of the tile before has been read
+        if constexpr (SHORT) ring_tile<kFmtI8, 256, 128, 2, 2, 3, 0, kEpiI8DequantSwiglu, false>(p, tc);
+        else dl_tile<kFmtI8, 256, 256, 2, 4, kEpiI8DequantSwiglu>(p, tc);
     }
+}
+__global__ __launch_bounds__(256) void i8_choice_prepare_kernel(const GroupTablesJob job, uint32_t w_tiles, uint32_t cus, uint32_t kblocks,
+                                                                int32_t* const short_tiles) {
+    fill_group_tables(job, 256, [=](uint32_t n128, uint32_t n256) -> bool {
+        const bool pay = short_tiles_pay(n128 * w_tiles, n256 * w_tiles, cus, kblocks);
+        if (threadIdx.x == 0) *short_tiles = pay ? 1 : 0;
+        return pay;
+    });
 }
 
 __global__ __launch_bounds__(256) void gmm_prepare_kernel(const GroupTablesJob job) { fill_group_tables(job); }
@@ -884,15 +897,33 @@ int launch_gemm_dl(const GemmParams& p, uint32_t max_m_tiles, hipStream_t s) {
     return CMX_OK;
 }
 
-int launch_i8_choice(const GemmParams& p, uint32_t max_m_tiles, hipStream_t s) {
-    if (int rc = allow_dynamic_lds<mx_gemm_i8_choice_kernel, kI8ChoiceLds>(); rc != CMX_OK) return rc;
-    const uint64_t tiles = (uint64_t)max_m_tiles * p.w_tiles;
-    CMX_REQUIRE(tiles > 0 && tiles < (1ull << 31), "tile count out of range");
+// tables of the chosen m-tiles and the choice itself (small groups have no tables of their own then: short_tiles lies in the place of those)
+int launch_i8_choice_tables(const GroupTablesJob& job, const GemmParams& p, int32_t* short_tiles, hipStream_t s) {
     int cus = 0;
     if (int rc = cu_count(&cus); rc != CMX_OK) return rc;
-    hipLaunchKernelGGL(mx_gemm_i8_choice_kernel, dim3((uint32_t)tiles), dim3(512), kI8ChoiceLds, s, p, (uint32_t)cus);
+    CMX_REQUIRE(job.small_rows == 0 && job.tile_m == 128, "tables of a choice: all groups, 128 rows first");
+    hipLaunchKernelGGL(i8_choice_prepare_kernel, dim3(1), dim3(256), 0, s, job, p.w_tiles, (uint32_t)cus, p.kblocks, short_tiles);
     CMX_LAUNCH_CHECK();
     return CMX_OK;
+}
+
+template <bool SHORT>
+int launch_i8_side(const GemmParams& p, const int32_t* short_tiles, uint32_t max_m_tiles, int cus, hipStream_t s) {
+    constexpr size_t smem = SHORT ? ring_lds_bytes(256, 128, 3, 0) : 2 * (256 + 256) * (kSlabBytes + 4);
+    constexpr auto kfn = mx_gemm_i8_choice_kernel<SHORT>;
+    if (int rc = allow_dynamic_lds<kfn, smem>(); rc != CMX_OK) return rc;
+    const uint64_t tiles = (uint64_t)max_m_tiles * p.w_tiles;
+    CMX_REQUIRE(tiles > 0 && tiles < (1ull << 31), "tile count out of range");
+    hipLaunchKernelGGL(kfn, dim3((uint32_t)std::min<uint64_t>(tiles, cus)), dim3(SHORT ? 256 : 512), smem, s, p, (uint32_t)cus, short_tiles);
+    CMX_LAUNCH_CHECK();
+    return CMX_OK;
+}
+// tiles128, tiles256: the most m-tiles that either side can have
+int launch_i8_choice(const GemmParams& p, const int32_t* short_tiles, uint32_t tiles128, uint32_t tiles256, hipStream_t s) {
+    int cus = 0;
+    if (int rc = cu_count(&cus); rc != CMX_OK) return rc;
+    if (int rc = launch_i8_side<true>(p, short_tiles, tiles128, cus, s); rc != CMX_OK) return rc;
+    return launch_i8_side<false>(p, short_tiles, tiles256, cus, s);
 }
 
 template <int FMT, int EPI, int TM, int WW, int WM, int NSLOT>
@@ -1095,8 +1126,8 @@ constexpr uint32_t kSmallGroupRows = 64;               // one m-tile of the 64 x
 //   32 experts, 1024 rows on 4      59    82    55      85    78    50      75    79    54
 //   32 experts, 1280 rows on 4      56    69    59      91    60    92      78    66    81
 // (256-row kernel: the three-slot 256 x 128 kernel for E4M3 SwiGLU, 256 x 256 tiles for INT8.  Since ring_groups has put the ring's tiles in their
-// place the rule's column reads, E4M3 SwiGLU and INT8: 32 on average, Zipf 1315 and 1318; 8192 rows on 8 experts 256 and 226, 2048 on 2 69 and 85;
-// 32 experts, 512 rows on 1 37 and 37, 1024 on 4 53 and 50, 1280 on 4 53 and 60.)
+// place the rule's column reads, E4M3 SwiGLU and INT8: 32 on average, Zipf 1315 and 1326; 8192 rows on 8 experts 256 and 242 on a box where the
+// 256-row kernel takes 242 too, 2048 on 2 69 and 81; 32 experts, 512 rows on 1 37 and 36, 1024 on 4 53 and 52, 1280 on 4 53 and 63.)
 // The empty one of the two launches costs 2-6 us.  A limit of 32 or 40 rows instead of 64: 1360 or 1308 against 1214 (random), 1349 or
 // 1298 against 1352 (Zipf).  8-bit problems whose K is no whole number of slabs go by size only past the 2048 tiles up to which the
 // split-K kernel beats the register-staged one (choose_ksplit).  Row-major and pre-tiled weights go by one rule, because they
@@ -1450,9 +1481,8 @@ uint32_t max_group_tiles(uint32_t m_total, uint32_t groups, uint32_t tile_m, uin
 // Problems of more tiles stay on the persistent kernels (32 x 194 rows, 7168, 4096: 287 against 311 with 128 x 256).
 // INT8, whose only other kernel has 256 x 256 tiles, one per workgroup (us, fp32 output):
 //   128 x 128    8 x 44 u, 4096, 2048 46.5 -> 21.6     8 x 200 u 47.7 -> 27.0     16 x 100 z, 7168, 1024 73.2 -> 34.8     16 x 44 u, 2048, 2048 29.7 -> 16.9
-//   256 x 128    32 x 44 u, 7168, 4096 222 -> 178       32 x 100 z 299 -> 232      32 x 100 z, 1152, 2048 46.3 -> 37.3: where the device chooses it
-//                (mx_gemm_i8_choice_kernel); not for more than 96 rows on average at K below 2048: 32 x 112, 1024, 4096 58 against 75 u, 73 against 71
-//                z, 28 against 47 on four groups, 64 x 100 112 against 111, 126 against 122, 53 against 87
+//   256 x 128    32 x 44 u, 7168, 4096 222 -> 178       32 x 100 z 299 -> 232      32 x 100 z, 1152, 2048 46.3 -> 37.3: from K = 512 on, and where the device
+//                chooses it (mx_gemm_i8_choice_kernel)
 //   128 x 256    16 x 200 u, 7168, 1024 71.8 -> 50.9; of more than a round 32 x 200 u, 7168, 4096 278 against 251, 16 x 2048 1077 against 1003
 // FP4, whose other kernels past the split-K sizes have tiles of 256 x 128 and 256 x 256 (us, bf16 output):
 //   128 x 128    8 x 70 u, 4096, 2048 31.6 -> 15.9     8 x 200 u 36.0 -> 18.4     16 x 100 z, 7168, 1024 46.9 -> 24.1     8 x 70 u, 7168, 4096 49 -> 26
@@ -1464,8 +1494,9 @@ int ring_groups(TileChoice* t, uint32_t m_total, uint32_t groups, uint32_t n, in
     int cus = 0;
     if (int rc = cu_count(&cus); rc != CMX_OK) return rc;
     const uint64_t w128 = ceil_div(n, 128);
+    const uint32_t k_min = eight_bit && swiglu ? 96 : 16;
     if (w128 * (m_total / 128 + groups) <= (uint64_t)cus) *t = {128, 128, kRing};
-    else if (t->tm <= 128 && (fmt == kFmtI8 ? kblocks >= 64 || ceil_div(m_total, groups) <= 96 : !swiglu || kblocks >= 96 || !eight_bit)) *t = {256, 128, kRing};
+    else if (t->tm <= 128 && kblocks >= k_min) *t = {256, 128, kRing};
     else if (t->tm == 256 && w128 * (m_total / 256 + groups * 3 / 4) <= (uint64_t)cus && (swiglu || kblocks >= 64 || !eight_bit)) *t = {128, 256, kRing};
     return CMX_OK;
 }
@@ -1639,24 +1670,27 @@ extern "C" int cmx_int8_gmm_dequant_swiglu(const int8_t* a, uint32_t lda, const 
         choice = !all_ksplit && t.waves == kRing && t.tw == 256;
     }
     if (t.waves != kRing) t.tm = 256;
-    // All kernels of the call take one tile per workgroup.  The choice goes by the sizes up to eight rounds; past them the 256 x 128 tiles lead
-    // on most loads (256 x 90 rows, 2048, 2048: 293 against 325 u, 330 against 369 z, 171 against 120 on four groups), but where the small groups
-    // go to the split-K kernel those that are left are large for their average (256 x 32, 7168, 4096, on eight groups 227 against 277).
+    // All kernels of the call take one tile per workgroup.  Past the rounds up to which they find it by the sizes, the launch that fills the
+    // tables makes the choice.  Where it would fill them for small groups as well, those that are left to the large tiles are large for
+    // their average (256 x 32, 7168, 4096, on eight groups 227 against 277).
     bool by_sizes = false;
     const uint64_t most = all_ksplit ? (uint64_t)(m_total / 64 + groups) * ceil_div(n, 64) : (uint64_t)(m_total / t.tm + groups) * ceil_div(n, t.tw);
-    if (int rc = tiles_by_sizes(&by_sizes, groups, choice && ks.small_rows == 0 ? most * 6 / 8 : most, all_ksplit ? 2 : 1); rc != CMX_OK) return rc;
-    if (choice && !by_sizes) {
+    // (a choice by the sizes is a second scan for every tile)
+    if (int rc = tiles_by_sizes(&by_sizes, groups, choice && ks.small_rows == 0 ? 3 * most : most, all_ksplit ? 2 : 1); rc != CMX_OK) return rc;
+    if (choice && !by_sizes && ks.small_rows != 0) {
         choice = false;
-        if (ks.small_rows != 0) t = {256, 256, 8};
+        t = {256, 256, 8};
     }
     const GroupTables tables(ws, groups);
-    const uint32_t tile_m = all_ksplit ? 16 * ks.tile.fm : t.tm;
-    if (int rc = prepare_groups(p, tables_job(tables, group_sizes, groups, m_total, tile_m, ks.small_rows), by_sizes, false, s); rc != CMX_OK) return rc;
+    const GroupTablesJob job = tables_job(tables, group_sizes, groups, m_total, all_ksplit ? 16 * ks.tile.fm : t.tm, ks.small_rows);
+    p.w_tiles = ceil_div(n / 2, t.tw / 2);
+    if (choice && !by_sizes)
+        if (int rc = launch_i8_choice_tables(job, p, tables.small_pref, s); rc != CMX_OK) return rc;
+    if (int rc = prepare_groups(p, job, by_sizes, choice, s); rc != CMX_OK) return rc;
     if (ks.tile.fw != 0)
         if (int rc = launch_grouped_ksplit(p, tables, ks, kFmtI8, kEpiI8DequantSwiglu, m_total, s); rc != CMX_OK || all_ksplit) return rc;
-    p.w_tiles = ceil_div(n / 2, t.tw / 2);
     const uint32_t max_m_tiles = max_group_tiles(m_total, groups, t.tm, ks.small_rows);
-    if (choice) return launch_i8_choice(p, max_m_tiles, s);
+    if (choice) return launch_i8_choice(p, tables.small_pref, max_m_tiles, max_group_tiles(m_total, groups, 256, ks.small_rows), s);
     if (t.waves == kRing) return launch_ring(p, {t.tw, t.tm}, kFmtI8, kEpiI8DequantSwiglu, false, max_m_tiles, s);
     // (hand-scheduled variants of this kernel were measured twice at 16 x 2048 x 7168 x 4096 and are not kept: two i8
     // MFMAs per step and accumulator in the 8-bit schedule 997 us, one per 32-K step in the 16-byte-fragment

@@ -133,9 +133,9 @@ __device__ __forceinline__ void interleave_xcd_walk(uint32_t total_tiles, uint32
 // One tile per workgroup (blockIdx.x < total_tiles).  Workgroups start in the order of their ids, ids congruent mod 8 on one
 // XCD.  Whole chunks of 256 tiles: the XCDs take blocks of 32 consecutive tiles of the chunk in turn, for the reason given
 // above (the INT8 operator on the 16-expert problem: 973-982 -> 942-945 us); the rest: a contiguous run per XCD.
-__device__ __forceinline__ uint32_t tile_of_workgroup(uint32_t total_tiles) {
+__device__ __forceinline__ uint32_t tile_of_workgroup(uint32_t total_tiles, uint32_t bid = blockIdx.x) {
     constexpr uint32_t kChunk = 32 * kXcds;
-    const uint32_t bid = blockIdx.x, full = total_tiles / kChunk * kChunk;
+    const uint32_t full = total_tiles / kChunk * kChunk;
     if (bid < full) return bid / kChunk * kChunk + (bid % kXcds) * 32 + (bid % kChunk) / kXcds;
     uint32_t count;
     const uint32_t k = bid - full;
@@ -244,7 +244,7 @@ __device__ __forceinline__ uint32_t tiles_of_group(const GemmParams& p, uint32_t
 }
 
 template <int TM>
-__device__ __forceinline__ bool locate_tile_by_sizes(const GemmParams& p, Tile& t) {
+__device__ __forceinline__ bool locate_tile_by_sizes(const GemmParams& p, Tile& t, uint32_t bid) {
     constexpr int kPer = kGroupsPerLane;
     uint32_t off[kPer + 1], tiles[kPer], all = 0;
     scan_group_rows(p, off);
@@ -255,8 +255,8 @@ __device__ __forceinline__ bool locate_tile_by_sizes(const GemmParams& p, Tile& 
     }
     const uint32_t pref = wave_scan(all, [](uint32_t a, uint32_t b) -> uint32_t { return a + b; });
     const uint32_t total = (uint32_t)__builtin_amdgcn_readlane((int)pref, 63) * p.w_tiles;
-    if (blockIdx.x >= total) return false;
-    const uint32_t L = tile_of_workgroup(total);
+    if (bid >= total) return false;
+    const uint32_t L = tile_of_workgroup(total, bid);
     const int at = (int)__builtin_ctzll(__ballot(pref * p.w_tiles > L));                         // lane of the tile's group
     uint32_t tp = (uint32_t)__builtin_amdgcn_readlane((int)(pref - all), at), g = kPer * at;
 #pragma unroll
@@ -276,22 +276,23 @@ __device__ __forceinline__ bool locate_tile_by_sizes(const GemmParams& p, Tile& 
 // K = 640, N = 3584: 15.9 against 14.1).
 enum class Locate { kDense, kTables, kSizes, kAny };
 
-// One tile per workgroup: maps the workgroup id to (group, m-tile, weight tile).  Returns false for ids past the last tile.
+// Maps the id of a workgroup (of one that goes on with further tiles: of the workgroup that would take this one if each took one) to
+// (group, m-tile, weight tile).  Returns false for ids past the last tile.
 template <int TM, Locate HOW>
-__device__ __forceinline__ bool locate_tile(const GemmParams& p, Tile& t) {
+__device__ __forceinline__ bool locate_tile(const GemmParams& p, Tile& t, uint32_t bid = blockIdx.x) {
     if constexpr (HOW == Locate::kDense) {
         const uint32_t m_tiles = (p.m + TM - 1) / TM, total_tiles = m_tiles * p.w_tiles;
-        if (blockIdx.x >= total_tiles) return false;
-        place_dense<TM>(p, m_tiles, tile_of_workgroup(total_tiles), t);
+        if (bid >= total_tiles) return false;
+        place_dense<TM>(p, m_tiles, tile_of_workgroup(total_tiles, bid), t);
         return true;
     }
-    if constexpr (HOW == Locate::kSizes) return locate_tile_by_sizes<TM>(p, t);
+    if constexpr (HOW == Locate::kSizes) return locate_tile_by_sizes<TM>(p, t, bid);
     if constexpr (HOW == Locate::kAny)
-        if (p.sizes != nullptr) return locate_tile_by_sizes<TM>(p, t);
+        if (p.sizes != nullptr) return locate_tile_by_sizes<TM>(p, t, bid);
     const uint32_t m_tiles_all = count_m_tiles<TM>(p);
     const uint32_t total_tiles = m_tiles_all * p.w_tiles;
-    if (blockIdx.x >= total_tiles) return false;
-    decode_tile<TM>(p, m_tiles_all, tile_of_workgroup(total_tiles), t);
+    if (bid >= total_tiles) return false;
+    decode_tile<TM>(p, m_tiles_all, tile_of_workgroup(total_tiles, bid), t);
     return true;
 }
 

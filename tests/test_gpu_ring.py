@@ -209,15 +209,18 @@ def test_grouped_int8_gives_the_bits_of_the_256_row_kernel(tile, out, counts, n,
 
 
 @pytest.mark.parametrize("counts,rows,n,k", [
-    ([110] * 20, 2200, 4096, 128),                                     # K < 2048, more than 96 rows each: 256 x 256 tiles without a choice
-    ([90] * 20, 1800, 4096, 128),                                      # the choice: two rounds of either, the ring's
-    ([1700, 0, 0, 90] + [3] * 16, 1838, 4096, 128),                    # two rounds of the ring's, one of the others'
-    ([100, 0, 130, 120] * 8, 2800, 2048, 2048),                        # the same by groups of a little more than 128 rows
-    ([2 ** 31 - 1, -4, 7, 2 ** 31 - 1] + [9] * 16, 1900, 4096, 128),   # sizes past the rows that there are, negative ones
-    ([128, 129] * 9, 2313, 3072, 4096),                                # K >= 4096
-    ([1100, 0, 64, 65, 1, 800, 33, 200] + [0] * 52, 2263, 4096, 128),  # small groups to split-K, the choice for the others
-    ([1, 200, 64, 65] * 64, 21120 - 9, 2048, 128),                     # more than eight rounds: tables, the ring's tiles
-    ([60, 70, 129, 5] * 75, 19800, 1024, 128)])                        # more groups than a scan takes: tables, the ring's tiles
+    # by the sizes (most tiles of two rounds), and by the launch that fills the tables; the 256 x 128 side, and the 256 x 256 one
+    ([90] * 12, 1080, 4096, 512),                                      # sizes, one round of either: 256 x 128
+    ([1300, 0, 0, 90] + [3] * 8, 1414, 4096, 512),                     # sizes, two rounds against one: 256 x 256
+    ([100, 130, 140] * 5, 1850, 4096, 2048),                           # K >= 2048, groups of a little more than 128 rows: 256 x 256
+    ([90] * 40, 3600, 4096, 512),                                      # tables, three rounds of either: 256 x 128
+    ([2000, 1500] + [0] * 38, 3500, 4096, 512),                        # tables, two rounds against one: 256 x 256
+    ([60, 70, 129, 5] * 75, 19800, 1024, 512),                         # tables of more groups than a scan takes: 256 x 128
+    ([9000, 0, 7000] + [1] * 298, 16298, 1024, 512),                   # the same, 256 x 256
+    ([2 ** 31 - 1, -4] + [9] * 8, 1200, 4096, 512),                    # sizes past the rows that there are, negative ones
+    ([2 ** 31 - 1, -4, 7, 2 ** 31 - 1] + [9] * 16, 1900, 4096, 512),   # the same in tables
+    ([1100, 0, 64, 65, 1, 800, 33, 200] + [0] * 52, 2263, 4096, 512),  # small groups to split-K, the choice for the others
+    ([110] * 20, 2200, 4096, 384)])                                    # K < 512: 256 x 256 tiles without a choice
 def test_chosen_int8_kernels(counts, rows, n, k):
     """Whatever of the 256 x 128 and 256 x 256 tiles the host or the device takes: one result, that of the 256-row kernel alone."""
     from catccos_amd import ops
