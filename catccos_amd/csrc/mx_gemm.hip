@@ -1478,6 +1478,8 @@ uint32_t max_group_tiles(uint32_t m_total, uint32_t groups, uint32_t tile_m, uin
 //                against 42.3 with weights in the memory-side cache; store 64 x 40 u, 1024, 4096 74.8 against 78.3
 //   128 x 256    8 x 200 u, 4096, 2048                       45.9 -> 34.5 / 43.1 -> 35.7    16 x 300 u, 7168, 1024   74 -> 57 / 69 -> 62
 //                8 x 500 u, 1024, 1024                       22.6 -> 18.6 / 20.0 against 19.9, so not for a store at K below 2048
+// Where n is at most 128, half of a 256-row tile would be empty: 128 x 128 for 256 x 128 (SwiGLU 256 x 68 z, 3072, 64 45 -> 34 where 256 x 128 takes
+// 48; FP4 256 x 128 u, 512, 64 20 -> 16, 23; INT8 256 x 128 u, 128, 128 17.5 -> 14.1, 20.1).
 // Problems of more tiles stay on the persistent kernels (32 x 194 rows, 7168, 4096: 287 against 311 with 128 x 256).
 // INT8, whose only other kernel has 256 x 256 tiles, one per workgroup (us, fp32 output):
 //   128 x 128    8 x 44 u, 4096, 2048 46.5 -> 21.6     8 x 200 u 47.7 -> 27.0     16 x 100 z, 7168, 1024 73.2 -> 34.8     16 x 44 u, 2048, 2048 29.7 -> 16.9
@@ -1496,7 +1498,7 @@ int ring_groups(TileChoice* t, uint32_t m_total, uint32_t groups, uint32_t n, in
     const uint64_t w128 = ceil_div(n, 128);
     const uint32_t k_min = eight_bit && swiglu ? 96 : 16;
     if (w128 * (m_total / 128 + groups) <= (uint64_t)cus) *t = {128, 128, kRing};
-    else if (t->tm <= 128 && kblocks >= k_min) *t = {256, 128, kRing};
+    else if (t->tm <= 128 && kblocks >= k_min) *t = {w128 == 1 ? 128 : 256, 128, kRing};
     else if (t->tm == 256 && w128 * (m_total / 256 + groups * 3 / 4) <= (uint64_t)cus && (swiglu || kblocks >= 64 || !eight_bit)) *t = {128, 256, kRing};
     return CMX_OK;
 }

@@ -220,7 +220,8 @@ def test_grouped_int8_gives_the_bits_of_the_256_row_kernel(tile, out, counts, n,
     ([2 ** 31 - 1, -4] + [9] * 8, 1200, 4096, 512),                    # sizes past the rows that there are, negative ones
     ([2 ** 31 - 1, -4, 7, 2 ** 31 - 1] + [9] * 16, 1900, 4096, 512),   # the same in tables
     ([1100, 0, 64, 65, 1, 800, 33, 200] + [0] * 52, 2263, 4096, 512),  # small groups to split-K, the choice for the others
-    ([110] * 20, 2200, 4096, 384)])                                    # K < 512: 256 x 256 tiles without a choice
+    ([110] * 20, 2200, 4096, 384),                                     # K < 512: 256 x 256 tiles without a choice
+    ([60, 70, 129, 5] * 75, 19800, 128, 512)])                         # n <= 128: 128 x 128 tiles of more than a round
 def test_chosen_int8_kernels(counts, rows, n, k):
     """Whatever of the 256 x 128 and 256 x 256 tiles the host or the device takes: one result, that of the 256-row kernel alone."""
     from catccos_amd import ops
@@ -235,6 +236,25 @@ def test_chosen_int8_kernels(counts, rows, n, k):
     hooks_lib().cmx_debug_force_ksplit(-1, 0, 0)
     hooks_lib().cmx_debug_force_tile(256, 256, 8)
     assert torch.equal(ops.int8_gmm_dequant_swiglu(*args), chosen) and chosen.abs().max() > 0
+
+
+@pytest.mark.parametrize("kind,k", [("E4M3", 512), ("E2M1", 512), ("SwiGLU", 3072), ("SwiGLU", 512)])
+@pytest.mark.parametrize("n", [64, 128, 192])
+def test_narrow_weights_in_many_groups(kind, k, n):
+    """More than a round of 128 x 128 tiles, which n <= 128 takes and 192 does not: the bits of the 256-row kernel."""
+    from catccos_amd import ops
+    g = torch.Generator(device="cuda")
+    g.manual_seed(n + k)
+    counts = torch.tensor([70, 0, 129, 128] * 60, dtype=torch.int32, device="cuda")
+    e, m, kb = len(counts), int(counts.sum()), k // 2 if kind == "E2M1" else k
+    codes = lambda *shape: torch.randint(0, 256, shape, dtype=torch.uint8, device="cuda", generator=g) & 0xF7
+    scales = lambda *shape: torch.randint(110, 125, shape, dtype=torch.uint8, device="cuda", generator=g)
+    args = (codes(m, kb), scales(m, k // 32), codes(e, n, kb), scales(e, n, k // 32), counts, k)
+    call = (lambda: ops.mx_gmm_swiglu_quant(*args)[:2]) if kind == "SwiGLU" else (lambda: [ops.mx_gmm(*args, kind)])
+    chosen = call()
+    hooks_lib().cmx_debug_force_tile(256, 256, 8)
+    for got, ref in zip(chosen, call()):
+        assert torch.equal(got.view(torch.uint8), ref.view(torch.uint8)) and bool((ref != 0).any())
 
 
 @pytest.mark.parametrize("kernel", ["ring", "split-K", "INT8"])
