@@ -7,15 +7,17 @@
 // split-K 50.4 us, 256 x 256 64, this kernel 36.4, of which its loads alone would take 28, its MFMAs alone 26 (the chip lowers its
 // clock under them: 32 workgroups alone 20) and start, prologue and epilogue 7.
 //   * Slabs of 128 bytes of K travel by LDS-DMA into a ring of three slots; one barrier per slab says both that slab s has been read and
-//     that slab s + 1 has arrived.  A fourth slot changes nothing (38.4 against 36.6).
+//     that slab s + 1 has arrived.  A fourth slot changes nothing (38.4 against 36.6); only INT8 at 128 x 128, which has no scales, has one.
 //   * One wavefront per SIMD issues in order, so the matrix pipe is busy only if LDS reads and loads stand between the MFMAs; the
 //     compiler puts the MFMAs of a slab together behind them (48 us at 64 rows, where the order below takes 30).  So each step of
 //     the loop is pinned (sched_barrier): an MFMA, its share of the fragment reads of the step after, its share of the loads.  The loads
 //     of a slab are spread over both steps (all of them in one: 37).
-//   * A loop without branches: past the last slab the loads go on from a buffer of no bytes.
+//   * Tile loads without branches: past the last slab they go on from a buffer of no bytes.  (The one branch of the loop asks for the next
+//     block of scales.)
 //   * Scales are a byte per 32 elements in rows of their own.  A dword per row and slab touches as many lines as the tile itself
-//     (320 lines a slab instead of 256: 4.5 us), so they come SPAN slabs at a time into one of two halves of an area behind the ring.
-//     SPAN is what the LDS has left: 32 slabs at TM = 128, 16 at 192, 4 at 256.
+//     (320 lines a slab instead of 256: 4.5 us), so they come SPAN dwords of a row at a time into one of two halves of an area behind the
+//     ring.  SPAN is what the LDS has left: 32 dwords at 128 x 128, 16 at 128 x 192, 4 at 128 x 256 and 256 x 128.  A slab takes one of them, of
+//     FP4 (256 elements) two.  INT8 has none: its scales are the epilogue's.
 //   * Weights stored [K, N] (KSLOW) are fetched as they lie, 128 columns of 128 K positions, and turned on the way from the LDS into
 //     the registers by ds_read_b64_tr_b8: 1024 x 4096 x 7168 38.9 us, where the pass that rewrites them takes 15 and a launch.
 // The K order of the sums is that of the 256-row kernels (one chain, the same instruction), and so are the bits.

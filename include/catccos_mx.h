@@ -232,9 +232,11 @@ int cmx_dispatch_ffn_combine_pretiled(cmx_stream_t stream, const uint8_t* x, con
  *
  * cmx_mx_gemm_ex / cmx_mx_gmm_ex are cmx_mx_gemm / cmx_mx_gmm for dense operands in either orientation
  * (trans_a = 1: A is [K, M]; trans_b = 0: B is [K, N] resp. [groups, K, N]); operands that are not K-contiguous
- * are normalised into the workspace first (one extra read and write of that operand).  The workspace
- * must be 256-byte aligned and hold *_ex_workspace_bytes bytes (for the grouped form this includes the
- * tile schedule metadata of cmx_mx_gmm).
+ * are normalised into the workspace first (one extra read and write of that operand).  Dense 8-bit weights stored
+ * [K, N] are read as they lie where that is the faster way (K a multiple of 128, N a multiple of 4): the call then leaves
+ * their part of the workspace alone, but asks for it all the same, because the size does not depend on the format and
+ * which way is the faster one depends on the device.  The workspace must be 256-byte aligned and hold
+ * *_ex_workspace_bytes bytes (for the grouped form this includes the tile schedule metadata of cmx_mx_gmm).
  * ---------------------------------------------------------------------------------------- */
 int cmx_mx_to_k_major(const uint8_t* src, uint32_t ld_src, const uint8_t* src_scale, uint8_t* dst, uint32_t ld_dst,
                       uint8_t* dst_scale, uint32_t ld_dst_scale, uint32_t k, uint32_t n, uint32_t batch,
