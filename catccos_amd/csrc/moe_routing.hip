@@ -364,15 +364,17 @@ __device__ __forceinline__ void zero_unmapped_rows(const ZeroJob& z, uint32_t bl
         }
     }
     __syncthreads();
-    const uint32_t lane = threadIdx.x & 63u;
-    for (uint32_t w = threadIdx.x / 64; w < words; w += THREADS / 64) {
+    // Beside the scatter, few wavefronts have the rows to clear: as many lanes to a row as it has vectors for, so that short rows are cleared
+    // several at a time (13044 tokens x 512, top 8, nine routes in ten dropped, 52.6 -> 42.3 us).
+    const uint32_t group = THREADS == kUnmappedThreads || z.nvec > 32 ? 64 : (z.nvec > 16 ? 32 : 16), lane = threadIdx.x & (group - 1);
+    for (uint32_t w = threadIdx.x / group; w < words; w += THREADS / group) {
         uint32_t miss = ~s_map[w];
         if (w == words - 1 && n % 32 != 0) miss &= (1u << (n % 32)) - 1u;
         while (miss != 0) {
             const size_t row = r0 + w * 32 + (uint32_t)__builtin_ctz(miss);
             miss &= miss - 1;
-            for (uint32_t v = lane; v < z.nvec; v += 64) *reinterpret_cast<uint4*>(out_codes + row * ld_out + v * 16) = make_uint4(0, 0, 0, 0);
-            for (uint32_t c = lane; c < z.scols; c += 64) out_scales[row * ld_outs + c] = 0;
+            for (uint32_t v = lane; v < z.nvec; v += group) *reinterpret_cast<uint4*>(out_codes + row * ld_out + v * 16) = make_uint4(0, 0, 0, 0);
+            for (uint32_t c = lane; c < z.scols; c += group) out_scales[row * ld_outs + c] = 0;
         }
     }
 }
