@@ -130,6 +130,18 @@ __device__ __forceinline__ void interleave_xcd_walk(uint32_t total_tiles, uint32
     end = total_tiles;
 }
 
+// The tile after tile_id of such a walk, or `end`.  In the last, partly filled round the XCDs take fewer tiles each, in whole bands of 8: in
+// blocks of 32 they would all lie on the first XCDs, and the L2s and links of the others would have nothing to do.  320 tiles on 256
+// workgroups (us): SwiGLU 8 x 1280 rows, K = 4096, N = 2048 124.5 -> 112.6, FP4 125.7 -> 117.2, dense 8192 x 5120 x 7168 (640 tiles) 281 -> 264; 384
+// tiles 128 -> 117.  In contiguous runs of any length, which cut across the bands, 65536 rows on 32 groups (17 rounds) lose 1.6 %.
+__device__ __forceinline__ uint32_t next_of_walk(uint32_t tile_id, uint32_t stride, uint32_t end) {
+    const uint32_t next = tile_id + stride;
+    if (stride != gridDim.x || next < end / stride * stride) return next;
+    const uint32_t full = end / stride * stride, per = ((end - full + kXcds - 1) / kXcds + 7) / 8 * 8, j = blockIdx.x / kXcds;
+    const uint32_t last = full + blockIdx.x % kXcds * per + j;
+    return tile_id < full && j < per && last < end ? last : end;
+}
+
 // One tile per workgroup (blockIdx.x < total_tiles).  Workgroups start in the order of their ids, ids congruent mod 8 on one
 // XCD.  Whole chunks of 256 tiles: the XCDs take blocks of 32 consecutive tiles of the chunk in turn, for the reason given
 // above (the INT8 operator on the 16-expert problem: 973-982 -> 942-945 us); the rest: a contiguous run per XCD.

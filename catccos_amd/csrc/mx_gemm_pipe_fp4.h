@@ -443,7 +443,7 @@ __global__ __launch_bounds__(256) void mx_gemm_pipe_fp4_kernel(const GemmParams 
                     __syncthreads();
                     next_id = run_first + tile_stride + __builtin_amdgcn_readfirstlane(*mailbox);
                 } else {
-                    next_id = tile_id + tile_stride;
+                    next_id = next_of_walk(tile_id, tile_stride, run_end);
                 }
                 next_ok = next_id < run_end;
                 if (next_ok) {
