@@ -352,6 +352,69 @@ __device__ __forceinline__ void lean_store_lines(const GemmParams& p, const Tile
     }
 }
 
+// INT8 dequant + SwiGLU of the persistent two-slot kernel, stored in whole lines like lean_store_lines: the 32 rows x 128 bytes that a
+// gate and an up fragment (16-bit outputs: two of each) give for one activation fragment go through `stage`.  The scales of the tile lie
+// in the LDS at `scales` ([256 channels][256 tokens] fp32, in the order of the tile's rows): a load from memory would wait, in order, for
+// the two slabs of operands in flight.
+template <int TW, int TM, int WW, int WM, int FW, int FM>
+__device__ __forceinline__ void i8_store_lines(const GemmParams& p, const Tile& tc, v16f (&acc)[FW][FM], uint32_t ww, uint32_t wm, uint32_t lane,
+                                               uint32_t stage, uint32_t scales) {
+    typedef int v16i __attribute__((ext_vector_type(16)));
+    static_assert(FW == 4, "two gate fragments and their up partners");
+    typedef const __attribute__((address_space(3))) v4f* lds_v4f;
+    typedef const __attribute__((address_space(3))) float* lds_float;
+    const uint32_t l32 = lane & 31u, lh = lane >> 5, half = p.n >> 1;
+    const uint32_t wr_row = stage + l32 * 128, x = l32 & 7u;
+    const uint32_t rd_r = lane >> 3, rd_p = lane & 7u;
+    const bool wide = p.out_type == CMX_OUT_FP32;
+#pragma unroll
+    for (int fm = 0; fm < FM; ++fm) {
+        const float tsv = *(lds_float)(uintptr_t)(scales + (TW + wm * (TM / WM) + fm * 32 + l32) * 4);
+#pragma unroll
+        for (int f = 0; f < FW / 2; ++f) {
+            const v16i ig = __builtin_bit_cast(v16i, acc[f][fm]), iu = __builtin_bit_cast(v16i, acc[f + FW / 2][fm]);
+            const uint32_t ch = scales + (ww * (TW / 2 / WW) + f * 32 + 4 * lh) * 4;
+#pragma unroll
+            for (int q = 0; q < 4; ++q) {
+                const v4f cg = *(lds_v4f)(uintptr_t)(ch + 32 * q), cu = *(lds_v4f)(uintptr_t)(ch + 32 * q + TW / 2 * 4);
+                float y[4];
+#pragma unroll
+                for (int i = 0; i < 4; ++i) {
+                    const float x0 = __fmul_rn(i8_dequant(ig[4 * q + i], cg[i]), tsv);
+                    const float gate = __fmul_rn(i8_dequant(iu[4 * q + i], cu[i]), tsv);
+                    y[i] = __fmul_rn(__fmul_rn(x0, __builtin_amdgcn_rcpf(1.0f + __expf(-x0))), gate);
+                }
+                if (wide) {
+                    asm volatile("ds_write_b128 %0, %1" ::"v"(wr_row + (((2 * q + lh) ^ x) << 4)), "v"((v4f){y[0], y[1], y[2], y[3]}) : "memory");
+                } else {
+                    uint32_t h[4];
+#pragma unroll
+                    for (int i = 0; i < 4; ++i)
+                        h[i] = p.out_type == CMX_OUT_FP16 ? __builtin_bit_cast(uint16_t, (_Float16)as_f32(y[i])) : (uint16_t)f32_to_bf16(y[i]);
+                    asm volatile("ds_write_b64 %0, %1" ::"v"(wr_row + (((4 * f + q) ^ x) << 4) + 8 * lh),
+                                 "v"((v2i){(int)(h[0] | h[1] << 16), (int)(h[2] | h[3] << 16)}) : "memory");
+                }
+            }
+            if (!wide && f == 0) continue;
+            asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+            v4i v[4];
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                const uint32_t r = 8 * j + rd_r;
+                asm volatile("ds_read_b128 %0, %1" : "=v"(v[j]) : "v"(stage + r * 128 + ((rd_p ^ (r & 7u)) << 4)) : "memory");
+            }
+            asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");       // also: the area is free for the next pieces
+            const uint32_t col = tc.wt * (TW / 2) + ww * (TW / 2 / WW) + (wide ? f * 32 + rd_p * 4 : rd_p * 8);
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                const uint32_t mloc = wm * (TM / WM) + fm * 32 + 8 * j + rd_r;
+                if (mloc < tc.rows_valid && col < half)                // n / 2 is a multiple of 32: a piece is in or out as a whole
+                    __builtin_nontemporal_store(v[j], reinterpret_cast<v4i*>(static_cast<uint8_t*>(p.c) + ((size_t)(tc.row0 + mloc) * p.ldc + col) * (wide ? 4 : 2)));
+            }
+        }
+    }
+}
+
 // TW/TM: tile rows (weights / activations); WW x WM wavefront grid over the tile (4 or 8 wavefronts).
 // FAST: K is a whole number of slabs and scale rows are dword aligned, so the main loop carries no
 // bounds checks at all.
@@ -809,26 +872,22 @@ __global__ __launch_bounds__(64 * WW * WM) void mx_gemm_dl_kernel(const GemmPara
     dl_tile<FMT, TW, TM, WW, WM, EPI>(p, tc);
 }
 
-#include "mx_gemm_pipe.h"
-#include "mx_gemm_wreg.h"
-#include "mx_gemm_pipe_fp4.h"
-
 // INT8 groups of up to 128 rows on average (but one round of 128 x 128 tiles): 256 x 128 tiles of the ring kernel, or 256 x 256 ones.
 // What decides is the number of rounds, of a workgroup per CU, that each takes, and with it how the rows lie, which the host does not
-// know: a round of the ring's tiles takes 0.73 (K < 2048) to 0.62 of one of the others, but where groups are a little longer than 128 rows,
+// know: a round of the ring's tiles takes 0.7 of one of the others, but where groups are a little longer than 128 rows,
 // or few of them hold all rows, there are up to twice as many.  So the device counts both from the sizes: in every workgroup up to two
 // rounds, in the launch that fills the tables beyond (a count costs each tile 1 us).  A kernel for each side, the one that the choice
 // leaves out finding nothing to do (2 us): both in one kernel share its registers, and the ring's loop comes out slower by a quarter
 // (8 groups x 76 rows u, 7168, 3072 58.8 against 41.5).  Below K = 512 the launches cost more than is won (64 x 128 u, 128, 3072 42 -> 51).
 // Measured (us, fp32 output, 256 x 256 alone / 256 x 128 alone / the choice; u: routes drawn uniformly, z: Zipf, c: all rows on four groups):
 //   K, N, groups x rows      u               z               c
-//   7168, 3072, 64 x 100     335 279 285     394 333 339     180 157 162
-//   7168, 3072, 32 x 90      201 152 161     202 178 191      83  97  87
-//   4096, 3072, 64 x 128     229 226 234     263 236 240     117 134 119
-//   2048, 3072, 32 x 90       63  46  51      66  61  69      33  40  38
-//   2048, 1024, 256 x 48     156 125 129     164 126 134      37  42  43
-//   1024, 3072, 64 x 100      73  57  61      83  73  77      44  47  50
-//    512, 3072, 128 x 70     104  77  78     107  88  87      42  53  44
+//   7168, 3072, 64 x 100     318 279 286     395 327 338     182 164 169
+//   7168, 3072, 32 x 90      200 154 161     195 183 190      81  99  87
+//   7168, 3072, 64 x 125     321 354 334     393 335 344     188 215 193
+//   2048, 3072, 32 x 90       65  48  52      67  60  66      32  40  38
+//   2048, 1024, 256 x 48     154 126 129     183 127 132      36  43  42
+//   1024, 3072, 64 x 100      71  58  62      91  70  77      47  47  52
+//    512, 3072, 128 x 70      99  77  79     113  90  89      37  52  42
 // tiles of 128 and of 256 rows that a problem has; cus: workgroups that run at a time
 __device__ __forceinline__ bool short_tiles_pay(uint32_t t128, uint32_t t256, uint32_t cus, uint32_t kblocks) {
     const uint32_t r128 = (t128 + cus - 1) / cus, r256 = (t256 + cus - 1) / cus;
@@ -846,18 +905,21 @@ __device__ __forceinline__ bool short_tiles_pay_by_sizes(const GemmParams& p, ui
     return short_tiles_pay((uint32_t)__builtin_amdgcn_readlane((int)wave_scan(n128, add), 63) * p.w_tiles,
                            (uint32_t)__builtin_amdgcn_readlane((int)wave_scan(n256, add), 63) * p.w_tiles, cus, p.kblocks);
 }
-// One side of the choice, which is left at once where it falls on the other.  A workgroup goes on with further tiles, so that there are no
-// more of them than run at a time: leaving takes each 0.3 us (256 groups x 48 rows c, 512, 1024, a workgroup for each tile 33.9, so 26.3).
-// short_tiles: the choice, where tables of its m-tiles have been filled (i8_choice_prepare_kernel).
-template <bool SHORT>
-__global__ __launch_bounds__(SHORT ? 256 : 512) void mx_gemm_i8_choice_kernel(const GemmParams p, const uint32_t cus, const int32_t* const short_tiles) {
-    const bool pay = p.sizes != nullptr ? short_tiles_pay_by_sizes(p, cus) : table_at(short_tiles, 0) != 0;
-    if ((__builtin_amdgcn_readfirstlane((int)pay) != 0) != SHORT) return;
+
+#include "mx_gemm_pipe.h"
+#include "mx_gemm_wreg.h"
+#include "mx_gemm_pipe_fp4.h"
+
+// The side of the 128-row tiles, which is left at once where the choice falls on the other (mx_gemm_pipe_kernel).  A workgroup goes on with
+// further tiles, so that there are no more of them than run at a time: leaving takes each 0.3 us (256 groups x 48 rows c, 512, 1024, a
+// workgroup for each tile 33.9, so 26.3).
+__global__ __launch_bounds__(256) void mx_gemm_i8_short_kernel(const GemmParams p) {
+    const bool pay = p.sizes != nullptr ? short_tiles_pay_by_sizes(p, p.choice_cus) : table_at(p.short_tiles, 0) != 0;
+    if (__builtin_amdgcn_readfirstlane((int)pay) == 0) return;
     Tile tc;
-    for (uint32_t id = blockIdx.x; locate_tile<SHORT ? 128 : 256, Locate::kAny>(p, tc, id); id += gridDim.x) {
+    for (uint32_t id = blockIdx.x; locate_tile<128, Locate::kAny>(p, tc, id); id += gridDim.x) {
         if (id != blockIdx.x) __syncthreads();                 // the LDS of the tile before has been read
-        if constexpr (SHORT) ring_tile<kFmtI8, 256, 128, 2, 2, 3, 0, kEpiI8DequantSwiglu, false>(p, tc);
-        else dl_tile<kFmtI8, 256, 256, 2, 4, kEpiI8DequantSwiglu>(p, tc);
+        ring_tile<kFmtI8, 256, 128, 2, 2, 3, 0, kEpiI8DequantSwiglu, false>(p, tc);
     }
 }
 __global__ __launch_bounds__(256) void i8_choice_prepare_kernel(const GroupTablesJob job, uint32_t w_tiles, uint32_t cus, uint32_t kblocks,
@@ -907,30 +969,12 @@ int launch_i8_choice_tables(const GroupTablesJob& job, const GemmParams& p, int3
     return CMX_OK;
 }
 
-template <bool SHORT>
-int launch_i8_side(const GemmParams& p, const int32_t* short_tiles, uint32_t max_m_tiles, int cus, hipStream_t s) {
-    constexpr size_t smem = SHORT ? ring_lds_bytes(256, 128, 3, 0) : 2 * (256 + 256) * (kSlabBytes + 4);
-    constexpr auto kfn = mx_gemm_i8_choice_kernel<SHORT>;
-    if (int rc = allow_dynamic_lds<kfn, smem>(); rc != CMX_OK) return rc;
-    const uint64_t tiles = (uint64_t)max_m_tiles * p.w_tiles;
-    CMX_REQUIRE(tiles > 0 && tiles < (1ull << 31), "tile count out of range");
-    hipLaunchKernelGGL(kfn, dim3((uint32_t)std::min<uint64_t>(tiles, cus)), dim3(SHORT ? 256 : 512), smem, s, p, (uint32_t)cus, short_tiles);
-    CMX_LAUNCH_CHECK();
-    return CMX_OK;
-}
-// tiles128, tiles256: the most m-tiles that either side can have
-int launch_i8_choice(const GemmParams& p, const int32_t* short_tiles, uint32_t tiles128, uint32_t tiles256, hipStream_t s) {
-    int cus = 0;
-    if (int rc = cu_count(&cus); rc != CMX_OK) return rc;
-    if (int rc = launch_i8_side<true>(p, short_tiles, tiles128, cus, s); rc != CMX_OK) return rc;
-    return launch_i8_side<false>(p, short_tiles, tiles256, cus, s);
-}
-
 template <int FMT, int EPI, int TM, int WW, int WM, int NSLOT>
 int launch_gemm_pipe(const GemmParams& p, uint32_t max_m_tiles, hipStream_t s) {
     // tile ring, scale ring (two-slot kernels: two blocks of 16 bytes per row), next-tile mailbox, 256-byte sink of the L2 prefetch loads
     // (+ the 16 KiB staging area of the whole-line stores, which overlays the last 512 bytes)
-    constexpr size_t smem = NSLOT * (256 + TM) * kSlabBytes + (NSLOT == 2 ? 2 * (256 + TM) * 16 : NSLOT * (256 + TM) * 4) +
+    // (INT8: the scales of two tiles instead of the scale ring, and a staging area of its own)
+    constexpr size_t smem = NSLOT * (256 + TM) * kSlabBytes + (FMT == kFmtI8 ? 2 * (256 + TM) * 4 + 16384 : NSLOT == 2 ? 2 * (256 + TM) * 16 : NSLOT * (256 + TM) * 4) +
                             (pipe_stages_stores(NSLOT, EPI, WW, WM) ? 16384 : 512);
     constexpr auto kfn = mx_gemm_pipe_kernel<FMT, EPI, TM, WW, WM, NSLOT>;
     if (int rc = allow_dynamic_lds<kfn, smem>(); rc != CMX_OK) return rc;
@@ -947,6 +991,18 @@ int launch_gemm_pipe(const GemmParams& p, uint32_t max_m_tiles, hipStream_t s) {
     hipLaunchKernelGGL(kfn, dim3(grid), dim3(256), smem, s, p);
     CMX_LAUNCH_CHECK();
     return CMX_OK;
+}
+
+// tiles128, tiles256: the most m-tiles that either side can have
+int launch_i8_choice(const GemmParams& p, uint32_t tiles128, uint32_t tiles256, hipStream_t s) {
+    constexpr size_t smem = ring_lds_bytes(256, 128, 3, 0);
+    constexpr auto kfn = mx_gemm_i8_short_kernel;
+    if (int rc = allow_dynamic_lds<kfn, smem>(); rc != CMX_OK) return rc;
+    const uint64_t tiles = (uint64_t)tiles128 * p.w_tiles;
+    CMX_REQUIRE(tiles > 0 && tiles < (1ull << 31), "tile count out of range");
+    hipLaunchKernelGGL(kfn, dim3((uint32_t)std::min<uint64_t>(tiles, p.choice_cus)), dim3(256), smem, s, p);
+    CMX_LAUNCH_CHECK();
+    return launch_gemm_pipe<kFmtI8, kEpiI8DequantSwiglu, 256, 2, 2, 2>(p, tiles256, s);
 }
 
 template <int FMT, int EPI, int TM>
@@ -1172,6 +1228,17 @@ TileChoice choose_tile(uint32_t m_hint, uint32_t n, int fmt, bool grouped) {
     return {256, 256, grouped && m_hint < 512 ? 5 : 4};
 }
 
+// 16-bit output whose rows start at whole 16-byte pieces takes the lean store epilogue, and with it the persistent kernels
+bool lean_store(const GemmParams& p) {
+    return p.out_type != CMX_OUT_FP32 && p.n % 8 == 0 && p.ldc % 8 == 0 && (reinterpret_cast<uintptr_t>(p.c) & 15u) == 0;
+}
+// Whether launch_tile takes a grouped problem to a persistent kernel that scans the group sizes by itself.
+bool scans_groups(const GemmParams& p, const TileChoice& t, int fmt, bool swiglu) {
+    if (g_disable_dl || p.w_pretiled || t.tw != 256 || t.tm != 256 || t.waves != 4 || !p.scale_vec16) return false;
+    if (swiglu) return p.act_bf16 == nullptr && p.kbytes % (4 * kSlabBytes) == 0;
+    return fmt == CMX_FMT_E2M1 && lean_store(p) && p.kbytes % (2 * kSlabBytes) == 0;
+}
+
 // Eight-wavefront shapes exist only as streaming kernels; when a problem is not eligible for
 // streaming (ragged K, unaligned scale rows) the four-wavefront register-staged kernel of the same
 // tile takes over.
@@ -1183,8 +1250,7 @@ int launch_tile(const GemmParams& p, int waves, uint32_t max_m_tiles, hipStream_
         if ((waves == 4 || waves == 5) && stream_ok && p.scale_vec16 && p.kbytes % (4 * kSlabBytes) == 0) {
             // plain 16-bit output with 8-element-aligned rows takes the lean store epilogue and with it the persistent kernel
             constexpr int kLeanBf16 = EPI == kEpiStore ? kEpiStoreBf16 : EPI, kLeanFp16 = EPI == kEpiStore ? kEpiStoreFp16 : EPI;
-            const bool lean = EPI == kEpiStore && p.out_type != CMX_OUT_FP32 && p.n % 8 == 0 && p.ldc % 8 == 0 &&
-                              (reinterpret_cast<uintptr_t>(p.c) & 15u) == 0;
+            const bool lean = EPI == kEpiStore && lean_store(p);
             // (the 4 x 1 layout with the lean store epilogue does not fit the register file without spilling
             // inside the loop, so the persistent store kernel is always 2 x 2)
             if (lean && p.out_type == CMX_OUT_BF16) return launch_gemm_pipe<FMT, kLeanBf16, 256, 2, 2, 2>(p, max_m_tiles, s);
@@ -1198,7 +1264,7 @@ int launch_tile(const GemmParams& p, int waves, uint32_t max_m_tiles, hipStream_
         if ((waves == 4 || waves == 5) && stream_ok && p.scale_vec16 && p.kbytes % (2 * kSlabBytes) == 0) {
             if constexpr (EPI == kEpiStore) {
                 // plain 16-bit output with 8-element-aligned rows: lean store epilogue, persistent kernel
-                const bool lean = p.out_type != CMX_OUT_FP32 && p.n % 8 == 0 && p.ldc % 8 == 0 && (reinterpret_cast<uintptr_t>(p.c) & 15u) == 0;
+                const bool lean = lean_store(p);
                 // (unlike the 8-bit kernel, whose fragments take twice the registers, the 4 x 1 layout fits here too)
                 if (lean && waves == 4 && p.out_type == CMX_OUT_BF16) return launch_gemm_pipe_fp4<kEpiStoreBf16, 2, 2>(p, max_m_tiles, s);
                 if (lean && waves == 4) return launch_gemm_pipe_fp4<kEpiStoreFp16, 2, 2>(p, max_m_tiles, s);
@@ -1481,10 +1547,10 @@ uint32_t max_group_tiles(uint32_t m_total, uint32_t groups, uint32_t tile_m, uin
 // Where n is at most 128, half of a 256-row tile would be empty: 128 x 128 for 256 x 128 (SwiGLU 256 x 68 z, 3072, 64 45 -> 34 where 256 x 128 takes
 // 48; FP4 256 x 128 u, 512, 64 20 -> 16, 23; INT8 256 x 128 u, 128, 128 17.5 -> 14.1, 20.1).
 // Problems of more tiles stay on the persistent kernels (32 x 194 rows, 7168, 4096: 287 against 311 with 128 x 256).
-// INT8, whose only other kernel has 256 x 256 tiles, one per workgroup (us, fp32 output):
+// INT8, whose other kernels have 256 x 256 tiles (us, fp32 output; against the streaming kernel, one of them per workgroup):
 //   128 x 128    8 x 44 u, 4096, 2048 46.5 -> 21.6     8 x 200 u 47.7 -> 27.0     16 x 100 z, 7168, 1024 73.2 -> 34.8     16 x 44 u, 2048, 2048 29.7 -> 16.9
 //   256 x 128    32 x 44 u, 7168, 4096 222 -> 178       32 x 100 z 299 -> 232      32 x 100 z, 1152, 2048 46.3 -> 37.3: from K = 512 on, and where the device
-//                chooses it (mx_gemm_i8_choice_kernel)
+//                chooses it (mx_gemm_i8_short_kernel)
 //   128 x 256    16 x 200 u, 7168, 1024 71.8 -> 50.9; of more than a round 32 x 200 u, 7168, 4096 278 against 251, 16 x 2048 1077 against 1003
 // FP4, whose other kernels past the split-K sizes have tiles of 256 x 128 and 256 x 256 (us, bf16 output):
 //   128 x 128    8 x 70 u, 4096, 2048 31.6 -> 15.9     8 x 200 u 36.0 -> 18.4     16 x 100 z, 7168, 1024 46.9 -> 24.1     8 x 70 u, 7168, 4096 49 -> 26
@@ -1549,8 +1615,10 @@ int gmm_common(GemmParams& p, const int32_t* group_sizes, uint32_t groups, uint3
     const TileChoice& t = plan.t;
     const bool all_ksplit = plan.all_ksplit();
     const GroupTables tables(workspace, groups);
-    bool by_sizes = false;                                     // (the persistent kernels walk from tile to tile through tables)
-    if (!tables_filled && (all_ksplit || t.waves == kRing)) {
+    bool by_sizes = false;
+    if (!tables_filled && !all_ksplit && ks.small_rows == 0 && scans_groups(p, t, fmt, swiglu)) {
+        by_sizes = groups <= kInlineGroups;                    // (the other persistent kernels walk from tile to tile through tables)
+    } else if (!tables_filled && (all_ksplit || t.waves == kRing)) {
         const uint64_t tiles = all_ksplit ? (uint64_t)(m_total / 64 + groups) * ceil_div(p.n, 64) : (uint64_t)(m_total / t.tm + groups) * ceil_div(p.n, t.tw);
         if (int rc = tiles_by_sizes(&by_sizes, groups, tiles, all_ksplit ? 2 : 1); rc != CMX_OK) return rc;
     }
@@ -1665,26 +1733,39 @@ extern "C" int cmx_int8_gmm_dequant_swiglu(const int8_t* a, uint32_t lda, const 
     if (int rc = choose_grouped_ksplit(m_total, groups, n, kFmtI8, p.kblocks, &ks); rc != CMX_OK) return rc;
     const bool all_ksplit = ks.tile.fw != 0 && ks.small_rows == 0;
     TileChoice t = {256, ceil_div(m_total, groups) <= 128 ? 128 : 256, 8};
+    // The persistent kernel of 256 x 256 tiles stores 16 bytes at a time and has the scales' offsets in 32 bits; the streaming kernel takes the rest.
+    const bool pipe = (!g_force_tile.tw || g_force_tile.waves == 4) && !g_disable_dl && k >= 2 * kSlabBytes && (uint64_t)ld_out * (out_type == CMX_OUT_FP32 ? 4 : 2) % 16 == 0 &&
+                      aligned16(out) && (uint64_t)n * channel_scale_stride * 4 < (1ull << 32);
     bool choice = false;                                       // 128- or 256-row tiles: the device chooses by the sizes
     if (g_force_tile.waves == kRing) t = g_force_tile;
     else if (!g_force_tile.tw && !g_disable_dl) {
         if (int rc = ring_groups(&t, m_total, groups, n, kFmtI8, p.kblocks, true); rc != CMX_OK) return rc;
-        choice = !all_ksplit && t.waves == kRing && t.tw == 256;
+        choice = !all_ksplit && t.waves == kRing && t.tw == 256 && pipe;
     }
     if (t.waves != kRing) t.tm = 256;
-    // All kernels of the call take one tile per workgroup.  Past the rounds up to which they find it by the sizes, the launch that fills the
-    // tables makes the choice.  Where it would fill them for small groups as well, those that are left to the large tiles are large for
-    // their average (256 x 32, 7168, 4096, on eight groups 227 against 277).
+    // Kernels of one tile per workgroup find it by the sizes up to some rounds; past those the launch that fills the tables makes the
+    // choice.  Where it would fill them for small groups as well, those that are left to the large tiles are large for
+    // their average (256 x 32, 7168, 4096, on eight groups 227 against 277).  The persistent kernel scans the sizes once.
     bool by_sizes = false;
-    const uint64_t most = all_ksplit ? (uint64_t)(m_total / 64 + groups) * ceil_div(n, 64) : (uint64_t)(m_total / t.tm + groups) * ceil_div(n, t.tw);
-    // (a choice by the sizes is a second scan for every tile)
-    if (int rc = tiles_by_sizes(&by_sizes, groups, choice && ks.small_rows == 0 ? 3 * most : most, all_ksplit ? 2 : 1); rc != CMX_OK) return rc;
+    if (pipe && !all_ksplit && t.waves != kRing && ks.small_rows == 0) {
+        by_sizes = groups <= kInlineGroups;
+    } else {
+        const uint64_t most = all_ksplit ? (uint64_t)(m_total / 64 + groups) * ceil_div(n, 64) : (uint64_t)(m_total / t.tm + groups) * ceil_div(n, t.tw);
+        // (a choice by the sizes is a second scan for every tile)
+        if (int rc = tiles_by_sizes(&by_sizes, groups, choice && ks.small_rows == 0 ? 3 * most : most, all_ksplit ? 2 : 1); rc != CMX_OK) return rc;
+    }
     if (choice && !by_sizes && ks.small_rows != 0) {
         choice = false;
         t = {256, 256, 8};
     }
     const GroupTables tables(ws, groups);
     const GroupTablesJob job = tables_job(tables, group_sizes, groups, m_total, all_ksplit ? 16 * ks.tile.fm : t.tm, ks.small_rows);
+    if (choice) {
+        int cus = 0;
+        if (int rc = cu_count(&cus); rc != CMX_OK) return rc;
+        p.choice_cus = (uint32_t)cus;
+        p.short_tiles = tables.small_pref;
+    }
     p.w_tiles = ceil_div(n / 2, t.tw / 2);
     if (choice && !by_sizes)
         if (int rc = launch_i8_choice_tables(job, p, tables.small_pref, s); rc != CMX_OK) return rc;
@@ -1692,11 +1773,10 @@ extern "C" int cmx_int8_gmm_dequant_swiglu(const int8_t* a, uint32_t lda, const 
     if (ks.tile.fw != 0)
         if (int rc = launch_grouped_ksplit(p, tables, ks, kFmtI8, kEpiI8DequantSwiglu, m_total, s); rc != CMX_OK || all_ksplit) return rc;
     const uint32_t max_m_tiles = max_group_tiles(m_total, groups, t.tm, ks.small_rows);
-    if (choice) return launch_i8_choice(p, tables.small_pref, max_m_tiles, max_group_tiles(m_total, groups, 256, ks.small_rows), s);
+    p.tile_ctr = nullptr;                                      // tiles of one cost: fixed strides
+    if (choice) return launch_i8_choice(p, max_m_tiles, max_group_tiles(m_total, groups, 256, ks.small_rows), s);
     if (t.waves == kRing) return launch_ring(p, {t.tw, t.tm}, kFmtI8, kEpiI8DequantSwiglu, false, max_m_tiles, s);
-    // (hand-scheduled variants of this kernel were measured twice at 16 x 2048 x 7168 x 4096 and are not kept: two i8
-    // MFMAs per step and accumulator in the 8-bit schedule 997 us, one per 32-K step in the 16-byte-fragment
-    // schedule shared with FP4, one tile per workgroup, 994-1000 us, against 967-975 us for this one)
+    if (pipe) return launch_gemm_pipe<kFmtI8, kEpiI8DequantSwiglu, 256, 2, 2, 2>(p, max_m_tiles, s);
     return launch_gemm_dl<kFmtI8, 256, 256, 2, 4, kEpiI8DequantSwiglu>(p, max_m_tiles, s);
 }
 

@@ -55,6 +55,8 @@ struct GemmParams {
     const int32_t* sizes;       // [groups] rows of the groups, in the place of row_off and tile_pref (at most kInlineGroups), or null
     uint32_t small_rows;        // with `sizes`: the limit between ...
     int group_class;            // ... the groups that this launch takes (GroupClass)
+    const int32_t* short_tiles; // INT8, 128- or 256-row tiles chosen on the device (choice_cus != 0): the choice, where tables have been filled
+    uint32_t choice_cus;        // ... and the workgroups that run at a time
 };
 
 __device__ __forceinline__ uint32_t swz(uint32_t row, uint32_t chunk) {
@@ -90,6 +92,7 @@ __device__ __forceinline__ float i8_dequant(int32_t sum, float channel_scale) {
 struct Tile {
     uint32_t g, mt, wt, row0, rows_valid;
     uint32_t rows_left;      // rows of the group (or problem) from row0 on
+    uint32_t group_tiles;    // m-tiles of the group (or problem)
 };
 
 // The group tables (row offsets, m-tile prefix) are written by gmm_prepare_kernel before the matmul kernel starts and
@@ -129,7 +132,6 @@ __device__ __forceinline__ void interleave_xcd_walk(uint32_t total_tiles, uint32
     stride = gridDim.x;
     end = total_tiles;
 }
-
 // The tile after tile_id of such a walk, or `end`.  In the last, partly filled round the XCDs take fewer tiles each, in whole bands of 8: in
 // blocks of 32 they would all lie on the first XCDs, and the L2s and links of the others would have nothing to do.  320 tiles on 256
 // workgroups (us): SwiGLU 8 x 1280 rows, K = 4096, N = 2048 124.5 -> 112.6, FP4 125.7 -> 117.2, dense 8192 x 5120 x 7168 (640 tiles) 281 -> 264; 384
@@ -161,6 +163,7 @@ __device__ __forceinline__ void place_in_group(const GemmParams& p, uint32_t g, 
                                                uint32_t L, Tile& t) {
     t.g = g;
     const uint32_t mtg = tp1 - tp;
+    t.group_tiles = mtg;
     const uint32_t local = L - tp * p.w_tiles;
     const uint32_t band = 8;
     const uint32_t per_band = band * p.w_tiles;
@@ -181,6 +184,7 @@ __device__ __forceinline__ void place_dense(const GemmParams& p, uint32_t m_tile
     const uint32_t b = L / per_band, within = L % per_band;
     const uint32_t band_rows = (m_tiles_all - b * band) < band ? (m_tiles_all - b * band) : band;
     t.g = 0;
+    t.group_tiles = m_tiles_all;
     t.mt = b * band + within % band_rows;
     t.wt = within / band_rows;
     t.row0 = t.mt * TM;
@@ -279,6 +283,42 @@ __device__ __forceinline__ bool locate_tile_by_sizes(const GemmParams& p, Tile& 
         tp += n;
     }
     return true;
+}
+
+// The same for persistent kernels: the groups are scanned once and stay in registers, so that the way to a further tile touches no memory.
+struct GroupScan {
+    uint32_t rows[kGroupsPerLane], row0, tile0;      // of the lane's groups: rows of each; first row and first m-tile of the first
+};
+// returns the m-tiles of all groups
+template <int TM>
+__device__ __forceinline__ uint32_t scan_groups(const GemmParams& p, GroupScan& gs) {
+    uint32_t off[kGroupsPerLane + 1], all = 0;
+    scan_group_rows(p, off);
+#pragma unroll
+    for (int j = 0; j < kGroupsPerLane; ++j) {
+        gs.rows[j] = off[j + 1] - off[j];
+        all += tiles_of_group(p, gs.rows[j], TM);
+    }
+    const uint32_t pref = wave_scan(all, [](uint32_t a, uint32_t b) -> uint32_t { return a + b; });
+    gs.row0 = off[0];
+    gs.tile0 = pref - all;
+    return (uint32_t)__builtin_amdgcn_readlane((int)pref, 63);
+}
+// tile L, which exists
+template <int TM>
+__device__ __forceinline__ void decode_scanned_tile(const GemmParams& p, const GroupScan& gs, uint32_t L, Tile& t) {
+    uint32_t end = gs.tile0;
+#pragma unroll
+    for (int j = 0; j < kGroupsPerLane; ++j) end += tiles_of_group(p, gs.rows[j], TM);
+    const int at = (int)__builtin_ctzll(__ballot(end * p.w_tiles > L));                          // lane of the tile's group
+    uint32_t tp = (uint32_t)__builtin_amdgcn_readlane((int)gs.tile0, at), r0 = (uint32_t)__builtin_amdgcn_readlane((int)gs.row0, at);
+#pragma unroll
+    for (int j = 0; j < kGroupsPerLane; ++j) {
+        const uint32_t rows = (uint32_t)__builtin_amdgcn_readlane((int)gs.rows[j], at), n = tiles_of_group(p, rows, TM);
+        if (L >= tp * p.w_tiles && L < (tp + n) * p.w_tiles) place_in_group<TM>(p, kGroupsPerLane * at + j, tp, tp + n, r0, r0 + rows, L, t);
+        tp += n;
+        r0 += rows;
+    }
 }
 
 // How a kernel finds its tiles: without a look for groups, in their tables (or none), by their sizes, or as the parameters say.  What a kernel

@@ -21,6 +21,11 @@
 // second half's weight fragments first, free the weight rows of the slot with a barrier after MFMA 4 (2 x 2) or 2 (4 x 1)
 // and send all eight weight loads of slab s+2 behind the following MFMAs; the persistent 2 x 2 kernels also issue two L2
 // prefetch loads per slab in step 1: see kWFirst and CMX_PIPE_PREFETCH below.)
+// INT8 (kFmtI8) runs on the same schedule with two v_mfma_i32_32x32x32_i8 in the place of a block-scaled MFMA, first the lower halves of all
+// fragments of a step, then the upper ones, so that no MFMA waits for the one before it; no block scales, and the epilogue's channel and
+// token scales travel to the LDS with the first slab of their tile.  Against the streaming kernel of eight wavefronts, one tile per
+// workgroup, that the call ran before (us, call with sort and quantise + scatter, fp32 output): 16 groups of 2048 rows (Zipf), K = 7168,
+// N = 4096 977 -> 840; 8 groups of 2048, 4096, 2048 148 -> 134, at K = 512 60 -> 51; one round of tiles 76.5 -> 73.
 // Every LDS address is a per-lane base register plus an immediate, every global address a per-lane
 // offset register plus a scalar slab offset: the loop contains no address arithmetic on the VALU.
 #pragma once
@@ -96,6 +101,12 @@ __device__ __forceinline__ void mfma_acc(v16f& acc, const v8i& w, const v8i& a, 
     }
 }
 #undef CMX_PIPE_MFMA
+// INT8: c0 += w0 x a0 and c1 += w0 x a1, 32 deep each (v_mfma_i32_32x32x32_i8), half the work of a 64-deep step on two accumulators: the
+// two halves of a step on ONE accumulator back to back would wait for each other
+__device__ __forceinline__ void mfma_acc_i8(v16f& c0, v16f& c1, const v4i& w, const v4i& a0, const v4i& a1) {
+    asm volatile("v_mfma_i32_32x32x32_i8 %0, %2, %3, %0\n\tv_mfma_i32_32x32x32_i8 %1, %2, %4, %1"
+                 : "+a"(c0), "+a"(c1) : "v"(w), "v"(a0), "v"(a1));
+}
 
 // MFMA sequence of a step: the operand with more fragments runs in the outer loop (weights on a tie).  The
 // fragments (0..FW-1 weights, FW..FW+FM-1 activations) are read in the order of their first use by it.
@@ -144,7 +155,8 @@ __host__ __device__ constexpr bool pipe_stages_stores(int nslot, int epi, int ww
 
 template <int FMT, int EPI, int TM, int WW, int WM, int NSLOT>
 __global__ __launch_bounds__(256) void mx_gemm_pipe_kernel(const GemmParams p) {
-    static_assert(FMT == CMX_FMT_E4M3 || FMT == CMX_FMT_E5M2, "8-bit element formats only");
+    constexpr bool kI8 = FMT == kFmtI8;                        // INT8: no block scales
+    static_assert(FMT == CMX_FMT_E4M3 || FMT == CMX_FMT_E5M2 || (kI8 && EPI == kEpiI8DequantSwiglu && NSLOT == 2 && WW == 2 && WM == 2), "8-bit element formats only");
     static_assert((TM == 256 && NSLOT == 2 && ((WW == 2 && WM == 2) || (WW == 4 && WM == 1))) ||
                       (TM == 128 && NSLOT == 3 && WW == 4 && WM == 1), "tile / ring / wavefront layout");
     constexpr int TW = 256, NW = 4, FW = TW / WW / 32, FM = TM / WM / 32, NF = FW + FM;
@@ -159,7 +171,8 @@ __global__ __launch_bounds__(256) void mx_gemm_pipe_kernel(const GemmParams p) {
     // the vector L1 as the tile data itself.  Their scale ring holds two such blocks, [block][row][4 dwords].
     // The three-slot kernel keeps one dword per row and slab, [slot][row].
     constexpr bool kSc4 = NSLOT == 2;
-    constexpr int kScaleSlotBytes = kSc4 ? kRows * 16 : kRows * 4;
+    // INT8: [tile parity][row], the fp32 channel and token scales of a tile, which its epilogue reads
+    constexpr int kScaleSlotBytes = kSc4 && !kI8 ? kRows * 16 : kRows * 4;
     constexpr int kScaleRingBytes = kSc4 ? 2 * kScaleSlotBytes : NSLOT * kScaleSlotBytes;
     constexpr int kTileLoads = kRows / (8 * NW);              // LDS-DMA loads per wavefront and slab (16 or 12)
     constexpr int kWTileLoads = TW / (8 * NW);                // the first 8 fetch weight rows
@@ -184,7 +197,20 @@ __global__ __launch_bounds__(256) void mx_gemm_pipe_kernel(const GemmParams p) {
     // workgroup (the general store epilogue with its three output types and edge cases needs too many
     // registers to sit inside the loop).
     constexpr bool kPersistent = pipe_is_persistent(NSLOT, EPI);
-    const uint32_t m_tiles_all = count_m_tiles<TM>(p);
+    // Grouped problems: the tiles come from tables (the FFN's, problems of more than kInlineGroups groups) or, in the fixed-stride walk of the
+    // persistent 2 x 2 kernels, from a scan of the sizes that stays in seven registers: the launch that fills the tables takes 5 us, the scan
+    // 1, about as long as the chain of table reads that it replaces.
+    // (The store epilogues leave those registers only to the FP4 kernel: here they would spill 249.)
+    constexpr bool kScan = kPersistent && WW == 2 && WM == 2 && (EPI == kEpiSwigluQuant || kI8);
+    const bool grouped = p.row_off != nullptr || (kScan && p.sizes != nullptr);
+    GroupScan groups = {};
+    if constexpr (kI8) {
+        if (p.choice_cus != 0) {
+            const bool pay = p.sizes != nullptr ? short_tiles_pay_by_sizes(p, p.choice_cus) : table_at(p.short_tiles, 0) != 0;
+            if (__builtin_amdgcn_readfirstlane((int)pay) != 0) return;
+        }
+    }
+    const uint32_t m_tiles_all = kScan && p.sizes != nullptr ? scan_groups<TM>(p, groups) : count_m_tiles<TM>(p);
     const uint32_t total_tiles = m_tiles_all * p.w_tiles;
     uint32_t run_count;
     const uint32_t run_first = xcd_run(total_tiles, blockIdx.x % kXcds, run_count);
@@ -214,20 +240,21 @@ __global__ __launch_bounds__(256) void mx_gemm_pipe_kernel(const GemmParams p) {
         return r;
     };
     auto aim_loads_at = [&](uint32_t L, uint32_t g_from) {
-        decode_tile<TM>(p, m_tiles_all, L, tq, g_from);
+        if (kScan && p.sizes != nullptr) decode_scanned_tile<TM>(p, groups, L, tq);
+        else decode_tile<TM>(p, m_tiles_all, L, tq, g_from);
         const uint32_t g = __builtin_amdgcn_readfirstlane(tq.g), wt = __builtin_amdgcn_readfirstlane(tq.wt);
         const uint32_t row0 = __builtin_amdgcn_readfirstlane(tq.row0);
         const uint32_t rows_valid = __builtin_amdgcn_readfirstlane(tq.rows_valid);
         tq.g = g; tq.wt = wt; tq.row0 = row0; tq.rows_valid = rows_valid;
         tq.mt = __builtin_amdgcn_readfirstlane(tq.mt);
         w_rs = make_rsrc(p.w + (size_t)g * p.n * p.ldw);
-        ws_rs = make_rsrc(p.w_scale + (size_t)g * p.n * p.ld_ws);
+        ws_rs = make_rsrc(p.w_scale + (size_t)g * p.n * p.ld_ws * (kI8 ? 4 : 1));
         a_rs = make_rsrc(p.a + (size_t)row0 * p.lda);
-        as_rs = make_rsrc(p.a_scale + (size_t)row0 * p.ld_as);
+        as_rs = make_rsrc(p.a_scale + (size_t)row0 * (kI8 ? 4 : p.ld_as));
         // global row of tile row r (rows past the edge re-read the last valid row; their results are never stored)
         auto wrow_of = [&](uint32_t r) -> uint32_t {
             uint32_t gr;
-            if (epi_is_swiglu_quant(EPI)) {
+            if (epi_pairs_gate_up(EPI)) {
                 const uint32_t half = p.n >> 1;
                 uint32_t rr = r < TW / 2 ? wt * (TW / 2) + r : wt * (TW / 2) + (r - TW / 2);
                 rr = rr < half ? rr : half - 1;
@@ -249,16 +276,16 @@ __global__ __launch_bounds__(256) void mx_gemm_pipe_kernel(const GemmParams p) {
         }
         // scale dwords: this wavefront fetches those of weight rows 64*wave.. and of activation rows
         // 64*(wave mod TM/64).. (with TM = 128 two wavefronts fetch the same rows to the same place)
-        sgoff_w = wrow_of(64 * wave + lane) * p.ld_ws;
-        sgoff_a = arow_of(64 * sa_blk + lane) * p.ld_as;
+        sgoff_w = wrow_of(64 * wave + lane) * p.ld_ws * (kI8 ? 4 : 1);
+        sgoff_a = arow_of(64 * sa_blk + lane) * (kI8 ? 4 : p.ld_as);
         if constexpr (kPf > 0) {
             static_assert(kPf == 0 || (TW == 256 && TM == 256), "the prefetch split assumes 256 + 256 rows");
             // The workgroups that run side by side on an XCD share operand panels (tile order: bands of m-tiles, m
             // fastest, across a run of weight tiles): the weight panel with the other m-tiles of the band.  Each
             // prefetches only its share of the panel's rows (row = position in the band, modulo the band's height);
             // the lanes left over repeat the last such row.
-            const uint32_t band = p.row_off != nullptr ? 8u : 4u;
-            const uint32_t mtg = p.row_off != nullptr ? (uint32_t)table_at(p.tile_pref, g + 1) - (uint32_t)table_at(p.tile_pref, g) : m_tiles_all;
+            const uint32_t band = grouped ? 8u : 4u;
+            const uint32_t mtg = tq.group_tiles;
             const uint32_t mt = tq.mt, b0 = mt / band * band;
             const uint32_t mod = __builtin_amdgcn_readfirstlane(mtg - b0 < band ? mtg - b0 : band);      // m-tiles that share the weight panel
             const uint32_t sel = __builtin_amdgcn_readfirstlane(mt - b0);
@@ -271,7 +298,7 @@ __global__ __launch_bounds__(256) void mx_gemm_pipe_kernel(const GemmParams p) {
                 // panels: 855.6 / 859.4 / 861.1 / 869.3 us.  Dense problems, whose workgroups run in lock step, lose 1-2 %.
                 // At most 86 rows: the two loads of wavefront 0 cover them, every other lane repeats the last one.
                 uint32_t r = sel + mod * (j * 64 + lane);
-                r = (r < 256u && wave == 0 && mod >= 3u && p.row_off != nullptr) ? r : last;
+                r = (r < 256u && wave == 0 && mod >= 3u && grouped) ? r : last;
                 pfoff[j] = mul_lo_u32(wrow_of(r), p.ldw);
             }
         }
@@ -280,9 +307,11 @@ __global__ __launch_bounds__(256) void mx_gemm_pipe_kernel(const GemmParams p) {
     Tile tc = tq;                               // tile of the MFMA stream / epilogue
 
     auto nslab_of = [](const GemmParams& q) -> uint32_t { return q.kbytes / kSlabBytes; };
-    const uint32_t nslab = nslab_of(p);
+    const uint32_t nslab_k = nslab_of(p);
+    // INT8 takes any number of slabs: an odd one is filled up with a slab of zeros
+    const uint32_t nslab = kI8 ? (nslab_k + 1) & ~1u : nslab_k;
     const uint32_t dma_base = __builtin_amdgcn_readfirstlane(lds0 + wave * 1024);
-    constexpr int kScaleRowBytes = kSc4 ? 16 : 4;
+    constexpr int kScaleRowBytes = kSc4 && !kI8 ? 16 : 4;
     const uint32_t sdma_base = __builtin_amdgcn_readfirstlane(lds0 + kScaleBase + wave * 64 * kScaleRowBytes);
     const uint32_t sdma_base_a = __builtin_amdgcn_readfirstlane(lds0 + kScaleBase + (TW + sa_blk * 64) * kScaleRowBytes);
 
@@ -300,13 +329,18 @@ __global__ __launch_bounds__(256) void mx_gemm_pipe_kernel(const GemmParams p) {
     auto issue_scale_block = [&](uint32_t blk) {
         const uint32_t pos = blocks_issued & 1u;
         ++blocks_issued;
+        if constexpr (kI8) {
+            dma_b32(sdma_base + pos * kScaleSlotBytes, sgoff_w, ws_rs, 0);
+            dma_b32(sdma_base_a + pos * kScaleSlotBytes, sgoff_a, as_rs, 0);
+            return;
+        }
         dma_b128(sdma_base + pos * kScaleSlotBytes, sgoff_w, ws_rs, blk * 16);
         dma_b128(sdma_base_a + pos * kScaleSlotBytes, sgoff_a, as_rs, blk * 16);
     };
     // the load stream is at slab q of its tile: block 0 goes out with slab 0, block b+1 with slab 4b+1 (the ring
     // position it takes was last read one slab earlier)
     const uint32_t nblk = nslab_of(p) / 4;
-    auto scale_block_due = [&](uint32_t q) -> bool { return q == 0 || ((q & 3u) == 1u && (q >> 2) + 1 < nblk); };
+    auto scale_block_due = [&](uint32_t q) -> bool { return kI8 ? q == 0 : q == 0 || ((q & 3u) == 1u && (q >> 2) + 1 < nblk); };
     auto scale_block_of = [&](uint32_t q) -> uint32_t { return q == 0 ? 0u : (q >> 2) + 1; };
     auto clamp_slab = [&](uint32_t slab) -> uint32_t { return slab < nslab ? slab : nslab - 1; };   // past the end: harmless reload
 
@@ -314,7 +348,7 @@ __global__ __launch_bounds__(256) void mx_gemm_pipe_kernel(const GemmParams p) {
     // a lane reads 16-byte chunks lh, lh+2 (step 0) and lh+4, lh+6 (step 1) of its row; all rows of a
     // lane share the low five bits l32, hence the swizzle term
     const uint32_t x = (l32 & 7u) ^ ((l32 >> 3) & 1u);
-    const uint32_t w_row_base = epi_is_swiglu_quant(EPI) ? ww * (TW / 2 / WW) : ww * (TW / WW);
+    const uint32_t w_row_base = epi_pairs_gate_up(EPI) ? ww * (TW / 2 / WW) : ww * (TW / WW);
     uint32_t wb[NSLOT][4], ab[NSLOT][4];       // [slot][chunk j]
 #pragma unroll
     for (int s = 0; s < NSLOT; ++s)
@@ -347,7 +381,7 @@ __global__ __launch_bounds__(256) void mx_gemm_pipe_kernel(const GemmParams p) {
     uint32_t sraw[NF], scur[NSLOT][NF];      // shifted scales alternate between two sets: a set is rewritten one slab after its last use
 
     // weight fragment f sits f*32 rows (SwiGLU: the gate fragments, then their up partners 128 rows on) below the base
-#define CMX_PIPE_WOFF(f) ((epi_is_swiglu_quant(EPI) ? ((f) < FW / 2 ? (f) * 32 : TW / 2 + ((f) - FW / 2) * 32) : (f) * 32))
+#define CMX_PIPE_WOFF(f) ((epi_pairs_gate_up(EPI) ? ((f) < FW / 2 ? (f) * 32 : TW / 2 + ((f) - FW / 2) * 32) : (f) * 32))
     // one 16-byte read: r = 2 * position in the read order + half (0: registers 0-3, 1: registers 4-7)
     // The two-slot grouped kernels (persistent 2 x 2, and 4 x 1) read the step-1 fragments weights first: the weight rows of a
     // slot are then free a few MFMAs into step 0 (four with 2 x 2 wavefronts, two with 4 x 1, whose wavefronts hold only two
@@ -394,7 +428,7 @@ __global__ __launch_bounds__(256) void mx_gemm_pipe_kernel(const GemmParams p) {
     if constexpr (kSc4) {
         // scale blocks first, so that the wait below can leave exactly the 16 tile loads of slab 1 in flight
         issue_scale_block(0);
-        if (nblk > 1) issue_scale_block(1);
+        if (!kI8 && nblk > 1) issue_scale_block(1);
 #pragma unroll
         for (int i = 0; i < kTileLoads; ++i) issue_tile_load(0, i, 0);
         const uint32_t k1 = clamp_slab(1);
@@ -407,7 +441,7 @@ __global__ __launch_bounds__(256) void mx_gemm_pipe_kernel(const GemmParams p) {
         }
         asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"n"(kTileLoads + kPf) : "memory");      // slab 0 and its scales have landed everywhere
         static_for<0, NF>([&](auto ic) { read_frag(I0{}, I0{}, ic, f0lo, f0hi); });
-        {
+        if constexpr (!kI8) {
             const uint32_t off = scale_read_offset();
             const uint32_t swb_at = swb + off, sab_at = sab + off;
             static_for<0, NF>([&](auto ic) { read_scale_at(swb_at, sab_at, ic); });
@@ -428,6 +462,7 @@ __global__ __launch_bounds__(256) void mx_gemm_pipe_kernel(const GemmParams p) {
 
     auto shift_scales = [&](auto set_c) {
         constexpr int set = decltype(set_c)::value;
+        if constexpr (kI8) return;
         (void)scur, (void)sraw, (void)sshift;      // asm operands alone do not make a generic lambda capture
 #pragma unroll
         for (int i = 0; i < NF; ++i) asm volatile("v_lshrrev_b32 %0, %1, %2" : "=v"(scur[set][i]) : "v"(sshift), "v"(sraw[i]));
@@ -441,8 +476,15 @@ __global__ __launch_bounds__(256) void mx_gemm_pipe_kernel(const GemmParams p) {
     uint32_t live = live_mask(tc.rows_valid);      // bit fm: block fm has valid rows
     auto step_mfma = [&](auto sel_c, auto i_c, v4i (&flo)[NF], v4i (&fhi)[NF], auto set_c) {
         constexpr int sel = decltype(sel_c)::value, i = decltype(i_c)::value, set = decltype(set_c)::value;
-        constexpr int fw = kMOuter ? i % FW : i / FM, fm = kMOuter ? i / FW : i % FM;
         (void)scur, (void)acc;
+        if constexpr (kI8) {
+            // first the lower halves of all fragments, then the upper ones, two accumulators a turn
+            constexpr int at = 2 * i % kM, w = at / FM, a = at % FM;
+            if constexpr (2 * i < kM) mfma_acc_i8(acc[w][a], acc[w][a + 1], flo[w], flo[FW + a], flo[FW + a + 1]);
+            else mfma_acc_i8(acc[w][a], acc[w][a + 1], fhi[w], fhi[FW + a], fhi[FW + a + 1]);
+            return;
+        }
+        constexpr int fw = kMOuter ? i % FW : i / FM, fm = kMOuter ? i / FW : i % FM;
         mfma_acc<FMT, sel, kSkip ? fm : -1>(acc[fw][fm], join8(flo[fw], fhi[fw]), join8(flo[FW + fm], fhi[FW + fm]), scur[set][fw],
                                             scur[set][FW + fm], live);
     };
@@ -458,6 +500,7 @@ __global__ __launch_bounds__(256) void mx_gemm_pipe_kernel(const GemmParams p) {
     auto pin_scales = [&](auto set_c) {
         constexpr int set = decltype(set_c)::value;
         (void)scur;
+        if constexpr (kI8) return;
 #pragma unroll
         for (int i = 0; i < NF; ++i) asm volatile("" ::"v"(scur[set][i]));
     };
@@ -480,6 +523,12 @@ __global__ __launch_bounds__(256) void mx_gemm_pipe_kernel(const GemmParams p) {
         static_assert(kM == 16 && kB1 + kScaleMfmas + 1 <= 14, "the scale shift must sit at least two MFMAs before the end of the step");
         using SlotT = std::integral_constant<int, slot>;
         using OtherT = std::integral_constant<int, slot ^ 1>;
+        if constexpr (kI8) {
+            // (a buffer of no bytes past K: its loads put zeros into the LDS)
+            const int range = __builtin_amdgcn_readfirstlane(koff < p.kbytes ? -1 : 0);
+            w_rs[2] = range;
+            a_rs[2] = range;
+        }
         const uint32_t sc_off = scale_read_offset();             // where the scales of the next slab sit
         const uint32_t swb_at = swb + sc_off, sab_at = sab + sc_off;
         ++scale_read_slab;
@@ -521,7 +570,7 @@ __global__ __launch_bounds__(256) void mx_gemm_pipe_kernel(const GemmParams p) {
                 constexpr int r = i * kR + decltype(jc)::value;
                 if constexpr (r < kReads) read_half(OtherT{}, I0{}, std::integral_constant<int, r>{}, f0lo, f0hi);
             });
-            if constexpr (i >= kB1 && i < kB1 + kScaleMfmas) {
+            if constexpr (!kI8 && i >= kB1 && i < kB1 + kScaleMfmas) {
                 read_scale_at(swb_at, sab_at, std::integral_constant<int, 2 * (i - kB1)>{});
                 if constexpr (2 * (i - kB1) + 1 < NF) read_scale_at(swb_at, sab_at, std::integral_constant<int, 2 * (i - kB1) + 1>{});
             }
@@ -636,6 +685,7 @@ __global__ __launch_bounds__(256) void mx_gemm_pipe_kernel(const GemmParams p) {
         uint32_t sq = 2;             // slab of the load stream within its tile
         bool next_ok = false;        // the load stream has moved on to a next tile
         uint32_t next_id = tile_id;
+        uint32_t scale_pos = 0;      // INT8: where the scales of the MFMA stream's tile lie
         for (;;) {
             if (sq == nslab) {
                 if (p.tile_ctr != nullptr) {
@@ -664,6 +714,10 @@ __global__ __launch_bounds__(256) void mx_gemm_pipe_kernel(const GemmParams p) {
                     // ago.)  No prefetch is issued again before two barriers of the next slab, when everyone is done here.
                     asm volatile("s_waitcnt vmcnt(0)\n\ts_barrier" ::: "memory");
                     lean_store_lines<TW, TM, WW, WM, EPI, FW, FM>(p, tc, acc, ww, wm, lane, lds0 + kScaleBase + kScaleRingBytes + wave * 4096);
+                } else if constexpr (kI8) {
+                    i8_store_lines<TW, TM, WW, WM, FW, FM>(p, tc, acc, ww, wm, lane, lds0 + kScaleBase + kScaleRingBytes + 512 + wave * 4096,
+                                                           lds0 + kScaleBase + scale_pos * kScaleSlotBytes);
+                    scale_pos ^= 1u;
                 } else {
                     epilogue<TW, TM, WW, WM, EPI, FW, FM>(p, tc, acc, ww, wm, lane);
                 }
@@ -683,7 +737,7 @@ __global__ __launch_bounds__(256) void mx_gemm_pipe_kernel(const GemmParams p) {
                 // The last slab has already read the new tile's first fragments and scales, but carrying them
                 // through the epilogue costs more registers than there are: read them again (slot 0, landed).
                 static_for<0, NF>([&](auto ic) { read_frag(I0{}, I0{}, ic, f0lo, f0hi); });
-                {
+                if constexpr (!kI8) {
                     --scale_read_slab;          // the slab whose scales the last body read: the new tile's slab 0
                     const uint32_t off = scale_read_offset();
                     const uint32_t swb_at = swb + off, sab_at = sab + off;

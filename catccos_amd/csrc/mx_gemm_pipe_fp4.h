@@ -101,7 +101,10 @@ __global__ __launch_bounds__(256) void mx_gemm_pipe_fp4_kernel(const GemmParams 
 
     // ---- tile sequence of this workgroup (see mx_gemm_pipe_kernel) ----
     constexpr bool kPersistent = pipe_is_persistent(2, EPI);
-    const uint32_t m_tiles_all = count_m_tiles<TM>(p);
+    constexpr bool kScan = kPersistent && WW == 2 && WM == 2;
+    const bool grouped = p.row_off != nullptr || (kScan && p.sizes != nullptr);
+    GroupScan groups = {};
+    const uint32_t m_tiles_all = kScan && p.sizes != nullptr ? scan_groups<TM>(p, groups) : count_m_tiles<TM>(p);
     const uint32_t total_tiles = m_tiles_all * p.w_tiles;
     uint32_t run_count;
     const uint32_t run_first = xcd_run(total_tiles, blockIdx.x % kXcds, run_count);
@@ -130,7 +133,8 @@ __global__ __launch_bounds__(256) void mx_gemm_pipe_fp4_kernel(const GemmParams 
         return r;
     };
     auto aim_loads_at = [&](uint32_t L, uint32_t g_from) {
-        decode_tile<TM>(p, m_tiles_all, L, tq, g_from);
+        if (kScan && p.sizes != nullptr) decode_scanned_tile<TM>(p, groups, L, tq);
+        else decode_tile<TM>(p, m_tiles_all, L, tq, g_from);
         const uint32_t g = __builtin_amdgcn_readfirstlane(tq.g), wt = __builtin_amdgcn_readfirstlane(tq.wt);
         const uint32_t row0 = __builtin_amdgcn_readfirstlane(tq.row0);
         const uint32_t rows_valid = __builtin_amdgcn_readfirstlane(tq.rows_valid);
@@ -158,8 +162,8 @@ __global__ __launch_bounds__(256) void mx_gemm_pipe_fp4_kernel(const GemmParams 
         sgoff_a = arow_of(64 * wave + lane) * p.ld_as;
         if constexpr (kPf > 0) {
             // each workgroup prefetches its share of the weight panel it has in common with the other m-tiles of its band
-            const uint32_t band = p.row_off != nullptr ? 8u : 4u;
-            const uint32_t mtg = p.row_off != nullptr ? (uint32_t)table_at(p.tile_pref, g + 1) - (uint32_t)table_at(p.tile_pref, g) : m_tiles_all;
+            const uint32_t band = grouped ? 8u : 4u;
+            const uint32_t mtg = tq.group_tiles;
             const uint32_t mt = tq.mt, b0 = mt / band * band;
             const uint32_t mod = __builtin_amdgcn_readfirstlane(mtg - b0 < band ? mtg - b0 : band);      // m-tiles that share the weight panel
             const uint32_t sel = __builtin_amdgcn_readfirstlane(mt - b0);
@@ -172,7 +176,7 @@ __global__ __launch_bounds__(256) void mx_gemm_pipe_fp4_kernel(const GemmParams 
                 // panels: 855.6 / 859.4 / 861.1 / 869.3 us.  Dense problems, whose workgroups run in lock step, lose 1-2 %.
                 // At most 86 rows: the two loads of wavefront 0 cover them, every other lane repeats the last one.
                 uint32_t r = sel + mod * (j * 64 + lane);
-                r = (r < 256u && wave == 0 && mod >= 3u && p.row_off != nullptr) ? r : last;
+                r = (r < 256u && wave == 0 && mod >= 3u && grouped) ? r : last;
                 pfoff[j] = mul_lo_u32(wrow_of(r), p.ldw);
             }
         }

@@ -38,7 +38,7 @@ FLAGS = ["--offload-arch=gfx950", "-O3", "-std=c++17", "-Xclang", "-target-featu
 
 # (explicit instantiation, the schedule's own vmcnt waits inside the stream: the early tile loads -- 7 or 8 (6 for FP4); the
 # persistent 2 x 2 kernels send all 8 weight loads early -- plus 2 prefetch loads in the persistent 2 x 2 kernels)
-#   mx_gemm_pipe_kernel<FMT, EPI, TM, WW, WM, NSLOT>; EPI 0 store, 1 SwiGLU + requant, 2 lean bf16, 4 lean fp16, 5 = 1 + bf16 activations
+#   mx_gemm_pipe_kernel<FMT, EPI, TM, WW, WM, NSLOT>; EPI 0 store, 1 SwiGLU + requant, 2 lean bf16, 3 INT8, 4 lean fp16, 5 = 1 + bf16 activations
 #   mx_gemm_pipe_fp4_kernel<EPI, WW, WM>
 #   mx_gemm_wreg_kernel<FMT, EPI, TM>: the wait at the start of a slab leaves the weight loads of the next slab and all loads of
 #   the one after in flight (8 + 16 or 17), and behind the slab that sent a scale block the loads of that block too
@@ -59,6 +59,7 @@ KERNELS = [
     ("mx_gemm_pipe_kernel<0, 5, 256, 4, 1, 2>", {8}),
     ("mx_gemm_pipe_kernel<0, 2, 256, 2, 2, 2>", {10}),
     ("mx_gemm_pipe_kernel<0, 4, 256, 2, 2, 2>", {10}),
+    ("mx_gemm_pipe_kernel<8, 3, 256, 2, 2, 2>", {10}),          # INT8 dequant + SwiGLU
     ("mx_gemm_pipe_kernel<0, 0, 256, 2, 2, 2>", {7}),
     ("mx_gemm_pipe_kernel<0, 0, 256, 4, 1, 2>", {8}),
     ("mx_gemm_pipe_kernel<0, 0, 128, 4, 1, 3>", {14}),

@@ -1,6 +1,6 @@
-"""The persistent 256 x 256 kernels with 2 x 2 wavefronts: their walk through more and less than whole rounds of tiles.
-Reference: the streaming kernel of the same tile, one tile per workgroup, whose K order is the
-same, so the outputs are the same bits."""
+"""The persistent 256 x 256 kernels with 2 x 2 wavefronts: their walk through more and less than whole rounds of tiles, groups found by a
+scan of the sizes, and the INT8 kernel.  Reference: the streaming kernel of the same tile, one tile per workgroup, whose K order (INT8:
+whole-number sums) is the same, so the outputs are the same bits."""
 import numpy as np
 import pytest
 import torch
@@ -52,3 +52,57 @@ def test_walk_through_rounds(kind, counts, n):
         return [ops.mx_gemm(a, a_s, w[0], w_s[0], k)]
     for got, ref in zip(*_pinned(call)):
         assert torch.equal(got.view(torch.uint8), ref.view(torch.uint8)) and bool((ref != 7).any())
+
+
+@pytest.mark.parametrize("sizes,rows", [([5, -3, 0, 700, 1], 706), ([40, 2 ** 31 - 1, 2 ** 31 - 1, 9], 300), ([0, 0, 0], 10), ([1] * 256, 256),
+                                        ([300, 0, 66, 1] * 64, 23000)])
+@pytest.mark.parametrize("kind", ["SwiGLU", "E2M1", "INT8"])
+def test_scanned_groups_are_those_of_the_tables(kind, sizes, rows):
+    """Up to 256 groups are scanned, more go through tables: empty groups behind the last one change nothing."""
+    from catccos_amd import ops
+    g = torch.Generator(device="cuda")
+    g.manual_seed(rows)
+    n, k, many = 64, 512, 300
+    kb = k // 2 if kind == "E2M1" else k
+    codes = lambda *shape: torch.randint(0, 256, shape, dtype=torch.uint8, device="cuda", generator=g) & 0xF7
+    a, w = codes(rows, kb), codes(many, n, kb)
+    a_s, w_s = (torch.randint(110, 125, s, dtype=torch.uint8, device="cuda", generator=g) for s in ((rows, k // 32), (many, n, k // 32)))
+    h = hooks_lib()
+    h.cmx_debug_force_ksplit(-1, 0, 0)
+    h.cmx_debug_force_tile(256, 256, 4)
+
+    def outputs(counts):
+        e, cnt = len(counts), dev(np.array(counts, dtype=np.int32))
+        if kind == "INT8":
+            return [ops.int8_gmm_dequant_swiglu(a.view(torch.int8), torch.ones(rows, device="cuda"), w[:e].view(torch.int8),
+                                                torch.full((e * n,), 1e-5, device="cuda"), cnt, n, k, 1, c=torch.zeros((rows, n // 2), device="cuda"))]
+        if kind == "SwiGLU":
+            outs = torch.zeros((rows, n // 2), dtype=torch.uint8, device="cuda"), torch.zeros((rows, 2), dtype=torch.uint8, device="cuda")
+            return ops.mx_gmm_swiglu_quant(a, a_s, w[:e], w_s[:e], cnt, k, outs=outs)[:2]
+        return [ops.mx_gmm(a, a_s, w[:e], w_s[:e], cnt, k, "E2M1", c=torch.zeros((rows, n), dtype=torch.bfloat16, device="cuda"))]
+    for got, want in zip(outputs(sizes), outputs(sizes + [0] * (many - len(sizes)))):
+        assert torch.equal(got, want) and (bool((got != 0).any()) or sum(sizes) == 0)
+
+
+# K of two slabs, of odd numbers of slabs and of whole blocks; a quarter of a tile along n, a tile and a half, whole ones; 300 groups (tables)
+@pytest.mark.parametrize("counts,n,k", [([300, 0, 257, 1], 64, 256), ([256] * 3 + [5], 384, 384), ([512, 31], 256, 1024),
+                                        ([700] * 40, 768, 640), ([1300, 0, 900] * 8, 2560, 128 * 9), ([290, 3] * 150, 128, 512)])
+@pytest.mark.parametrize("out", ["fp32", "bf16", "fp16"])
+def test_int8_gives_the_bits_of_the_streaming_kernel(out, counts, n, k):
+    from catccos_amd import ops
+    g = torch.Generator(device="cuda")
+    g.manual_seed(n + k)
+    e, m = len(counts), sum(counts)
+    dtype = {"fp32": torch.float32, "bf16": torch.bfloat16, "fp16": torch.float16}[out]
+    a = torch.randint(-127, 128, (m, k), dtype=torch.int8, device="cuda", generator=g)
+    w = torch.randint(-127, 128, (e, n, k), dtype=torch.int8, device="cuda", generator=g)
+    channel, token = torch.rand(e * n * 2, device="cuda", generator=g) * 1e-4, torch.rand(m, device="cuda", generator=g)
+    cnt = dev(np.array(counts, dtype=np.int32))
+
+    def call():
+        c = torch.full((m + 3, n // 2), 7.0, dtype=dtype, device="cuda")
+        ops.int8_gmm_dequant_swiglu(a, token, w, channel, cnt, n, k, 1, out, scale_stride=2, c=c[:m])
+        assert bool((c[m:] == 7.0).all())
+        return c
+    got, ref = _pinned(call)
+    assert torch.equal(got, ref) and not bool((ref[:m] == 7.0).all(dim=1).any())
