@@ -40,8 +40,9 @@ typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
 enum WeightLayout { kRowMajor = 0, kTiled = 1, kKSlow = 2 };
 
 constexpr int ks_scale_steps(int fmt) { return fmt == kFmtI8 ? 0 : (fmt == CMX_FMT_E2M1 ? 2 : 1); }   // scale dwords per row and slab
-// slabs in the register ring: what fits beside the accumulators, one slab of fragments in MFMA order, their scales and
-// addresses in 256 registers (two wavefronts per SIMD).  The scale pieces in flight before the K loop (sreg, treg: up to 32
+// slabs in the register ring: what fits beside the accumulators, a slab on its way through the exchange, their scales and
+// addresses in 256 registers (two wavefronts per SIMD).  (Fragments change places in the registers that they have, but rings that count on all
+// of that room spill 30 registers: FP4, 32 experts x 16 rows 90 -> 104 us.)  The scale pieces in flight before the K loop (sreg, treg: up to 32
 // registers at 8 wavefronts) are not counted; by the compiler's report they cost 16 x 16 tiles 3-4 spilled registers and 16 x 32
 // tiles 7 (FP4 12), stored and reloaded before the loop, and no other tile more than one.
 constexpr int ks_ring(int fmt, int fw, int fm) {
@@ -49,10 +50,11 @@ constexpr int ks_ring(int fmt, int fw, int fm) {
     const int n = room / ((fw + fm) * 8), most = fw + fm == 2 ? 8 : (fw + fm == 3 ? 5 : 4);
     return n < 1 ? 1 : (n > most ? most : n);
 }
-// activation rows whose partial sums go through the LDS at a time (the NW partial tiles of all rows may exceed it)
+// activation rows whose partial sums go through the LDS at a time: all of them where the workgroup is alone on its CU (eight
+// wavefronts) or where two still fit (1000 x 1000 x 960: four passes of 16 rows, half of the threads idle, took 2.7 us, one 2.5)
 constexpr int ks_pass_frags(int fw, int fm, int nw) {
     int n = fm;
-    while (n > 1 && nw * n * 16 * (16 * fw + 4) * 4 > 65536) n /= 2;
+    while (n > 1 && nw * n * 16 * (16 * fw + 4) * 4 > (nw == 8 ? 140 : 70) * 1024) n /= 2;
     return n;
 }
 // exchange buffers of a wavefront (2 KiB, one fragment): four, used in turn; K-slow weights change places a whole slab at a time, in
@@ -90,13 +92,12 @@ __device__ __forceinline__ v4f ks_mfma(const v4i (&w)[2], const v4i (&a)[2], v4f
     }
 }
 
-// STREAM: weights are loaded non-temporal (KsplitWeights)
-template <int FMT, int FW, int FM, int NW, int EPI, int LAYOUT, bool STREAM>
+// STREAM: weights are loaded non-temporal (KsplitWeights); PD: slabs in the ring
+template <int FMT, int FW, int FM, int NW, int EPI, int LAYOUT, bool STREAM, int PD = ks_ring(FMT, FW, FM)>
 __device__ __forceinline__ void ks_tile(const GemmParams& p, const Tile& tc, uint8_t* smem) {
     constexpr int NT = 64 * NW, TW = 16 * FW;
     constexpr int kS = ks_scale_steps(FMT);
     constexpr int kSA = kS ? kS : 1;
-    constexpr int PD = ks_ring(FMT, FW, FM);
     constexpr bool TILED = LAYOUT == kTiled, KSLOW = LAYOUT == kKSlow;
     constexpr int kScaleW = KSLOW ? 0 : TW, kRows = kScaleW + 16 * FM;            // rows of scales: weights (unless K-slow), activations
     static_assert(!KSLOW || (FW == 4 && kS == 1 && EPI == kEpiStore), "K-slow weights: 64 columns, 8-bit formats");
@@ -300,7 +301,6 @@ __device__ __forceinline__ void ks_tile(const GemmParams& p, const Tile& tc, uin
             request16(i0);
             deposit16(i0);
         }
-        __syncthreads();
     }
     const uint8_t* const sw_row = smem + r * pitch * 4 + g;
     const uint8_t* const sa_row = smem + (kScaleW + r) * pitch * 4 + g;
@@ -362,20 +362,15 @@ __device__ __forceinline__ void ks_tile(const GemmParams& p, const Tile& tc, uin
                     out[f][h][2 * j + 1] = v[1];
                 }
     };
-    auto multiply = [&](const v4i (&wl)[FW][2], const v4i (&al)[FM][2], uint32_t s) {
-        v4i w[FW][2], a[FM][2];
+    // a slab from the order of the loads to that of the MFMA, in the registers that it has
+    auto arrange = [&](v4i (&w)[FW][2], v4i (&a)[FM][2]) {
 #pragma unroll
-        for (int f = 0; f < FM; ++f) exchange(f, al[f], a[f]);
-        if constexpr (KSLOW) exchange_kslow(wl, w);
+        for (int f = 0; f < FM; ++f) exchange(f, a[f], a[f]);
+        if constexpr (KSLOW) exchange_kslow(w, w);
 #pragma unroll
-        for (int f = 0; f < FW && !KSLOW; ++f) {
-            if constexpr (TILED) {
-                w[f][0] = wl[f][0];
-                w[f][1] = wl[f][1];
-            } else {
-                exchange(FM + f, wl[f], w[f]);
-            }
-        }
+        for (int f = 0; f < FW && !KSLOW && !TILED; ++f) exchange(FM + f, w[f], w[f]);
+    };
+    auto multiply = [&](const v4i (&w)[FW][2], const v4i (&a)[FM][2], uint32_t s) {
         uint32_t sw[FW][2] = {}, sa[FM][2] = {};
 #pragma unroll
         for (int j = 0; j < kS; ++j) {
@@ -392,17 +387,30 @@ __device__ __forceinline__ void ks_tile(const GemmParams& p, const Tile& tc, uin
 
     // ---- K loop --------------------------------------------------------------------------------------------------------
     const uint32_t mine = nslab > wave ? (nslab - wave + NW - 1) / NW : 0u;          // slabs of this wavefront
+    // Eight wavefronts, which are alone on their CU, arrange the slabs of the first turn while the scales are on their way: with the scales
+    // in front, the exchange of all slabs (16 x 4096 x 7168: 1.5 us of LDS time) stood between the arrival of the last operands and the
+    // first MFMA.  Quantizer included, us: 16 x 4096 x 7168 10.2 -> 9.3, 200 x 2048 x 4096 13.4 -> 12.4, 512 x 512 x 4096 11.5 -> 10.7, [K, N] 64 x
+    // 4096 x 4096 15.0 -> 13.5.  Beside a second workgroup of four wavefronts nothing is gained (32 experts x 60 rows 87.1 against 88.3).
+    constexpr bool kFirst = NW == 8;
+#pragma unroll
+    for (int d = 0; d < PD && kFirst; ++d)
+        if ((uint32_t)d < mine) arrange(wf[d], af[d]);
+    if constexpr (kS != 0) __syncthreads();
     uint32_t i = 0;
     for (; i + PD < mine; i += PD) {
 #pragma unroll
         for (int d = 0; d < PD; ++d) {
+            if (!kFirst || i != 0) arrange(wf[d], af[d]);
             multiply(wf[d], af[d], wave + NW * (i + d));
             load_slot(d, wave + NW * (i + PD + d));
         }
     }
 #pragma unroll
     for (int d = 0; d < PD; ++d)
-        if (i + d < mine) multiply(wf[d], af[d], wave + NW * (i + d));
+        if (i + d < mine) {
+            if (!kFirst || i != 0) arrange(wf[d], af[d]);
+            multiply(wf[d], af[d], wave + NW * (i + d));
+        }
     // K not a whole number of slabs: the rest, zeros past K
     if constexpr (FMT != kFmtI8 && LAYOUT == kRowMajor) {
         if (p.kbytes % kSlabBytes != 0 && nslab % NW == wave) {
@@ -421,6 +429,7 @@ __device__ __forceinline__ void ks_tile(const GemmParams& p, const Tile& tc, uin
                     if (in) af[0][f][h] = __builtin_bit_cast(v4i, __builtin_amdgcn_raw_buffer_load_b128(a_rs, (int)aoff[f][h], kb, 0));
                 }
             }
+            arrange(wf[0], af[0]);
             multiply(wf[0], af[0], nslab);
         }
     }
@@ -471,6 +480,13 @@ __device__ __forceinline__ void ks_rows(const GemmParams& p, const Tile& tc, uin
     }
     if constexpr (FM >= 2) {
         if (tc.rows_valid <= 16 * FM / 2) return ks_tile<FMT, FW, FM / 2, NW, EPI, LAYOUT, STREAM>(p, tc, smem);
+    }
+    // A slot without a slab costs the vector cache its loads all the same, so a short K gets a short ring (us, quantizer included: 30 x 1000 x
+    // 512, five slots for one slab 7.1 -> 5.7; 5 x 4096 x 2048 7.5 -> 6.1; 1 x 4096 x 4096, eight for four 7.7 -> 6.9).
+    if constexpr (NW == 8 && ks_ring(FMT, FW, FM) >= 4) {
+        if (p.kbytes <= 2 * NW * kSlabBytes) return ks_tile<FMT, FW, FM, NW, EPI, LAYOUT, STREAM, 2>(p, tc, smem);
+        if constexpr (ks_ring(FMT, FW, FM) > 4)
+            if (p.kbytes <= 4 * NW * kSlabBytes) return ks_tile<FMT, FW, FM, NW, EPI, LAYOUT, STREAM, 4>(p, tc, smem);
     }
     ks_tile<FMT, FW, FM, NW, EPI, LAYOUT, STREAM>(p, tc, smem);
 }

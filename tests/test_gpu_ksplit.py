@@ -45,6 +45,25 @@ def test_dense_tiles(shape, fmt, m, n, k):
     assert bad == 0, (bad, worst)
 
 
+# the last K of a ring of two and of four slots, the first of the next, a slab in part behind either
+@pytest.mark.parametrize("shape", [(1, 1, 8), (1, 2, 8), (2, 1, 8), (2, 2, 8)])
+@pytest.mark.parametrize("fmt,k", [("E4M3", 2048), ("E4M3", 2080), ("E5M2", 2176), ("E4M3", 4096), ("E4M3", 4128), ("E4M3", 4224), ("E2M1", 4096), ("E2M1", 4352),
+                                   ("E2M1", 8192), ("E2M1", 8448)])
+def test_rings_of_every_length(shape, fmt, k):
+    """Against the 64 x 64 tile, whose ring has one length: eight partial sums on either, so the same bits."""
+    from catccos_amd import ops
+    rng = np.random.default_rng(k)
+    m, n = 21, 40
+    aq, asc = _mx(rng, m, k, fmt)
+    bq, bsc = _mx(rng, n, k, fmt)
+    pack = O.pack_fp4 if fmt == "E2M1" else (lambda x: x)
+    args = dev(pack(aq)), dev(asc), dev(pack(bq)), dev(bsc), k, fmt, "fp32"
+    hooks_lib().cmx_debug_force_ksplit(4, 4, 8)
+    want = host(ops.mx_gemm(*args))
+    hooks_lib().cmx_debug_force_ksplit(*shape)
+    assert np.array_equal(host(ops.mx_gemm(*args)), want) and np.abs(want).max() > 0
+
+
 def test_scale_rows_that_are_not_dword_aligned_and_an_output_pitch():
     """K = 96: three scales a row, fewer than the dword that longer rows end in, at a pitch of 5.  Output rows wider than n: the rest
     keeps its poison."""
