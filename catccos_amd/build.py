@@ -23,6 +23,7 @@ NATIVE_SRC = os.path.join(CSRC, "native_call.cpp")
 NATIVE = os.path.join(HERE, "_native_call" + sysconfig.get_config_var("EXT_SUFFIX"))
 
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
+ROCM = os.environ.get("ROCM_PATH", "/opt/rocm")
 FLAGS = [
     "--offload-arch=gfx950", "-O3", "-std=c++17", "-fPIC",
     "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
@@ -85,10 +86,10 @@ def build_native(force: bool = False) -> str:
     import torch
     t = os.path.dirname(torch.__file__)
     cmd = ["g++", "-O2", "-std=c++17", "-fPIC", "-shared", f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}",
-           f'-DCMX_TORCH_VERSION="{torch.__version__}"',
+           f'-DCMX_TORCH_VERSION="{torch.__version__}"', "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM",
            "-isystem", os.path.join(t, "include"), "-isystem", os.path.join(t, "include", "torch", "csrc", "api", "include"),
-           "-isystem", sysconfig.get_paths()["include"], NATIVE_SRC,
-           "-L" + os.path.join(t, "lib"), "-ltorch_python", "-ltorch", "-ltorch_cpu", "-lc10"]
+           "-isystem", os.path.join(ROCM, "include"), "-isystem", sysconfig.get_paths()["include"], NATIVE_SRC,
+           "-L" + os.path.join(t, "lib"), "-ltorch_python", "-ltorch", "-ltorch_cpu", "-lc10", "-lc10_hip", "-ltorch_hip"]
     stamp, want = os.path.join(OBJ, "native_call.stamp"), "\n".join([sys.version, *cmd])
     if (not force and os.path.exists(NATIVE) and os.path.getmtime(NATIVE) >= os.path.getmtime(NATIVE_SRC)
             and os.path.exists(stamp) and open(stamp).read() == want):

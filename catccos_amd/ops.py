@@ -62,16 +62,13 @@ def _p(t: torch.Tensor):
 
 
 def _launch(name, *args):
-    """The entry point `name` on these tensors (GPU tensors, or ValueError), integers and Nones, and torch's current stream.  A whole number
-    that the caller gives goes through index() first: as a tensor of one element it would be passed by its address."""
-    try:
-        stream = _stream()
-    except RuntimeError:                       # a process without a GPU has no stream; its tensors are refused as such
-        _need_cuda(*(t for t in args if isinstance(t, torch.Tensor)))
-        raise
-    rc = _run(_lib.entries()[name], *args, stream)
-    if rc != 0:
-        _lib.check(rc)
+    """The entry point `name` on these tensors (GPU tensors, or ValueError), integers and Nones, and torch's current stream (...); a tuple (dtype,
+    sizes) stands for a new tensor.  Returns the new tensors.  A whole number that the caller gives goes through index() first: as a tensor of one
+    element it would be passed by its address."""
+    out = _run(_lib.entries()[name], *args, ...)
+    if out.__class__ is int:
+        _lib.check(out)
+    return out
 
 
 def _brought(t):
@@ -102,9 +99,7 @@ def mx_quant(x: torch.Tensor, fmt: str = "E4M3", mode: str | None = None):
         mode = "lut" if fp4 else "rne"
     ccols = (cols + 1) // 2 if fp4 else cols
     scols = scale_cols(cols)
-    codes, scales = _empty(x, torch.uint8, rows, ccols), _empty(x, torch.uint8, rows, scols)
-    _launch("cmx_mx_quant", x, pitch, codes, ccols, scales, scols, rows, cols, FMT[fmt], ROUND[mode])
-    return codes, scales
+    return _launch("cmx_mx_quant", x, pitch, (torch.uint8, rows, ccols), ccols, (torch.uint8, rows, scols), scols, rows, cols, FMT[fmt], ROUND[mode])
 
 
 def mx_dequant(codes: torch.Tensor, scales: torch.Tensor, cols: int, fmt: str = "E4M3") -> torch.Tensor:
@@ -121,10 +116,8 @@ def mx_gemm(a, a_scale, b, b_scale, k: int, fmt: str = "E4M3", out: str = "bf16"
     """C[m,n] = deq(a)[m,k] . deq(b)[n,k]^T"""
     k = index(k)
     m, n = a.size(0), b.size(0)
-    c = _empty(a, _OUT_DTYPE[out], m, n)
-    _launch("cmx_mx_gemm", a, a.stride(0), a_scale, a_scale.stride(0), b, b.stride(0), b_scale, b_scale.stride(0), c, n, m, n, k, FMT[fmt],
-            OUT[out])
-    return c
+    return _launch("cmx_mx_gemm", a, a.stride(0), a_scale, a_scale.stride(0), b, b.stride(0), b_scale, b_scale.stride(0), (_OUT_DTYPE[out], m, n), n,
+                   m, n, k, FMT[fmt], OUT[out])
 
 
 def mx_to_k_major(src, src_scale, k: int, n: int):
@@ -162,9 +155,7 @@ def mx_gemm_ex(a, a_scale, b, b_scale, m: int, n: int, k: int, fmt: str = "E4M3"
     assert a.is_contiguous() and a_scale.is_contiguous() and b.is_contiguous() and b_scale.is_contiguous()
     need = _lib.load().cmx_mx_gemm_ex_workspace_bytes(m, n, k, trans_a, trans_b)
     ws = _empty(a, torch.uint8, max(need, 1))
-    c = _empty(a, _OUT_DTYPE[out], m, n)
-    _launch("cmx_mx_gemm_ex", a, a_scale, b, b_scale, c, n, m, n, k, FMT[fmt], OUT[out], trans_a, trans_b, ws)
-    return c
+    return _launch("cmx_mx_gemm_ex", a, a_scale, b, b_scale, (_OUT_DTYPE[out], m, n), n, m, n, k, FMT[fmt], OUT[out], trans_a, trans_b, ws)
 
 
 def mx_gmm_ex(a, a_scale, b, b_scale, group_sizes, n: int, k: int, fmt: str = "E4M3", out: str = "bf16",
@@ -188,9 +179,7 @@ def int8_quant_scatter(x: torch.Tensor, src2sorted, top_k: int = 1):
     tokens, k = x.shape
     pitch, step = x.stride()
     assert step == 1
-    codes, scales = _empty(x, torch.int8, tokens * top_k, k), _empty(x, torch.float32, tokens * top_k)
-    _launch("cmx_int8_quant_scatter", x, pitch, src2sorted, codes, k, scales, tokens, k, top_k)
-    return codes, scales
+    return _launch("cmx_int8_quant_scatter", x, pitch, src2sorted, (torch.int8, tokens * top_k, k), k, (torch.float32, tokens * top_k), tokens, k, top_k)
 
 
 def int8_gmm_dequant_swiglu(a, token_scale, b, channel_scale, group_sizes, n: int, k: int, trans_b: int = 0,
@@ -308,11 +297,8 @@ def moe_init_routing(expert_idx: torch.Tensor, experts: int):
     assert expert_idx.dtype == torch.int32 and expert_idx.is_contiguous()
     t, top_k = expert_idx.shape
     routes = t * top_k
-    s2s, inv = _empty(expert_idx, torch.int32, routes), _empty(expert_idx, torch.int32, routes)
-    counts = _empty(expert_idx, torch.int32, experts)
     ws = _empty(expert_idx, torch.uint8, _lib.load().cmx_moe_routing_workspace_bytes(routes, experts))
-    _launch("cmx_moe_init_routing", expert_idx, t, top_k, experts, s2s, inv, counts, ws)
-    return s2s, inv, counts
+    return _launch("cmx_moe_init_routing", expert_idx, t, top_k, experts, (torch.int32, routes), (torch.int32, routes), (torch.int32, experts), ws)
 
 
 def quant_scatter(x: torch.Tensor, src2sorted: torch.Tensor, top_k: int, packed: bool = False, out=None):
@@ -333,9 +319,7 @@ def quant_scatter(x: torch.Tensor, src2sorted: torch.Tensor, top_k: int, packed:
                                          top_k, _stream()))
         return buf
     scols = scale_cols(k)
-    codes, scales = _empty(x, torch.uint8, rows, k), _empty(x, torch.uint8, rows, scols)
-    _launch("cmx_quant_scatter_zeroed", x, x.stride(0), src2sorted, codes, k, scales, scols, t, k, top_k)
-    return codes, scales
+    return _launch("cmx_quant_scatter_zeroed", x, x.stride(0), src2sorted, (torch.uint8, rows, k), k, (torch.uint8, rows, scols), scols, t, k, top_k)
 
 
 def moe_token_unpermute(y: torch.Tensor, src2sorted: torch.Tensor, probs: torch.Tensor) -> torch.Tensor:

@@ -188,6 +188,37 @@ def test_outputs_and_errors_on_the_gpu():
 
 
 @pytest.mark.gpu
+def test_new_tensors_and_the_current_stream_reach_the_entry_point():
+    got, rc = [], [0]
+    proto = C.CFUNCTYPE(C.c_int, *[C.c_uint64] * 24)
+
+    @proto
+    def callee(*args):
+        got.append(args)
+        return rc[0]
+    address = C.cast(callee, C.c_void_p).value
+    x = torch.zeros(4, device="cuda")
+    side = torch.cuda.Stream()
+    with torch.cuda.stream(side):
+        a, b = _native_call.run(address, 1, (torch.uint8, 3, 5), x, (torch.float32, 7), ...)
+    assert a.shape == (3, 5) and a.dtype == torch.uint8 and b.shape == (7,) and b.dtype == torch.float32 and a.device == b.device == x.device
+    assert got[0][:6] == (1, a.data_ptr(), x.data_ptr(), b.data_ptr(), side.cuda_stream, 0)
+    one = _native_call.run(address, x, (torch.int32, 2, 0), ...)
+    assert one.shape == (2, 0) and got[1][2] == torch.cuda.current_stream().cuda_stream
+    rc[0] = -5
+    assert _native_call.run(address, x, (torch.uint8, 1)) == -5
+    for bad in (lambda: _native_call.run(address, x, ("u8", 1)), lambda: _native_call.run(address, x, (torch.uint8,)),
+                lambda: _native_call.run(address, x, *[(torch.uint8, 1)] * 5)):
+        with pytest.raises(TypeError):
+            bad()
+    with pytest.raises(ValueError, match="expected a GPU tensor"):
+        _native_call.run(address, 1, (torch.uint8, 1))
+    with pytest.raises(RuntimeError):
+        _native_call.run(address, x, (torch.uint8, -2))
+    assert len(got) == 3
+
+
+@pytest.mark.gpu
 def test_buffers_that_the_caller_brings_may_be_pinned():
     """Weights, outputs and workspaces in pinned host memory give the results that device buffers give (no kernel of these small problems uses
     the workspace); other host memory, and inputs in host memory, are refused."""
