@@ -352,14 +352,77 @@ __device__ __forceinline__ void ring_tile(const GemmParams& p, Tile tc) {
         }
         return;
     }
+    if constexpr (EPI == kEpiStore) {
+        if (stores_pieces(p)) {
+            // A thread keeps its eight columns from row to row, so that a piece costs two LDS reads, four conversions and a store: with one
+            // wavefront per SIMD the general loop below is bound by its instructions (1024 x 4096, 2.5 us of it; K = 1024, the call XXX us).
+            constexpr uint32_t kPieces8 = TW / 8, kTurn = NT / kPieces8;
+            static_assert(NT % kPieces8 == 0 && TM % kTurn == 0, "whole rows a turn");
+            const uint32_t q = tid % kPieces8, m0 = tid / kPieces8;
+            uint32_t ncol = tc.wt * TW + 8 * q;
+            if constexpr (KSLOW) ncol = ncol / 16 * 16 < p.n ? wcol_of(q / 2) + 8 * (q % 2) : p.n;
+            if (ncol >= p.n) return;
+            auto store_rows = [&](auto out_c) {
+                uint16_t* o = reinterpret_cast<uint16_t*>(p.c) + (size_t)(tc.row0 + m0) * p.ldc + ncol;
+#pragma unroll
+                for (uint32_t i = 0; i < TM / kTurn; ++i) {
+                    const float* const s = sums + (m0 + i * kTurn) * kPitch + 8 * q;
+                    const uint4 v = pack_piece<decltype(out_c)::value>(*reinterpret_cast<const v4f*>(s), *reinterpret_cast<const v4f*>(s + 4));
+                    if (m0 + i * kTurn < tc.rows_valid) *reinterpret_cast<uint4*>(o) = v;
+                    o += (size_t)kTurn * p.ldc;
+                }
+            };
+            if (p.out_type == CMX_OUT_BF16) store_rows(std::integral_constant<int, CMX_OUT_BF16>{});
+            else store_rows(std::integral_constant<int, CMX_OUT_FP16>{});
+            return;
+        }
+    }
+    if constexpr (epi_is_swiglu_quant(EPI)) {
+        // The same: eight activation columns of a thread, its rows one after the other.
+        constexpr uint32_t kPieces8 = TW / 16, kTurn = NT / kPieces8;
+        static_assert(NT % kPieces8 == 0 && TM % kTurn == 0, "whole rows a turn");
+        const uint32_t q = tid % kPieces8, m0 = tid / kPieces8;
+        const uint32_t ncol = tc.wt * (TW / 2) + 8 * q, blk = ncol / 32, blocks = half / 32;
+        const bool aligned8 = p.ld_act % 8 == 0 && (reinterpret_cast<uintptr_t>(p.act_codes) & 7u) == 0;
+#pragma unroll 2
+        for (uint32_t i = 0; i < TM / kTurn; ++i) {
+            const uint32_t m = m0 + i * kTurn;
+            const float* const s = sums + m * kPitch + 8 * q;
+            const v4f g[2] = {*reinterpret_cast<const v4f*>(s), *reinterpret_cast<const v4f*>(s + 4)};
+            const v4f u[2] = {*reinterpret_cast<const v4f*>(s + TW / 2), *reinterpret_cast<const v4f*>(s + TW / 2 + 4)};
+            uint32_t pk[4];
+            uint2 codes;
+            const int e = swiglu_quant_piece(g, u, pk, codes);                       // (all lanes: they hold the blocks together)
+            if (m >= tc.rows_valid || ncol >= half) continue;                        // n is a multiple of 64: a block is in or out as a whole
+            const size_t mrow = tc.row0 + m;
+            if constexpr (EPI == kEpiSwigluQuantAct) {
+                if (p.act_bf16) {
+                    uint16_t* const o = p.act_bf16 + mrow * half + ncol;
+#pragma unroll
+                    for (int j = 0; j < 8; ++j) o[j] = (uint16_t)(pk[j >> 1] >> (16 * (j & 1)));
+                }
+            }
+            uint8_t* const o = p.act_codes + mrow * p.ld_act + ncol;
+            if (aligned8) {
+                *reinterpret_cast<uint2*>(o) = codes;
+            } else {
+                *reinterpret_cast<uint32_t*>(o) = codes.x;
+                *reinterpret_cast<uint32_t*>(o + 4) = codes.y;
+            }
+            if (q % 4 == 0) {
+                uint8_t* const srow = p.act_scales + mrow * p.ld_acts;
+                srow[blk] = (uint8_t)(e + 127);
+                if (blk == blocks - 1 && (blocks & 1u)) srow[blocks] = 127;
+            }
+        }
+        return;
+    }
 #pragma unroll 4
     for (uint32_t it = tid; it < TM * kQuads; it += NT) {
         const uint32_t m = it / kQuads, q = it % kQuads;
-        if (m >= tc.rows_valid && !epi_is_swiglu_quant(EPI)) continue;
-        const v4f v = *reinterpret_cast<const v4f*>(sums + m * kPitch + 4 * q);
-        v4f u = v;
-        if constexpr (epi_pairs_gate_up(EPI)) u = *reinterpret_cast<const v4f*>(sums + m * kPitch + TW / 2 + 4 * q);
-        uint32_t ncol = tc.wt * (epi_pairs_gate_up(EPI) ? TW / 2 : TW) + 4 * q;
+        if (m >= tc.rows_valid) continue;
+        const v4f v = *reinterpret_cast<const v4f*>(sums + m * kPitch + 4 * q), u = v;
+        uint32_t ncol = tc.wt * TW + 4 * q;
         if constexpr (KSLOW) {
             const uint32_t col = tc.wt * TW + 16 * (q / 4);
             ncol = col < p.n ? wcol_of(q / 4) + 4 * (q % 4) : p.n;

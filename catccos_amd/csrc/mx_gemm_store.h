@@ -49,6 +49,22 @@ __device__ __forceinline__ void store_i8_quad(const GemmParams& p, size_t mrow, 
     }
 }
 
+// Whether rows of 16-bit output are whole 16-byte pieces, so that eight columns from a multiple of eight on are in or out together.
+__device__ __forceinline__ bool stores_pieces(const GemmParams& p) {
+    return p.out_type != CMX_OUT_FP32 && p.n % 8 == 0 && p.ldc % 8 == 0 && (reinterpret_cast<uintptr_t>(p.c) & 15u) == 0;
+}
+// eight sums as such a piece
+template <int OUT>
+__device__ __forceinline__ uint4 pack_piece(const v4f& lo, const v4f& hi) {
+    if constexpr (OUT == CMX_OUT_BF16) {
+        return make_uint4(cvt_pk_bf16(lo[0], lo[1]), cvt_pk_bf16(lo[2], lo[3]), cvt_pk_bf16(hi[0], hi[1]), cvt_pk_bf16(hi[2], hi[3]));
+    } else {
+        typedef _Float16 v8h __attribute__((ext_vector_type(8)));
+        return __builtin_bit_cast(uint4, (v8h){(_Float16)lo[0], (_Float16)lo[1], (_Float16)lo[2], (_Float16)lo[3],
+                                               (_Float16)hi[0], (_Float16)hi[1], (_Float16)hi[2], (_Float16)hi[3]});
+    }
+}
+
 // Sums of one output row, four consecutive columns from ncol on (SwiGLU kinds: four gate columns and their up partners, ncol the
 // activation column), to memory.  SwiGLU + requant: eight neighbouring lanes hold the 32 columns of an MX block.
 template <int EPI>
@@ -125,6 +141,29 @@ __device__ __forceinline__ void store_quad(const GemmParams& p, const Tile& tc, 
             if (blk == nblk - 1 && (nblk & 1u)) srow[nblk] = 127;
         }
     }
+}
+
+// SwiGLU on the bf16-rounded sums of eight gate and up columns of one row, bf16 again, then the MX block of 32 columns, which four neighbouring
+// lanes hold: its scale exponent, and the lane's eight codes (pk: the bf16 values, in pairs)
+__device__ __forceinline__ int swiglu_quant_piece(const v4f (&g)[2], const v4f (&u)[2], uint32_t (&pk)[4], uint2& codes) {
+    uint32_t m = 0;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+        const uint32_t g2 = cvt_pk_bf16(g[j / 2][j % 2 * 2], g[j / 2][j % 2 * 2 + 1]), u2 = cvt_pk_bf16(u[j / 2][j % 2 * 2], u[j / 2][j % 2 * 2 + 1]);
+        pk[j] = cvt_pk_bf16(silu_mul(__uint_as_float(g2 << 16), __uint_as_float(u2 << 16)),
+                            silu_mul(__uint_as_float(g2 & 0xFFFF0000u), __uint_as_float(u2 & 0xFFFF0000u)));
+        m = pk_max_u16(m, pk[j] & 0x7FFF7FFFu);
+    }
+    m = pk_max_u16(m, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)m, 0xB1, 0xF, 0xF, true));     // lane ^ 1
+    m = pk_max_u16(m, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)m, 0x4E, 0xF, 0xF, true));     // lane ^ 2
+    const int e = block_exp_from_bf16_amax(max(m & 0xFFFFu, m >> 16), kEmaxE4M3);
+    const uint32_t lim = (((uint32_t)(e + kEmaxE4M3 + 127) << 7) | 0x60u) * 0x10001u;
+    const float scale = __uint_as_float((uint32_t)(e + 127) << 23);
+    uint32_t c[4];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) c[j] = pk_min_u16(pk[j] & 0x7FFF7FFFu, lim) | (pk[j] & 0x80008000u);
+    codes = make_uint2(cvt_scaled_pk4<CMX_FMT_E4M3>(c[0], c[1], scale), cvt_scaled_pk4<CMX_FMT_E4M3>(c[2], c[3], scale));
+    return e;
 }
 
 #endif  // __HIPCC__
