@@ -1103,26 +1103,21 @@ bool takes_128_tile(uint32_t m, uint32_t n, int fmt, uint32_t kblocks, int cus) 
 // the split-K kernel runs in two rounds of a workgroup per CU, and few enough tiles of 128 x 128, 192 or 256 for one round of
 // the ring kernel's.  Its sums are the 256-row kernels' (one chain over K), so the limit to those is a matter of time only; the limit
 // to split-K (whose sums differ in the last bits) goes by sizes alone.
-// Measured (us, E4M3, bf16 out, operands of three calls in turn; before -> ring, [K, N] = on weights stored [K, N], where
-// the other kernels need a pass of 9 (K = 4096) to 15 (7168) before them):
-//   n = 4096:      K = 512         1024            2048            4096            7168            3968 (no multiple of 512)
-//   m = 512    7.6 against 9.4  8.9   10.8     12.0   14.4     19.8   23.1     27.2   31.4     19.5   22.0       split-K stays
-//   700        9.5 ->  9.5     12.8 -> 11.3    18.1 -> 14.8    26.7 -> 24.0    40.3 -> 33.8    27.5 -> 22.8       128
-//   1024      10.0 ->  9.9     13.3 -> 11.8    19.0 -> 15.5    33.2 -> 25.3    50.4 -> 36.4    33.9 -> 23.8       128
-//   1280      11.7 against 11.8 15.7 -> 14.1   23.5 -> 18.6    38.9 -> 29.0    62.7 -> 44.0    51.3 -> 28.3       192
-//   1536      11.8 against 12.2 15.8 -> 14.7   24.4 -> 19.5    38.9 -> 30.7    62.3 -> 47.1    50.4 -> 30.6       192
-//   2048      12.1 against 14.9 16.3 against 18.0 24.1 against 24.9 39.7 -> 38.6 63.2 -> 59.8  52.0 -> 38.8       256
-//   2560      (two rounds)      16.6   24.8    25.3   33.9     43.2   57.4     70     86       54.3   55.6       256-row kernels
-//   2048, [K, N]  12 + 4 -> 16.7   16 + 5 -> 19.8  24 + 6 -> 26.9  40 + 9 -> 40.8  63 + 15 -> 62.4
-int ring_rows(uint32_t m, uint32_t n, int fmt, uint32_t kblocks, int cus, bool k_slow) {
+// Measured (us, E4M3, bf16 out, operands of three calls in turn; split-K 64 x 64 or 256-row kernels -> ring; on weights stored [K, N] the
+// other kernels need a pass of 4 (K = 512) to 9 (K = 4096) before them):
+//   n = 4096:      K = 512         1024            2048            4096
+//   m = 512    7.0 against 7.1  8.6    8.6     11.8   12.0     17.6   18.7       split-K stays
+//   768       10.1 ->  7.4     12.8 ->  9.2    17.2 -> 12.7    25.4 -> 19.9       128
+//   1024      11.8 ->  7.8     15.4 ->  9.6    20.4 -> 13.2    31.5 -> 21.4       128
+//   1280      12.1 ->  9.0     15.9 -> 10.9    23.4 -> 15.4    38.9 -> 25.1       192
+//   1536      12.1 ->  9.4     15.9 -> 11.3    23.5 -> 16.2    38.7 -> 26.8       192
+//   2048      12.5 -> 11.0     16.6 -> 13.8    24.3 -> 20.6    39.7 -> 34.4       256
+// Past one round the 256-row kernels are the faster ones (2560 x 4096, ring in two rounds: K = 1024 24.8 against 16.6, 4096 57.4 against 43.2).
+int ring_rows(uint32_t m, uint32_t n, int fmt, uint32_t kblocks, int cus) {
     if (fmt == CMX_FMT_E2M1 || kblocks % 4 != 0 || kblocks < 16) return 0;
     if ((uint64_t)ceil_div(n, 64) * ceil_div(m, 64) <= 2 * (uint64_t)cus) return 0;
     const auto one_round = [&](uint32_t tm) { return (uint64_t)ceil_div(n, 128) * ceil_div(m, tm) <= (uint64_t)cus; };
-    const bool slow_256 = k_slow || kblocks % 16 != 0;        // the 256-row kernels need a pass first, or are the streaming ones
-    if (one_round(128)) return 128;
-    if (one_round(192) && (slow_256 || kblocks >= 32)) return 192;
-    if (one_round(256) && (slow_256 || kblocks >= 128)) return 256;
-    return 0;
+    return one_round(128) ? 128 : (one_round(192) ? 192 : (one_round(256) ? 256 : 0));
 }
 
 // Whether a problem goes to the split-K kernels (mx_gemm_ksplit.hip), and with which tile; fw == 0: no.  The choice depends
@@ -1151,7 +1146,7 @@ int choose_ksplit(uint32_t m, uint32_t n, int fmt, uint32_t kblocks, KsplitTile*
         }
     const KsplitTile t = {4, 4, 4};
     const uint64_t per_cu = fmt != CMX_FMT_E2M1 && kblocks % 4 != 0 ? 8 : 4;
-    if (tiles(t) <= per_cu * cus && !takes_128_tile(m, n, fmt, kblocks, cus) && ring_rows(m, n, fmt, kblocks, cus, false) == 0 && fits(t)) *out = t;
+    if (tiles(t) <= per_cu * cus && !takes_128_tile(m, n, fmt, kblocks, cus) && ring_rows(m, n, fmt, kblocks, cus) == 0 && fits(t)) *out = t;
     return CMX_OK;
 }
 
@@ -1408,7 +1403,7 @@ extern "C" int cmx_mx_gemm(const uint8_t* a, uint32_t lda, const uint8_t* a_scal
     if (rc = cu_count(&cus); rc != CMX_OK) return rc;
     TileChoice t = choose_tile(m, n, fmt, false);
     if (!g_force_tile.tw && !g_disable_dl) {
-        if (const int tm = ring_rows(m, n, fmt, p.kblocks, cus, false)) return ring_gemm(p, {128, tm}, fmt, false, s);
+        if (const int tm = ring_rows(m, n, fmt, p.kblocks, cus)) return ring_gemm(p, {128, tm}, fmt, false, s);
         if (takes_128_tile(m, n, fmt, p.kblocks, cus)) t = {128, 128, 4};
     }
     if (t.waves == kRing) return ring_gemm(p, {t.tw, t.tm}, fmt, false, s);
@@ -1458,7 +1453,7 @@ int cmx::gemm_k_slow(const uint8_t* a, const uint8_t* a_scale, const uint8_t* b,
     if (ks.fw != 0) {
         if (!k_slow_pays(m, n, k, ks, cus) || !ksplit_k_slow_tile(&ks, m, n, fmt, k / 32, cus)) return CMX_OK;
     } else {
-        tm = g_force_tile.waves == kRing ? g_force_tile.tm : (g_force_tile.tw || g_disable_dl ? 0 : ring_rows(m, n, fmt, k / 32, cus, true));
+        tm = g_force_tile.waves == kRing ? g_force_tile.tm : (g_force_tile.tw || g_disable_dl ? 0 : ring_rows(m, n, fmt, k / 32, cus));
         if (tm == 0) return CMX_OK;
     }
     CMX_REQUIRE(a && a_scale && b && b_scale && aligned16(a), "operand rows must be 16-byte aligned");
@@ -1539,11 +1534,10 @@ uint32_t max_group_tiles(uint32_t m_total, uint32_t groups, uint32_t tile_m, uin
 //   128 x 128    8 experts x 64 rows u, K = 1024, N = 1024   14.6 -> 13.9 / 18.3 -> 13.7    x 200 z   22.1 -> 14.3 / 19.7 -> 14.5
 //                8 x 100 u, 4096, 2048                       35.7 -> 25.0 / 40.1 -> 25.4    16 x 64 z, 7168, 1024   56.8 -> 36.8 / 61.5 -> 36.7
 //   256 x 128    32 x 100 u, 7168, 4096                      206 -> 190 / 221 -> 204        32 x 128 z   320 -> 279 / 327 -> 284
-//                16 x 100 u, 2048, 2048                      23.4 against 24.0 / 28.2 -> 25.2, so not for SwiGLU at K below 3072 (at 1152
-//                22.6 against 24.2); 32 x 128 z, 4096, 1024 57.0 -> 48.6 / 47.1 -> 47.1.  The most that this line loses: 64 x 64 u, 3072, 1024 40.4
-//                against 42.3 with weights in the memory-side cache; store 64 x 40 u, 1024, 4096 74.8 against 78.3
+//                SwiGLU 32 x 100 u, K = 1024, N = 2048 21.5 -> 18.5, 4096 36.8 -> 34.5; 2048, 4096 61.2 -> 54.8; 64 x 90 z, 2048, 2048 71.9 -> 66.9; in many
+//                rounds at K = 1024 it loses a little: 128 x 70, 4096 u 141.8 against 143.7, z 163.3 against 167.2 (below K = 1024 not measured)
 //   128 x 256    8 x 200 u, 4096, 2048                       45.9 -> 34.5 / 43.1 -> 35.7    16 x 300 u, 7168, 1024   74 -> 57 / 69 -> 62
-//                8 x 500 u, 1024, 1024                       22.6 -> 18.6 / 20.0 against 19.9, so not for a store at K below 2048
+//                8 x 500 u, 1024, 1024                       22.6 -> 18.6 / 19.4 -> 12.9; store 8 x 200 u, 512, 2048 15.3 -> 9.6, 16 x 300 u, 512, 1024 16.5 -> 11.3
 // Where n is at most 128, half of a 256-row tile would be empty: 128 x 128 for 256 x 128 (SwiGLU 256 x 68 z, 3072, 64 45 -> 34 where 256 x 128 takes
 // 48; FP4 256 x 128 u, 512, 64 20 -> 16, 23; INT8 256 x 128 u, 128, 128 17.5 -> 14.1, 20.1).
 // Problems of more tiles stay on the persistent kernels (32 x 194 rows, 7168, 4096: 287 against 311 with 128 x 256).
@@ -1562,10 +1556,10 @@ int ring_groups(TileChoice* t, uint32_t m_total, uint32_t groups, uint32_t n, in
     int cus = 0;
     if (int rc = cu_count(&cus); rc != CMX_OK) return rc;
     const uint64_t w128 = ceil_div(n, 128);
-    const uint32_t k_min = eight_bit && swiglu ? 96 : 16;
+    const uint32_t k_min = eight_bit && swiglu ? 32 : 16;
     if (w128 * (m_total / 128 + groups) <= (uint64_t)cus) *t = {128, 128, kRing};
     else if (t->tm <= 128 && kblocks >= k_min) *t = {w128 == 1 ? 128 : 256, 128, kRing};
-    else if (t->tm == 256 && w128 * (m_total / 256 + groups * 3 / 4) <= (uint64_t)cus && (swiglu || kblocks >= 64 || !eight_bit)) *t = {128, 256, kRing};
+    else if (t->tm == 256 && w128 * (m_total / 256 + groups * 3 / 4) <= (uint64_t)cus) *t = {128, 256, kRing};
     return CMX_OK;
 }
 
@@ -1629,8 +1623,9 @@ int gmm_common(GemmParams& p, const int32_t* group_sizes, uint32_t groups, uint3
     }
     // The persistent kernels draw their next tile from a per-XCD counter when tiles differ in cost (4 x 1 wavefronts skip
     // the MFMAs of absent rows).  With 2 x 2 wavefronts every tile costs the same, so those kernels walk their XCD's run in
-    // fixed strides instead: no atomic whose result has to be waited for with everything else in flight.
-    if (t.waves == 4) p.tile_ctr = nullptr;
+    // fixed strides instead: no atomic whose result has to be waited for with everything else in flight.  (8-bit stores have 2 x 2 wavefronts
+    // whatever `waves` says: 16 groups x 300 rows, K = 512, N = 2048 18.6 -> 16.8 us, 4096 28.4 -> 25.9.)
+    if (t.waves == 4 || (!swiglu && fmt != CMX_FMT_E2M1 && !p.w_pretiled)) p.tile_ctr = nullptr;
     p.w_tiles = swiglu ? ceil_div(p.n / 2, t.tw / 2) : ceil_div(p.n, t.tw);
     const uint32_t max_m_tiles = max_group_tiles(m_total, groups, t.tm, ks.small_rows);
     if (p.w_pretiled) return t.tm == 288 ? launch_pretiled<288>(p, fmt, swiglu, max_m_tiles, s) : launch_pretiled<256>(p, fmt, swiglu, max_m_tiles, s);
