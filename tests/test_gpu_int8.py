@@ -12,7 +12,8 @@ from tests.gpu_util import dev, host, bf16_dev
 pytestmark = pytest.mark.gpu
 
 
-@pytest.mark.parametrize("tokens,k,top_k", [(5, 64, 1), (33, 7168, 4), (16, 264, 3), (300, 2048, 8)])
+@pytest.mark.parametrize("tokens,k,top_k", [(5, 64, 1), (33, 7168, 4), (16, 264, 3), (300, 2048, 8), (9, 2056, 2), (6, 4032, 9), (3, 8192, 20),
+                                            (4, 8200, 2)])
 def test_quant_scatter_bit_exact(tokens, k, top_k):
     from catccos_amd import ops
     xb = W.activations_with_outliers(tokens, k, seed=tokens + k)

@@ -37,9 +37,10 @@ def test_sort_all_routes_to_one_expert_and_repeats():
     assert np.array_equal(host(s2s), O.moe_init_routing(bal, 16)[0])
 
 
-@pytest.mark.parametrize("routes,experts", [(63, 1), (1024, 512), (1025, 512), (1025, 513), (5000, 3), (131072, 64), (131073, 64)])
+@pytest.mark.parametrize("routes,experts", [(1, 1), (63, 1), (64, 64), (65, 200), (200, 65), (1, 512), (1023, 3), (1024, 512), (1025, 512), (1025, 513), (5000, 3), (131072, 64), (131073, 64)])
 def test_sort_at_the_edges_of_the_single_launch(routes, experts):
-    """Workgroups of 1024 routes, 512 experts and 131072 routes at most in one launch, three launches beyond; keys outside
+    """One workgroup of as many wavefronts as routes or experts need, workgroups of 1024 routes, three launches past 512 experts or 131072
+    routes; keys outside
     0 .. experts - 1 are dropped on both sides."""
     from catccos_amd import ops
     keys = np.random.default_rng(routes).integers(-1, experts + 1, routes).astype(np.int32)
