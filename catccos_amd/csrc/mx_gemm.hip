@@ -969,14 +969,14 @@ int launch_i8_choice_tables(const GroupTablesJob& job, const GemmParams& p, int3
     return CMX_OK;
 }
 
-template <int FMT, int EPI, int TM, int WW, int WM, int NSLOT>
+template <int FMT, int EPI, int TM, int WW, int WM, int NSLOT, bool SCAN = FMT == kFmtI8>
 int launch_gemm_pipe(const GemmParams& p, uint32_t max_m_tiles, hipStream_t s) {
     // tile ring, scale ring (two-slot kernels: two blocks of 16 bytes per row), next-tile mailbox, 256-byte sink of the L2 prefetch loads
     // (+ the 16 KiB staging area of the whole-line stores, which overlays the last 512 bytes)
     // (INT8: the scales of two tiles instead of the scale ring, and a staging area of its own)
     constexpr size_t smem = NSLOT * (256 + TM) * kSlabBytes + (FMT == kFmtI8 ? 2 * (256 + TM) * 4 + 16384 : NSLOT == 2 ? 2 * (256 + TM) * 16 : NSLOT * (256 + TM) * 4) +
                             (pipe_stages_stores(NSLOT, EPI, WW, WM) ? 16384 : 512);
-    constexpr auto kfn = mx_gemm_pipe_kernel<FMT, EPI, TM, WW, WM, NSLOT>;
+    constexpr auto kfn = mx_gemm_pipe_kernel<FMT, EPI, TM, WW, WM, NSLOT, SCAN>;
     if (int rc = allow_dynamic_lds<kfn, smem>(); rc != CMX_OK) return rc;
     const uint64_t tiles = (uint64_t)max_m_tiles * p.w_tiles;
     CMX_REQUIRE(tiles > 0 && tiles < (1ull << 31), "tile count out of range");
@@ -1022,12 +1022,12 @@ int launch_gemm_wreg(const GemmParams& p, uint32_t max_m_tiles, hipStream_t s) {
     return CMX_OK;
 }
 
-template <int EPI, int WW, int WM>
+template <int EPI, int WW, int WM, bool SCAN = false>
 int launch_gemm_pipe_fp4(const GemmParams& p, uint32_t max_m_tiles, hipStream_t s) {
     // tile ring, ring of two scale blocks, next-tile mailbox and sink of the L2 prefetch loads (or the 16 KiB staging area of the
     // whole-line stores, which overlays those 512 bytes)
     constexpr size_t smem = 2 * 512 * kSlabBytes + 2 * 512 * 16 + (pipe_stages_stores(2, EPI, WW, WM) ? 16384 : 512);
-    constexpr auto kfn = mx_gemm_pipe_fp4_kernel<EPI, WW, WM>;
+    constexpr auto kfn = mx_gemm_pipe_fp4_kernel<EPI, WW, WM, SCAN>;
     if (int rc = allow_dynamic_lds<kfn, smem>(); rc != CMX_OK) return rc;
     const uint64_t tiles = (uint64_t)max_m_tiles * p.w_tiles;
     CMX_REQUIRE(tiles > 0 && tiles < (1ull << 31), "tile count out of range");
@@ -1250,6 +1250,8 @@ int launch_tile(const GemmParams& p, int waves, uint32_t max_m_tiles, hipStream_
             // inside the loop, so the persistent store kernel is always 2 x 2)
             if (lean && p.out_type == CMX_OUT_BF16) return launch_gemm_pipe<FMT, kLeanBf16, 256, 2, 2, 2>(p, max_m_tiles, s);
             if (lean) return launch_gemm_pipe<FMT, kLeanFp16, 256, 2, 2, 2>(p, max_m_tiles, s);
+            if constexpr (EPI == kEpiSwigluQuant)
+                if (waves == 4 && p.sizes != nullptr) return launch_gemm_pipe<FMT, EPI, 256, 2, 2, 2, true>(p, max_m_tiles, s);
             if (waves == 4) return launch_gemm_pipe<FMT, EPI, 256, 2, 2, 2>(p, max_m_tiles, s);
             return launch_gemm_pipe<FMT, EPI, 256, 4, 1, 2>(p, max_m_tiles, s);
         }
@@ -1261,6 +1263,8 @@ int launch_tile(const GemmParams& p, int waves, uint32_t max_m_tiles, hipStream_
                 // plain 16-bit output with 8-element-aligned rows: lean store epilogue, persistent kernel
                 const bool lean = lean_store(p);
                 // (unlike the 8-bit kernel, whose fragments take twice the registers, the 4 x 1 layout fits here too)
+                if (lean && waves == 4 && p.sizes != nullptr)
+                    return p.out_type == CMX_OUT_BF16 ? launch_gemm_pipe_fp4<kEpiStoreBf16, 2, 2, true>(p, max_m_tiles, s) : launch_gemm_pipe_fp4<kEpiStoreFp16, 2, 2, true>(p, max_m_tiles, s);
                 if (lean && waves == 4 && p.out_type == CMX_OUT_BF16) return launch_gemm_pipe_fp4<kEpiStoreBf16, 2, 2>(p, max_m_tiles, s);
                 if (lean && waves == 4) return launch_gemm_pipe_fp4<kEpiStoreFp16, 2, 2>(p, max_m_tiles, s);
                 if (lean && p.out_type == CMX_OUT_BF16) return launch_gemm_pipe_fp4<kEpiStoreBf16, 4, 1>(p, max_m_tiles, s);
@@ -1610,9 +1614,8 @@ int gmm_common(GemmParams& p, const int32_t* group_sizes, uint32_t groups, uint3
     const bool all_ksplit = plan.all_ksplit();
     const GroupTables tables(workspace, groups);
     bool by_sizes = false;
-    if (!tables_filled && !all_ksplit && ks.small_rows == 0 && scans_groups(p, t, fmt, swiglu)) {
-        by_sizes = groups <= kInlineGroups;                    // (the other persistent kernels walk from tile to tile through tables)
-    } else if (!tables_filled && (all_ksplit || t.waves == kRing)) {
+    // (the other persistent kernels walk from tile to tile through tables)
+    if (!tables_filled && (all_ksplit || t.waves == kRing || (ks.small_rows == 0 && scans_groups(p, t, fmt, swiglu)))) {
         const uint64_t tiles = all_ksplit ? (uint64_t)(m_total / 64 + groups) * ceil_div(p.n, 64) : (uint64_t)(m_total / t.tm + groups) * ceil_div(p.n, t.tw);
         if (int rc = tiles_by_sizes(&by_sizes, groups, tiles, all_ksplit ? 2 : 1); rc != CMX_OK) return rc;
     }
@@ -1624,8 +1627,9 @@ int gmm_common(GemmParams& p, const int32_t* group_sizes, uint32_t groups, uint3
     // The persistent kernels draw their next tile from a per-XCD counter when tiles differ in cost (4 x 1 wavefronts skip
     // the MFMAs of absent rows).  With 2 x 2 wavefronts every tile costs the same, so those kernels walk their XCD's run in
     // fixed strides instead: no atomic whose result has to be waited for with everything else in flight.  (8-bit stores have 2 x 2 wavefronts
-    // whatever `waves` says: 16 groups x 300 rows, K = 512, N = 2048 18.6 -> 16.8 us, 4096 28.4 -> 25.9.)
-    if (t.waves == 4 || (!swiglu && fmt != CMX_FMT_E2M1 && !p.w_pretiled)) p.tile_ctr = nullptr;
+    // whatever `waves` says: 16 groups x 300 rows, K = 512, N = 2048 18.6 -> 16.8 us, 4096 28.4 -> 25.9; behind the FFN's first matmul, where the
+    // counters cost no launch, they are the better walk by half a per cent of the chain.)
+    if (t.waves == 4 || (!swiglu && fmt != CMX_FMT_E2M1 && !p.w_pretiled && !tables_filled)) p.tile_ctr = nullptr;
     p.w_tiles = swiglu ? ceil_div(p.n / 2, t.tw / 2) : ceil_div(p.n, t.tw);
     const uint32_t max_m_tiles = max_group_tiles(m_total, groups, t.tm, ks.small_rows);
     if (p.w_pretiled) return t.tm == 288 ? launch_pretiled<288>(p, fmt, swiglu, max_m_tiles, s) : launch_pretiled<256>(p, fmt, swiglu, max_m_tiles, s);

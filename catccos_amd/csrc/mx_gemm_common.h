@@ -136,9 +136,10 @@ __device__ __forceinline__ void interleave_xcd_walk(uint32_t total_tiles, uint32
 // blocks of 32 they would all lie on the first XCDs, and the L2s and links of the others would have nothing to do.  320 tiles on 256
 // workgroups (us): SwiGLU 8 x 1280 rows, K = 4096, N = 2048 124.5 -> 112.6, FP4 125.7 -> 117.2, dense 8192 x 5120 x 7168 (640 tiles) 281 -> 264; 384
 // tiles 128 -> 117.  In contiguous runs of any length, which cut across the bands, 65536 rows on 32 groups (17 rounds) lose 1.6 %.
+constexpr uint32_t kSpreadRounds = 6;              // (five rounds 337 -> 333; at eight the workgroups have drifted apart and the order makes no difference)
 __device__ __forceinline__ uint32_t next_of_walk(uint32_t tile_id, uint32_t stride, uint32_t end) {
     const uint32_t next = tile_id + stride;
-    if (stride != gridDim.x || next < end / stride * stride) return next;
+    if (stride != gridDim.x || end >= kSpreadRounds * stride || next < end / stride * stride) return next;
     const uint32_t full = end / stride * stride, per = ((end - full + kXcds - 1) / kXcds + 7) / 8 * 8, j = blockIdx.x / kXcds;
     const uint32_t last = full + blockIdx.x % kXcds * per + j;
     return tile_id < full && j < per && last < end ? last : end;
@@ -158,14 +159,15 @@ __device__ __forceinline__ uint32_t tile_of_workgroup(uint32_t total_tiles, uint
 
 // Tile L of group g, whose m-tiles are tp .. tp1 - 1 and whose rows r_begin .. r_end - 1.  Bands of 8 m-tiles share a run of weight tiles
 // (m fastest inside a band): the 32 tiles that an XCD works on at a time then touch 8 + 4 operand panels instead of mtg + 32/mtg
-template <int TM>
+// SHORT: groups of one m-tile, which is what short groups are, without a division
+template <int TM, bool SHORT = false>
 __device__ __forceinline__ void place_in_group(const GemmParams& p, uint32_t g, uint32_t tp, uint32_t tp1, uint32_t r_begin, uint32_t r_end,
                                                uint32_t L, Tile& t) {
     t.g = g;
     const uint32_t mtg = tp1 - tp;
     t.group_tiles = mtg;
     const uint32_t local = L - tp * p.w_tiles;
-    if (mtg == 1) {                            // (what short groups are: no division)
+    if (SHORT && mtg == 1) {
         t.mt = 0;
         t.wt = local;
         t.row0 = r_begin;
@@ -320,7 +322,7 @@ __device__ __forceinline__ bool locate_tile_by_sizes(const GemmParams& p, Tile& 
     for (int j = 0; j < kPer; ++j) {
         const uint32_t n = (uint32_t)__builtin_amdgcn_readlane((int)tiles[j], at);
         const uint32_t r0 = (uint32_t)__builtin_amdgcn_readlane((int)off[j], at), r1 = (uint32_t)__builtin_amdgcn_readlane((int)off[j + 1], at);
-        if (L >= tp * p.w_tiles && L < (tp + n) * p.w_tiles) place_in_group<TM>(p, g + j, tp, tp + n, r0, r1, L, t);
+        if (L >= tp * p.w_tiles && L < (tp + n) * p.w_tiles) place_in_group<TM, true>(p, g + j, tp, tp + n, r0, r1, L, t);
         tp += n;
     }
     return true;

@@ -153,7 +153,8 @@ __host__ __device__ constexpr bool pipe_stages_stores(int nslot, int epi, int ww
 #endif
 
 
-template <int FMT, int EPI, int TM, int WW, int WM, int NSLOT>
+// SCAN: grouped problems whose groups are scanned (GroupScan) instead of looked up in tables
+template <int FMT, int EPI, int TM, int WW, int WM, int NSLOT, bool SCAN = FMT == kFmtI8>
 __global__ __launch_bounds__(256) void mx_gemm_pipe_kernel(const GemmParams p) {
     constexpr bool kI8 = FMT == kFmtI8;                        // INT8: no block scales
     static_assert(FMT == CMX_FMT_E4M3 || FMT == CMX_FMT_E5M2 || (kI8 && EPI == kEpiI8DequantSwiglu && NSLOT == 2 && WW == 2 && WM == 2), "8-bit element formats only");
@@ -197,12 +198,13 @@ __global__ __launch_bounds__(256) void mx_gemm_pipe_kernel(const GemmParams p) {
     // workgroup (the general store epilogue with its three output types and edge cases needs too many
     // registers to sit inside the loop).
     constexpr bool kPersistent = pipe_is_persistent(NSLOT, EPI);
-    // Grouped problems: the tiles come from tables (the FFN's, problems of more than kInlineGroups groups) or, in the fixed-stride walk of the
-    // persistent 2 x 2 kernels, from a scan of the sizes that stays in seven registers: the launch that fills the tables takes 5 us, the scan
-    // 1, about as long as the chain of table reads that it replaces.
-    // (The store epilogues leave those registers only to the FP4 kernel: here they would spill 249.)
-    constexpr bool kScan = kPersistent && WW == 2 && WM == 2 && (EPI == kEpiSwigluQuant || kI8);
-    const bool grouped = p.row_off != nullptr || (kScan && p.sizes != nullptr);
+    // Grouped problems: the tiles come from tables (the FFN's, problems of many groups or rounds) or, in the fixed-stride walk of the persistent
+    // 2 x 2 kernels, from a scan of the sizes that stays in seven registers: the launch that fills the tables takes 5 us, the scan 1, about as
+    // long as the chain of table reads that it replaces.  A kernel for each way: the scan costs every tile a little (16 groups x 2048 rows, eight
+    // rounds, 0.7 %), and in the 8-bit store kernel it would spill 249 registers.  INT8, which has no block scales, has room for both.
+    static_assert(!SCAN || (kPersistent && WW == 2 && WM == 2 && (EPI == kEpiSwigluQuant || kI8)), "scanned groups");
+    const bool scanned = SCAN && (!kI8 || p.sizes != nullptr);
+    const bool grouped = p.row_off != nullptr || scanned;
     GroupScan groups = {};
     if constexpr (kI8) {
         if (p.choice_cus != 0) {
@@ -210,7 +212,7 @@ __global__ __launch_bounds__(256) void mx_gemm_pipe_kernel(const GemmParams p) {
             if (__builtin_amdgcn_readfirstlane((int)pay) != 0) return;
         }
     }
-    const uint32_t m_tiles_all = kScan && p.sizes != nullptr ? scan_groups<TM>(p, groups) : count_m_tiles<TM>(p);
+    const uint32_t m_tiles_all = scanned ? scan_groups<TM>(p, groups) : count_m_tiles<TM>(p);
     const uint32_t total_tiles = m_tiles_all * p.w_tiles;
     uint32_t run_count;
     const uint32_t run_first = xcd_run(total_tiles, blockIdx.x % kXcds, run_count);
@@ -240,7 +242,7 @@ __global__ __launch_bounds__(256) void mx_gemm_pipe_kernel(const GemmParams p) {
         return r;
     };
     auto aim_loads_at = [&](uint32_t L, uint32_t g_from) {
-        if (kScan && p.sizes != nullptr) decode_scanned_tile<TM>(p, groups, L, tq);
+        if (scanned) decode_scanned_tile<TM>(p, groups, L, tq);
         else decode_tile<TM>(p, m_tiles_all, L, tq, g_from);
         const uint32_t g = __builtin_amdgcn_readfirstlane(tq.g), wt = __builtin_amdgcn_readfirstlane(tq.wt);
         const uint32_t row0 = __builtin_amdgcn_readfirstlane(tq.row0);
@@ -694,7 +696,7 @@ __global__ __launch_bounds__(256) void mx_gemm_pipe_kernel(const GemmParams p) {
                     __syncthreads();
                     next_id = run_first + tile_stride + __builtin_amdgcn_readfirstlane(*mailbox);
                 } else {
-                    next_id = next_of_walk(tile_id, tile_stride, run_end);
+                    next_id = WM == 2 ? next_of_walk(tile_id, tile_stride, run_end) : tile_id + tile_stride;
                 }
                 next_ok = next_id < run_end;
                 if (next_ok) {

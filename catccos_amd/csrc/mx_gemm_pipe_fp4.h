@@ -71,7 +71,7 @@ __device__ __forceinline__ void mfma_acc_fp4(v16f& acc, const v4i& w, const v4i&
 }
 
 // WW x WM = 2 x 2 (dense) or 4 x 1 (grouped: skips the MFMAs of activation blocks without valid rows)
-template <int EPI, int WW, int WM>
+template <int EPI, int WW, int WM, bool SCAN = false>              // SCAN: as in mx_gemm_pipe_kernel
 __global__ __launch_bounds__(256) void mx_gemm_pipe_fp4_kernel(const GemmParams p) {
     static_assert((WW == 2 && WM == 2) || (WW == 4 && WM == 1), "wavefront layout");
     static_assert(!epi_pairs_gate_up(EPI), "store epilogues only");
@@ -101,10 +101,10 @@ __global__ __launch_bounds__(256) void mx_gemm_pipe_fp4_kernel(const GemmParams 
 
     // ---- tile sequence of this workgroup (see mx_gemm_pipe_kernel) ----
     constexpr bool kPersistent = pipe_is_persistent(2, EPI);
-    constexpr bool kScan = kPersistent && WW == 2 && WM == 2;
-    const bool grouped = p.row_off != nullptr || (kScan && p.sizes != nullptr);
+    static_assert(!SCAN || (kPersistent && WW == 2 && WM == 2), "scanned groups");
+    const bool grouped = p.row_off != nullptr || SCAN;
     GroupScan groups = {};
-    const uint32_t m_tiles_all = kScan && p.sizes != nullptr ? scan_groups<TM>(p, groups) : count_m_tiles<TM>(p);
+    const uint32_t m_tiles_all = SCAN ? scan_groups<TM>(p, groups) : count_m_tiles<TM>(p);
     const uint32_t total_tiles = m_tiles_all * p.w_tiles;
     uint32_t run_count;
     const uint32_t run_first = xcd_run(total_tiles, blockIdx.x % kXcds, run_count);
@@ -133,7 +133,7 @@ __global__ __launch_bounds__(256) void mx_gemm_pipe_fp4_kernel(const GemmParams 
         return r;
     };
     auto aim_loads_at = [&](uint32_t L, uint32_t g_from) {
-        if (kScan && p.sizes != nullptr) decode_scanned_tile<TM>(p, groups, L, tq);
+        if constexpr (SCAN) decode_scanned_tile<TM>(p, groups, L, tq);
         else decode_tile<TM>(p, m_tiles_all, L, tq, g_from);
         const uint32_t g = __builtin_amdgcn_readfirstlane(tq.g), wt = __builtin_amdgcn_readfirstlane(tq.wt);
         const uint32_t row0 = __builtin_amdgcn_readfirstlane(tq.row0);
@@ -447,7 +447,7 @@ __global__ __launch_bounds__(256) void mx_gemm_pipe_fp4_kernel(const GemmParams 
                     __syncthreads();
                     next_id = run_first + tile_stride + __builtin_amdgcn_readfirstlane(*mailbox);
                 } else {
-                    next_id = next_of_walk(tile_id, tile_stride, run_end);
+                    next_id = WM == 2 ? next_of_walk(tile_id, tile_stride, run_end) : tile_id + tile_stride;
                 }
                 next_ok = next_id < run_end;
                 if (next_ok) {

@@ -38,8 +38,8 @@ FLAGS = ["--offload-arch=gfx950", "-O3", "-std=c++17", "-Xclang", "-target-featu
 
 # (explicit instantiation, the schedule's own vmcnt waits inside the stream: the early tile loads -- 7 or 8 (6 for FP4); the
 # persistent 2 x 2 kernels send all 8 weight loads early -- plus 2 prefetch loads in the persistent 2 x 2 kernels)
-#   mx_gemm_pipe_kernel<FMT, EPI, TM, WW, WM, NSLOT>; EPI 0 store, 1 SwiGLU + requant, 2 lean bf16, 3 INT8, 4 lean fp16, 5 = 1 + bf16 activations
-#   mx_gemm_pipe_fp4_kernel<EPI, WW, WM>
+#   mx_gemm_pipe_kernel<FMT, EPI, TM, WW, WM, NSLOT, SCAN>; EPI 0 store, 1 SwiGLU + requant, 2 lean bf16, 3 INT8, 4 lean fp16, 5 = 1 + bf16 activations
+#   mx_gemm_pipe_fp4_kernel<EPI, WW, WM, SCAN>
 #   mx_gemm_wreg_kernel<FMT, EPI, TM>: the wait at the start of a slab leaves the weight loads of the next slab and all loads of
 #   the one after in flight (8 + 16 or 17), and behind the slab that sent a scale block the loads of that block too
 KERNELS = [
@@ -54,6 +54,7 @@ KERNELS = [
     ("mx_gemm_wreg_kernel<1, 2, 288>", {25, 29}),
     ("mx_gemm_wreg_kernel<1, 4, 288>", {25, 29}),
     ("mx_gemm_pipe_kernel<0, 1, 256, 2, 2, 2>", {10}),
+    ("mx_gemm_pipe_kernel<0, 1, 256, 2, 2, 2, true>", {10}),
     ("mx_gemm_pipe_kernel<0, 1, 256, 4, 1, 2>", {8}),
     ("mx_gemm_pipe_kernel<0, 5, 256, 2, 2, 2>", {10}),          # SwiGLU + requant that also writes the bf16 activations
     ("mx_gemm_pipe_kernel<0, 5, 256, 4, 1, 2>", {8}),
@@ -66,6 +67,8 @@ KERNELS = [
     ("mx_gemm_pipe_kernel<0, 1, 128, 4, 1, 3>", {14}),
     ("mx_gemm_pipe_fp4_kernel<2, 2, 2>", {10}),
     ("mx_gemm_pipe_fp4_kernel<4, 2, 2>", {10}),
+    ("mx_gemm_pipe_fp4_kernel<2, 2, 2, true>", {10}),
+    ("mx_gemm_pipe_fp4_kernel<4, 2, 2, true>", {10}),
     ("mx_gemm_pipe_fp4_kernel<2, 4, 1>", {8}),
     ("mx_gemm_pipe_fp4_kernel<4, 4, 1>", {8}),
     ("mx_gemm_pipe_fp4_kernel<0, 2, 2>", {6}),
