@@ -3,6 +3,7 @@
 #pragma once
 
 #include "mx_common.h"
+#include "tile_walk.h"
 
 namespace cmx {
 

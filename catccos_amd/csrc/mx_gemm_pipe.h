@@ -308,10 +308,8 @@ __global__ __launch_bounds__(256) void mx_gemm_pipe_kernel(const GemmParams p) {
     aim_loads_at(tile_id, 0);
     Tile tc = tq;                               // tile of the MFMA stream / epilogue
 
-    auto nslab_of = [](const GemmParams& q) -> uint32_t { return q.kbytes / kSlabBytes; };
-    const uint32_t nslab_k = nslab_of(p);
-    // INT8 takes any number of slabs: an odd one is filled up with a slab of zeros
-    const uint32_t nslab = kI8 ? (nslab_k + 1) & ~1u : nslab_k;
+    const KSlabs slabs = k_slabs(p.kbytes, kSlabBytes, kI8);
+    const uint32_t nslab = slabs.walked;
     const uint32_t dma_base = __builtin_amdgcn_readfirstlane(lds0 + wave * 1024);
     constexpr int kScaleRowBytes = kSc4 && !kI8 ? 16 : 4;
     const uint32_t sdma_base = __builtin_amdgcn_readfirstlane(lds0 + kScaleBase + wave * 64 * kScaleRowBytes);
@@ -341,10 +339,10 @@ __global__ __launch_bounds__(256) void mx_gemm_pipe_kernel(const GemmParams p) {
     };
     // the load stream is at slab q of its tile: block 0 goes out with slab 0, block b+1 with slab 4b+1 (the ring
     // position it takes was last read one slab earlier)
-    const uint32_t nblk = nslab_of(p) / 4;
+    const uint32_t nblk = slabs.real / 4;
     auto scale_block_due = [&](uint32_t q) -> bool { return kI8 ? q == 0 : q == 0 || ((q & 3u) == 1u && (q >> 2) + 1 < nblk); };
     auto scale_block_of = [&](uint32_t q) -> uint32_t { return q == 0 ? 0u : (q >> 2) + 1; };
-    auto clamp_slab = [&](uint32_t slab) -> uint32_t { return slab < nslab ? slab : nslab - 1; };   // past the end: harmless reload
+    auto clamp_slab = [&](uint32_t slab) -> uint32_t { return load_slab(slab, slabs); };
 
     // ---- fragment read addresses ------------------------------------------------------------------
     // a lane reads 16-byte chunks lh, lh+2 (step 0) and lh+4, lh+6 (step 1) of its row; all rows of a
@@ -437,7 +435,7 @@ __global__ __launch_bounds__(256) void mx_gemm_pipe_kernel(const GemmParams p) {
 #pragma unroll
         for (int i = 0; i < kTileLoads; ++i) issue_tile_load(1, i, k1 * kSlabBytes);
         if constexpr (kPf > 0) {
-            const uint32_t kp = clamp_slab(1 + kPfAhead) * kSlabBytes;
+            const uint32_t kp = prefetch_slab(1 + kPfAhead, slabs) * kSlabBytes;
             issue_prefetch(0, kp);
             issue_prefetch(1, kp);
         }
@@ -527,7 +525,7 @@ __global__ __launch_bounds__(256) void mx_gemm_pipe_kernel(const GemmParams p) {
         using OtherT = std::integral_constant<int, slot ^ 1>;
         if constexpr (kI8) {
             // (a buffer of no bytes past K: its loads put zeros into the LDS)
-            const int range = __builtin_amdgcn_readfirstlane(koff < p.kbytes ? -1 : 0);
+            const int range = __builtin_amdgcn_readfirstlane(slab_in_memory(koff / kSlabBytes, slabs) ? -1 : 0);
             w_rs[2] = range;
             a_rs[2] = range;
         }
@@ -676,8 +674,8 @@ __global__ __launch_bounds__(256) void mx_gemm_pipe_kernel(const GemmParams p) {
         fence_accumulators();
         epilogue<TW, TM, WW, WM, EPI, FW, FM>(p, tc, acc, ww, wm, lane);
     } else {
-        // The host only selects this kernel for a slab count that is a multiple of four.  The load stream runs two slabs ahead of
-        // the MFMA stream: when it reaches the end of the tile it is aimed at the workgroup's next tile (or keeps
+        // An even number of slabs is walked: whole blocks of four, or, for INT8, any number from two on, filled up with a slab that is not in
+        // memory (KSlabs).  The load stream runs two slabs ahead of the MFMA stream: when it reaches the end of the tile it is aimed at the workgroup's next tile (or keeps
         // re-requesting the last slab when there is none), so the loads and the fragment reads run on through
         // the tile boundary and only the epilogue and the clearing of the accumulators interrupt the MFMAs.
         // One loop holds every case so that the register assignment of the scheduled part never changes.
@@ -704,8 +702,8 @@ __global__ __launch_bounds__(256) void mx_gemm_pipe_kernel(const GemmParams p) {
                     sq = 0;
                 }
             }
-            slab_body2(I0{}, clamp_slab(sq) * kSlabBytes, sq < nslab ? sq : kNoSlab, clamp_slab(sq + kPfAhead) * kSlabBytes);
-            slab_body2(I1{}, clamp_slab(sq + 1) * kSlabBytes, sq + 1 < nslab ? sq + 1 : kNoSlab, clamp_slab(sq + 1 + kPfAhead) * kSlabBytes);
+            slab_body2(I0{}, clamp_slab(sq) * kSlabBytes, sq < nslab ? sq : kNoSlab, prefetch_slab(sq + kPfAhead, slabs) * kSlabBytes);
+            slab_body2(I1{}, clamp_slab(sq + 1) * kSlabBytes, sq + 1 < nslab ? sq + 1 : kNoSlab, prefetch_slab(sq + 1 + kPfAhead, slabs) * kSlabBytes);
             sq += 2;
             sm += 2;
             if (sm == nslab) {
