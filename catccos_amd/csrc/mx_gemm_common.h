@@ -11,7 +11,6 @@ namespace cmx {
 
 constexpr int kSlabBytes = 128;     // K bytes per LDS slab and row
 constexpr int kChunks = kSlabBytes / 16;
-constexpr int kXcds = 8;
 
 // kEpiStoreBf16 / kEpiStoreFp16: 16-bit output whose rows and row pitch are multiples of eight elements (16-byte
 // stores, no per-element edge handling): small enough to sit inside a persistent kernel's tile loop.  Two epilogues, not one with a run-time switch: a second copy of the store loop inside the kernel costs
@@ -117,33 +116,6 @@ __device__ __forceinline__ uint32_t xcd_run(uint32_t total_tiles, uint32_t x, ui
     const uint32_t base = total_tiles / kXcds, rem = total_tiles % kXcds;
     count = base + (x < rem ? 1u : 0u);
     return x * base + (x < rem ? x : rem);
-}
-
-// Persistent kernels that walk in fixed strides (no tile counter), with at least one full round of tiles: instead of
-// owning a contiguous run, the XCDs take turns at blocks of (workgroups per XCD) consecutive tiles, workgroup j of XCD x
-// walking tiles x * per + j, + grid, + 2 * grid, ...  The whole chip then works on one stretch of `grid` consecutive
-// tiles at a time -- two bands of m-tiles across all their weight tiles -- so an activation panel is wanted by four XCDs
-// and a weight panel by two at about the same time (the memory-side cache can serve the repeats), and every block of 32
-// tiles starts on a multiple of 32, where the contiguous runs cut across the bands.  Zipf-routed 16-expert problem: 16 %
-// fewer L2 misses, 1.7-3.3 % less time.  Problems of less than a round keep the contiguous runs, which spread few tiles
-// over all eight L2s.
-__device__ __forceinline__ void interleave_xcd_walk(uint32_t total_tiles, uint32_t& tile_id, uint32_t& stride, uint32_t& end) {
-    if (total_tiles < gridDim.x) return;
-    tile_id = (blockIdx.x % kXcds) * (gridDim.x / kXcds) + blockIdx.x / kXcds;
-    stride = gridDim.x;
-    end = total_tiles;
-}
-// The tile after tile_id of such a walk, or `end`.  In the last, partly filled round the XCDs take fewer tiles each, in whole bands of 8: in
-// blocks of 32 they would all lie on the first XCDs, and the L2s and links of the others would have nothing to do.  320 tiles on 256
-// workgroups (us): SwiGLU 8 x 1280 rows, K = 4096, N = 2048 124.5 -> 112.6, FP4 125.7 -> 117.2, dense 8192 x 5120 x 7168 (640 tiles) 281 -> 264; 384
-// tiles 128 -> 117.  In contiguous runs of any length, which cut across the bands, 65536 rows on 32 groups (17 rounds) lose 1.6 %.
-constexpr uint32_t kSpreadRounds = 6;              // (five rounds 337 -> 333; at eight the workgroups have drifted apart and the order makes no difference)
-__device__ __forceinline__ uint32_t next_of_walk(uint32_t tile_id, uint32_t stride, uint32_t end) {
-    const uint32_t next = tile_id + stride;
-    if (stride != gridDim.x || end >= kSpreadRounds * stride || next < end / stride * stride) return next;
-    const uint32_t full = end / stride * stride, per = ((end - full + kXcds - 1) / kXcds + 7) / 8 * 8, j = blockIdx.x / kXcds;
-    const uint32_t last = full + blockIdx.x % kXcds * per + j;
-    return tile_id < full && j < per && last < end ? last : end;
 }
 
 // One tile per workgroup (blockIdx.x < total_tiles).  Workgroups start in the order of their ids, ids congruent mod 8 on one

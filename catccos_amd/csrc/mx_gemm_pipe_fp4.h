@@ -111,7 +111,7 @@ __global__ __launch_bounds__(256) void mx_gemm_pipe_fp4_kernel(const GemmParams 
     uint32_t run_end = run_first + run_count;
     uint32_t tile_stride = kPersistent ? gridDim.x / kXcds : total_tiles;      // one tile only when not persistent
     uint32_t tile_id = run_first + blockIdx.x / kXcds;
-    if (kPersistent && p.tile_ctr == nullptr) interleave_xcd_walk(total_tiles, tile_id, tile_stride, run_end);
+    if (kPersistent && p.tile_ctr == nullptr) interleave_xcd_walk(total_tiles, blockIdx.x, gridDim.x, tile_id, tile_stride, run_end);
     if (!kPersistent && blockIdx.x < total_tiles) {
         tile_id = tile_of_workgroup(total_tiles);
         run_end = total_tiles;
@@ -447,7 +447,7 @@ __global__ __launch_bounds__(256) void mx_gemm_pipe_fp4_kernel(const GemmParams 
                     __syncthreads();
                     next_id = run_first + tile_stride + __builtin_amdgcn_readfirstlane(*mailbox);
                 } else {
-                    next_id = WM == 2 ? next_of_walk(tile_id, tile_stride, run_end) : tile_id + tile_stride;
+                    next_id = WM == 2 ? next_of_walk(tile_id, tile_stride, run_end, blockIdx.x, gridDim.x) : tile_id + tile_stride;
                 }
                 next_ok = next_id < run_end;
                 if (next_ok) {

@@ -1,5 +1,6 @@
 // A host's walk through the index arithmetic of the persistent kernels.  Prints what is wrong; exit status 1 if anything is.
 #include <cstdio>
+#include <vector>
 
 #include "../../catccos_amd/csrc/tile_walk.h"
 
@@ -38,9 +39,31 @@ void check_slabs(uint32_t real, bool fill_to_even) {
     }
 }
 
+// Every tile of `total` goes to one workgroup of `grid`, in the walk of at least a round of tiles.
+void check_tiles(uint32_t grid, uint32_t total) {
+    std::vector<int> visits(total);
+    bool outside = false;
+    for (uint32_t wg = 0; wg < grid; ++wg) {
+        uint32_t tile = total, stride = 0, end = 0;
+        interleave_xcd_walk(total, wg, grid, tile, stride, end);
+        for (uint32_t turn = 0; tile < end && turn <= total; tile = next_of_walk(tile, stride, end, wg, grid), ++turn) {
+            if (tile < total) ++visits[tile];
+            else outside = true;
+        }
+    }
+    uint32_t lost = 0, twice = 0;
+    for (int v : visits) lost += v == 0, twice += v > 1;
+    if (lost == 0 && twice == 0 && !outside) return;
+    ++faults;
+    std::printf("%u tiles on %u workgroups: %u with nobody, %u more than once%s\n", total, grid, lost, twice, outside ? ", some that do not exist" : "");
+}
+
 }  // namespace
 
 int main() {
+    // (launches take a multiple of eight workgroups)
+    for (uint32_t grid = 8; grid <= 304; grid += 8)
+        for (uint32_t total = grid; total <= (kSpreadRounds + 1) * grid; ++total) check_tiles(grid, total);
     for (uint32_t real = 2; real <= 64; ++real) {
         check_slabs(real, true);
         if (real % 4 == 0) check_slabs(real, false);

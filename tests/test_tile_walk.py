@@ -1,5 +1,5 @@
-"""The index arithmetic of the persistent matmul kernels (catccos_amd/csrc/tile_walk.h), walked on the host: every slab that they ask memory for
-lies within K, whatever the number of slabs."""
+"""The index arithmetic of the persistent matmul kernels (catccos_amd/csrc/tile_walk.h), walked on the host: every tile goes to one
+workgroup, whatever the number of CUs, and every slab that they ask memory for lies within K, whatever the number of slabs."""
 import os
 import shutil
 import subprocess
