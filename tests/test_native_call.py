@@ -219,6 +219,38 @@ def test_new_tensors_and_the_current_stream_reach_the_entry_point():
 
 
 @pytest.mark.gpu
+def test_new_tensors_are_those_of_torch_empty():
+    """Filled where deterministic algorithms are asked for, seen by a dispatch mode, inference tensors in inference mode."""
+    from torch.utils._python_dispatch import TorchDispatchMode
+    x = torch.zeros(4, device="cuda")
+    routes = torch.tensor([[0, -1], [7, 1]], dtype=torch.int32, device="cuda")          # two of four dropped
+    was = torch.are_deterministic_algorithms_enabled()
+    torch.use_deterministic_algorithms(True)
+    try:
+        assert bool(_native_call.empty(x, torch.float32, 5, 3).isnan().all())
+        assert ops.moe_init_routing(routes, 2)[0].tolist() == [0, 3, 2 ** 31 - 1, 2 ** 31 - 1]
+    finally:
+        torch.use_deterministic_algorithms(was)
+
+    class Seen(TorchDispatchMode):
+        def __init__(self, give=None):
+            super().__init__()
+            self.calls, self.give = [], give
+
+        def __torch_dispatch__(self, func, types, args=(), kwargs=None):
+            self.calls.append(func)
+            return func(*args, **(kwargs or {})) if self.give is None else self.give
+    with Seen() as mode:
+        ops.moe_init_routing(routes, 2)
+    assert mode.calls == [torch.ops.aten.empty.memory_format] * 4                       # workspace and three outputs
+    with Seen(torch.zeros(5)), pytest.raises(ValueError, match="expected a GPU tensor"):
+        _native_call.empty(x, torch.float32, 5)
+    with torch.inference_mode():
+        assert ops.moe_init_routing(routes, 2)[2].is_inference()
+    assert not ops.moe_init_routing(routes, 2)[2].is_inference()
+
+
+@pytest.mark.gpu
 def test_buffers_that_the_caller_brings_may_be_pinned():
     """Weights, outputs and workspaces in pinned host memory give the results that device buffers give (no kernel of these small problems uses
     the workspace); other host memory, and inputs in host memory, are refused."""
