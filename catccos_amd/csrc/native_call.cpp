@@ -139,6 +139,10 @@ PyObject* run(PyObject*, PyObject* const* args, Py_ssize_t n) {
             continue;
         }
         if (args[i] == Py_Ellipsis) {
+            if (stream >= 0) {
+                PyErr_SetString(PyExc_TypeError, "an Ellipsis stands for the stream, once");
+                return nullptr;
+            }
             stream = i - 1;
             continue;
         }

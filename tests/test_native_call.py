@@ -175,6 +175,19 @@ def test_entries_follow_the_active_library():
     assert set(_lib.entries()) == set(_lib.SIGNATURES) and all(_lib.entries().values())
 
 
+def test_an_ellipsis_in_the_place_of_a_tensor_is_refused():
+    """Only the front end puts one, behind the other arguments; one that the caller gives would leave a null pointer in its place."""
+    got = []
+
+    @C.CFUNCTYPE(C.c_int, *[C.c_uint64] * 24)
+    def callee(*args):
+        got.append(args)
+        return 0
+    with pytest.raises(TypeError, match="Ellipsis"):
+        _native_call.run(C.cast(callee, C.c_void_p).value, ..., 1, ...)
+    assert not got
+
+
 @pytest.mark.gpu
 def test_outputs_and_errors_on_the_gpu():
     x = torch.randn(3, 64, device="cuda").to(torch.bfloat16)
