@@ -77,6 +77,13 @@ def _brought(t):
     return t if isinstance(t, torch.Tensor) and (t.is_cuda or not t.is_pinned()) else t.data_ptr()
 
 
+def _no_new(*ts):
+    """What a caller gives where _launch gets it as it is, and where a tuple would stand for a new tensor."""
+    for t in ts:
+        if isinstance(t, tuple):
+            raise TypeError("expected a tensor, not a tuple")
+
+
 def _need_cuda(*ts):
     for t in ts:
         if t is not None and not t.is_cuda:
@@ -179,6 +186,7 @@ def int8_quant_scatter(x: torch.Tensor, src2sorted, top_k: int = 1):
     tokens, k = x.shape
     pitch, step = x.stride()
     assert step == 1
+    _no_new(src2sorted)
     return _launch("cmx_int8_quant_scatter", x, pitch, src2sorted, (torch.int8, tokens * top_k, k), k, (torch.float32, tokens * top_k), tokens, k, top_k)
 
 
@@ -187,6 +195,7 @@ def int8_gmm_dequant_swiglu(a, token_scale, b, channel_scale, group_sizes, n: in
     """a int8 [rows, k]; b int8 [G, k, n] (trans_b = 0) or [G, n, k] (trans_b = 1); channel_scale fp32 [G*n*scale_stride]."""
     n, k, trans_b, scale_stride = index(n), index(k), index(trans_b), index(scale_stride)
     assert a.is_contiguous() and b.is_contiguous() and group_sizes.dtype == torch.int32
+    _no_new(token_scale, channel_scale)
     rows, g = a.size(0), b.size(0)
     ws = _empty(a, torch.uint8, _lib.load().cmx_int8_gmm_workspace_bytes(g, n, k, trans_b))
     if c is None:

@@ -188,6 +188,17 @@ def test_an_ellipsis_in_the_place_of_a_tensor_is_refused():
     assert not got
 
 
+def test_a_tuple_in_the_place_of_a_tensor_is_refused():
+    """Only the front end puts one, for a new tensor; one that the caller gives would reach the kernel as a tensor of anything."""
+    spec, x = (torch.int32, 8), torch.zeros((8, 64), dtype=torch.bfloat16)
+    with pytest.raises(TypeError, match="tuple"):
+        ops.int8_quant_scatter(x, spec, 1)
+    a, w, scale, sizes = x.view(torch.int16).to(torch.int8), torch.zeros((1, 64, 64), dtype=torch.int8), torch.ones(64), torch.zeros(1, dtype=torch.int32)
+    for token, channel in (spec, scale), (scale, spec):
+        with pytest.raises(TypeError, match="tuple"):
+            ops.int8_gmm_dequant_swiglu(a, token, w, channel, sizes, 64, 64, 1)
+
+
 @pytest.mark.gpu
 def test_outputs_and_errors_on_the_gpu():
     x = torch.randn(3, 64, device="cuda").to(torch.bfloat16)
