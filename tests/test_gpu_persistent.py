@@ -106,3 +106,25 @@ def test_int8_gives_the_bits_of_the_streaming_kernel(out, counts, n, k):
         return c
     got, ref = _pinned(call)
     assert torch.equal(got, ref) and not bool((ref[:m] == 7.0).all(dim=1).any())
+
+
+@pytest.mark.parametrize("out", ["fp32", "bf16", "fp16"])
+def test_int8_rounds_special_values_like_the_streaming_kernel(out):
+    """Token scales that make outputs zero, denormal, halfway between neighbours, infinite and NaN."""
+    from catccos_amd import ops
+    g = torch.Generator(device="cuda")
+    g.manual_seed(3)
+    counts, n, k = [256, 300], 256, 512
+    m = sum(counts)
+    a = torch.randint(-127, 128, (m, k), dtype=torch.int8, device="cuda", generator=g)
+    w = torch.randint(-127, 128, (2, n, k), dtype=torch.int8, device="cuda", generator=g)
+    w[:, 0], w[:, n // 2] = 0, 0                                                     # sums of zero, which infinite scales make NaN
+    token = torch.rand(m, device="cuda", generator=g)
+    special = [0.0, -0.0, float("inf"), -float("inf"), float("nan"), 1e-38, 1e-42, 1e-20, 2.0 ** -12, 2.0 ** -13, 3.0, 1e4, 1e30, 3e38]
+    token[:16 * len(special)] = torch.tensor(special, device="cuda").repeat(16)
+    token[-1], token[-2] = torch.tensor([0x7F80_0001, -1], dtype=torch.int32).view(torch.float32).cuda()            # other NaNs
+    channel = torch.full((2 * n,), 2.0 ** -10, device="cuda")
+    channel[::7] = torch.rand(channel[::7].numel(), device="cuda", generator=g)
+    call = lambda: ops.int8_gmm_dequant_swiglu(a, token, w, channel, dev(np.array(counts, dtype=np.int32)), n, k, 1, out)
+    got, ref = _pinned(call)
+    assert torch.equal(got.view(torch.int16), ref.view(torch.int16)) and bool(ref.isnan().any()) and bool(ref.isinf().any())

@@ -21,3 +21,12 @@ pytestmark = pytest.mark.skipif(not (os.path.exists(chk.HIPCC) or shutil.which("
 def test_scheduled_stream_is_free_of_spills_and_foreign_waits(kernel, own_waits, tmp_path):
     problems = chk.check(kernel, own_waits, str(tmp_path))
     assert not problems, "\n".join(problems[:10])
+
+
+def test_int8_epilogue_branches_by_the_piece(tmp_path):
+    """The INT8 kernel stores 32 pieces of four values: a handful of branches for each, not one for every value, on the output type."""
+    chk.check("mx_gemm_pipe_kernel<8, 3, 256, 2, 2, 2>", set(), str(tmp_path))
+    code = [ln.strip() for ln in open(tmp_path / "one_kernel.s")]
+    stores = code[max(i for i, ln in enumerate(code) if ln.startswith("v_mfma")):]
+    assert sum(ln.startswith("v_exp_f32") for ln in stores) == 128                                   # values of a thread
+    assert sum(ln.startswith(("s_cbranch", "s_branch")) for ln in stores) < 6 * 32
