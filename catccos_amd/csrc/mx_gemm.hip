@@ -1699,6 +1699,29 @@ extern "C" size_t cmx_int8_gmm_workspace_bytes(uint32_t groups, uint32_t n, uint
     return meta + (trans_b ? 0 : cmx::round_up_sz((size_t)groups * n * k, 256));
 }
 
+namespace cmx {
+namespace {
+// Takes fp32 outputs of up to two rounds of 256 x 256 tiles and short K from the persistent kernel (*pipe) where it is slower than the streaming
+// one.  With an odd number of slabs it walks one more, a microsecond a round (K below 2048); where groups average 256 rows or less, the tiles of
+// a second round are few and its longer start shows (K up to 1536; K = 256: up to 512 rows).  With 16-bit outputs it is the faster one throughout.
+// Measured (us, streaming against persistent; u: routes drawn uniformly, z: Zipf; N = 2048):
+//   groups x rows   K = 256         384           512           640           1152          1536          1920          2048          3072
+//   16 x 300 u      16.3  17.8   18.1  19.7   19.8  20.1   21.8  22.3   28.2  29.0   32.5  32.1   36.9  37.4   38.7  37.6   50.2  48.6
+//   32 x 140 z      26.4  28.6   29.8  32.8   32.2  34.5   34.9  38.9   44.1  47.9   51.1  53.0   58.8  62.4   61.0  62.4   81.6  82.1
+//   24 x 150 z      16.0  17.4   17.9  19.3   19.7  20.0                27.8  29.0   32.3  32.2   36.6  37.4   38.8  37.6   49.0  48.4
+//   8 x 1000 u      29.6  29.4   32.6  33.6   34.7  33.9   37.8  38.7   47.3  48.3   54.8  53.7   63.0  63.5   65.2  63.3   86.6  83.4
+//   16 x 700 z      31.7  30.1   35.3  35.3   37.2  36.1   40.6  41.5   51.3  52.2   59.5  58.4   68.5  69.2   70.8  69.2   93.5  91.6
+//   8 x 1900 u (past two rounds)  45.2  38.3                54.0  45.2   62.7  56.0
+int i8_streams(bool* pipe, uint64_t most_tiles, uint32_t mean_rows, uint32_t nslab) {
+    int cus = 0;
+    if (int rc = cu_count(&cus); rc != CMX_OK) return rc;
+    const bool slower = nslab % 2 != 0 ? nslab < 16 : nslab <= 12 && mean_rows <= (nslab == 2 ? 512u : 256u);
+    if (slower && most_tiles <= 2 * (uint64_t)cus) *pipe = false;
+    return CMX_OK;
+}
+}  // namespace
+}  // namespace cmx
+
 extern "C" int cmx_int8_gmm_dequant_swiglu(const int8_t* a, uint32_t lda, const float* token_scale, const int8_t* b,
                                            const float* channel_scale, uint32_t channel_scale_stride, void* out,
                                            uint32_t ld_out, int out_type, const int32_t* group_sizes, uint32_t groups,
@@ -1739,8 +1762,8 @@ extern "C" int cmx_int8_gmm_dequant_swiglu(const int8_t* a, uint32_t lda, const 
     const bool all_ksplit = ks.tile.fw != 0 && ks.small_rows == 0;
     TileChoice t = {256, ceil_div(m_total, groups) <= 128 ? 128 : 256, 8};
     // The persistent kernel of 256 x 256 tiles stores 16 bytes at a time and has the scales' offsets in 32 bits; the streaming kernel takes the rest.
-    const bool pipe = (!g_force_tile.tw || g_force_tile.waves == 4) && !g_disable_dl && k >= 2 * kSlabBytes && (uint64_t)ld_out * (out_type == CMX_OUT_FP32 ? 4 : 2) % 16 == 0 &&
-                      aligned16(out) && (uint64_t)n * channel_scale_stride * 4 < (1ull << 32);
+    bool pipe = (!g_force_tile.tw || g_force_tile.waves == 4) && !g_disable_dl && k >= 2 * kSlabBytes && (uint64_t)ld_out * (out_type == CMX_OUT_FP32 ? 4 : 2) % 16 == 0 &&
+                aligned16(out) && (uint64_t)n * channel_scale_stride * 4 < (1ull << 32);
     bool choice = false;                                       // 128- or 256-row tiles: the device chooses by the sizes
     if (g_force_tile.waves == kRing) t = g_force_tile;
     else if (!g_force_tile.tw && !g_disable_dl) {
@@ -1748,6 +1771,9 @@ extern "C" int cmx_int8_gmm_dequant_swiglu(const int8_t* a, uint32_t lda, const 
         choice = !all_ksplit && t.waves == kRing && t.tw == 256 && pipe;
     }
     if (t.waves != kRing) t.tm = 256;
+    const uint64_t most_tiles = (uint64_t)max_group_tiles(m_total, groups, 256, ks.small_rows) * ceil_div(n, 256);
+    if (t.waves != kRing && !g_force_tile.tw && out_type == CMX_OUT_FP32)
+        if (int rc = i8_streams(&pipe, most_tiles, ceil_div(m_total, groups), k / kSlabBytes); rc != CMX_OK) return rc;
     // Kernels of one tile per workgroup find it by the sizes up to some rounds; past those the launch that fills the tables makes the
     // choice.  Where it would fill them for small groups as well, those that are left to the large tiles are large for
     // their average (256 x 32, 7168, 4096, on eight groups 227 against 277).  The persistent kernel scans the sizes once.

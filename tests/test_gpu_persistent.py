@@ -1,6 +1,8 @@
 """The persistent 256 x 256 kernels with 2 x 2 wavefronts: their walk through more and less than whole rounds of tiles, groups found by a
 scan of the sizes, and the INT8 kernel.  Reference: the streaming kernel of the same tile, one tile per workgroup, whose K order (INT8:
 whole-number sums) is the same, so the outputs are the same bits."""
+import ctypes
+
 import numpy as np
 import pytest
 import torch
@@ -128,3 +130,47 @@ def test_int8_rounds_special_values_like_the_streaming_kernel(out):
     call = lambda: ops.int8_gmm_dequant_swiglu(a, token, w, channel, dev(np.array(counts, dtype=np.int32)), n, k, 1, out)
     got, ref = _pinned(call)
     assert torch.equal(got.view(torch.int16), ref.view(torch.int16)) and bool(ref.isnan().any()) and bool(ref.isinf().any())
+
+
+class _KernelNode(ctypes.Structure):
+    _fields_ = [("block", ctypes.c_uint32 * 3), ("extra", ctypes.c_void_p), ("func", ctypes.c_void_p), ("grid", ctypes.c_uint32 * 3),
+                ("params", ctypes.c_void_p), ("shared", ctypes.c_uint32)]
+
+
+def _kernels_of(call):
+    """the kernels that a call launches, in no order, read from a capture of it"""
+    hip = ctypes.CDLL("libamdhip64.so")
+    call()                                             # (limits of the LDS are raised at the first launch)
+    graph, n = torch.cuda.CUDAGraph(keep_graph=True), ctypes.c_size_t()
+    with torch.cuda.graph(graph):
+        call()
+    raw = ctypes.c_void_p(graph.raw_cuda_graph())
+    assert hip.hipGraphGetNodes(raw, None, ctypes.byref(n)) == 0
+    nodes = (ctypes.c_void_p * n.value)()
+    assert hip.hipGraphGetNodes(raw, nodes, ctypes.byref(n)) == 0
+    out = []
+    for node in nodes:
+        k = _KernelNode()
+        assert hip.hipGraphKernelNodeGetParams(ctypes.c_void_p(node), ctypes.byref(k)) == 0
+        out.append(k.func)
+    return sorted(out)
+
+
+# at most two rounds of tiles: an odd number of slabs, one past the K up to which it counts, even; short groups; 16-bit output; past two rounds
+@pytest.mark.parametrize("e,rows,n,k,out,waves", [(16, 300, 2048, 384, "fp32", 8), (16, 300, 2048, 1920, "fp32", 8), (16, 300, 2048, 2176, "fp32", 4), (16, 300, 2048, 512, "fp32", 4),
+                                                  (16, 300, 2048, 256, "fp32", 8), (32, 140, 2048, 1536, "fp32", 8), (32, 140, 2048, 1792, "fp32", 4), (16, 300, 2048, 384, "bf16", 4),
+                                                  (8, 1900, 2048, 384, "fp32", 4)])
+def test_int8_kernel_by_size(e, rows, n, k, out, waves):
+    """waves: 8 the streaming kernel, 4 the persistent one"""
+    from catccos_amd import ops
+    a, w = torch.zeros((e * rows, k), dtype=torch.int8, device="cuda"), torch.zeros((e, n, k), dtype=torch.int8, device="cuda")
+    token, channel, cnt = torch.ones(e * rows, device="cuda"), torch.ones(e * n, device="cuda"), dev(np.full(e, rows, dtype=np.int32))
+    c = torch.empty((e * rows, n // 2), dtype=torch.float32 if out == "fp32" else torch.bfloat16, device="cuda")
+    call = lambda: ops.int8_gmm_dequant_swiglu(a, token, w, channel, cnt, n, k, 1, out, c=c)
+    h = hooks_lib()
+    h.cmx_debug_force_ksplit(-1, 0, 0)
+    got, pinned = _kernels_of(call), {}
+    for v in (4, 8):
+        h.cmx_debug_force_tile(256, 256, v)
+        pinned[v] = _kernels_of(call)
+    assert pinned[4][-1:] != pinned[8][-1:] and got == pinned[waves]
