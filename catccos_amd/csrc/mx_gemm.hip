@@ -1544,8 +1544,10 @@ uint32_t max_group_tiles(uint32_t m_total, uint32_t groups, uint32_t tile_m, uin
 //   128 x 128    8 experts x 64 rows u, K = 1024, N = 1024   14.6 -> 13.9 / 18.3 -> 13.7    x 200 z   22.1 -> 14.3 / 19.7 -> 14.5
 //                8 x 100 u, 4096, 2048                       35.7 -> 25.0 / 40.1 -> 25.4    16 x 64 z, 7168, 1024   56.8 -> 36.8 / 61.5 -> 36.7
 //   256 x 128    32 x 100 u, 7168, 4096                      206 -> 190 / 221 -> 204        32 x 128 z   320 -> 279 / 327 -> 284
-//                SwiGLU 32 x 100 u, K = 1024, N = 2048 21.5 -> 18.5, 4096 36.8 -> 34.5; 2048, 4096 61.2 -> 54.8; 64 x 90 z, 2048, 2048 71.9 -> 66.9; in many
-//                rounds at K = 1024 it loses a little: 128 x 70, 4096 u 141.8 against 143.7, z 163.3 against 167.2 (below K = 1024 not measured)
+//                SwiGLU 32 x 100 u, K = 1024, N = 2048 21.5 -> 18.5, 4096 36.9 -> 35.8; 2048, 4096 61.2 -> 54.8; 64 x 90 z, 2048, 2048 71.9 -> 66.9; below K = 1536
+//                only up to eight rounds: 64 x 110 u, 1024, 4096 83.6 -> 82.5, but 128 x 70, 1024, 4096 u 138.7 against 141.1, z 165.2 against 171.0; 256 x 50 u, 1024,
+//                2048 136.8 against 140.7; 128 x 90 z, 1152, 4096 199.8 against 206.8 (K = 1536, 128 x 70 u 190.8 and 191.5).  Between two and eight rounds
+//                it is within -3 and +4 % there (K = 1024: 32 x 70 z 42.3 and 42.7, 64 x 60 z, 2048 42.9 and 41.7, 64 x 70 u 66.3 and 69.1), to K = 1023 not measured
 //   128 x 256    8 x 200 u, 4096, 2048                       45.9 -> 34.5 / 43.1 -> 35.7    16 x 300 u, 7168, 1024   74 -> 57 / 69 -> 62
 //                8 x 500 u, 1024, 1024                       22.6 -> 18.6 / 19.4 -> 12.9; store 8 x 200 u, 512, 2048 15.3 -> 9.6, 16 x 300 u, 512, 1024 16.5 -> 11.3
 // Where n is at most 128, half of a 256-row tile would be empty: 128 x 128 for 256 x 128 (SwiGLU 256 x 68 z, 3072, 64 45 -> 34 where 256 x 128 takes
@@ -1568,7 +1570,7 @@ int ring_groups(TileChoice* t, uint32_t m_total, uint32_t groups, uint32_t n, in
     const uint64_t w128 = ceil_div(n, 128);
     const uint32_t k_min = eight_bit && swiglu ? 32 : 16;
     if (w128 * (m_total / 128 + groups) <= (uint64_t)cus) *t = {128, 128, kRing};
-    else if (t->tm <= 128 && kblocks >= k_min) *t = {w128 == 1 ? 128 : 256, 128, kRing};
+    else if (t->tm <= 128 && kblocks >= k_min && (!eight_bit || !swiglu || kblocks >= 48 || (uint64_t)ceil_div(n, 256) * (m_total / 128 + groups) <= 8 * (uint64_t)cus)) *t = {w128 == 1 ? 128 : 256, 128, kRing};
     else if (t->tm == 256 && w128 * (m_total / 256 + groups * 3 / 4) <= (uint64_t)cus) *t = {128, 256, kRing};
     return CMX_OK;
 }

@@ -174,3 +174,21 @@ def test_int8_kernel_by_size(e, rows, n, k, out, waves):
         h.cmx_debug_force_tile(256, 256, v)
         pinned[v] = _kernels_of(call)
     assert pinned[4][-1:] != pinned[8][-1:] and got == pinned[waves]
+
+
+# 8-bit SwiGLU in groups of at most 128 rows: the ring kernel, but for many rounds of its tiles at K below 1536
+@pytest.mark.parametrize("e,rows,n,k,waves", [(256, 40, 2048, 1024, 5), (256, 40, 2048, 1408, 5), (256, 40, 2048, 1536, 6), (160, 40, 2048, 1024, 6), (32, 100, 2048, 1024, 6)])
+def test_swiglu_kernel_of_short_groups_by_size(e, rows, n, k, waves):
+    """waves: 5 the three-slot kernel, 6 the ring kernel"""
+    from catccos_amd import ops
+    z = lambda *shape: torch.zeros(shape, dtype=torch.uint8, device="cuda")
+    a, a_s, w, w_s, cnt = z(e * rows, k), z(e * rows, k // 32), z(e, n, k), z(e, n, k // 32), dev(np.full(e, rows, dtype=np.int32))
+    outs, ws = (z(e * rows, n // 2), z(e * rows, ops.scale_cols(n // 2))), ops.gmm_workspace(e, "cuda")
+    call = lambda: ops.mx_gmm_swiglu_quant(a, a_s, w, w_s, cnt, k, workspace=ws, outs=outs)
+    h = hooks_lib()
+    h.cmx_debug_force_ksplit(-1, 0, 0)
+    got, pinned = _kernels_of(call), {}
+    for v in (5, 6):
+        h.cmx_debug_force_tile(256, 128, v)
+        pinned[v] = _kernels_of(call)
+    assert pinned[5] != pinned[6] and got == pinned[waves]
