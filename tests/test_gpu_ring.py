@@ -288,3 +288,32 @@ def test_tiles_located_by_sizes_are_those_of_the_tables(kernel, sizes, rows):
     if kernel == "ring":
         done = min(sum(max(s, 0) for s in sizes), rows)
         assert bool((got[done:].float() == 7.0).all()) and not bool((got[:done].float() == 7.0).all(dim=1).any())
+
+
+@pytest.mark.parametrize("tw,tm", [(128, 128), (256, 128), (128, 256)])
+@pytest.mark.parametrize("want_bf16", [False, True])
+def test_activation_codes_in_rows_of_four_byte_alignment(tw, tm, want_bf16):
+    """A thread's eight codes leave in one store where rows start at eight bytes, else in two; what lies between the rows is left alone."""
+    from catccos_amd import ops
+    counts, n, k = [130, 0, 257, 3], 320, 640
+    m, g = sum(counts) + 2, torch.Generator(device="cuda")
+    g.manual_seed(tw + tm)
+    codes = lambda *shape: torch.randint(0, 256, shape, dtype=torch.uint8, device="cuda", generator=g) & 0x77
+    scales = lambda *shape: torch.randint(112, 124, shape, dtype=torch.uint8, device="cuda", generator=g)
+    a, a_s, w, w_s = codes(m, k), scales(m, k // 32), codes(len(counts), n, k), scales(len(counts), n, k // 32)
+    cnt = dev(np.array(counts, dtype=np.int32))
+    hooks_lib().cmx_debug_force_tile(tw, tm, 6)
+
+    def outputs(pad, start):
+        """codes in rows of n / 2 + pad bytes, the first row `start` bytes behind a multiple of 16"""
+        buf = torch.full((m * (n // 2 + pad) + 16,), 0x55, dtype=torch.uint8, device="cuda")
+        rows = buf[start:start + m * (n // 2 + pad)].view(m, -1)
+        s = torch.full((m, ops.scale_cols(n // 2)), 0x55, dtype=torch.uint8, device="cuda")
+        act = ops.mx_gmm_swiglu_quant(a, a_s, w, w_s, cnt, k, want_bf16=want_bf16, outs=(rows[:, :n // 2], s))[2]
+        assert bool((rows[:, n // 2:] == 0x55).all()) and bool((buf[:start] == 0x55).all()) and bool((buf[start + rows.numel():] == 0x55).all())
+        return [rows[:, :n // 2], s] + ([act] if want_bf16 else [])
+    want = outputs(0, 0)
+    assert bool((want[0][:m - 2] != 0x55).any(dim=1).all()) and bool((want[0][m - 2:] == 0x55).all())
+    for pad, start in (4, 0), (8, 4), (0, 4):
+        for x, y in zip(outputs(pad, start), want):
+            assert torch.equal(x, y)
