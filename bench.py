@@ -259,7 +259,7 @@ def main() -> int:
         o8 = torch.empty((rows, N // 2), dtype=torch.float32, device=dev)
         t8 = hip_time(lambda: ops.int8_gmm_dequant_swiglu(a8, ts8, w8, ch8, counts, N, H, 1, "fp32", c=o8))
         extra["int8_gmm_dequant_swiglu_cfg3_shape"] = {
-            "kernel": "mx_gemm_dl_kernel<INT8, dequant+swiglu epilogue, 256x256 tile, 8 wavefronts> (grouped)", "bound": "mfma",
+            "kernel": "mx_gemm_pipe_kernel<INT8, dequant+swiglu epilogue, 2x2 wavefronts, persistent> (grouped, 256x256 tile)", "bound": "mfma",
             "achieved": flop / t8 / 1e12, "peak": INT8_PEAK_TOPS, "unit": "TOP/s", "frac": flop / t8 / 1e12 / INT8_PEAK_TOPS,
             "avg_launch_us": t8 * 1e6}
         log(f"[int8 gmm+dequant+swiglu, cfg3 shape] {t8*1e6:.1f} us -> {flop/t8/1e12:.0f} TOP/s")

@@ -944,6 +944,7 @@ int launch_gemm_impl(const GemmParams& p, uint32_t max_m_tiles, hipStream_t s) {
     constexpr int kScaleDw = FMT == CMX_FMT_E2M1 ? 2 : 1;
     constexpr size_t smem = 2 * ((TW + TM) * kSlabBytes + (TW + TM) * 4 * kScaleDw);
     constexpr auto kfn = mx_gemm_kernel<FMT, TW, TM, WW, WM, EPI, FAST>;
+    CMX_REQUIRE(p.sizes == nullptr, "groups by their sizes: not this kernel");
     if (int rc = allow_dynamic_lds<kfn, smem>(); rc != CMX_OK) return rc;
     const uint64_t tiles = (uint64_t)max_m_tiles * p.w_tiles;
     CMX_REQUIRE(tiles > 0 && tiles < (1ull << 31), "tile count out of range");
@@ -957,6 +958,7 @@ int launch_gemm_dl(const GemmParams& p, uint32_t max_m_tiles, hipStream_t s) {
     constexpr int kScaleDw = FMT == CMX_FMT_E2M1 ? 2 : 1;
     constexpr size_t smem = 2 * (TW + TM) * kSlabBytes + 2 * (TW + TM) * kScaleDw * 4;
     constexpr auto kfn = mx_gemm_dl_kernel<FMT, TW, TM, WW, WM, EPI>;
+    CMX_REQUIRE(FMT == kFmtI8 || p.sizes == nullptr, "groups by their sizes: not this kernel");
     if (int rc = allow_dynamic_lds<kfn, smem>(); rc != CMX_OK) return rc;
     const uint64_t tiles = (uint64_t)max_m_tiles * p.w_tiles;
     CMX_REQUIRE(tiles > 0 && tiles < (1ull << 31), "tile count out of range");
@@ -983,6 +985,7 @@ int launch_gemm_pipe(const GemmParams& p, uint32_t max_m_tiles, hipStream_t s) {
     constexpr size_t smem = NSLOT * (256 + TM) * kSlabBytes + (FMT == kFmtI8 ? 2 * (256 + TM) * 4 + 16384 : NSLOT == 2 ? 2 * (256 + TM) * 16 : NSLOT * (256 + TM) * 4) +
                             (pipe_stages_stores(NSLOT, EPI, WW, WM) ? 16384 : 512);
     constexpr auto kfn = mx_gemm_pipe_kernel<FMT, EPI, TM, WW, WM, NSLOT, SCAN>;
+    CMX_REQUIRE(SCAN || p.sizes == nullptr, "groups by their sizes: not this kernel");
     if (int rc = allow_dynamic_lds<kfn, smem>(); rc != CMX_OK) return rc;
     const uint64_t tiles = (uint64_t)max_m_tiles * p.w_tiles;
     CMX_REQUIRE(tiles > 0 && tiles < (1ull << 31), "tile count out of range");
@@ -1034,6 +1037,7 @@ int launch_gemm_pipe_fp4(const GemmParams& p, uint32_t max_m_tiles, hipStream_t 
     // whole-line stores, which overlays those 512 bytes)
     constexpr size_t smem = 2 * 512 * kSlabBytes + 2 * 512 * 16 + (pipe_stages_stores(2, EPI, WW, WM) ? 16384 : 512);
     constexpr auto kfn = mx_gemm_pipe_fp4_kernel<EPI, WW, WM, SCAN>;
+    CMX_REQUIRE(SCAN || p.sizes == nullptr, "groups by their sizes: not this kernel");
     if (int rc = allow_dynamic_lds<kfn, smem>(); rc != CMX_OK) return rc;
     const uint64_t tiles = (uint64_t)max_m_tiles * p.w_tiles;
     CMX_REQUIRE(tiles > 0 && tiles < (1ull << 31), "tile count out of range");
@@ -1118,6 +1122,12 @@ bool takes_128_tile(uint32_t m, uint32_t n, int fmt, uint32_t kblocks, int cus) 
 //   1280      12.1 ->  9.0     15.9 -> 10.9    23.4 -> 15.4    38.9 -> 25.1       192
 //   1536      12.1 ->  9.4     15.9 -> 11.3    23.5 -> 16.2    38.7 -> 26.8       192
 //   2048      12.5 -> 11.0     16.6 -> 13.8    24.3 -> 20.6    39.7 -> 34.4       256
+// On weights stored [K, N], the 256-row kernels with their pass / split-K 64 x 64 in place / ring:
+//   n = 4096:      K = 512             1024                2048                4096                7168
+//   m = 768    16.6 11.5  7.7    21.9 15.1  9.7    33.0 20.9 13.3    54.1 32.8 21.0     90.7  50.5 32.4
+//   1024       16.7 13.2  8.0    22.1 17.4 10.5    33.0 24.6 14.0    53.7 39.5 21.8     90.6  63.6 34.5
+//   1536       17.1 18.3  9.4    23.5 24.0 12.2    34.6 34.0 17.1    54.6 55.8 27.4     89.3  94.6 44.2
+//   2048       17.1 22.9 11.2    23.2 30.4 14.3    34.1 43.2 20.9    54.2 69.6 33.2     88.8 121.7 54.4
 // Past one round the 256-row kernels are the faster ones (2560 x 4096, ring in two rounds: K = 1024 24.8 against 16.6, 4096 57.4 against 43.2).
 int ring_rows(uint32_t m, uint32_t n, int fmt, uint32_t kblocks, int cus) {
     if (fmt == CMX_FMT_E2M1 || kblocks % 4 != 0 || kblocks < 16) return 0;
@@ -1547,17 +1557,18 @@ uint32_t max_group_tiles(uint32_t m_total, uint32_t groups, uint32_t tile_m, uin
 //                SwiGLU 32 x 100 u, K = 1024, N = 2048 21.5 -> 18.5, 4096 36.9 -> 35.8; 2048, 4096 61.2 -> 54.8; 64 x 90 z, 2048, 2048 71.9 -> 66.9; below K = 1536
 //                only up to eight rounds: 64 x 110 u, 1024, 4096 83.6 -> 82.5, but 128 x 70, 1024, 4096 u 138.7 against 141.1, z 165.2 against 171.0; 256 x 50 u, 1024,
 //                2048 136.8 against 140.7; 128 x 90 z, 1152, 4096 199.8 against 206.8 (K = 1536, 128 x 70 u 190.8 and 191.5).  Between two and eight rounds
-//                it is within -3 and +4 % there (K = 1024: 32 x 70 z 42.3 and 42.7, 64 x 60 z, 2048 42.9 and 41.7, 64 x 70 u 66.3 and 69.1), to K = 1023 not measured
+//                it is within -3 and +4 % there (K = 1024: 32 x 70 z 42.3 and 42.7, 64 x 60 z, 2048 42.9 and 41.7, 64 x 70 u 66.3 and 69.1); below K = 1024 not measured
 //   128 x 256    8 x 200 u, 4096, 2048                       45.9 -> 34.5 / 43.1 -> 35.7    16 x 300 u, 7168, 1024   74 -> 57 / 69 -> 62
 //                8 x 500 u, 1024, 1024                       22.6 -> 18.6 / 19.4 -> 12.9; store 8 x 200 u, 512, 2048 15.3 -> 9.6, 16 x 300 u, 512, 1024 16.5 -> 11.3
 // Where n is at most 128, half of a 256-row tile would be empty: 128 x 128 for 256 x 128 (SwiGLU 256 x 68 z, 3072, 64 45 -> 34 where 256 x 128 takes
-// 48; FP4 256 x 128 u, 512, 64 20 -> 16, 23; INT8 256 x 128 u, 128, 128 17.5 -> 14.1, 20.1).
+// 48; FP4 256 x 128 u, 512, 64 20 -> 16, 23).
 // Problems of more tiles stay on the persistent kernels (32 x 194 rows, 7168, 4096: 287 against 311 with 128 x 256).
-// INT8, whose other kernels have 256 x 256 tiles (us, fp32 output; against the streaming kernel, one of them per workgroup):
-//   128 x 128    8 x 44 u, 4096, 2048 46.5 -> 21.6     8 x 200 u 47.7 -> 27.0     16 x 100 z, 7168, 1024 73.2 -> 34.8     16 x 44 u, 2048, 2048 29.7 -> 16.9
-//   256 x 128    32 x 44 u, 7168, 4096 222 -> 178       32 x 100 z 299 -> 232      32 x 100 z, 1152, 2048 46.3 -> 37.3: from K = 512 on, and where the device
+// INT8, whose other kernels have 256 x 256 tiles (us, fp32 output; the faster of the persistent and the streaming one -> ring):
+//   128 x 128    8 x 44 u, 4096, 2048 43.4 -> 17.6     16 x 100 z, 7168, 1024 70.2 -> 30.4
+//   256 x 128    32 x 44 u, 7168, 4096 223 -> 174       32 x 100 z 284 -> 213      32 x 100 z, 1152, 2048 41.7 -> 30.4: from K = 512 on, and where the device
 //                chooses it (mx_gemm_i8_short_kernel)
-//   128 x 256    16 x 200 u, 7168, 1024 71.8 -> 50.9; of more than a round 32 x 200 u, 7168, 4096 278 against 251, 16 x 2048 1077 against 1003
+//   128 x 256    16 x 200 u, 7168, 1024 70.7 -> 42.7    8 x 200 u, 4096, 2048 45.6 -> 28.5    8 x 500 u, 1024, 1024 20.3 -> 15.5    16 x 300 u, 512, 1024 16.5 -> 13.9;
+//                of more than a round 32 x 200 u, 7168, 4096 281 against 247, 16 x 2048 1062 against 889
 // FP4, whose other kernels past the split-K sizes have tiles of 256 x 128 and 256 x 256 (us, bf16 output):
 //   128 x 128    8 x 70 u, 4096, 2048 31.6 -> 15.9     8 x 200 u 36.0 -> 18.4     16 x 100 z, 7168, 1024 46.9 -> 24.1     8 x 70 u, 7168, 4096 49 -> 26
 //   256 x 128    32 x 70 u, 7168, 4096 144 -> 111       32 x 100 z 196 -> 141      32 x 100 z, 1280, 2048 29.9 -> 26.9
@@ -1568,9 +1579,10 @@ int ring_groups(TileChoice* t, uint32_t m_total, uint32_t groups, uint32_t n, in
     int cus = 0;
     if (int rc = cu_count(&cus); rc != CMX_OK) return rc;
     const uint64_t w128 = ceil_div(n, 128);
+    const bool short_k = eight_bit && swiglu && kblocks < 48, many = (uint64_t)ceil_div(n, 256) * (m_total / 128 + groups) > 8 * (uint64_t)cus;
     const uint32_t k_min = eight_bit && swiglu ? 32 : 16;
     if (w128 * (m_total / 128 + groups) <= (uint64_t)cus) *t = {128, 128, kRing};
-    else if (t->tm <= 128 && kblocks >= k_min && (!eight_bit || !swiglu || kblocks >= 48 || (uint64_t)ceil_div(n, 256) * (m_total / 128 + groups) <= 8 * (uint64_t)cus)) *t = {w128 == 1 ? 128 : 256, 128, kRing};
+    else if (t->tm <= 128 && kblocks >= k_min && !(short_k && many)) *t = {w128 == 1 ? 128 : 256, 128, kRing};
     else if (t->tm == 256 && w128 * (m_total / 256 + groups * 3 / 4) <= (uint64_t)cus) *t = {128, 256, kRing};
     return CMX_OK;
 }
@@ -1766,7 +1778,10 @@ extern "C" int cmx_int8_gmm_dequant_swiglu(const int8_t* a, uint32_t lda, const 
     // The persistent kernel of 256 x 256 tiles stores 16 bytes at a time and has the scales' offsets in 32 bits; the streaming kernel takes the rest.
     bool pipe = (!g_force_tile.tw || g_force_tile.waves == 4) && !g_disable_dl && k >= 2 * kSlabBytes && (uint64_t)ld_out * (out_type == CMX_OUT_FP32 ? 4 : 2) % 16 == 0 &&
                 aligned16(out) && (uint64_t)n * channel_scale_stride * 4 < (1ull << 32);
-    bool choice = false;                                       // 128- or 256-row tiles: the device chooses by the sizes
+    // 128- or 256-row tiles: the device chooses by the sizes.  Not for outputs that the persistent kernel cannot store: against the streaming kernel
+    // the ring's tiles alone win wherever the rows lie (rows at 4 bytes, us, ring / choice: 64 x 100, 7168, 3072 u 317 325, z 338 349, on four groups
+    // 157 164; 32 x 90, 2048, 3072 45 51, 62 67, 40 47; 64 x 128, 4096, 3072 232 266, 232 236, 133 147; only 32 x 90, 7168, 3072 on four 95 91).
+    bool choice = false;
     if (g_force_tile.waves == kRing) t = g_force_tile;
     else if (!g_force_tile.tw && !g_disable_dl) {
         if (int rc = ring_groups(&t, m_total, groups, n, kFmtI8, p.kblocks, true); rc != CMX_OK) return rc;
@@ -1778,7 +1793,8 @@ extern "C" int cmx_int8_gmm_dequant_swiglu(const int8_t* a, uint32_t lda, const 
         if (int rc = i8_streams(&pipe, most_tiles, ceil_div(m_total, groups), k / kSlabBytes); rc != CMX_OK) return rc;
     // Kernels of one tile per workgroup find it by the sizes up to some rounds; past those the launch that fills the tables makes the
     // choice.  Where it would fill them for small groups as well, those that are left to the large tiles are large for
-    // their average (256 x 32, 7168, 4096, on eight groups 227 against 277).  The persistent kernel scans the sizes once.
+    // their average (256 x 32, 7168, 4096, on eight groups 227 against 277).  The persistent kernel scans the sizes once,
+    // in any number of rounds (scan / tables, us: 16 x 2048, K = 512, N = 4096, 8 rounds 150 155; 32 x 2048, 1024, 17 rounds 384 386; 32 x 4096, 33 rounds 741 739).
     bool by_sizes = false;
     if (pipe && !all_ksplit && t.waves != kRing && ks.small_rows == 0) {
         by_sizes = groups <= kInlineGroups;

@@ -120,7 +120,8 @@ __device__ __forceinline__ uint32_t xcd_run(uint32_t total_tiles, uint32_t x, ui
 
 // One tile per workgroup (blockIdx.x < total_tiles).  Workgroups start in the order of their ids, ids congruent mod 8 on one
 // XCD.  Whole chunks of 256 tiles: the XCDs take blocks of 32 consecutive tiles of the chunk in turn, for the reason given
-// above (the INT8 operator on the 16-expert problem: 973-982 -> 942-945 us); the rest: a contiguous run per XCD.
+// at interleave_xcd_walk (the INT8 operator on the 16-expert problem, when it ran on the streaming kernel: 973-982 -> 942-945 us); the rest: a
+// contiguous run per XCD.
 __device__ __forceinline__ uint32_t tile_of_workgroup(uint32_t total_tiles, uint32_t bid = blockIdx.x) {
     constexpr uint32_t kChunk = 32 * kXcds;
     const uint32_t full = total_tiles / kChunk * kChunk;

@@ -675,9 +675,9 @@ __global__ __launch_bounds__(256) void mx_gemm_pipe_kernel(const GemmParams p) {
         epilogue<TW, TM, WW, WM, EPI, FW, FM>(p, tc, acc, ww, wm, lane);
     } else {
         // An even number of slabs is walked: whole blocks of four, or, for INT8, any number from two on, filled up with a slab that is not in
-        // memory (KSlabs).  The load stream runs two slabs ahead of the MFMA stream: when it reaches the end of the tile it is aimed at the workgroup's next tile (or keeps
-        // re-requesting the last slab when there is none), so the loads and the fragment reads run on through
-        // the tile boundary and only the epilogue and the clearing of the accumulators interrupt the MFMAs.
+        // memory (KSlabs).  The load stream runs two slabs ahead of the MFMA stream: when it reaches the end of the tile it is aimed at
+        // the workgroup's next tile (or keeps re-requesting the last slab when there is none), so the loads and the fragment reads run on
+        // through the tile boundary and only the epilogue and the clearing of the accumulators interrupt the MFMAs.
         // One loop holds every case so that the register assignment of the scheduled part never changes.
         // Next tile: with a counter array (grouped problems in the 4 x 1 layout, whose tiles differ in cost) the workgroups of an
         // XCD draw from that XCD's run in order; without one the walk is strided.

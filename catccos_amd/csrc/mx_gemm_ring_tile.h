@@ -355,7 +355,8 @@ __device__ __forceinline__ void ring_tile(const GemmParams& p, Tile tc) {
     if constexpr (EPI == kEpiStore) {
         if (stores_pieces(p)) {
             // A thread keeps its eight columns from row to row, so that a piece costs two LDS reads, four conversions and a store: with one
-            // wavefront per SIMD the general loop below is bound by its instructions (1024 x 4096, 2.5 us of it; K = 1024, the call XXX us).
+            // wavefront per SIMD the general loop below is bound by its instructions (1024 x 4096, 2.5 us of it;
+            // at K = 1024, quantizer and matmul 14.5 -> 12.8 us).
             constexpr uint32_t kPieces8 = TW / 8, kTurn = NT / kPieces8;
             static_assert(NT % kPieces8 == 0 && TM % kTurn == 0, "whole rows a turn");
             const uint32_t q = tid % kPieces8, m0 = tid / kPieces8;

@@ -105,16 +105,6 @@ bool to_word(PyObject* o, Py_ssize_t i, uint64_t& v) {
     return false;
 }
 
-template <class F>
-auto call_without_gil(F fn, const uint64_t (&v)[kMaxArgs]) {
-    decltype(fn(0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0)) rc;
-    Py_BEGIN_ALLOW_THREADS
-    rc = fn(v[0], v[1], v[2], v[3], v[4], v[5], v[6], v[7], v[8], v[9], v[10], v[11], v[12], v[13], v[14], v[15], v[16], v[17], v[18], v[19],
-            v[20], v[21], v[22], v[23]);
-    Py_END_ALLOW_THREADS
-    return rc;
-}
-
 PyObject* run(PyObject*, PyObject* const* args, Py_ssize_t n) {
     HANDLE_TH_ERRORS
     if (n < 1 || n > 1 + kMaxArgs) {
@@ -199,7 +189,7 @@ PyObject* empty(PyObject*, PyObject* const* args, Py_ssize_t n) {
 }
 
 PyMethodDef methods[] = {
-    {"run", reinterpret_cast<PyCFunction>(reinterpret_cast<void*>(run)), METH_FASTCALL, "run(address, *args) -> int"},
+    {"run", reinterpret_cast<PyCFunction>(reinterpret_cast<void*>(run)), METH_FASTCALL, "run(address, *args) -> int, or the new tensors"},
     {"empty", reinterpret_cast<PyCFunction>(reinterpret_cast<void*>(empty)), METH_FASTCALL, "empty(like, dtype, *size) -> Tensor"},
     {nullptr, nullptr, 0, nullptr}};
 PyModuleDef module = {PyModuleDef_HEAD_INIT, "_native_call", nullptr, -1, methods};
